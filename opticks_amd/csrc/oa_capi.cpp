@@ -123,6 +123,7 @@ struct mi_sim {
     /* geometry */
     int64_t n_inst = 0, n_prim = 0, n_tlas = 0;
     uint32_t tlas_depth = 0, blas_depth = 0, blas_stack = 0;
+    int32_t stack_depth = OA_STACK_DEPTH;           /* traversal stack entries a walk can reach (build_tlas) */
     uint32_t front_leaf = OA_BVH_EMPTY;             /* items of the front instances (build_tlas) */
     int32_t tlas_empty = 0;                         /* every instance is a front instance */
     std::vector<char> h_is_front;                   /* per instance: kept out of the TLAS */
@@ -440,6 +441,7 @@ static int build_tlas(mi_sim* sim, int leaf)
     nt.release(); ni.release(); nb.release();
     sim->h_is_front = is_front;
     sim->tlas_depth = tb.max_depth;
+    sim->stack_depth = (int32_t)(tb.stack_need + sim->blas_stack + 1);
     sim->n_tlas = (int64_t)tlas.size();
     sim->front_leaf = front_leaf;
     sim->tlas_empty = titems.empty() ? 1 : 0;
@@ -716,6 +718,7 @@ static SimParams base_params(const mi_sim* sim)
     P.node = sim->node.p; P.itra = sim->itra.p; P.plan = sim->plan.p; P.ext_leaves = sim->ext_leaves; P.inst = sim->inst.p; P.prim = sim->prim.p;
     P.tlas = sim->tlas.p; P.tlas_items = sim->tlas_items.p; P.blas = sim->blas.p; P.blas_prims = sim->blas_prims.p;
     P.front_leaf = sim->front_leaf; P.tlas_empty = sim->tlas_empty; P.free_ball = sim->free_ball.p;
+    P.stack_depth = sim->stack_depth;
     P.bnd = sim->bnd.p; P.optical = sim->optical.p; P.icdf = sim->icdf.p;
     P.n_wl = sim->n_wl; P.wl_low = sim->wl_low; P.wl_step = sim->wl_step;
     P.n_icdf = sim->n_icdf; P.n_icdf_layer = sim->n_icdf_layer; P.icdf_hd = sim->icdf_hd;
@@ -769,13 +772,24 @@ static int xorwow_table(mi_sim* sim, const int32_t* event_ids, int32_t n_event, 
     return MI_OK;
 }
 
+/* threads per propagation block: the configured size, halved while its LDS would pass the
+   64 KB a launch may ask for (a deep geometry with 256-thread blocks; results do not
+   depend on it) */
+static int sim_block(const mi_sim* sim)
+{
+    int b = sim->cfg.block_size;
+    while (b > 64 && oa_launch::sim_lds(b, sim->stack_depth) > 65536u) b /= 2;
+    return b;
+}
+
 /* persistent grid: every resident slot of every CU (occupancy API), or the
    configured waves per CU */
 static int wave_grid(const mi_sim* sim)
 {
-    const int waves_per_block = sim->cfg.block_size / 64;
+    const int block = sim_block(sim);
+    const int waves_per_block = block / 64;
     if (sim->cfg.waves_per_cu > 0) return std::max(1, sim->n_cu * sim->cfg.waves_per_cu / waves_per_block);
-    int nb = oa_launch::wave_blocks_per_cu(sim->cfg.block_size, sim->cfg.rng_kind);
+    int nb = oa_launch::wave_blocks_per_cu(block, sim->cfg.rng_kind, sim->stack_depth);
     if (nb <= 0) nb = std::max(1, 8 / waves_per_block);
     return std::max(1, sim->n_cu * nb);
 }
@@ -800,7 +814,7 @@ static int launch(mi_sim* sim, SimParams& P, hipStream_t s)
         HIPCHECK(oa_launch::zero_u64(sim->words.p, n_words, s));
         HIPCHECK(oa_launch::zero_u64(sim->next.p, 1, s));
     }
-    HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim->cfg.block_size, wave_grid(sim), s));
+    HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s));
     return MI_OK;
 }
 
@@ -1028,7 +1042,7 @@ int mi_sim_simulate_device_noalloc(mi_sim* sim, int32_t event_id, const void* d_
     P.hitwords = words;
     P.next = next;
     if (sim->cfg.kernel == MI_KERNEL_WAVEFRONT) HIPCHECK(oa_launch::zero_u64(words, n_words, s));
-    HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim->cfg.block_size, wave_grid(sim), s));
+    HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s));
     HIPCHECK(hipEventRecord(sim->ev[2], s));
     const int64_t nb = (n_words + 255) / 256;
     HIPCHECK(oa_launch::compact_hits(words, n_words, word_prefix, block_total, (const float4*)d_photon,
@@ -1398,7 +1412,7 @@ int mi_sim_adjoint_device(mi_sim* sim, int32_t event_id, const void* d_gensteps,
     HIPCHECK(sim->adj_tmp.reserve(tmp_bytes));
     HIPCHECK(sim->adj_seg.reserve((size_t)n_det + 1));
     /* persistent replay over every resident block slot */
-    const int replay_grid = sim->n_cu * std::max(1, oa_launch::adjoint_blocks_per_cu(sim->cfg.rng_kind));
+    const int replay_grid = sim->n_cu * std::max(1, oa_launch::adjoint_blocks_per_cu(sim->cfg.rng_kind, sim->stack_depth));
     double replay_ms = 0.0, reduce_ms = 0.0;
     oa_launch::AdjBufs ab;
     ab.mat_block = sim->adj_mat_block.p; ab.n_mat = adj->n_mat;
@@ -1557,7 +1571,7 @@ static hipError_t batch_work(mi_batch* b, const SimParams& P, const void* d_gens
         if ((e = oa_launch::zero_u64(b->words.p, b->n_words, s)) != hipSuccess) return e;
         if ((e = oa_launch::zero_u64(b->next.p, 1, s)) != hipSuccess) return e;
     }
-    if ((e = oa_launch::simulate(P, sim->cfg.kernel, sim->cfg.block_size, wave_grid(sim), s)) != hipSuccess) return e;
+    if ((e = oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s)) != hipSuccess) return e;
     if ((e = oa_launch::compact_hits(b->words.p, b->n_words, b->word_prefix.p, b->block_total.p,
                                      (const float4*)d_photon, (float4*)d_hit, d_hit ? b->hit_capacity : 0, s)) != hipSuccess)
         return e;
@@ -1574,7 +1588,7 @@ static hipError_t batch_work(mi_batch* b, const SimParams& P, const void* d_gens
 static hipError_t batch_adjoint_work(mi_batch* b, SimParams P, const void* d_hit, hipStream_t s)
 {
     const mi_sim* sim = b->sim;
-    const int grid = sim->n_cu * std::max(1, oa_launch::adjoint_blocks_per_cu(sim->cfg.rng_kind));
+    const int grid = sim->n_cu * std::max(1, oa_launch::adjoint_blocks_per_cu(sim->cfg.rng_kind, sim->stack_depth));
     hipError_t e;
     oa_launch::AdjBufs ab;
     ab.mat_block = b->mat_block.p; ab.n_mat = b->n_mat;

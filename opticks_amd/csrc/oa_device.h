@@ -169,7 +169,8 @@ struct Photon {
     v3 pos; float time;
     v3 mom; uint32_t hitcount_iindex;
     v3 pol; float wavelength;
-    uint32_t obf, identity, index, flagmask;   /* orient_boundary_flag ... (sysrap/sphoton.h:171-246) */
+    uint32_t obf, identity, flagmask;          /* orient_boundary_flag ... (sysrap/sphoton.h:171-246); the index
+                                                  is parked with the random stream (oa_sim.h) */
 };
 
 OA_D uint32_t ph_flag(const Photon& p) { return p.obf & 0xffffu; }

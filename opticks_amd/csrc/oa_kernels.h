@@ -9,7 +9,8 @@ hipError_t seed_map(const int64_t* d_prefix, int64_t n_gs, int64_t n_photon, uin
                     const int64_t* d_ev_gs_begin, int32_t n_event, int32_t* d_gs_event, hipStream_t s);
 hipError_t gs_prefix(const float* d_gs, int64_t n_gs, int64_t* d_prefix, hipStream_t s);
 hipError_t simulate(const SimParams& P, int kernel, int block, int grid, hipStream_t s);
-int wave_blocks_per_cu(int block, int rng_kind);   /* resident blocks of the persistent kernel per CU */
+int wave_blocks_per_cu(int block, int rng_kind, int stack_depth);   /* resident blocks of the persistent kernel per CU */
+unsigned sim_lds(int block, int stack_depth);      /* LDS bytes of a propagation block */
 hipError_t prefix_check(const int64_t* a, const int64_t* b, int64_t n, unsigned long long* flag, hipStream_t s);
 hipError_t zero_u64(unsigned long long* p, int64_t n, hipStream_t s);
 hipError_t compact_hits(const unsigned long long* d_words, int64_t n_words, int32_t* d_word_prefix,
@@ -50,7 +51,7 @@ hipError_t adjoint_chunk(const SimParams& P, const AdjBufs& a, int64_t begin, in
    parameters than it handles, OA_TAPE_NJ_MAX x 256) */
 #define OA_TAPE_NJ_MAX 4
 int tape_reduce_rows(int32_t n_param);
-int adjoint_blocks_per_cu(int rng_kind);
+int adjoint_blocks_per_cu(int rng_kind, int stack_depth);
 /* no-allocation entry point: the device address of the per-GPU scratch array
    (call with `device` current), and the per-launch event setup kernel */
 hipError_t noalloc_scratch(int device, void** ptr);

@@ -319,16 +319,18 @@ hipError_t gs_prefix(const float* d_gs, int64_t n_gs, int64_t* d_prefix, hipStre
     (P.rng_kind == 1 ? fn##_##B##_1(__VA_ARGS__) : P.rng_kind == 2 ? fn##_##B##_2(__VA_ARGS__) \
                                                  : fn##_##B##_0(__VA_ARGS__))
 
-int wave_blocks_per_cu(int block, int rng_kind)
+int wave_blocks_per_cu(int block, int rng_kind, int stack_depth)
 {
     const int k = rng_kind;
     switch (block) {
-        case 64: return k == 1 ? sim_occupancy_64_1() : k == 2 ? sim_occupancy_64_2() : sim_occupancy_64_0();
-        case 128: return k == 1 ? sim_occupancy_128_1() : k == 2 ? sim_occupancy_128_2() : sim_occupancy_128_0();
-        case 256: return k == 1 ? sim_occupancy_256_1() : k == 2 ? sim_occupancy_256_2() : sim_occupancy_256_0();
+        case 64: return k == 1 ? sim_occupancy_64_1(stack_depth) : k == 2 ? sim_occupancy_64_2(stack_depth) : sim_occupancy_64_0(stack_depth);
+        case 128: return k == 1 ? sim_occupancy_128_1(stack_depth) : k == 2 ? sim_occupancy_128_2(stack_depth) : sim_occupancy_128_0(stack_depth);
+        case 256: return k == 1 ? sim_occupancy_256_1(stack_depth) : k == 2 ? sim_occupancy_256_2(stack_depth) : sim_occupancy_256_0(stack_depth);
         default: return 0;
     }
 }
+
+unsigned sim_lds(int block, int stack_depth) { return oa_sim_lds(block, stack_depth); }
 
 hipError_t simulate(const SimParams& P, int kernel, int block, int grid, hipStream_t s)
 {
@@ -727,9 +729,10 @@ __global__ void __launch_bounds__(256) k_tape_det_reduce(SimParams P, AdjParams 
 
 namespace oa_launch {
 
-int adjoint_blocks_per_cu(int rng_kind)
+int adjoint_blocks_per_cu(int rng_kind, int stack_depth)
 {
-    return rng_kind == 1 ? adjoint_occupancy_128_1() : rng_kind == 2 ? adjoint_occupancy_128_2() : adjoint_occupancy_128_0();
+    return rng_kind == 1 ? adjoint_occupancy_128_1(stack_depth)
+         : rng_kind == 2 ? adjoint_occupancy_128_2(stack_depth) : adjoint_occupancy_128_0(stack_depth);
 }
 
 static int det_key_bits(uint32_t n_det)

@@ -24,7 +24,8 @@
 
 #define OA_BVH_LEAF_BIT 0x80000000u
 #define OA_BVH_EMPTY    0xffffffffu
-#define OA_STACK_DEPTH  48
+#define OA_STACK_DEPTH  48      /* most traversal stack entries a geometry may need */
+#define OA_PARK_WORDS   27      /* LDS words of a photon kept beside the stack while it runs (oa_sim.h) */
 #define OA_BVH_WIDTH    4
 #define OA_CSG_MAX_HEIGHT 7
 #define OA_MAX_FRONT    4       /* instances tested before the TLAS walk (world-sized boxes) */
@@ -102,6 +103,7 @@ struct SimParams {
     const PrimRec* blas_prims;    /* prim records in BLAS leaf order (PrimRec.index: the prim) */
     uint32_t front_leaf;          /* leaf link to the front instances' items (tested first), or empty */
     int32_t tlas_empty;           /* the TLAS holds no instance: every instance is front */
+    int32_t stack_depth;          /* traversal stack entries this geometry needs (at most OA_STACK_DEPTH) */
     const float4* free_ball;      /* (cx, cy, cz, r^2): a ball no TLAS instance box meets (r^2 <= 0: none) */
     /* physics */
     const float4*  bnd;

@@ -68,6 +68,7 @@ enum : int { SEG_SAIL = 0, SEG_ABSORB = 1, SEG_SCATTER = 2 };
    segment call (propagate -> to_boundary), so a photon's step number is its
    segment number: `at` names it before the step, `finish` gets the count. */
 struct NoTape {
+    static constexpr bool keeps_seq = true;
     __device__ inline __attribute__((always_inline)) void at(const SimParams&, int64_t, int) {}
     __device__ inline __attribute__((always_inline)) void seg(const SimParams&, int, float, float, float, float, int) {}
     __device__ inline __attribute__((always_inline)) void finish(const SimParams&, int64_t, int) {}
@@ -82,6 +83,7 @@ struct NoTape {
    and step number the lane keeps anyway, and forms the record address from them
    and the launch fields only at the store. */
 struct RecordTape {
+    static constexpr bool keeps_seq = true;
     int64_t g;
     int32_t step;
     __device__ inline __attribute__((always_inline)) void at(const SimParams&, int64_t g_, int step_)
@@ -402,7 +404,7 @@ enum : uint32_t { T_DISC = 1, T_LINE = 2, T_POINT = 3, T_CIRCLE = 4, T_RECTANGLE
 
 OA_D void zero_flags_set(Photon& p, uint32_t flag)
 {
-    p.obf = 0u; p.identity = 0u; p.index = 0u; p.flagmask = 0u; p.hitcount_iindex = 0u;
+    p.obf = 0u; p.identity = 0u; p.flagmask = 0u; p.hitcount_iindex = 0u;
     set_flag(p, flag);
 }
 

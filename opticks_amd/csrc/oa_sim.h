@@ -40,25 +40,124 @@ template <class R, bool LITE>
 struct Lane {
     Photon p;
     R rng;
-    uint64_t sh0, sh1, sb0, sb1;
     int bounce;
     int64_t g;
     LiteState<LITE> lite;
 };
 
-template <class R, bool LITE>
-OA_D void seq_add(Lane<R, LITE>& L, unsigned slot, uint32_t flag, uint32_t boundary)
+/*
+ * Parked lane state. A trace reads only the photon's position, direction and flag,
+ * and it is what needs the registers (node tests, CSG trees). Everything else a
+ * photon carries is kept in LDS while it runs: stored by park() at the end of a
+ * step, read back by unpark() after the trace. Left to the compiler these values
+ * were spilled to scratch memory, whose slots (152 B a lane, 3.7 MB of the resident
+ * waves of an XCD, nearly its whole L2) missed the vector L1: a lone wave spent half
+ * of a step waiting on memory. Word i of a lane is at base[i * STRIDE], so the lanes
+ * of a wave are in different banks and pairs of words move in one instruction.
+ */
+enum : int { PK_TIME, PK_POLX, PK_POLY, PK_POLZ, PK_WL, PK_IDENT, PK_MASK, PK_HITCOUNT, PK_BOUNCE, PK_G, PK_G_HI,
+             PK_SEQ, PK_RNG = PK_SEQ + 8 };
+static_assert(PK_RNG + 8 == OA_PARK_WORDS, "parked words");
+
+/* park_fixed: what stays as it is from the photon's start to its end, its 32-bit index
+   (sphoton::set_index) at word index_word<R> among it */
+template <class R> struct index_word { static constexpr int value = 7; };
+template <> struct index_word<PhiloxRng> { static constexpr int value = 0; };
+template <> struct index_word<PhiloxRngInline> { static constexpr int value = 0; };
+
+template <int STRIDE> OA_D void park_fixed(uint32_t* w, const oa_philox_stream& s)
 {
-    /* sseq::add_nibble (sysrap/sseq.h:174-183) */
-    const unsigned iseq = slot / 16u;
-    const unsigned shift = 4u * (slot - iseq * 16u);
-    const uint64_t f = (uint64_t)((flag ? (uint32_t)__builtin_ffs((int)flag) : 0u) & 0xfu) << shift;
-    const uint64_t bn = (uint64_t)(boundary & 0xfu) << shift;
-    /* value selects, not a branch per field: a pointer phi would pin Lane to scratch */
-    L.sh0 |= iseq == 0u ? f : 0ull;
-    L.sb0 |= iseq == 0u ? bn : 0ull;
-    L.sh1 |= iseq == 1u ? f : 0ull;
-    L.sb1 |= iseq == 1u ? bn : 0ull;
+    w[0] = (uint32_t)s.photon; w[STRIDE] = (uint32_t)(s.photon >> 32);
+}
+template <int STRIDE> OA_D void park_rng(uint32_t* w, const oa_philox_stream& s)
+{
+    w[2 * STRIDE] = (uint32_t)s.pos; w[3 * STRIDE] = (uint32_t)(s.pos >> 32);
+    w[4 * STRIDE] = s.b0; w[5 * STRIDE] = s.b1; w[6 * STRIDE] = s.b2; w[7 * STRIDE] = s.b3;
+}
+template <int STRIDE> OA_D void unpark_rng(const SimParams& P, const uint32_t* w, oa_philox_stream& s)
+{
+    s.key = P.seed;
+    s.photon = (uint64_t)w[0] | ((uint64_t)w[STRIDE] << 32);
+    s.pos = (uint64_t)w[2 * STRIDE] | ((uint64_t)w[3 * STRIDE] << 32);
+    s.b0 = w[4 * STRIDE]; s.b1 = w[5 * STRIDE]; s.b2 = w[6 * STRIDE]; s.b3 = w[7 * STRIDE];
+}
+template <int STRIDE> OA_D void park_fixed(uint32_t* w, const PhiloxRng& r) { park_fixed<STRIDE>(w, r.ph); }
+template <int STRIDE> OA_D void park_rng(uint32_t* w, const PhiloxRng& r) { park_rng<STRIDE>(w, r.ph); }
+template <int STRIDE> OA_D void unpark_rng(const SimParams& P, const uint32_t* w, PhiloxRng& r) { unpark_rng<STRIDE>(P, w, r.ph); }
+template <int STRIDE> OA_D void park_fixed(uint32_t* w, const PhiloxRngInline& r) { park_fixed<STRIDE>(w, r.ph); }
+template <int STRIDE> OA_D void park_rng(uint32_t* w, const PhiloxRngInline& r) { park_rng<STRIDE>(w, r.ph); }
+template <int STRIDE> OA_D void unpark_rng(const SimParams& P, const uint32_t* w, PhiloxRngInline& r) { unpark_rng<STRIDE>(P, w, r.ph); }
+template <int STRIDE> OA_D void park_fixed(uint32_t*, const XorwowRng&) {}
+template <int STRIDE> OA_D void park_rng(uint32_t* w, const XorwowRng& r)
+{
+    w[0] = r.xw.x0; w[STRIDE] = r.xw.x1; w[2 * STRIDE] = r.xw.x2; w[3 * STRIDE] = r.xw.x3; w[4 * STRIDE] = r.xw.x4;
+    w[5 * STRIDE] = r.xw.d;
+}
+template <int STRIDE> OA_D void unpark_rng(const SimParams&, const uint32_t* w, XorwowRng& r)
+{
+    r.xw.x0 = w[0]; r.xw.x1 = w[STRIDE]; r.xw.x2 = w[2 * STRIDE]; r.xw.x3 = w[3 * STRIDE]; r.xw.x4 = w[4 * STRIDE];
+    r.xw.d = w[5 * STRIDE];
+}
+template <int STRIDE> OA_D void park_fixed(uint32_t* w, const PrecookedRng& r)
+{
+    const uint64_t a = (uint64_t)(uintptr_t)r.row;
+    w[0] = (uint32_t)a; w[STRIDE] = (uint32_t)(a >> 32);
+}
+template <int STRIDE> OA_D void park_rng(uint32_t* w, const PrecookedRng& r) { w[2 * STRIDE] = (uint32_t)r.cursor; }
+template <int STRIDE> OA_D void unpark_rng(const SimParams& P, const uint32_t* w, PrecookedRng& r)
+{
+    r.row = (const float*)(uintptr_t)((uint64_t)w[0] | ((uint64_t)w[STRIDE] << 32));
+    r.cursor = (int32_t)w[2 * STRIDE];
+    r.nk = (int32_t)P.pre_nk;
+}
+
+template <int STRIDE, class R, bool LITE>
+OA_D void park(uint32_t* w, const Lane<R, LITE>& L)
+{
+    w[PK_TIME * STRIDE] = fbits(L.p.time);
+    w[PK_POLX * STRIDE] = fbits(L.p.pol.x);
+    w[PK_POLY * STRIDE] = fbits(L.p.pol.y);
+    w[PK_POLZ * STRIDE] = fbits(L.p.pol.z);
+    w[PK_WL * STRIDE] = fbits(L.p.wavelength);
+    w[PK_IDENT * STRIDE] = L.p.identity;
+    w[PK_MASK * STRIDE] = L.p.flagmask;
+    w[PK_HITCOUNT * STRIDE] = L.p.hitcount_iindex;
+    w[PK_BOUNCE * STRIDE] = (uint32_t)L.bounce;
+    park_rng<STRIDE>(w + PK_RNG * STRIDE, L.rng);
+    /* the values above are not carried over a trace in registers */
+    asm volatile("" ::: "memory");
+}
+
+template <int STRIDE, class R, bool LITE>
+OA_D void unpark(const SimParams& P, const uint32_t* w, Lane<R, LITE>& L)
+{
+    L.p.time = __uint_as_float(w[PK_TIME * STRIDE]);
+    L.p.pol = mk(__uint_as_float(w[PK_POLX * STRIDE]), __uint_as_float(w[PK_POLY * STRIDE]),
+                 __uint_as_float(w[PK_POLZ * STRIDE]));
+    L.p.wavelength = __uint_as_float(w[PK_WL * STRIDE]);
+    L.p.identity = w[PK_IDENT * STRIDE];
+    L.p.flagmask = w[PK_MASK * STRIDE];
+    L.p.hitcount_iindex = w[PK_HITCOUNT * STRIDE];
+    L.bounce = (int)w[PK_BOUNCE * STRIDE];
+    unpark_rng<STRIDE>(P, w + PK_RNG * STRIDE, L.rng);
+}
+
+/* photon index of the launch: written at the start, read where the photon ends */
+template <int STRIDE> OA_D int64_t parked_g(const uint32_t* w)
+{
+    return (int64_t)((uint64_t)w[PK_G * STRIDE] | ((uint64_t)w[PK_G_HI * STRIDE] << 32));
+}
+
+/* sseq::add_nibble (sysrap/sseq.h:174-183) on the parked history: words 0..3 hold
+   seqhis, 4..7 seqbnd, eight slots a word */
+template <int STRIDE>
+OA_D void seq_add(uint32_t* w, unsigned slot, uint32_t flag, uint32_t boundary)
+{
+    if (slot >= 32u) return;
+    uint32_t* s = w + (PK_SEQ + (int)(slot >> 3)) * STRIDE;
+    const unsigned shift = 4u * (slot & 7u);
+    atomicOr(s, ((flag ? (uint32_t)__builtin_ffs((int)flag) : 0u) & 0xfu) << shift);
+    atomicOr(s + 4 * STRIDE, (boundary & 0xfu) << shift);
 }
 
 OA_D int64_t upper_index(const int64_t* a, int64_t lo, int64_t hi, int64_t v)
@@ -101,9 +200,18 @@ OA_D void rng_start(const SimParams& P, PrecookedRng& r, int, uint64_t photon_id
     r.nk = (int32_t)P.pre_nk;
 }
 
-/* generation for global photon g: genstep lookup, RNG stream, generate_photon */
+/* whether the CSGOptiX7.cu:477-509 loop takes another step */
 template <class R, bool LITE>
-OA_D void lane_start(const SimParams& P, Lane<R, LITE>& L, int64_t g)
+OA_D bool lane_alive(const SimParams& P, const Lane<R, LITE>& L)
+{
+    return L.bounce < P.max_bounce && L.p.time < P.max_time;
+}
+
+/* generation for global photon g: genstep lookup, RNG stream, generate_photon; the
+   history starts in the parked words, the rest is parked by the caller. Returns
+   whether the photon takes a step at all. */
+template <int STRIDE, class Tape, class R, bool LITE>
+OA_D bool lane_start(const SimParams& P, Lane<R, LITE>& L, int64_t g, uint32_t* w)
 {
     L.g = g;
     int e = 0;
@@ -124,23 +232,33 @@ OA_D void lane_start(const SimParams& P, Lane<R, LITE>& L, int64_t g)
     if (gencode == 6) gen_torch(L.p, L.rng, gq, photon_idx);
     else if (gencode == 15 || gencode == 18) gen_cerenkov(P, L.p, L.rng, gq);
     else gen_scint(P, L.p, L.rng, gq);
-    /* sphoton::set_index (sysrap/sphoton.h:230-237) */
-    L.p.index = (uint32_t)(photon_idx & 0xffffffffu);
+    /* sphoton::set_index (sysrap/sphoton.h:230-237); the index word is parked below */
     L.p.identity = ((uint32_t)((photon_idx >> 32) & 0xffu) << 24) | (L.p.identity & 0xffffffu);
-    L.sh0 = L.sh1 = L.sb0 = L.sb1 = 0ull;
     L.bounce = 0;
     if constexpr (LITE) { L.lite.lcost = 0.f; L.lite.lx = 0.f; L.lite.ly = __uint_as_float(0x7fc00000u); }
-    seq_add(L, 0u, ph_flag(L.p), ph_boundary(L.p));
+    w[PK_G * STRIDE] = (uint32_t)g;
+    w[PK_G_HI * STRIDE] = (uint32_t)((uint64_t)g >> 32);
+    w[(PK_RNG + index_word<R>::value) * STRIDE] = (uint32_t)photon_idx;
+    park_fixed<STRIDE>(w + PK_RNG * STRIDE, L.rng);
+    if constexpr (Tape::keeps_seq) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[(PK_SEQ + i) * STRIDE] = 0u;
+        seq_add<STRIDE>(w, 0u, ph_flag(L.p), ph_boundary(L.p));
+    }
+    return lane_alive(P, L);
 }
 
-/* one iteration of the CSGOptiX7.cu:477-509 loop; returns true when the photon is done */
+/* one iteration of the CSGOptiX7.cu:477-509 loop from the parked state w, which the
+   caller parks again for the next; returns true when the photon is done */
 template <int STRIDE, class Tape, bool LITE, bool EXT, class R>
-OA_D bool lane_step(const SimParams& P, Lane<R, LITE>& L, uint32_t* stk, Tape& tape)
+OA_D bool lane_step(const SimParams& P, Lane<R, LITE>& L, uint32_t* w, uint32_t* stk, Tape& tape)
 {
-    if (!(L.bounce < P.max_bounce && L.p.time < P.max_time)) return true;
     const float tmin = (L.p.obf & P.eps0_mask) ? P.tmin0 : P.tmin;
     Prd prd;
     trace<STRIDE, EXT>(P, stk, L.p.pos, L.p.mom, tmin, P.tmax, prd);
+    asm volatile("" ::: "memory");
+    unpark<STRIDE>(P, w, L);
+    L.g = parked_g<STRIDE>(w);
     if constexpr (LITE) { L.lite.lcost = prd.lposcost; L.lite.lx = prd.lx; L.lite.ly = prd.ly; }
     if (prd.boundary == 0xffffu) return true;
     prd.normal = normalize(prd.normal);
@@ -149,9 +267,9 @@ OA_D bool lane_step(const SimParams& P, Lane<R, LITE>& L, uint32_t* stk, Tape& t
     tape.at(P, L.g, L.bounce);
     const int command = propagate(P, L.rng, L.p, prd, tape);
     L.bounce++;
-    seq_add(L, (unsigned)L.bounce, ph_flag(L.p), ph_boundary(L.p));
+    if constexpr (Tape::keeps_seq) seq_add<STRIDE>(w, (unsigned)L.bounce, ph_flag(L.p), ph_boundary(L.p));
     if (command == CMD_BREAK) return true;
-    return !(L.bounce < P.max_bounce && L.p.time < P.max_time);
+    return !lane_alive(P, L);
 }
 
 /* sphotonlite::init + set_lpos (sysrap/sphotonlite.h:192-198,234-244) from the
@@ -167,8 +285,8 @@ OA_D uint4 make_lite(const Lane<R, true>& L)
                       ((uint32_t)qc << 16) | (uint32_t)qf, L.p.flagmask);
 }
 
-template <class R, bool LITE>
-OA_D void lane_finish(const SimParams& P, const Lane<R, LITE>& L)
+template <int STRIDE, class R, bool LITE>
+OA_D void lane_finish(const SimParams& P, const Lane<R, LITE>& L, const uint32_t* w)
 {
     const int64_t g = L.g;
     if constexpr (LITE) {
@@ -180,12 +298,16 @@ OA_D void lane_finish(const SimParams& P, const Lane<R, LITE>& L)
         o[1] = make_float4(L.p.mom.x, L.p.mom.y, L.p.mom.z, __uint_as_float(L.p.hitcount_iindex));
         o[2] = make_float4(L.p.pol.x, L.p.pol.y, L.p.pol.z, L.p.wavelength);
         o[3] = make_float4(__uint_as_float(L.p.obf), __uint_as_float(L.p.identity),
-                           __uint_as_float(L.p.index), __uint_as_float(L.p.flagmask));
+                           __uint_as_float(w[(PK_RNG + index_word<R>::value) * STRIDE]), __uint_as_float(L.p.flagmask));
     }
     if (P.seq) {
         ulonglong2* s = reinterpret_cast<ulonglong2*>(P.seq + 4 * g);
-        s[0] = make_ulonglong2(L.sh0, L.sh1);
-        s[1] = make_ulonglong2(L.sb0, L.sb1);
+        uint64_t q[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            q[i] = (uint64_t)w[(PK_SEQ + 2 * i) * STRIDE] | ((uint64_t)w[(PK_SEQ + 2 * i + 1) * STRIDE] << 32);
+        s[0] = make_ulonglong2(q[0], q[1]);
+        s[1] = make_ulonglong2(q[2], q[3]);
     }
 }
 
@@ -197,16 +319,20 @@ template <int BLOCK, int F, class R>
 __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_plain(SimParams P)
 {
     using namespace oa;
-    __shared__ uint32_t s_stack[OA_STACK_DEPTH * BLOCK];
-    uint32_t* stk = s_stack + threadIdx.x;
+    extern __shared__ uint32_t s_lane[];           /* OA_PARK_WORDS parked words, then the stack, of each lane */
+    uint32_t* park_w = s_lane + threadIdx.x;
+    uint32_t* stk = park_w + OA_PARK_WORDS * BLOCK;
     const int64_t g = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     bool hit = false;
     if (g < P.n_photon) {
         Lane<R, (F & 1) != 0> L;
         NoTape tape;
-        lane_start(P, L, g);
-        while (!lane_step<BLOCK, NoTape, (F & 1) != 0, (F & 2) != 0>(P, L, stk, tape)) {}
-        lane_finish(P, L);
+        bool more = lane_start<BLOCK, NoTape>(P, L, g, park_w);
+        while (more) {
+            park<BLOCK>(park_w, L);
+            more = !lane_step<BLOCK, NoTape, (F & 1) != 0, (F & 2) != 0>(P, L, park_w, stk, tape);
+        }
+        lane_finish<BLOCK>(P, L, park_w);
         hit = (L.p.flagmask & P.hit_mask) != 0u;
     }
     const unsigned long long m = __ballot(hit);
@@ -219,8 +345,9 @@ template <int BLOCK, int F, class R, class T = oa::NoTape>
 __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_wave(SimParams P)
 {
     using namespace oa;
-    __shared__ uint32_t s_stack[OA_STACK_DEPTH * BLOCK];
-    uint32_t* stk = s_stack + threadIdx.x;
+    extern __shared__ uint32_t s_lane[];           /* OA_PARK_WORDS parked words, then the stack, of each lane */
+    uint32_t* park_w = s_lane + threadIdx.x;
+    uint32_t* stk = park_w + OA_PARK_WORDS * BLOCK;
     const int lane = threadIdx.x & 63;
     Lane<R, (F & 1) != 0> L;
     T tape;
@@ -231,6 +358,11 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_wave(SimParams P)
        same iteration from one genstep stay in step (the same boundary at the same
        bounce), so the CSG tests of a detector shell run with more lanes at once */
     const int batch = P.refill_batch > 1 ? P.refill_batch : 1;
+    const auto finish = [&](const Lane<R, (F & 1) != 0>& L) {
+        lane_finish<BLOCK>(P, L, park_w);
+        tape.finish(P, L.g, L.bounce);
+        if ((L.p.flagmask & P.hit_mask) != 0u) atomicOr(P.hitwords + (L.g >> 6), 1ull << (L.g & 63));
+    };
     for (int iter = 0;; ++iter) {
         OA_CYC_MARK(c_iter);
         const unsigned long long idle = __ballot(!active);
@@ -245,25 +377,28 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_wave(SimParams P)
                 const unsigned long long below = idle & ((1ull << lane) - 1ull);
                 const int64_t g = (int64_t)(base + (unsigned long long)__popcll(below));
                 if (g < P.n_photon) {
-                    lane_start(P, L, g);
-                    active = true;
+                    active = lane_start<BLOCK, T>(P, L, g, park_w);
+                    if (active) park<BLOCK>(park_w, L);
+                    else finish(L);
                 }
             }
             if ((int64_t)(base + (unsigned long long)n_idle) >= P.n_photon) exhausted = true;
         }
         const unsigned long long act = __ballot(active);
-        if (act == 0ull) break;
+        if (act == 0ull) {
+            if (exhausted) break;
+            continue;
+        }
 #ifdef OA_STATS
         if (lane == 0) { OA_COUNT(OA_ST_ITER); OA_COUNT_N(OA_ST_ACTIVE, __popcll(act)); }
 #endif
         OA_CYC_ADD(OA_ST_C_REFILL, c_iter);
         if (active) {
-            if (lane_step<BLOCK, T, (F & 1) != 0, (F & 2) != 0>(P, L, stk, tape)) {
-                lane_finish(P, L);
-                tape.finish(P, L.g, L.bounce);
-                if ((L.p.flagmask & P.hit_mask) != 0u)
-                    atomicOr(P.hitwords + (L.g >> 6), 1ull << (L.g & 63));
+            if (lane_step<BLOCK, T, (F & 1) != 0, (F & 2) != 0>(P, L, park_w, stk, tape)) {
+                finish(L);
                 active = false;
+            } else {
+                park<BLOCK>(park_w, L);
             }
         }
         OA_CYC_ADD(OA_ST_C_ITER, c_iter);
@@ -303,6 +438,7 @@ struct ScoreTerm {
 };
 
 struct ScoreTape {
+    static constexpr bool keeps_seq = false;
     const int32_t* optical;
     int32_t n_wl;
     float wl_low, wl_step;
@@ -400,8 +536,9 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_adjoint_wave(SimParams P, AdjP
                                                                int32_t n_ev, int64_t hit_cap, float* S)
 {
     using namespace oa;
-    __shared__ uint32_t s_stack[OA_STACK_DEPTH * BLOCK];
-    uint32_t* stk = s_stack + threadIdx.x;
+    extern __shared__ uint32_t s_lane[];           /* OA_PARK_WORDS parked words, then the stack, of each lane */
+    uint32_t* park_w = s_lane + threadIdx.x;
+    uint32_t* stk = park_w + OA_PARK_WORDS * BLOCK;
     const int lane = threadIdx.x & 63;
     /* with the segment tape, only photons it could not hold are replayed: none, when
        the ordering pass (k_hit_det) raised no flag */
@@ -431,12 +568,12 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_adjoint_wave(SimParams P, AdjP
                     const int64_t g = hit_photon(P, hits, begin + i, hit_off, n_ev);
                     /* a hit whose segments are all on the tape was scored from it */
                     if (g >= 0 && !(P.tape_n && (int32_t)P.tape_n[g] <= P.tape_k)) {
-                        lane_start(P, L, g);
+                        active = lane_start<BLOCK, ScoreTape>(P, L, g, park_w);
+                        park<BLOCK>(park_w, L);
                         tape.row = S + i * (int64_t)A.n_param;
                         /* with the tape the rows are not cleared beforehand: only these hits use them */
                         if (P.tape)
                             for (int32_t k = 0; k < A.n_param; ++k) tape.row[k] = 0.f;
-                        active = true;
                     }
                 }
             }
@@ -447,7 +584,10 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_adjoint_wave(SimParams P, AdjP
             if (exhausted) break;
             continue;
         }
-        if (active && lane_step<BLOCK, ScoreTape, false, EXT>(P, L, stk, tape)) active = false;
+        if (active) {
+            active = !lane_step<BLOCK, ScoreTape, false, EXT>(P, L, park_w, stk, tape);
+            park<BLOCK>(park_w, L);
+        }
     }
 }
 

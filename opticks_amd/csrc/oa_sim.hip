@@ -28,35 +28,36 @@ namespace oa_launch {
 hipError_t OA_SIM_NAME(sim_launch, OA_SIM_BLOCK, OA_SIM_RNG)(const SimParams& P, int kernel, int grid, hipStream_t s)
 {
     constexpr int B = OA_SIM_BLOCK;
+    const unsigned lds = oa_sim_lds(B, P.stack_depth);
     const int f = (P.photonlite ? 1 : 0) | (P.ext_leaves ? 2 : 0);
     if (kernel == 0) {
         const unsigned nb = (unsigned)((P.n_photon + B - 1) / B);
         switch (f) {
-            case 0: hipLaunchKernelGGL((k_sim_plain<B, 0, OA_SIM_R>), dim3(nb), dim3(B), 0, s, P); break;
-            case 1: hipLaunchKernelGGL((k_sim_plain<B, 1, OA_SIM_R>), dim3(nb), dim3(B), 0, s, P); break;
-            case 2: hipLaunchKernelGGL((k_sim_plain<B, 2, OA_SIM_R>), dim3(nb), dim3(B), 0, s, P); break;
-            default: hipLaunchKernelGGL((k_sim_plain<B, 3, OA_SIM_R>), dim3(nb), dim3(B), 0, s, P); break;
+            case 0: hipLaunchKernelGGL((k_sim_plain<B, 0, OA_SIM_R>), dim3(nb), dim3(B), lds, s, P); break;
+            case 1: hipLaunchKernelGGL((k_sim_plain<B, 1, OA_SIM_R>), dim3(nb), dim3(B), lds, s, P); break;
+            case 2: hipLaunchKernelGGL((k_sim_plain<B, 2, OA_SIM_R>), dim3(nb), dim3(B), lds, s, P); break;
+            default: hipLaunchKernelGGL((k_sim_plain<B, 3, OA_SIM_R>), dim3(nb), dim3(B), lds, s, P); break;
         }
     } else if (P.tape) {
         /* a forward for a following adjoint: segment records on the tape (no lite output) */
-        if (f & 2) hipLaunchKernelGGL((k_sim_wave<B, 2, OA_SIM_RT, oa::RecordTape>), dim3((unsigned)grid), dim3(B), 0, s, P);
-        else hipLaunchKernelGGL((k_sim_wave<B, 0, OA_SIM_RT, oa::RecordTape>), dim3((unsigned)grid), dim3(B), 0, s, P);
+        if (f & 2) hipLaunchKernelGGL((k_sim_wave<B, 2, OA_SIM_RT, oa::RecordTape>), dim3((unsigned)grid), dim3(B), lds, s, P);
+        else hipLaunchKernelGGL((k_sim_wave<B, 0, OA_SIM_RT, oa::RecordTape>), dim3((unsigned)grid), dim3(B), lds, s, P);
     } else {
         switch (f) {
-            case 0: hipLaunchKernelGGL((k_sim_wave<B, 0, OA_SIM_R>), dim3((unsigned)grid), dim3(B), 0, s, P); break;
-            case 1: hipLaunchKernelGGL((k_sim_wave<B, 1, OA_SIM_R>), dim3((unsigned)grid), dim3(B), 0, s, P); break;
-            case 2: hipLaunchKernelGGL((k_sim_wave<B, 2, OA_SIM_R>), dim3((unsigned)grid), dim3(B), 0, s, P); break;
-            default: hipLaunchKernelGGL((k_sim_wave<B, 3, OA_SIM_R>), dim3((unsigned)grid), dim3(B), 0, s, P); break;
+            case 0: hipLaunchKernelGGL((k_sim_wave<B, 0, OA_SIM_R>), dim3((unsigned)grid), dim3(B), lds, s, P); break;
+            case 1: hipLaunchKernelGGL((k_sim_wave<B, 1, OA_SIM_R>), dim3((unsigned)grid), dim3(B), lds, s, P); break;
+            case 2: hipLaunchKernelGGL((k_sim_wave<B, 2, OA_SIM_R>), dim3((unsigned)grid), dim3(B), lds, s, P); break;
+            default: hipLaunchKernelGGL((k_sim_wave<B, 3, OA_SIM_R>), dim3((unsigned)grid), dim3(B), lds, s, P); break;
         }
     }
     return hipGetLastError();
 }
 
-int OA_SIM_NAME(sim_occupancy, OA_SIM_BLOCK, OA_SIM_RNG)()
+int OA_SIM_NAME(sim_occupancy, OA_SIM_BLOCK, OA_SIM_RNG)(int stack_depth)
 {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sim_wave<OA_SIM_BLOCK, 0, OA_SIM_R>, OA_SIM_BLOCK, 0) !=
-        hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sim_wave<OA_SIM_BLOCK, 0, OA_SIM_R>, OA_SIM_BLOCK,
+                                                     oa_sim_lds(OA_SIM_BLOCK, stack_depth)) != hipSuccess)
         return 0;
     return nb;
 }
@@ -67,20 +68,21 @@ hipError_t OA_SIM_NAME(adjoint_launch, OA_ADJ_BLOCK, OA_SIM_RNG)(const SimParams
                                                                  const int64_t* hit_off, int32_t n_ev, int64_t hit_cap,
                                                                  float* S, int grid, hipStream_t s)
 {
+    const unsigned lds = oa_sim_lds(OA_ADJ_BLOCK, P.stack_depth);
     if (P.ext_leaves)
-        hipLaunchKernelGGL((k_adjoint_wave<OA_ADJ_BLOCK, true, OA_SIM_R>), dim3((unsigned)grid), dim3(OA_ADJ_BLOCK), 0,
+        hipLaunchKernelGGL((k_adjoint_wave<OA_ADJ_BLOCK, true, OA_SIM_R>), dim3((unsigned)grid), dim3(OA_ADJ_BLOCK), lds,
                            s, P, A, hits, begin, n_max, hit_off, n_ev, hit_cap, S);
     else
-        hipLaunchKernelGGL((k_adjoint_wave<OA_ADJ_BLOCK, false, OA_SIM_R>), dim3((unsigned)grid), dim3(OA_ADJ_BLOCK), 0,
+        hipLaunchKernelGGL((k_adjoint_wave<OA_ADJ_BLOCK, false, OA_SIM_R>), dim3((unsigned)grid), dim3(OA_ADJ_BLOCK), lds,
                            s, P, A, hits, begin, n_max, hit_off, n_ev, hit_cap, S);
     return hipGetLastError();
 }
 
-int OA_SIM_NAME(adjoint_occupancy, OA_ADJ_BLOCK, OA_SIM_RNG)()
+int OA_SIM_NAME(adjoint_occupancy, OA_ADJ_BLOCK, OA_SIM_RNG)(int stack_depth)
 {
     int nb = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_adjoint_wave<OA_ADJ_BLOCK, false, OA_SIM_R>, OA_ADJ_BLOCK,
-                                                     0) != hipSuccess)
+                                                     oa_sim_lds(OA_ADJ_BLOCK, stack_depth)) != hipSuccess)
         return 0;
     return nb;
 }

@@ -11,7 +11,13 @@ struct AdjParams;
 
 #define OA_SIM_DECLARE(B, K)                                                                   \
     hipError_t sim_launch_##B##_##K(const SimParams& P, int kernel, int grid, hipStream_t s); \
-    int sim_occupancy_##B##_##K();
+    int sim_occupancy_##B##_##K(int stack_depth);
+
+/* LDS bytes of a propagation block: each thread's parked photon words and traversal stack */
+inline unsigned oa_sim_lds(int block, int stack_depth)
+{
+    return (unsigned)(OA_PARK_WORDS + stack_depth) * 4u * (unsigned)block;
+}
 
 namespace oa_launch {
 OA_SIM_DECLARE(64, 0)
@@ -28,7 +34,7 @@ OA_SIM_DECLARE(256, 2)
     hipError_t adjoint_launch_128_##K(const SimParams& P, const AdjParams& A, const float4* hits, int64_t begin, \
                                       int64_t n_max, const int64_t* hit_off, int32_t n_ev, int64_t hit_cap,    \
                                       float* S, int grid, hipStream_t s);                                      \
-    int adjoint_occupancy_128_##K();
+    int adjoint_occupancy_128_##K(int stack_depth);
 OA_ADJ_DECLARE(0)
 OA_ADJ_DECLARE(1)
 OA_ADJ_DECLARE(2)

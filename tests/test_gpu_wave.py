@@ -1,0 +1,57 @@
+"""The propagation kernels' launch shapes against the CPU checker (MI355X only): geometries
+whose traversal stack is far deeper than a detector's, which changes the LDS of a block."""
+import numpy as np
+import pytest
+
+import pyoracle as po
+from opticks_amd import configs
+from opticks_amd import _lib as L
+from opticks_amd.foundry import Foundry, Node
+from opticks_amd.physics import BoundaryLib, Material, Surface, gaussian_icdf
+from opticks_amd.qsim import QSim, SEventConfig
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+if not torch.cuda.is_available():
+    pytest.skip("no GPU", allow_module_level=True)
+
+
+def onions(shells, num_photon=20_000, seed=42):
+    """Two instances of a solid of concentric spheres, radii growing by 11%, in a water box:
+    each SAH split of such a solid takes the largest sphere off, so its BLAS is a chain and
+    the traversal stack holds about one entry a shell."""
+    lib = BoundaryLib()
+    lib.add_material(Material("Water", 1.33, 20000.0, 30000.0))
+    lib.add_material(Material("Acrylic", 1.36, 1e6, 1e6))
+    lib.add_surface(Surface("wallSurf", detect=0.5, absorb=0.5))
+    b_world = lib.boundary("Water/wallSurf/wallSurf/Water")
+    b_obj = lib.boundary("Water///Acrylic")
+    fd = Foundry()
+    s0 = fd.addSolid("world", [fd.addPrim(Node.box3(6000.0, 6000.0, 6000.0), b_world)])
+    s1 = fd.addSolid("onion", [fd.addPrim(Node.sphere(10.0 * 1.11 ** k), b_obj) for k in range(shells)])
+    fd.addInstance(np.eye(4), s0)
+    for x in (-1100.0, 1100.0):
+        t = np.eye(4)
+        t[3, 0] = x
+        fd.addInstance(t, s1)
+    phys = lib.arrays()
+    phys["icdf"], phys["icdf_hd_factor"] = gaussian_icdf()
+    gs = np.stack([configs.torch_genstep(num_photon // 2, configs.T_POINT_ISO, pos=p, wavelength=300.0, weight=300.0)
+                   for p in ((0.0, 0.0, 0.0), (-1100.0, 3.0, 2.0))]).astype(np.float32)
+    return configs.Workload("onions", fd.arrays(), phys, gs, seed=seed)
+
+
+# 3 shells: a shallow stack; 40: 27 + 41 words a lane, past 64 KB for a 256-thread block
+@pytest.mark.parametrize("shells", [3, 40])
+@pytest.mark.parametrize("block", [64, 128, 256])
+@pytest.mark.parametrize("kernel", [L.MI_KERNEL_PLAIN, L.MI_KERNEL_WAVEFRONT])
+def test_stack_depths_match_checker(shells, block, kernel):
+    w = onions(shells)
+    sim = QSim(w.geometry, w.physics, SEventConfig(seed=w.seed, block_size=block, kernel=kernel))
+    hits = sim.simulate(w.gensteps, 0)
+    photon, seq = po.World(w.geometry, w.physics).simulate(w.gensteps, seed=w.seed)
+    assert np.array_equal(sim.seq, seq)
+    assert np.array_equal(sim.photon.view(np.uint32), photon.view(np.uint32))
+    assert len(hits) == np.count_nonzero(photon[:, 3, 3].view(np.uint32) & 0x40)
+    sim.close()
