@@ -778,7 +778,7 @@ static int xorwow_table(mi_sim* sim, const int32_t* event_ids, int32_t n_event, 
 static int sim_block(const mi_sim* sim)
 {
     int b = sim->cfg.block_size;
-    while (b > 64 && oa_launch::sim_lds(b, sim->stack_depth) > 65536u) b /= 2;
+    while (b > 64 && oa_launch::sim_lds(b, sim->cfg.rng_kind, sim->stack_depth) > 65536u) b /= 2;
     return b;
 }
 

@@ -104,14 +104,15 @@ enum : uint32_t { TC_ZERO = 0, TC_UNION = 1, TC_INTERSECTION = 2, TC_DIFFERENCE 
    each kernel instantiation carries only the state of its own kind. */
 enum : int { RNG_PHILOX = 0, RNG_PRECOOKED = 1, RNG_XORWOW = 2 };
 
-struct PhiloxRng { oa_philox_stream ph; };
-/* the same stream with its block generated inline at each draw site (the taped
-   forward's instantiation, whose register allocation measured better with it) */
-struct PhiloxRngInline { oa_philox_stream ph; };
-/* whether the physics of a kernel drawing from R calls the table-index wrap's integer
-   divisions out of line (a smaller kernel), or inline (the taped forward) */
-template <class R> struct wrap_ool { static constexpr bool value = true; };
-template <> struct wrap_ool<PhiloxRngInline> { static constexpr bool value = false; };
+/*
+ * Philox is counter-based, so its state is the word position alone: a draw of N words
+ * generates the block they start in, and the next one where they run over its end. The
+ * words are those of oa_rng_uniform called N times. The draws of a step are taken in
+ * groups: with a buffered block and one word at a time, every draw site of the physics
+ * ran the ten rounds for the lanes that had used their block up, a different quarter of
+ * the wave each time.
+ */
+struct PhiloxRng { uint64_t key, photon, pos; };
 struct XorwowRng { oa_xorwow_state xw; };
 /* precooked uniforms (the reference's s_seq aligned-randoms mode): a row of nk
    values per photon; the cursor wraps modulo nk as s_seq::flat recycles
@@ -121,31 +122,49 @@ struct PrecookedRng {
     int32_t cursor, nk;
 };
 
-/* the Philox block out of line: one copy of its ten rounds instead of one per draw site */
-__device__ static __attribute__((noinline)) uint4 philox_block(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
-                                                                uint32_t k0, uint32_t k1)
+#define OA_DRAW_MAX 5       /* words of one draw: the block they start in and the next hold them */
+
+struct PhiloxWords { uint32_t v[OA_DRAW_MAX]; };
+
+/* the n <= OA_DRAW_MAX words from word position pos (the rest of v: unspecified) */
+OA_D PhiloxWords philox_words(uint64_t key, uint64_t photon, uint64_t pos, uint32_t n)
 {
-    oa_u32x4 c;
-    c.v[0] = c0; c.v[1] = c1; c.v[2] = c2; c.v[3] = c3;
-    const oa_u32x4 o = oa_philox4x32_10(c, k0, k1);
-    return make_uint4(o.v[0], o.v[1], o.v[2], o.v[3]);
-}
-/* oa_rng_uniform with the block generated out of line (the same words) */
-OA_D float uni(PhiloxRng& r)
-{
-    oa_philox_stream* s = &r.ph;
-    const uint32_t x = s->b0;
-    s->b0 = s->b1; s->b1 = s->b2; s->b2 = s->b3;
-    s->pos += 1u;
-    if ((s->pos & 3u) == 0u) {
-        const uint64_t block = s->pos >> 2;
-        const uint4 o = philox_block((uint32_t)block, (uint32_t)(block >> 32), (uint32_t)s->photon,
-                                     (uint32_t)(s->photon >> 32), (uint32_t)s->key, (uint32_t)(s->key >> 32));
-        s->b0 = o.x; s->b1 = o.y; s->b2 = o.z; s->b3 = o.w;
+    const uint32_t o = (uint32_t)pos & 3u;
+    oa_u32x4 c, a, b;
+    c.v[0] = (uint32_t)(pos >> 2); c.v[1] = (uint32_t)(pos >> 34);
+    c.v[2] = (uint32_t)photon; c.v[3] = (uint32_t)(photon >> 32);
+    a = oa_philox4x32_10(c, (uint32_t)key, (uint32_t)(key >> 32));
+    b.v[0] = b.v[1] = b.v[2] = b.v[3] = 0u;
+    if (o + n > 4u) {
+        const uint64_t next = (pos + 4u) >> 2;
+        c.v[0] = (uint32_t)next; c.v[1] = (uint32_t)(next >> 32);
+        b = oa_philox4x32_10(c, (uint32_t)key, (uint32_t)(key >> 32));
     }
-    return oa_u32_to_uniform(x);
+    /* scalars, not arrays: selects of array elements became indexed scratch accesses */
+    const bool s2 = (o & 2u) != 0u, s1 = (o & 1u) != 0u;
+    const uint32_t a0 = a.v[0], a1 = a.v[1], a2 = a.v[2], a3 = a.v[3], b0 = b.v[0], b1 = b.v[1], b2 = b.v[2], b3 = b.v[3];
+    const uint32_t x0 = s2 ? a2 : a0, x1 = s2 ? a3 : a1, x2 = s2 ? b0 : a2, x3 = s2 ? b1 : a3, x4 = s2 ? b2 : b0,
+                   x5 = s2 ? b3 : b1;
+    PhiloxWords r;
+    r.v[0] = s1 ? x1 : x0; r.v[1] = s1 ? x2 : x1; r.v[2] = s1 ? x3 : x2; r.v[3] = s1 ? x4 : x3; r.v[4] = s1 ? x5 : x4;
+    return r;
 }
-OA_D float uni(PhiloxRngInline& r) { return oa_rng_uniform(&r.ph); }
+/* one copy of the rounds for all draw sites but a step's first (code size) */
+__device__ static __attribute__((noinline)) PhiloxWords philox_words_call(uint64_t key, uint64_t photon, uint64_t pos,
+                                                                          uint32_t n)
+{
+    return philox_words(key, photon, pos, n);
+}
+
+/* the next N uniforms */
+template <int N> OA_D void draw(PhiloxRng& r, float (&u)[N])
+{
+    static_assert(N <= OA_DRAW_MAX, "draw");
+    const PhiloxWords w = philox_words_call(r.key, r.photon, r.pos, N);
+    r.pos += N;
+#pragma unroll
+    for (int i = 0; i < N; ++i) u[i] = oa_u32_to_uniform(w.v[i]);
+}
 OA_D float uni(XorwowRng& r) { return oa_xorwow_uniform(&r.xw); }
 OA_D float uni(PrecookedRng& r)
 {
@@ -153,6 +172,41 @@ OA_D float uni(PrecookedRng& r)
     r.cursor = r.cursor + 1 == r.nk ? 0 : r.cursor + 1;
     return v;
 }
+template <int N, class R> OA_D void draw(R& r, float (&u)[N])
+{
+#pragma unroll
+    for (int i = 0; i < N; ++i) u[i] = uni(r);
+}
+template <class R> OA_D float draw1(R& r)
+{
+    float u[1];
+    draw<1>(r, u);
+    return u[0];
+}
+
+/* the two uniforms every step draws, and a third that most steps draw: taken by
+   maybe_third() where it is needed. Sequential generators draw it there. */
+struct MaybeThird { float u; };
+OA_D MaybeThird draw2_maybe3(PhiloxRng& r, float& u0, float& u1)
+{
+    const PhiloxWords w = philox_words(r.key, r.photon, r.pos, 3u);
+    r.pos += 2u;
+    u0 = oa_u32_to_uniform(w.v[0]);
+    u1 = oa_u32_to_uniform(w.v[1]);
+    MaybeThird m;
+    m.u = oa_u32_to_uniform(w.v[2]);
+    return m;
+}
+template <class R> OA_D MaybeThird draw2_maybe3(R& r, float& u0, float& u1)
+{
+    u0 = uni(r);
+    u1 = uni(r);
+    MaybeThird m;
+    m.u = 0.f;
+    return m;
+}
+OA_D float maybe_third(PhiloxRng& r, MaybeThird m) { r.pos += 1u; return m.u; }
+template <class R> OA_D float maybe_third(R& r, MaybeThird) { return uni(r); }
 
 /* Rejection loops of the reference (marsaglia, Rayleigh, torch sphere,
    Cerenkov position) are unbounded; here each stops after OA_MAX_TRIALS

@@ -83,12 +83,16 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_simtrace(SimParams P, float4* 
     const int64_t gsi = upper_index(P.gs_prefix, 0, P.n_gs, idx);
     const float4* gq = reinterpret_cast<const float4*>(P.gensteps + 24 * gsi);
     PhiloxRng rng;
-    oa_rng_init(&rng.ph, P.seed, P.rng_offset, P.skipahead, 0ull, (uint64_t)idx);
+    rng.key = P.seed;
+    rng.photon = (uint64_t)idx;
+    rng.pos = P.rng_offset;
+    float u[2];
+    draw<2>(rng, u);
     const uint32_t gridaxes = __float_as_uint(gq[0].y);
-    const float u0 = uni(rng);
+    const float u0 = u[0];
     float sinPhi, cosPhi;
     oa_sincosf(2.f * OA_PI_F * u0, &sinPhi, &cosPhi);
-    const float u1 = uni(rng);
+    const float u1 = u[1];
     const float cosTheta = 2.f * u1 - 1.f;
     const float sinTheta = sqrtf(1.f - cosTheta * cosTheta);
     v3 dir = gridaxes == 1u ? mk(0.f, cosPhi, sinPhi)
@@ -330,7 +334,12 @@ int wave_blocks_per_cu(int block, int rng_kind, int stack_depth)
     }
 }
 
-unsigned sim_lds(int block, int stack_depth) { return oa_sim_lds(block, stack_depth); }
+unsigned sim_lds(int block, int rng_kind, int stack_depth)
+{
+    const unsigned b64 = rng_kind == 1 ? sim_lds_64_1(stack_depth) : rng_kind == 2 ? sim_lds_64_2(stack_depth)
+                                                                                   : sim_lds_64_0(stack_depth);
+    return b64 * (unsigned)(block / 64);
+}
 
 hipError_t simulate(const SimParams& P, int kernel, int block, int grid, hipStream_t s)
 {

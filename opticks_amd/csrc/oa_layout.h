@@ -25,7 +25,6 @@
 #define OA_BVH_LEAF_BIT 0x80000000u
 #define OA_BVH_EMPTY    0xffffffffu
 #define OA_STACK_DEPTH  48      /* most traversal stack entries a geometry may need */
-#define OA_PARK_WORDS   27      /* LDS words of a photon kept beside the stack while it runs (oa_sim.h) */
 #define OA_BVH_WIDTH    4
 #define OA_CSG_MAX_HEIGHT 7
 #define OA_MAX_FRONT    4       /* instances tested before the TLAS walk (world-sized boxes) */

@@ -24,19 +24,15 @@ namespace oa {
    outside the table (wavelengths beyond the domain), the results are the same. */
 __device__ static __attribute__((noinline)) int wrap_index(int i, int n) { return ((i % n) + n) % n; }
 
-/* OOL: the integer divisions out of line (a smaller kernel; the taped forward's register
-   allocation does better with them inline: wrap_ool) */
-template <bool OOL = true>
 OA_D void wrap_pair(int i, int n, int& i0, int& i1)
 {
     i0 = i;
-    if (i0 < 0 || i0 >= n) i0 = OOL ? wrap_index(i0, n) : ((i0 % n) + n) % n;
+    if (i0 < 0 || i0 >= n) i0 = wrap_index(i0, n);
     i1 = i0 + 1 == n ? 0 : i0 + 1;
 }
 
 /* One lerped float4 of bnd row (2*line+k) at wavelength nm: the FP32 form of
    the linearly filtered, wrap-addressed texture fetch of qbnd::boundary_lookup. */
-template <bool OOL = true>
 OA_D float4 bnd_lookup(const SimParams& P, float nm, int line, int k)
 {
     const int nwl = P.n_wl;
@@ -44,7 +40,7 @@ OA_D float4 bnd_lookup(const SimParams& P, float nm, int line, int k)
     float fl = floorf(fx);
     float a = fx - fl;
     int i0, i1;
-    wrap_pair<OOL>((int)fl, nwl, i0, i1);
+    wrap_pair((int)fl, nwl, i0, i1);
     const float4* row = P.bnd + (int64_t)(2 * line + k) * nwl;
     float4 v0 = row[i0];
     float4 v1 = row[i1];
@@ -114,7 +110,6 @@ OA_D const uint32_t* tape_record(const SimParams& P, int64_t g, int j)
     return P.tape + 3 * ((int64_t)j * P.tape_stride + g);
 }
 
-template <bool OOL = true>
 OA_D void fill(const SimParams& P, State& s, uint32_t boundary, float wl, float cosTheta)
 {
     const int line = (int)boundary * 4;
@@ -122,14 +117,13 @@ OA_D void fill(const SimParams& P, State& s, uint32_t boundary, float wl, float 
     const int m2_line = cosTheta > 0.f ? line + 0 : line + 3;
     const int su_line = cosTheta > 0.f ? line + 2 : line + 1;
     s.m1_line = m1_line;
-    s.material1 = bnd_lookup<OOL>(P, wl, m1_line, 0);
-    s.group_velocity = bnd_lookup<OOL>(P, wl, m1_line, 1).x;
-    s.n2 = bnd_lookup<OOL>(P, wl, m2_line, 0).x;
+    s.material1 = bnd_lookup(P, wl, m1_line, 0);
+    s.group_velocity = bnd_lookup(P, wl, m1_line, 1).x;
+    s.n2 = bnd_lookup(P, wl, m2_line, 0).x;
     s.ems = P.optical[4 * su_line + 1];
-    s.surface = (s.ems != EMS_NOSURFACE) ? bnd_lookup<OOL>(P, wl, su_line, 0) : make_float4(0.f, 0.f, 0.f, 0.f);
+    s.surface = (s.ems != EMS_NOSURFACE) ? bnd_lookup(P, wl, su_line, 0) : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-template <bool OOL = true>
 OA_D float icdf_tex(const SimParams& P, float x, int layer)
 {
     const int n = P.n_icdf;
@@ -137,26 +131,25 @@ OA_D float icdf_tex(const SimParams& P, float x, int layer)
     float fl = floorf(xb);
     float a = xb - fl;
     int i0, i1;
-    wrap_pair<OOL>((int)fl, n, i0, i1);
+    wrap_pair((int)fl, n, i0, i1);
     int L = layer < P.n_icdf_layer ? layer : 0;
     const float* row = P.icdf + (int64_t)L * n;
     float v0 = row[i0], v1 = row[i1];
     return v0 + a * (v1 - v0);
 }
 
-template <bool OOL = true>
 OA_D float scint_wavelength(const SimParams& P, float u0)
 {
-    if (P.icdf_hd == 0) return icdf_tex<OOL>(P, u0, 0);
+    if (P.icdf_hd == 0) return icdf_tex(P, u0, 0);
     if (P.icdf_hd == 10) {
         bool lhs = u0 < 0.1f, rhs = u0 > 0.9f;
         float x = lhs ? (u0 * 10.f) : (rhs ? (u0 - 0.9f) * 10.f : u0);
-        return icdf_tex<OOL>(P, x, lhs ? 1 : (rhs ? 2 : 0));
+        return icdf_tex(P, x, lhs ? 1 : (rhs ? 2 : 0));
     }
     if (P.icdf_hd == 20) {
         bool lhs = u0 < 0.05f, rhs = u0 > 0.95f;
         float x = lhs ? (u0 * 20.f) : (rhs ? (u0 - 0.95f) * 20.f : u0);
-        return icdf_tex<OOL>(P, x, lhs ? 1 : (rhs ? 2 : 0));
+        return icdf_tex(P, x, lhs ? 1 : (rhs ? 2 : 0));
     }
     return 0.f;
 }
@@ -194,10 +187,10 @@ OA_D void marsaglia(v3& dir, R& rng)
     float u, v, b, a;
     int trials = 0;
     do {
-        float u0 = uni(rng);
-        float u1 = uni(rng);
-        u = 2.f * u0 - 1.f;
-        v = 2.f * u1 - 1.f;
+        float w[2];
+        draw<2>(rng, w);
+        u = 2.f * w[0] - 1.f;
+        v = 2.f * w[1] - 1.f;
         b = u * u + v * v;
     } while (b > 1.f && ++trials < OA_MAX_TRIALS);
     if (b > 1.f) { u = 0.f; v = 0.f; b = 0.f; }   /* bound reached: (0, 0, -1) */
@@ -215,7 +208,7 @@ OA_D void lambertian(v3& dir, v3 normal, float orient, R& rng)
         marsaglia(dir, rng);
         ndotv = dot(dir, normal) * orient;
         if (ndotv < 0.f) { dir = -1.f * dir; ndotv = -1.f * ndotv; }
-        u = uni(rng);
+        u = draw1(rng);
     } while (!(u < ndotv) && (count < 1024));
 }
 
@@ -226,7 +219,9 @@ OA_D void rayleigh(Photon& p, R& rng)
     bool looping = true;
     int trials = 0;
     do {
-        float u0 = uni(rng), u1 = uni(rng), u2 = uni(rng), u3 = uni(rng), u4 = uni(rng);
+        float u[5];
+        draw<5>(rng, u);
+        const float u0 = u[0], u1 = u[1], u2 = u[2], u3 = u[3], u4 = u[4];
         float cosTheta = u0;
         float sinTheta = sqrtf(1.0f - u0 * u0);
         if (u1 < 0.5f) cosTheta = -cosTheta;
@@ -255,14 +250,15 @@ OA_D void rayleigh(Photon& p, R& rng)
 /* ----------------------------------------------------------- physics */
 
 template <class R, class Tape>
-OA_D int to_boundary(const SimParams& P, uint32_t& flag, R& rng, Photon& p, const State& s, float dist, Tape& tape)
+OA_D int to_boundary(const SimParams& P, uint32_t& flag, R& rng, Photon& p, const State& s, float dist, Tape& tape,
+                     MaybeThird& third)
 {
     const float absorption_length = s.material1.y;
     const float scattering_length = s.material1.z;
     const float reemission_prob = s.material1.w;
     const float gv = s.group_velocity;
-    const float u_scattering = uni(rng);
-    const float u_absorption = uni(rng);
+    float u_scattering, u_absorption;
+    third = draw2_maybe3(rng, u_scattering, u_absorption);
     const float scattering_distance = -scattering_length * oa_logf(u_scattering);
     const float absorption_distance = -absorption_length * oa_logf(u_absorption);
     /* the step's one segment: its length and the process that ends it (the
@@ -278,12 +274,13 @@ OA_D int to_boundary(const SimParams& P, uint32_t& flag, R& rng, Photon& p, cons
         if (absorption_distance <= dist) {
             p.time += absorption_distance / gv;
             p.pos = p.pos + absorption_distance * p.mom;
-            float u_reemit = reemission_prob == 0.f ? 2.f : uni(rng);
+            float u_reemit = reemission_prob == 0.f ? 2.f : maybe_third(rng, third);
             if (u_reemit < reemission_prob) {
-                float u_wl = uni(rng), u_mph = uni(rng), u_mct = uni(rng), u_pph = uni(rng), u_pct = uni(rng);
-                p.wavelength = scint_wavelength<wrap_ool<R>::value>(P, u_wl);
-                p.mom = uniform_sphere(u_mph, u_mct);
-                p.pol = normalize(cross(uniform_sphere(u_pph, u_pct), p.mom));
+                float u[5];     /* wavelength, direction (2), polarization (2) */
+                draw<5>(rng, u);
+                p.wavelength = scint_wavelength(P, u[0]);
+                p.mom = uniform_sphere(u[1], u[2]);
+                p.pol = normalize(cross(uniform_sphere(u[3], u[4]), p.mom));
                 flag = F_BULK_REEMIT;
                 return CMD_CONTINUE;
             }
@@ -303,7 +300,7 @@ OA_D int to_boundary(const SimParams& P, uint32_t& flag, R& rng, Photon& p, cons
 }
 
 template <class R>
-OA_D int at_boundary(uint32_t& flag, R& rng, Photon& p, float n1, float n2, v3 normal)
+OA_D int at_boundary(uint32_t& flag, R& rng, MaybeThird third, Photon& p, float n1, float n2, v3 normal)
 {
     const float eta = n1 / n2;
     const float _c1 = -dot(p.mom, normal);
@@ -329,7 +326,7 @@ OA_D int at_boundary(uint32_t& flag, R& rng, Photon& p, float n1, float n2, v3 n
     const float invR = 1.0f / sqrtf(E2_rx * E2_rx + E2_ry * E2_ry);
     const float invT = 1.0f / sqrtf(E2_tx * E2_tx + E2_ty * E2_ty);
     const float TransCoeff = (tir || n1c1 == 0.f) ? 0.f : n2c2 * (E2_tx * E2_tx + E2_ty * E2_ty) / n1c1;
-    const float u_reflect = uni(rng);
+    const float u_reflect = maybe_third(rng, third);
     const bool reflect = u_reflect > TransCoeff;
     p.mom = reflect ? p.mom + (2.0f * c1) * on : eta * p.mom + (eta * c1 - c2) * on;
     const v3 A_paral = normalize(cross(p.mom, A_trans));
@@ -345,10 +342,10 @@ OA_D int at_boundary(uint32_t& flag, R& rng, Photon& p, float n1, float n2, v3 n
 }
 
 template <class R>
-OA_D int at_surface(uint32_t& flag, R& rng, Photon& p, const State& s, v3 normal)
+OA_D int at_surface(uint32_t& flag, R& rng, MaybeThird third, Photon& p, const State& s, v3 normal)
 {
     const float detect = s.surface.x, absorb = s.surface.y, diffuse = s.surface.w;
-    const float u_surface = uni(rng);
+    const float u_surface = maybe_third(rng, third);
     const int action = u_surface < absorb + detect ? CMD_BREAK : CMD_CONTINUE;
     if (action == CMD_BREAK) {
         flag = u_surface < absorb ? F_SURFACE_ABSORB : F_SURFACE_DETECT;
@@ -384,14 +381,15 @@ OA_D int propagate(const SimParams& P, R& rng, Photon& p, const Prd& prd, Tape& 
     p.obf = (p.obf & 0x7fffffffu) | ((cosTheta < 0.f ? 0x1u : 0x0u) << 31);
     p.hitcount_iindex = 0x00010000u | (0x0000ffffu & iindex);
     State s;
-    fill<wrap_ool<R>::value>(P, s, boundary, p.wavelength, cosTheta);
+    fill(P, s, boundary, p.wavelength, cosTheta);
     uint32_t flag = 0u;
-    int command = to_boundary(P, flag, rng, p, s, prd.t, tape);
+    MaybeThird third;
+    int command = to_boundary(P, flag, rng, p, s, prd.t, tape, third);
     if (command == CMD_BOUNDARY) {
-        if (s.ems == EMS_NOSURFACE) command = at_boundary(flag, rng, p, s.material1.x, s.n2, normal);
-        else if (s.ems == EMS_SURFACE) command = at_surface(flag, rng, p, s, normal);
-        else if (prd.lposcost < 0.f) command = at_surface(flag, rng, p, s, normal);
-        else if (s.ems == EMS_ZPLUS_SENSOR_A) { (void)uni(rng); flag = F_SURFACE_DETECT; command = CMD_BREAK; }
+        if (s.ems == EMS_NOSURFACE) command = at_boundary(flag, rng, third, p, s.material1.x, s.n2, normal);
+        else if (s.ems == EMS_SURFACE) command = at_surface(flag, rng, third, p, s, normal);
+        else if (prd.lposcost < 0.f) command = at_surface(flag, rng, third, p, s, normal);
+        else if (s.ems == EMS_ZPLUS_SENSOR_A) { (void)maybe_third(rng, third); flag = F_SURFACE_DETECT; command = CMD_BREAK; }
     }
     set_flag(p, flag);
     return command;
@@ -425,8 +423,10 @@ OA_D void gen_torch(Photon& p, R& rng, const float4* gq, uint64_t photon_id)
     p.wavelength = 0.f;
     if (type == T_SPHERE || type == T_POINT_ISO) {
         p.wavelength = gwl; p.time = gtime;
-        float u_zenith = zx + uni(rng) * (zy - zx);
-        float u_azimuth = ax + uni(rng) * (ay - ax);
+        float u0, u1;
+        const MaybeThird third = draw2_maybe3(rng, u0, u1);
+        float u_zenith = zx + u0 * (zy - zx);
+        float u_azimuth = ax + u1 * (ay - ax);
         float phi = 2.f * OA_PI_F * u_azimuth;
         float sinPhi, cosPhi; oa_sincosf(phi, &sinPhi, &cosPhi);
         float cosTheta = 1.f - 2.0f * u_zenith;
@@ -441,12 +441,14 @@ OA_D void gen_torch(Photon& p, R& rng, const float4* gq, uint64_t photon_id)
         rotateUz(p.pol, p.mom);
         if (type == T_POINT_ISO) {
             p.pos = p.pos + gpos;
-            if (gweight > 0.f) p.wavelength = gwl + uni(rng) * gweight;
+            if (gweight > 0.f) p.wavelength = gwl + maybe_third(rng, third) * gweight;
         }
     } else if (type == T_DISC) {
         p.wavelength = gwl; p.time = gtime; p.mom = gmom;
-        float u_zenith = zx + uni(rng) * (zy - zx);
-        float u_azimuth = ax + uni(rng) * (ay - ax);
+        float u2[2];
+        draw<2>(rng, u2);
+        float u_zenith = zx + u2[0] * (zy - zx);
+        float u_azimuth = ax + u2[1] * (ay - ax);
         float r = radius * u_zenith;
         float phi = 2.f * OA_PI_F * u_azimuth;
         float sinPhi, cosPhi; oa_sincosf(phi, &sinPhi, &cosPhi);
@@ -460,8 +462,10 @@ OA_D void gen_torch(Photon& p, R& rng, const float4* gq, uint64_t photon_id)
         float u, v, b, a;
         int trials = 0;
         do {
-            float u0z = zx + uni(rng) * (zy - zx);
-            float u1a = ax + uni(rng) * (ay - ax);
+            float u2[2];
+            draw<2>(rng, u2);
+            float u0z = zx + u2[0] * (zy - zx);
+            float u1a = ax + u2[1] * (ay - ax);
             u = 2.f * u0z - 1.f; v = 2.f * u1a - 1.f; b = u * u + v * v;
         } while (b > 1.f && ++trials < OA_MAX_TRIALS);
         if (b > 1.f) { u = 0.f; v = 0.f; b = 0.f; }
@@ -531,7 +535,9 @@ OA_D void gen_torch(Photon& p, R& rng, const float4* gq, uint64_t photon_id)
 template <class R>
 OA_D void gen_scint(const SimParams& P, Photon& p, R& rng, const float4* gq)
 {
-    float u0 = uni(rng), u1 = uni(rng), u2 = uni(rng), u3 = uni(rng);
+    float ug[4];
+    draw<4>(rng, ug);
+    const float u0 = ug[0], u1 = ug[1], u2 = ug[2], u3 = ug[3];
     float cost = 1.f - 2.f * u0;
     float sint = sqrtf((1.f - cost) * (1.f + cost));
     float phi = 2.f * OA_PI_F * u1;
@@ -541,12 +547,15 @@ OA_D void gen_scint(const SimParams& P, Photon& p, R& rng, const float4* gq)
     phi = 2.f * OA_PI_F * u2;
     oa_sincosf(phi, &sinp, &cosp);
     p.pol = normalize(cosp * p.pol + sinp * cross(p.mom, p.pol));
-    p.wavelength = scint_wavelength<wrap_ool<R>::value>(P, u3);
+    p.wavelength = scint_wavelength(P, u3);
     const float4 q1 = gq[1], q2 = gq[2], q3 = gq[3], q5 = gq[5];
     const float charge = q3.y, meanVelocity = q3.w, step_length = q2.w, scint_time = q5.x;
-    float fraction = charge == 0.f ? 1.f : uni(rng);
+    float ut[2];                    /* position along the step (charged), then the decay time */
+    if (charge == 0.f) { ut[0] = 1.f; ut[1] = draw1(rng); }
+    else draw<2>(rng, ut);
+    const float fraction = ut[0];
     p.pos = mk(q1.x, q1.y, q1.z) + fraction * mk(q2.x, q2.y, q2.z);
-    float u4 = uni(rng);
+    const float u4 = ut[1];
     float deltaTime = fraction * step_length / meanVelocity - scint_time * oa_logf(u4);
     p.time = q1.w + deltaTime;
     zero_flags_set(p, F_SCINTILLATION);
@@ -569,20 +578,19 @@ OA_D void gen_cerenkov(const SimParams& P, Photon& p, R& rng, const float4* gq)
     float wavelength, cosTheta, sin2Theta, u_maxSin2;
     unsigned count = 0;
     do {
-        const float u0 = uni(rng);
-        const float w = Wmin + u0 * (Wmax - Wmin);
+        float u[2];
+        draw<2>(rng, u);
+        const float w = Wmin + u[0] * (Wmax - Wmin);
         wavelength = Wmin * Wmax / w;
-        const float4 props = bnd_lookup<wrap_ool<R>::value>(P, wavelength, matline, 0);
+        const float4 props = bnd_lookup(P, wavelength, matline, 0);
         const float sampledRI = props.x;
         cosTheta = BetaInverse / sampledRI;
         sin2Theta = fmaxf(0.f, (1.f - cosTheta) * (1.f + cosTheta));
-        const float u1 = uni(rng);
-        u_maxSin2 = u1 * maxSin2;
+        u_maxSin2 = u[1] * maxSin2;
         count += 1;
     } while (u_maxSin2 > sin2Theta && count < 100);
     const float sinTheta = sqrtf(sin2Theta);
-    const float u0 = uni(rng);
-    const float phi = 2.f * OA_PI_F * u0;
+    const float phi = 2.f * OA_PI_F * draw1(rng);
     float sinPhi, cosPhi;
     oa_sincosf(phi, &sinPhi, &cosPhi);
     p.mom = mk(sinTheta * cosPhi, sinTheta * sinPhi, cosTheta);
@@ -590,16 +598,17 @@ OA_D void gen_cerenkov(const SimParams& P, Photon& p, R& rng, const float4* gq)
     p.pol = mk(cosTheta * cosPhi, cosTheta * sinPhi, -sinTheta);
     rotateUz(p.pol, p0);
     p.wavelength = wavelength;
-    float fraction, delta, NumberOfPhotons, N, u;
+    float fraction, delta, NumberOfPhotons, N;
     const float MeanNumberOfPhotonsMax = fmaxf(N1, N2);
     const float DeltaN = (N1 - N2);
     int trials = 0;
     do {
-        fraction = uni(rng);
+        float w[2];
+        draw<2>(rng, w);
+        fraction = w[0];
         delta = fraction * step_length;
         NumberOfPhotons = N1 - fraction * DeltaN;
-        u = uni(rng);
-        N = u * MeanNumberOfPhotonsMax;
+        N = w[1] * MeanNumberOfPhotonsMax;
     } while (N > NumberOfPhotons && ++trials < OA_MAX_TRIALS);
     const float midVelocity = preVelocity + fraction * (postVelocity - preVelocity) * 0.5f;
     p.time = q1.w + delta / midVelocity;

@@ -57,36 +57,31 @@ struct Lane {
  */
 enum : int { PK_TIME, PK_POLX, PK_POLY, PK_POLZ, PK_WL, PK_IDENT, PK_MASK, PK_HITCOUNT, PK_BOUNCE, PK_G, PK_G_HI,
              PK_SEQ, PK_RNG = PK_SEQ + 8 };
-static_assert(PK_RNG + 8 == OA_PARK_WORDS, "parked words");
 
 /* park_fixed: what stays as it is from the photon's start to its end, its 32-bit index
    (sphoton::set_index) at word index_word<R> among it */
-template <class R> struct index_word { static constexpr int value = 7; };
+template <class R> struct index_word;
 template <> struct index_word<PhiloxRng> { static constexpr int value = 0; };
-template <> struct index_word<PhiloxRngInline> { static constexpr int value = 0; };
+template <> struct index_word<PrecookedRng> { static constexpr int value = 3; };
+template <> struct index_word<XorwowRng> { static constexpr int value = 6; };
+/* LDS words of a lane's parked state */
+template <class R> struct park_words { static constexpr int value = PK_RNG + 4; };
+template <> struct park_words<XorwowRng> { static constexpr int value = PK_RNG + 7; };
 
-template <int STRIDE> OA_D void park_fixed(uint32_t* w, const oa_philox_stream& s)
+template <int STRIDE> OA_D void park_fixed(uint32_t* w, const PhiloxRng& r)
 {
-    w[0] = (uint32_t)s.photon; w[STRIDE] = (uint32_t)(s.photon >> 32);
+    w[0] = (uint32_t)r.photon; w[STRIDE] = (uint32_t)(r.photon >> 32);
 }
-template <int STRIDE> OA_D void park_rng(uint32_t* w, const oa_philox_stream& s)
+template <int STRIDE> OA_D void park_rng(uint32_t* w, const PhiloxRng& r)
 {
-    w[2 * STRIDE] = (uint32_t)s.pos; w[3 * STRIDE] = (uint32_t)(s.pos >> 32);
-    w[4 * STRIDE] = s.b0; w[5 * STRIDE] = s.b1; w[6 * STRIDE] = s.b2; w[7 * STRIDE] = s.b3;
+    w[2 * STRIDE] = (uint32_t)r.pos; w[3 * STRIDE] = (uint32_t)(r.pos >> 32);
 }
-template <int STRIDE> OA_D void unpark_rng(const SimParams& P, const uint32_t* w, oa_philox_stream& s)
+template <int STRIDE> OA_D void unpark_rng(const SimParams& P, const uint32_t* w, PhiloxRng& r)
 {
-    s.key = P.seed;
-    s.photon = (uint64_t)w[0] | ((uint64_t)w[STRIDE] << 32);
-    s.pos = (uint64_t)w[2 * STRIDE] | ((uint64_t)w[3 * STRIDE] << 32);
-    s.b0 = w[4 * STRIDE]; s.b1 = w[5 * STRIDE]; s.b2 = w[6 * STRIDE]; s.b3 = w[7 * STRIDE];
+    r.key = P.seed;
+    r.photon = (uint64_t)w[0] | ((uint64_t)w[STRIDE] << 32);
+    r.pos = (uint64_t)w[2 * STRIDE] | ((uint64_t)w[3 * STRIDE] << 32);
 }
-template <int STRIDE> OA_D void park_fixed(uint32_t* w, const PhiloxRng& r) { park_fixed<STRIDE>(w, r.ph); }
-template <int STRIDE> OA_D void park_rng(uint32_t* w, const PhiloxRng& r) { park_rng<STRIDE>(w, r.ph); }
-template <int STRIDE> OA_D void unpark_rng(const SimParams& P, const uint32_t* w, PhiloxRng& r) { unpark_rng<STRIDE>(P, w, r.ph); }
-template <int STRIDE> OA_D void park_fixed(uint32_t* w, const PhiloxRngInline& r) { park_fixed<STRIDE>(w, r.ph); }
-template <int STRIDE> OA_D void park_rng(uint32_t* w, const PhiloxRngInline& r) { park_rng<STRIDE>(w, r.ph); }
-template <int STRIDE> OA_D void unpark_rng(const SimParams& P, const uint32_t* w, PhiloxRngInline& r) { unpark_rng<STRIDE>(P, w, r.ph); }
 template <int STRIDE> OA_D void park_fixed(uint32_t*, const XorwowRng&) {}
 template <int STRIDE> OA_D void park_rng(uint32_t* w, const XorwowRng& r)
 {
@@ -177,12 +172,9 @@ OA_D int64_t upper_index(const int64_t* a, int64_t lo, int64_t hi, int64_t v)
    (qudarap/qrng.h:84-89,131-137) */
 OA_D void rng_start(const SimParams& P, PhiloxRng& r, int e, uint64_t photon_idx)
 {
-    oa_rng_init(&r.ph, P.seed, P.rng_offset, P.skipahead, (uint64_t)P.ev_id[e], photon_idx);
-}
-
-OA_D void rng_start(const SimParams& P, PhiloxRngInline& r, int e, uint64_t photon_idx)
-{
-    oa_rng_init(&r.ph, P.seed, P.rng_offset, P.skipahead, (uint64_t)P.ev_id[e], photon_idx);
+    r.key = P.seed;
+    r.photon = photon_idx;
+    r.pos = P.rng_offset + P.skipahead * (uint64_t)P.ev_id[e];
 }
 
 OA_D void rng_start(const SimParams& P, XorwowRng& r, int e, uint64_t photon_idx)
@@ -311,6 +303,12 @@ OA_D void lane_finish(const SimParams& P, const Lane<R, LITE>& L, const uint32_t
     }
 }
 
+/* LDS bytes of a block: parked words and traversal stack of each thread */
+template <class R> inline unsigned block_lds(int block, int stack_depth)
+{
+    return (unsigned)(park_words<R>::value + stack_depth) * 4u * (unsigned)block;
+}
+
 } // namespace oa
 
 /* ----------------------------------------------------- plain kernel */
@@ -319,9 +317,9 @@ template <int BLOCK, int F, class R>
 __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_plain(SimParams P)
 {
     using namespace oa;
-    extern __shared__ uint32_t s_lane[];           /* OA_PARK_WORDS parked words, then the stack, of each lane */
+    extern __shared__ uint32_t s_lane[];           /* each lane's parked words, then its stack */
     uint32_t* park_w = s_lane + threadIdx.x;
-    uint32_t* stk = park_w + OA_PARK_WORDS * BLOCK;
+    uint32_t* stk = park_w + park_words<R>::value * BLOCK;
     const int64_t g = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     bool hit = false;
     if (g < P.n_photon) {
@@ -345,9 +343,9 @@ template <int BLOCK, int F, class R, class T = oa::NoTape>
 __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_wave(SimParams P)
 {
     using namespace oa;
-    extern __shared__ uint32_t s_lane[];           /* OA_PARK_WORDS parked words, then the stack, of each lane */
+    extern __shared__ uint32_t s_lane[];           /* each lane's parked words, then its stack */
     uint32_t* park_w = s_lane + threadIdx.x;
-    uint32_t* stk = park_w + OA_PARK_WORDS * BLOCK;
+    uint32_t* stk = park_w + park_words<R>::value * BLOCK;
     const int lane = threadIdx.x & 63;
     Lane<R, (F & 1) != 0> L;
     T tape;
@@ -536,9 +534,9 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_adjoint_wave(SimParams P, AdjP
                                                                int32_t n_ev, int64_t hit_cap, float* S)
 {
     using namespace oa;
-    extern __shared__ uint32_t s_lane[];           /* OA_PARK_WORDS parked words, then the stack, of each lane */
+    extern __shared__ uint32_t s_lane[];           /* each lane's parked words, then its stack */
     uint32_t* park_w = s_lane + threadIdx.x;
-    uint32_t* stk = park_w + OA_PARK_WORDS * BLOCK;
+    uint32_t* stk = park_w + park_words<R>::value * BLOCK;
     const int lane = threadIdx.x & 63;
     /* with the segment tape, only photons it could not hold are replayed: none, when
        the ordering pass (k_hit_det) raised no flag */

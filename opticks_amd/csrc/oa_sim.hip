@@ -14,13 +14,10 @@
 
 #if OA_SIM_RNG == 0
 #define OA_SIM_R oa::PhiloxRng
-#define OA_SIM_RT oa::PhiloxRngInline     /* the taped forward: the same stream, block inlined */
 #elif OA_SIM_RNG == 1
 #define OA_SIM_R oa::PrecookedRng
-#define OA_SIM_RT OA_SIM_R
 #else
 #define OA_SIM_R oa::XorwowRng
-#define OA_SIM_RT OA_SIM_R
 #endif
 
 namespace oa_launch {
@@ -28,7 +25,7 @@ namespace oa_launch {
 hipError_t OA_SIM_NAME(sim_launch, OA_SIM_BLOCK, OA_SIM_RNG)(const SimParams& P, int kernel, int grid, hipStream_t s)
 {
     constexpr int B = OA_SIM_BLOCK;
-    const unsigned lds = oa_sim_lds(B, P.stack_depth);
+    const unsigned lds = oa::block_lds<OA_SIM_R>(B, P.stack_depth);
     const int f = (P.photonlite ? 1 : 0) | (P.ext_leaves ? 2 : 0);
     if (kernel == 0) {
         const unsigned nb = (unsigned)((P.n_photon + B - 1) / B);
@@ -40,8 +37,8 @@ hipError_t OA_SIM_NAME(sim_launch, OA_SIM_BLOCK, OA_SIM_RNG)(const SimParams& P,
         }
     } else if (P.tape) {
         /* a forward for a following adjoint: segment records on the tape (no lite output) */
-        if (f & 2) hipLaunchKernelGGL((k_sim_wave<B, 2, OA_SIM_RT, oa::RecordTape>), dim3((unsigned)grid), dim3(B), lds, s, P);
-        else hipLaunchKernelGGL((k_sim_wave<B, 0, OA_SIM_RT, oa::RecordTape>), dim3((unsigned)grid), dim3(B), lds, s, P);
+        if (f & 2) hipLaunchKernelGGL((k_sim_wave<B, 2, OA_SIM_R, oa::RecordTape>), dim3((unsigned)grid), dim3(B), lds, s, P);
+        else hipLaunchKernelGGL((k_sim_wave<B, 0, OA_SIM_R, oa::RecordTape>), dim3((unsigned)grid), dim3(B), lds, s, P);
     } else {
         switch (f) {
             case 0: hipLaunchKernelGGL((k_sim_wave<B, 0, OA_SIM_R>), dim3((unsigned)grid), dim3(B), lds, s, P); break;
@@ -53,11 +50,16 @@ hipError_t OA_SIM_NAME(sim_launch, OA_SIM_BLOCK, OA_SIM_RNG)(const SimParams& P,
     return hipGetLastError();
 }
 
+unsigned OA_SIM_NAME(sim_lds, OA_SIM_BLOCK, OA_SIM_RNG)(int stack_depth)
+{
+    return oa::block_lds<OA_SIM_R>(OA_SIM_BLOCK, stack_depth);
+}
+
 int OA_SIM_NAME(sim_occupancy, OA_SIM_BLOCK, OA_SIM_RNG)(int stack_depth)
 {
     int nb = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sim_wave<OA_SIM_BLOCK, 0, OA_SIM_R>, OA_SIM_BLOCK,
-                                                     oa_sim_lds(OA_SIM_BLOCK, stack_depth)) != hipSuccess)
+                                                     oa::block_lds<OA_SIM_R>(OA_SIM_BLOCK, stack_depth)) != hipSuccess)
         return 0;
     return nb;
 }
@@ -68,7 +70,7 @@ hipError_t OA_SIM_NAME(adjoint_launch, OA_ADJ_BLOCK, OA_SIM_RNG)(const SimParams
                                                                  const int64_t* hit_off, int32_t n_ev, int64_t hit_cap,
                                                                  float* S, int grid, hipStream_t s)
 {
-    const unsigned lds = oa_sim_lds(OA_ADJ_BLOCK, P.stack_depth);
+    const unsigned lds = oa::block_lds<OA_SIM_R>(OA_ADJ_BLOCK, P.stack_depth);
     if (P.ext_leaves)
         hipLaunchKernelGGL((k_adjoint_wave<OA_ADJ_BLOCK, true, OA_SIM_R>), dim3((unsigned)grid), dim3(OA_ADJ_BLOCK), lds,
                            s, P, A, hits, begin, n_max, hit_off, n_ev, hit_cap, S);
@@ -82,7 +84,7 @@ int OA_SIM_NAME(adjoint_occupancy, OA_ADJ_BLOCK, OA_SIM_RNG)(int stack_depth)
 {
     int nb = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_adjoint_wave<OA_ADJ_BLOCK, false, OA_SIM_R>, OA_ADJ_BLOCK,
-                                                     oa_sim_lds(OA_ADJ_BLOCK, stack_depth)) != hipSuccess)
+                                                     oa::block_lds<OA_SIM_R>(OA_ADJ_BLOCK, stack_depth)) != hipSuccess)
         return 0;
     return nb;
 }
@@ -91,4 +93,3 @@ int OA_SIM_NAME(adjoint_occupancy, OA_ADJ_BLOCK, OA_SIM_RNG)(int stack_depth)
 } // namespace oa_launch
 
 #undef OA_SIM_R
-#undef OA_SIM_RT

@@ -11,13 +11,8 @@ struct AdjParams;
 
 #define OA_SIM_DECLARE(B, K)                                                                   \
     hipError_t sim_launch_##B##_##K(const SimParams& P, int kernel, int grid, hipStream_t s); \
+    unsigned sim_lds_##B##_##K(int stack_depth);                                               \
     int sim_occupancy_##B##_##K(int stack_depth);
-
-/* LDS bytes of a propagation block: each thread's parked photon words and traversal stack */
-inline unsigned oa_sim_lds(int block, int stack_depth)
-{
-    return (unsigned)(OA_PARK_WORDS + stack_depth) * 4u * (unsigned)block;
-}
 
 namespace oa_launch {
 OA_SIM_DECLARE(64, 0)
