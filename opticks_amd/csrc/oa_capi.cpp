@@ -127,6 +127,8 @@ struct mi_sim {
     uint32_t front_leaf = OA_BVH_EMPTY;             /* items of the front instances (build_tlas) */
     int32_t tlas_empty = 0;                         /* every instance is a front instance */
     std::vector<char> h_is_front;                   /* per instance: kept out of the TLAS */
+    std::vector<char> h_link_plain;                 /* per instance: its record links one leaf of plain prims */
+    int32_t front_plain = 0;                        /* front instances are such (SimParams.front_plain) */
     std::vector<uint32_t> solid_blas_root;
     std::vector<uint32_t> h_inst_blas_root;
     std::vector<std::array<double, 6>> solid_box;   /* padded solid-frame prim box per solid */
@@ -401,6 +403,15 @@ static float4 free_ball(const mi_sim* sim, const std::vector<oa_bvh::Item>& all,
     return make_float4((float)b.c[0], (float)b.c[1], (float)b.c[2], (float)b.r2);
 }
 
+/* whether trace_front can test the front instances: each links one leaf of all its prims,
+   and those are leaves of the common types */
+static void set_front_plain(mi_sim* sim)
+{
+    sim->front_plain = sim->front_leaf != OA_BVH_EMPTY && sim->h_link_plain.size() == sim->h_is_front.size();
+    for (size_t i = 0; sim->front_plain && i < sim->h_is_front.size(); ++i)
+        if (sim->h_is_front[i] && !sim->h_link_plain[i]) sim->front_plain = 0;
+}
+
 /* host SAH build of the TLAS over instance boxes with the given leaf size, uploaded
    into new buffers that replace the handle's only when every step succeeded */
 static int build_tlas(mi_sim* sim, int leaf)
@@ -445,6 +456,7 @@ static int build_tlas(mi_sim* sim, int leaf)
     sim->n_tlas = (int64_t)tlas.size();
     sim->front_leaf = front_leaf;
     sim->tlas_empty = titems.empty() ? 1 : 0;
+    set_front_plain(sim);
     sim->generation++;
     return MI_OK;
 }
@@ -527,12 +539,21 @@ static int build_and_upload_geometry(mi_sim* sim, const mi_geometry* g)
        nearest hit does not depend on the order or on box pruning (ties go to the
        smaller key). The link is valid for any instance, so a later TLAS rebuild
        that changes which instances are front changes no result. */
+    sim->h_link_plain.assign((size_t)ni, 0);
     for (int64_t i = 0; i < ni; ++i) {
         if (!sim->h_is_front[i]) continue;
         int32_t gas;
         std::memcpy(&gas, g->inst + 16 * i + 7, 4);
         inst[i].m[11] = f32_of(solid_flat[gas]);
+        bool plain = (solid_flat[gas] & OA_BVH_LEAF_BIT) != 0u;
+        for (int32_t k = 0; k < sim->h_solid_prims[gas].second; ++k) {
+            const int32_t* pr = (const int32_t*)(g->prim + 16 * (sim->h_solid_prims[gas].first + k));
+            const uint32_t tc = ((const uint32_t*)(g->node + 16 * (int64_t)pr[1]))[14];
+            plain = plain && (tc == 101 || tc == 103 || tc == 105 || tc == 110);  /* sphere, zsphere, cylinder, box3 */
+        }
+        sim->h_link_plain[i] = plain;
     }
+    set_front_plain(sim);
 
     std::vector<PrimRec> prim(g->n_prim);
     for (int64_t p = 0; p < g->n_prim; ++p) {
@@ -717,7 +738,7 @@ static SimParams base_params(const mi_sim* sim)
     std::memset(&P, 0, sizeof(P));
     P.node = sim->node.p; P.itra = sim->itra.p; P.plan = sim->plan.p; P.ext_leaves = sim->ext_leaves; P.inst = sim->inst.p; P.prim = sim->prim.p;
     P.tlas = sim->tlas.p; P.tlas_items = sim->tlas_items.p; P.blas = sim->blas.p; P.blas_prims = sim->blas_prims.p;
-    P.front_leaf = sim->front_leaf; P.tlas_empty = sim->tlas_empty; P.free_ball = sim->free_ball.p;
+    P.front_leaf = sim->front_leaf; P.front_plain = sim->front_plain; P.tlas_empty = sim->tlas_empty; P.free_ball = sim->free_ball.p;
     P.stack_depth = sim->stack_depth;
     P.bnd = sim->bnd.p; P.optical = sim->optical.p; P.icdf = sim->icdf.p;
     P.n_wl = sim->n_wl; P.wl_low = sim->wl_low; P.wl_step = sim->wl_step;

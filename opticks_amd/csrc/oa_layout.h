@@ -101,6 +101,7 @@ struct SimParams {
     const BvhNode* blas;
     const PrimRec* blas_prims;    /* prim records in BLAS leaf order (PrimRec.index: the prim) */
     uint32_t front_leaf;          /* leaf link to the front instances' items (tested first), or empty */
+    int32_t front_plain;          /* the front instances' prims are all leaves that trace_front tests */
     int32_t tlas_empty;           /* the TLAS holds no instance: every instance is front */
     int32_t stack_depth;          /* traversal stack entries this geometry needs (at most OA_STACK_DEPTH) */
     const float4* free_ball;      /* (cx, cy, cz, r^2): a ball no TLAS instance box meets (r^2 <= 0: none) */

@@ -693,9 +693,8 @@ OA_D uint32_t visit(const BvhNode* nodes, uint32_t idx, v3 inv, v3 oi, float tmi
     return t0 < INFINITY ? c0 : OA_BVH_EMPTY;
 }
 
-OA_D void inst_ray(const float4* m, v3 o, v3 d, v3& oo, v3& od)
+OA_D void inst_ray_rows(float4 r0, float4 r1, float4 r2, float4 r3, v3 o, v3 d, v3& oo, v3& od)
 {
-    const float4 r0 = m[0], r1 = m[1], r2 = m[2], r3 = m[3];
     oo = mk(r0.x * o.x + r1.x * o.y + r2.x * o.z + r3.x,
             r0.y * o.x + r1.y * o.y + r2.y * o.z + r3.y,
             r0.z * o.x + r1.z * o.y + r2.z * o.z + r3.z);
@@ -703,6 +702,7 @@ OA_D void inst_ray(const float4* m, v3 o, v3 d, v3& oo, v3& od)
             r0.y * d.x + r1.y * d.y + r2.y * d.z,
             r0.z * d.x + r1.z * d.y + r2.z * d.z);
 }
+OA_D void inst_ray(const float4* m, v3 o, v3 d, v3& oo, v3& od) { inst_ray_rows(m[0], m[1], m[2], m[3], o, d, oo, od); }
 
 /* one prim of one instance (entry k of the BLAS-ordered prim records) against the
    nearest hit so far (t, then the (instance, prim) key) */
@@ -720,6 +720,73 @@ OA_D void consider_prim(const SimParams& P, uint32_t ii, uint32_t k, v3 oo, v3 o
     const uint64_t key = ((uint64_t)ii << 32) | (uint64_t)pi;
     if (is.w < best_t || (is.w == best_t && key < best_key)) {
         best_t = is.w; best_key = key; best_inst = ii; best_prim = pi; best_is = is;
+    }
+}
+
+/* Whether a ray has anything to find in the TLAS beyond its nearest front hit at best_t, and
+   from where (tlo): a lane whose segment from the origin to that hit lies in the free ball,
+   which no TLAS instance meets, has nothing; one whose origin lies in it can meet an instance
+   only after leaving it, so its box tests start there (boxes only prune: the prim tests keep
+   tmin). */
+OA_D bool beyond_free_ball(float4 fb, v3 o, v3 d, float tmin, float best_t, float& tlo)
+{
+    if (!(fb.w > 0.f)) return true;
+    const v3 c = mk(fb.x, fb.y, fb.z);
+    const v3 a = o - c, b = o + best_t * d - c;
+    const float qa = dot(a, a) - fb.w;
+    if (qa < 0.f) {
+        if (dot(b, b) < fb.w) return false;
+        const float dd = dot(d, d), bb = dot(a, d);
+        const float t_exit = (sqrtf(bb * bb - dd * qa) - bb) / dd;
+        tlo = fmaxf(tmin, t_exit);
+    }
+    return true;
+}
+
+/* Geometry records that are the same for a whole wave, read through the scalar cache: the
+   constant address space tells the compiler that nothing writes them during the launch. */
+typedef float cf4 __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(4))) cf4* cptr4;
+typedef const __attribute__((address_space(4))) uint32_t* cptr1;
+OA_D cptr4 const_ptr(const void* p) { return (cptr4)(uintptr_t)p; }
+OA_D float4 const_load(cptr4 p) { const cf4 v = *p; return make_float4(v.x, v.y, v.z, v.w); }
+
+/*
+ * The front instances (world-sized, tested by every trace), where their solids are leaf
+ * prims of the common types: P.front_plain. Every lane tests the same prims, so their
+ * records come by scalar loads and the leaf type is a scalar branch, where the leaf phase
+ * below chains vector loads (item, instance, prim record, node) with a switch per lane.
+ */
+OA_D void trace_front(const SimParams& P, v3 o, v3 d, float tmin, float& best_t, uint64_t& best_key, uint32_t& best_inst,
+                      uint32_t& best_prim, Isect& best_is)
+{
+    const uint32_t first = P.front_leaf & 0x00ffffffu, count = (P.front_leaf >> 24) & 0x7fu;
+    for (uint32_t k = 0; k < count; ++k) {
+        const uint32_t ii = ((cptr1)(uintptr_t)P.tlas_items)[first + k];
+        const cptr4 m = const_ptr(P.inst + ii);
+        OA_COUNT(OA_ST_INST);
+        const float4 r0 = const_load(m), r1 = const_load(m + 1), r2 = const_load(m + 2), r3 = const_load(m + 3);
+        v3 oo, od;
+        inst_ray_rows(r0, r1, r2, r3, o, d, oo, od);
+        const uint32_t link = __float_as_uint(r2.w);       /* a front instance's link: one leaf of all its prims */
+        const uint32_t bf = link & 0x00ffffffu, bn = (link >> 24) & 0x7fu;
+        for (uint32_t j = 0; j < bn; ++j) {
+            OA_COUNT(OA_ST_PRIM);
+            OA_WAVE_COUNT(OA_ST_W_PRIM, OA_ST_L_PRIM);
+            const float4 pr = const_load(const_ptr(P.blas_prims + bf + j));
+            const uint32_t pi = __float_as_uint(pr.w);
+            const cptr4 nd = const_ptr(P.node + 4u * __float_as_uint(pr.x));
+            const float4 q0 = const_load(nd), q1 = const_load(nd + 1), q3 = const_load(nd + 3);
+            Isect is;
+            if (!intersect_leaf_q<false>(is, q0, q1, __float_as_uint(q3.z), __float_as_uint(q3.w), P.itra, P.plan, tmin,
+                                         oo, od))
+                continue;
+            if (!(is.w >= tmin)) continue;
+            const uint64_t key = ((uint64_t)ii << 32) | (uint64_t)pi;
+            if (is.w < best_t || (is.w == best_t && key < best_key)) {
+                best_t = is.w; best_key = key; best_inst = ii; best_prim = pi; best_is = is;
+            }
+        }
     }
 }
 
@@ -748,13 +815,17 @@ OA_D void trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float
     Isect best_is; best_is.x = best_is.y = best_is.z = best_is.w = 0.f;
     int sp = 0;
     uint32_t cur = P.tlas_empty ? OA_BVH_EMPTY : 0u;    /* TLAS root node */
-    /* the first leaf phase tests the front instances (world-sized boxes kept out
-       of the TLAS) on every lane together; the walk then starts with their
-       nearest hit as tmax */
-    uint32_t leaf = P.front_leaf;
+    /* the front instances (world-sized boxes kept out of the TLAS) are tested on every
+       lane together, by trace_front or as the first leaf phase; the walk then starts with
+       their nearest hit as tmax */
+    uint32_t leaf = P.front_plain ? OA_BVH_EMPTY : P.front_leaf;
     /* lower bound of the node and BLAS box tests of TLAS instances (set after the front phase) */
     float tlo = tmin;
     bool done = false;
+    if (P.front_plain) {
+        trace_front(P, o, d, tmin, best_t, best_key, best_inst, best_prim, best_is);
+        done = !(cur == 0u && beyond_free_ball(const_load(const_ptr(P.free_ball)), o, d, tmin, best_t, tlo));
+    }
 #ifdef OA_STATS
     uint32_t n1 = 0, n2 = 0;
 #endif
@@ -850,28 +921,8 @@ OA_D void trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float
         }
         OA_CYC_ADD(OA_ST_C_P2, c_p2);
         __builtin_amdgcn_s_setprio(0);
-        /* after the front phase (the TLAS walk not begun: cur is still the root): a lane
-           whose segment from the origin to the nearest front hit lies in the free ball,
-           which no TLAS instance meets, has nothing to find in the TLAS; one whose origin
-           lies in it can meet an instance only after leaving it, so its box tests start
-           there (boxes only prune: the prim tests keep tmin) */
-        if (cur == 0u) {
-            const float4 fb = *P.free_ball;
-            if (fb.w > 0.f) {
-                const v3 c = mk(fb.x, fb.y, fb.z);
-                const v3 a = o - c, b = o + best_t * d - c;
-                const float qa = dot(a, a) - fb.w;
-                if (qa < 0.f) {
-                    if (dot(b, b) < fb.w) {
-                        cur = OA_BVH_EMPTY;
-                    } else {
-                        const float dd = dot(d, d), bb = dot(a, d);
-                        const float t_exit = (sqrtf(bb * bb - dd * qa) - bb) / dd;
-                        tlo = fmaxf(tmin, t_exit);
-                    }
-                }
-            }
-        }
+        /* after a front leaf phase (the TLAS walk not begun: cur is still the root) */
+        if (cur == 0u && !beyond_free_ball(*P.free_ball, o, d, tmin, best_t, tlo)) cur = OA_BVH_EMPTY;
     }
     OA_CYC_ADD(OA_ST_C_TRACE, c_trace);
 #ifdef OA_STATS

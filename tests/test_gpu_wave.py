@@ -55,3 +55,48 @@ def test_stack_depths_match_checker(shells, block, kernel):
     assert np.array_equal(sim.photon.view(np.uint32), photon.view(np.uint32))
     assert len(hits) == np.count_nonzero(photon[:, 3, 3].view(np.uint32) & 0x40)
     sim.close()
+
+
+def front_world(kind, num_photon=40_000, seed=42):
+    """A world solid of several large prims tested ahead of the TLAS, with eight small spheres
+    inside it. `plain`: leaves of every type the scalar front test takes, one of them under a
+    node transform; `tree`: also a Boolean tree, which sends the front solid down the general
+    path."""
+    from opticks_amd.foundry import CSG_DIFFERENCE
+    lib = BoundaryLib()
+    lib.add_material(Material("Water", 1.33, 20000.0, 30000.0))
+    lib.add_material(Material("Acrylic", 1.50, 1e6, 1e6))
+    lib.add_surface(Surface("wallSurf", detect=0.5, absorb=0.5))
+    b_world = lib.boundary("Water/wallSurf/wallSurf/Water")
+    b_obj = lib.boundary("Water///Acrylic")
+    fd = Foundry()
+    tilted = Node.cylinder(2500.0, -2500.0, 2500.0)
+    tilted.transform = configs.rotation_z_to([0.3, -0.5, 0.81])
+    tilted.transform[3, :3] = (40.0, -60.0, 20.0)
+    prims = [fd.addPrim(Node.box3(9000.0, 9000.0, 9000.0), b_world), fd.addPrim(tilted, b_obj),
+             fd.addPrim(Node.zsphere(2300.0, -1900.0, 2100.0), b_obj), fd.addPrim(Node.sphere(1500.0), b_obj)]
+    if kind == "tree":
+        prims.append(fd.addPrim(Node.op(CSG_DIFFERENCE, Node.sphere(1300.0), Node.sphere(1200.0)), b_obj))
+    s0 = fd.addSolid("world", prims)
+    s1 = fd.addSolid("ball", [fd.addPrim(Node.sphere(150.0), b_world)])
+    fd.addInstance(np.eye(4), s0)
+    for k in range(8):
+        t = np.eye(4)
+        t[3, :3] = [(800.0 if k >> a & 1 else -700.0) for a in range(3)]
+        fd.addInstance(t, s1, sensor_identifier=k, sensor_index=k)
+    phys = lib.arrays()
+    phys["icdf"], phys["icdf_hd_factor"] = gaussian_icdf()
+    gs = np.stack([configs.torch_genstep(num_photon // 2, configs.T_POINT_ISO, pos=p, wavelength=300.0, weight=300.0)
+                   for p in ((0.0, 0.0, 0.0), (30.0, -2900.0, 100.0))]).astype(np.float32)
+    return configs.Workload("front_world", fd.arrays(), phys, gs, seed=seed)
+
+
+@pytest.mark.parametrize("kind", ["plain", "tree"])
+def test_front_solids_match_checker(kind):
+    w = front_world(kind)
+    sim = QSim(w.geometry, w.physics, SEventConfig(seed=w.seed))
+    sim.simulate(w.gensteps, 0)
+    photon, seq = po.World(w.geometry, w.physics).simulate(w.gensteps, seed=w.seed)
+    assert np.array_equal(sim.seq, seq)
+    assert np.array_equal(sim.photon.view(np.uint32), photon.view(np.uint32))
+    sim.close()
