@@ -800,9 +800,14 @@ OA_D void trace_front(const SimParams& P, v3 o, v3 d, float tmin, float& best_t,
  * an instance leaf or is finished, then all pending leaves (instance ray
  * transform, BLAS walk, CSG prim tests) run together, so the expensive CSG
  * code executes with most lanes of the wave active instead of once per lane.
+ *
+ * Returns false, with nothing found out, for a lane that needs the TLAS walk while fewer
+ * than walk_min lanes of the wave do and some lane does not: it is traced again, front
+ * instances included, with its wave's next step (they are tested on the whole wave anyway).
+ * Such a wave always has a lane whose trace ended, so it gets on.
  */
 template <int STRIDE, bool EXT = false>
-OA_D void trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float tmax, Prd& prd)
+OA_D bool trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float tmax, Prd& prd, int walk_min = 0)
 {
     OA_COUNT(OA_ST_TRACE);
     OA_WAVE_COUNT(OA_ST_W_TRACE, OA_ST_L_TRACE);
@@ -825,6 +830,12 @@ OA_D void trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float
     if (P.front_plain) {
         trace_front(P, o, d, tmin, best_t, best_key, best_inst, best_prim, best_is);
         done = !(cur == 0u && beyond_free_ball(const_load(const_ptr(P.free_ball)), o, d, tmin, best_t, tlo));
+        /* the TLAS walk and the CSG trees behind it run for as long as their slowest lane:
+           lanes that need them wait for company while others of the wave have a step to do */
+        const unsigned long long walkers = __ballot(!done);
+        if (__popcll(walkers) < walk_min && walkers != __ballot(1)) {
+            if (!done) return false;
+        }
     }
 #ifdef OA_STATS
     uint32_t n1 = 0, n2 = 0;
@@ -941,7 +952,7 @@ OA_D void trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float
         prd.normal = mk(0.f, 0.f, 0.f); prd.t = 0.f; prd.lposcost = 0.f;
         prd.lx = 0.f; prd.ly = __uint_as_float(0x7fc00000u); prd.gprim = 0xffffu;
         prd.iindex_identity = 0xffffffffu; prd.boundary = 0xffffu;
-        return;
+        return true;
     }
     const float4* m = reinterpret_cast<const float4*>(P.inst + best_inst);
     const float4 r0 = m[0], r1 = m[1], r2 = m[2];
@@ -959,6 +970,7 @@ OA_D void trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float
     prd.iindex_identity = ((best_inst & 0xffffu) << 16) | (ident & 0xffffu);
     prd.boundary = P.prim[best_prim].boundary & 0xffffu;
     prd.gprim = P.prim[best_prim].global_prim;
+    return true;
 }
 
 } // namespace oa

@@ -240,19 +240,37 @@ OA_D bool lane_start(const SimParams& P, Lane<R, LITE>& L, int64_t g, uint32_t* 
     return lane_alive(P, L);
 }
 
-/* one iteration of the CSGOptiX7.cu:477-509 loop from the parked state w, which the
-   caller parks again for the next; returns true when the photon is done */
+/*
+ * Lanes that must need the TLAS walk before a wave runs it (trace's walk_min). On a detector
+ * shell a third of the steps leave the free ball, so about 20 lanes of a full wave walked at
+ * each step, 8 of them on average at any time, and the walk with its CSG trees took 60% of
+ * the kernel. Waiting for 36 runs it half as often; lanes that wait are idle for the cheap
+ * part of the step meanwhile. 24 / 32 / 36 / 40 / 44: 36.1 / 34.7 / 34.3 / 34.4 / 35.0 ms on 64
+ * events of 20,000 detectors (51.6 without), 6.21 / 6.14 / 6.08 / 6.24 / 6.40 ms on 10M photons
+ * and 2,000 detectors (9.09 without). Once the photons have run out lanes are not refilled
+ * and waiting only lengthens the last histories: 8 there (0 is 5% slower on one event of 1M
+ * photons, 24 is 3% slower on 12,000).
+ */
+#ifndef OA_WALK_MIN
+#define OA_WALK_MIN 36
+#define OA_WALK_MIN_TAIL 8
+#endif
+
+/* one iteration of the CSGOptiX7.cu:477-509 loop from the parked state w, parked again for
+   the next (STEP_MORE) or not (STEP_DONE: the photon ended); STEP_WAITS: nothing was done */
+enum : int { STEP_MORE, STEP_DONE, STEP_WAITS };
 template <int STRIDE, class Tape, bool LITE, bool EXT, class R>
-OA_D bool lane_step(const SimParams& P, Lane<R, LITE>& L, uint32_t* w, uint32_t* stk, Tape& tape)
+OA_D int lane_step(const SimParams& P, Lane<R, LITE>& L, uint32_t* w, uint32_t* stk, Tape& tape, int walk_min = 0)
 {
     const float tmin = (L.p.obf & P.eps0_mask) ? P.tmin0 : P.tmin;
     Prd prd;
-    trace<STRIDE, EXT>(P, stk, L.p.pos, L.p.mom, tmin, P.tmax, prd);
+    const bool traced = trace<STRIDE, EXT>(P, stk, L.p.pos, L.p.mom, tmin, P.tmax, prd, walk_min);
     asm volatile("" ::: "memory");
-    unpark<STRIDE>(P, w, L);
+    unpark<STRIDE>(P, w, L);                      /* by waiting lanes too: their old values need not outlive the trace */
+    if (!traced) return STEP_WAITS;
     L.g = parked_g<STRIDE>(w);
     if constexpr (LITE) { L.lite.lcost = prd.lposcost; L.lite.lx = prd.lx; L.lite.ly = prd.ly; }
-    if (prd.boundary == 0xffffu) return true;
+    if (prd.boundary == 0xffffu) return STEP_DONE;
     prd.normal = normalize(prd.normal);
     OA_COUNT(OA_ST_STEP);
     OA_WAVE_COUNT(OA_ST_W_PHYS, OA_ST_L_PHYS);
@@ -260,8 +278,9 @@ OA_D bool lane_step(const SimParams& P, Lane<R, LITE>& L, uint32_t* w, uint32_t*
     const int command = propagate(P, L.rng, L.p, prd, tape);
     L.bounce++;
     if constexpr (Tape::keeps_seq) seq_add<STRIDE>(w, (unsigned)L.bounce, ph_flag(L.p), ph_boundary(L.p));
-    if (command == CMD_BREAK) return true;
-    return !lane_alive(P, L);
+    if (command == CMD_BREAK || !lane_alive(P, L)) return STEP_DONE;
+    park<STRIDE>(w, L);
+    return STEP_MORE;
 }
 
 /* sphotonlite::init + set_lpos (sysrap/sphotonlite.h:192-198,234-244) from the
@@ -326,10 +345,8 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_plain(SimParams P)
         Lane<R, (F & 1) != 0> L;
         NoTape tape;
         bool more = lane_start<BLOCK, NoTape>(P, L, g, park_w);
-        while (more) {
-            park<BLOCK>(park_w, L);
-            more = !lane_step<BLOCK, NoTape, (F & 1) != 0, (F & 2) != 0>(P, L, park_w, stk, tape);
-        }
+        if (more) park<BLOCK>(park_w, L);
+        while (more) more = lane_step<BLOCK, NoTape, (F & 1) != 0, (F & 2) != 0>(P, L, park_w, stk, tape) == STEP_MORE;
         lane_finish<BLOCK>(P, L, park_w);
         hit = (L.p.flagmask & P.hit_mask) != 0u;
     }
@@ -392,11 +409,10 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_wave(SimParams P)
 #endif
         OA_CYC_ADD(OA_ST_C_REFILL, c_iter);
         if (active) {
-            if (lane_step<BLOCK, T, (F & 1) != 0, (F & 2) != 0>(P, L, park_w, stk, tape)) {
+            if (lane_step<BLOCK, T, (F & 1) != 0, (F & 2) != 0>(P, L, park_w, stk, tape,
+                                                                exhausted ? OA_WALK_MIN_TAIL : OA_WALK_MIN) == STEP_DONE) {
                 finish(L);
                 active = false;
-            } else {
-                park<BLOCK>(park_w, L);
             }
         }
         OA_CYC_ADD(OA_ST_C_ITER, c_iter);
@@ -582,10 +598,9 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_adjoint_wave(SimParams P, AdjP
             if (exhausted) break;
             continue;
         }
-        if (active) {
-            active = !lane_step<BLOCK, ScoreTape, false, EXT>(P, L, park_w, stk, tape);
-            park<BLOCK>(park_w, L);
-        }
+        if (active)
+            active = lane_step<BLOCK, ScoreTape, false, EXT>(P, L, park_w, stk, tape,
+                                                             exhausted ? OA_WALK_MIN_TAIL : OA_WALK_MIN) != STEP_DONE;
     }
 }
 

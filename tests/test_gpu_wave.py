@@ -100,3 +100,17 @@ def test_front_solids_match_checker(kind):
     assert np.array_equal(sim.seq, seq)
     assert np.array_equal(sim.photon.view(np.uint32), photon.view(np.uint32))
     sim.close()
+
+
+# the smallest events (one wave, partly filled), a wave and a lane, and enough photons for
+# refills to mix lanes that wait for the instance walk with fresh ones
+@pytest.mark.parametrize("n", [1, 63, 65, 4097, 600_001])
+@pytest.mark.parametrize("batch", [1, 16, 64])
+def test_waiting_lanes_keep_results(n, batch):
+    w = configs.config1(num_gs=1, per_gs=n)
+    sim = QSim(w.geometry, w.physics, SEventConfig(seed=7, refill_batch=batch))
+    sim.simulate(w.gensteps, 3)
+    photon, seq = po.World(w.geometry, w.physics).simulate(w.gensteps, event_idx=3, seed=7)
+    assert np.array_equal(sim.seq, seq)
+    assert np.array_equal(sim.photon.view(np.uint32), photon.view(np.uint32))
+    sim.close()
