@@ -90,7 +90,8 @@ enum : uint32_t {
     F_SURFACE_DREFLECT = 0x1u << 8, F_SURFACE_SREFLECT = 0x1u << 9,
     F_BOUNDARY_REFLECT = 0x1u << 10, F_BOUNDARY_TRANSMIT = 0x1u << 11
 };
-enum : int { CMD_BREAK = 1, CMD_CONTINUE = 2, CMD_BOUNDARY = 3 };
+enum : int { CMD_BREAK = 1, CMD_CONTINUE = 2, CMD_BOUNDARY = 3,
+             CMD_REEMIT = 4, CMD_SCATTER = 5 };   /* the photon's new direction is still to be drawn (redirect) */
 enum : int { EMS_NOSURFACE = 1, EMS_SURFACE = 2, EMS_ZPLUS_SENSOR_A = 3 };
 enum : uint32_t { TC_ZERO = 0, TC_UNION = 1, TC_INTERSECTION = 2, TC_DIFFERENCE = 3, TC_NODE = 11,
                   TC_CONTIGUOUS = 11, TC_DISCONTIGUOUS = 12, TC_OVERLAP = 13,

@@ -212,39 +212,55 @@ OA_D void lambertian(v3& dir, v3 normal, float orient, R& rng)
     } while (!(u < ndotv) && (count < 1024));
 }
 
-template <class R>
-OA_D void rayleigh(Photon& p, R& rng)
+/* one trial of the rejection loop of qsim::rayleigh_scatter: whether it is accepted, and the
+   direction and polarization it proposes */
+OA_D bool rayleigh_trial(const Photon& p, const float (&u)[5], v3& direction, v3& polarization)
 {
+    const float u0 = u[0], u1 = u[1], u2 = u[2], u3 = u[3], u4 = u[4];
+    float cosTheta = u0;
+    float sinTheta = sqrtf(1.0f - u0 * u0);
+    if (u1 < 0.5f) cosTheta = -cosTheta;
+    float sinPhi, cosPhi;
+    oa_sincosf(2.f * OA_PI_F * u2, &sinPhi, &cosPhi);
+    direction = mk(sinTheta * cosPhi, sinTheta * sinPhi, cosTheta);
+    rotateUz(direction, p.mom);
+    float constant = -dot(direction, p.pol);
+    polarization = mk(p.pol.x + constant * direction.x, p.pol.y + constant * direction.y,
+                      p.pol.z + constant * direction.z);
+    if (dot(polarization, polarization) == 0.f) {
+        oa_sincosf(2.f * OA_PI_F * u3, &sinPhi, &cosPhi);
+        polarization = mk(cosPhi, sinPhi, 0.f);
+        rotateUz(polarization, direction);
+    } else {
+        if (u3 < 0.5f) polarization = -polarization;
+    }
+    polarization = normalize(polarization);
+    float doCosTheta = dot(polarization, p.pol);
+    return !(doCosTheta * doCosTheta < u4);
+}
+
+/* the new direction of a reemitted photon, or one trial of a scattered one's (the trial-th,
+   from 0): false when another trial is needed */
+template <class R>
+OA_D bool redirect(const SimParams& P, int command, int trial, uint32_t& flag, R& rng, Photon& p)
+{
+    float u[5];
+    draw<5>(rng, u);
+    if (command == CMD_REEMIT) {        /* wavelength, direction (2), polarization (2) */
+        p.wavelength = scint_wavelength(P, u[0]);
+        p.mom = uniform_sphere(u[1], u[2]);
+        p.pol = normalize(cross(uniform_sphere(u[3], u[4]), p.mom));
+        flag = F_BULK_REEMIT;
+        return true;
+    }
     v3 direction, polarization;
-    bool looping = true;
-    int trials = 0;
-    do {
-        float u[5];
-        draw<5>(rng, u);
-        const float u0 = u[0], u1 = u[1], u2 = u[2], u3 = u[3], u4 = u[4];
-        float cosTheta = u0;
-        float sinTheta = sqrtf(1.0f - u0 * u0);
-        if (u1 < 0.5f) cosTheta = -cosTheta;
-        float sinPhi, cosPhi;
-        oa_sincosf(2.f * OA_PI_F * u2, &sinPhi, &cosPhi);
-        direction = mk(sinTheta * cosPhi, sinTheta * sinPhi, cosTheta);
-        rotateUz(direction, p.mom);
-        float constant = -dot(direction, p.pol);
-        polarization = mk(p.pol.x + constant * direction.x, p.pol.y + constant * direction.y,
-                          p.pol.z + constant * direction.z);
-        if (dot(polarization, polarization) == 0.f) {
-            oa_sincosf(2.f * OA_PI_F * u3, &sinPhi, &cosPhi);
-            polarization = mk(cosPhi, sinPhi, 0.f);
-            rotateUz(polarization, direction);
-        } else {
-            if (u3 < 0.5f) polarization = -polarization;
-        }
-        polarization = normalize(polarization);
-        float doCosTheta = dot(polarization, p.pol);
-        looping = doCosTheta * doCosTheta < u4;
-    } while (looping && ++trials < OA_MAX_TRIALS);
-    p.mom = direction;
-    p.pol = polarization;
+    const bool accepted = rayleigh_trial(p, u, direction, polarization) || trial + 1 >= OA_MAX_TRIALS;
+    if (accepted) {
+        p.mom = direction;
+        p.pol = polarization;
+        flag = F_BULK_SCATTER;
+    }
+    return accepted;
 }
 
 /* ----------------------------------------------------------- physics */
@@ -275,24 +291,14 @@ OA_D int to_boundary(const SimParams& P, uint32_t& flag, R& rng, Photon& p, cons
             p.time += absorption_distance / gv;
             p.pos = p.pos + absorption_distance * p.mom;
             float u_reemit = reemission_prob == 0.f ? 2.f : maybe_third(rng, third);
-            if (u_reemit < reemission_prob) {
-                float u[5];     /* wavelength, direction (2), polarization (2) */
-                draw<5>(rng, u);
-                p.wavelength = scint_wavelength(P, u[0]);
-                p.mom = uniform_sphere(u[1], u[2]);
-                p.pol = normalize(cross(uniform_sphere(u[3], u[4]), p.mom));
-                flag = F_BULK_REEMIT;
-                return CMD_CONTINUE;
-            }
+            if (u_reemit < reemission_prob) return CMD_REEMIT;
             flag = F_BULK_ABSORB;
             return CMD_BREAK;
         }
     } else if (scattering_distance <= dist) {
         p.time += scattering_distance / gv;
         p.pos = p.pos + scattering_distance * p.mom;
-        rayleigh(p, rng);
-        flag = F_BULK_SCATTER;
-        return CMD_CONTINUE;
+        return CMD_SCATTER;
     }
     p.pos = p.pos + dist * p.mom;
     p.time += dist / gv;
@@ -367,8 +373,10 @@ OA_D int at_surface(uint32_t& flag, R& rng, MaybeThird third, Photon& p, const S
     return action;
 }
 
+/* up to the photon's fate in this step; CMD_REEMIT and CMD_SCATTER leave its new direction
+   and flag to redirect() */
 template <class R, class Tape>
-OA_D int propagate(const SimParams& P, R& rng, Photon& p, const Prd& prd, Tape& tape)
+OA_D int propagate(const SimParams& P, uint32_t& flag, R& rng, Photon& p, const Prd& prd, Tape& tape)
 {
     const uint32_t boundary = prd.boundary;
     const uint32_t identity = prd.iindex_identity & 0xffffu;
@@ -382,7 +390,6 @@ OA_D int propagate(const SimParams& P, R& rng, Photon& p, const Prd& prd, Tape& 
     p.hitcount_iindex = 0x00010000u | (0x0000ffffu & iindex);
     State s;
     fill(P, s, boundary, p.wavelength, cosTheta);
-    uint32_t flag = 0u;
     MaybeThird third;
     int command = to_boundary(P, flag, rng, p, s, prd.t, tape, third);
     if (command == CMD_BOUNDARY) {
@@ -391,7 +398,6 @@ OA_D int propagate(const SimParams& P, R& rng, Photon& p, const Prd& prd, Tape& 
         else if (prd.lposcost < 0.f) command = at_surface(flag, rng, third, p, s, normal);
         else if (s.ems == EMS_ZPLUS_SENSOR_A) { (void)maybe_third(rng, third); flag = F_SURFACE_DETECT; command = CMD_BREAK; }
     }
-    set_flag(p, flag);
     return command;
 }
 
@@ -802,12 +808,13 @@ OA_D void trace_front(const SimParams& P, v3 o, v3 d, float tmin, float& best_t,
  * code executes with most lanes of the wave active instead of once per lane.
  *
  * Returns false, with nothing found out, for a lane that needs the TLAS walk while fewer
- * than walk_min lanes of the wave do and some lane does not: it is traced again, front
- * instances included, with its wave's next step (they are tested on the whole wave anyway).
- * Such a wave always has a lane whose trace ended, so it gets on.
+ * than walk_min lanes of the wave do and some lane does not, or others of the wave have
+ * something else to do (`others`): it is traced again, front instances included, with its
+ * wave's next step (they are tested on the whole wave anyway). Such a wave always has a
+ * lane that gets on.
  */
 template <int STRIDE, bool EXT = false>
-OA_D bool trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float tmax, Prd& prd, int walk_min = 0)
+OA_D bool trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float tmax, Prd& prd, int walk_min = 0, bool others = false)
 {
     OA_COUNT(OA_ST_TRACE);
     OA_WAVE_COUNT(OA_ST_W_TRACE, OA_ST_L_TRACE);
@@ -833,7 +840,7 @@ OA_D bool trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float
         /* the TLAS walk and the CSG trees behind it run for as long as their slowest lane:
            lanes that need them wait for company while others of the wave have a step to do */
         const unsigned long long walkers = __ballot(!done);
-        if (__popcll(walkers) < walk_min && walkers != __ballot(1)) {
+        if (__popcll(walkers) < walk_min && (others || walkers != __ballot(1))) {
             if (!done) return false;
         }
     }

@@ -41,6 +41,7 @@ struct Lane {
     Photon p;
     R rng;
     int bounce;
+    int trial;                    /* Rayleigh trials made of a scatter that has none accepted yet (lane_step) */
     int64_t g;
     LiteState<LITE> lite;
 };
@@ -67,6 +68,7 @@ template <> struct index_word<XorwowRng> { static constexpr int value = 6; };
 /* LDS words of a lane's parked state */
 template <class R> struct park_words { static constexpr int value = PK_RNG + 4; };
 template <> struct park_words<XorwowRng> { static constexpr int value = PK_RNG + 7; };
+#define OA_LITE_WORDS 3      /* the lite instantiations also park the last trace's local position */
 
 template <int STRIDE> OA_D void park_fixed(uint32_t* w, const PhiloxRng& r)
 {
@@ -115,10 +117,14 @@ OA_D void park(uint32_t* w, const Lane<R, LITE>& L)
     w[PK_POLZ * STRIDE] = fbits(L.p.pol.z);
     w[PK_WL * STRIDE] = fbits(L.p.wavelength);
     w[PK_IDENT * STRIDE] = L.p.identity;
-    w[PK_MASK * STRIDE] = L.p.flagmask;
+    w[PK_MASK * STRIDE] = L.p.flagmask | ((uint32_t)L.trial << 16);    /* flags are 16 bits, trials fewer than 2^16 */
     w[PK_HITCOUNT * STRIDE] = L.p.hitcount_iindex;
     w[PK_BOUNCE * STRIDE] = (uint32_t)L.bounce;
     park_rng<STRIDE>(w + PK_RNG * STRIDE, L.rng);
+    if constexpr (LITE) {
+        uint32_t* k = w + park_words<R>::value * STRIDE;
+        k[0] = fbits(L.lite.lcost); k[STRIDE] = fbits(L.lite.lx); k[2 * STRIDE] = fbits(L.lite.ly);
+    }
     /* the values above are not carried over a trace in registers */
     asm volatile("" ::: "memory");
 }
@@ -131,10 +137,15 @@ OA_D void unpark(const SimParams& P, const uint32_t* w, Lane<R, LITE>& L)
                  __uint_as_float(w[PK_POLZ * STRIDE]));
     L.p.wavelength = __uint_as_float(w[PK_WL * STRIDE]);
     L.p.identity = w[PK_IDENT * STRIDE];
-    L.p.flagmask = w[PK_MASK * STRIDE];
+    L.p.flagmask = w[PK_MASK * STRIDE] & 0xffffu;
+    L.trial = (int)(w[PK_MASK * STRIDE] >> 16);
     L.p.hitcount_iindex = w[PK_HITCOUNT * STRIDE];
     L.bounce = (int)w[PK_BOUNCE * STRIDE];
     unpark_rng<STRIDE>(P, w + PK_RNG * STRIDE, L.rng);
+    if constexpr (LITE) {
+        const uint32_t* k = w + park_words<R>::value * STRIDE;
+        L.lite.lcost = __uint_as_float(k[0]); L.lite.lx = __uint_as_float(k[STRIDE]); L.lite.ly = __uint_as_float(k[2 * STRIDE]);
+    }
 }
 
 /* photon index of the launch: written at the start, read where the photon ends */
@@ -227,6 +238,7 @@ OA_D bool lane_start(const SimParams& P, Lane<R, LITE>& L, int64_t g, uint32_t* 
     /* sphoton::set_index (sysrap/sphoton.h:230-237); the index word is parked below */
     L.p.identity = ((uint32_t)((photon_idx >> 32) & 0xffu) << 24) | (L.p.identity & 0xffffffu);
     L.bounce = 0;
+    L.trial = 0;
     if constexpr (LITE) { L.lite.lcost = 0.f; L.lite.lx = 0.f; L.lite.ly = __uint_as_float(0x7fc00000u); }
     w[PK_G * STRIDE] = (uint32_t)g;
     w[PK_G_HI * STRIDE] = (uint32_t)((uint64_t)g >> 32);
@@ -256,26 +268,52 @@ OA_D bool lane_start(const SimParams& P, Lane<R, LITE>& L, int64_t g, uint32_t* 
 #define OA_WALK_MIN_TAIL 8
 #endif
 
-/* one iteration of the CSGOptiX7.cu:477-509 loop from the parked state w, parked again for
-   the next (STEP_MORE) or not (STEP_DONE: the photon ended); STEP_WAITS: nothing was done */
+/*
+ * One iteration of the CSGOptiX7.cu:477-509 loop from the parked state w, parked again for
+ * the next (STEP_MORE) or not (STEP_DONE: the photon ended); STEP_WAITS: nothing was done.
+ *
+ * A Rayleigh scatter draws trials until one is accepted, a third of them fail. They are made
+ * one an iteration (`scattering`: some were made, none accepted yet): a lane whose trial fails
+ * makes its next one with the lanes that scatter in the wave's next step, where a loop in
+ * place ran until the unluckiest lane of the wave was done.
+ */
 enum : int { STEP_MORE, STEP_DONE, STEP_WAITS };
 template <int STRIDE, class Tape, bool LITE, bool EXT, class R>
-OA_D int lane_step(const SimParams& P, Lane<R, LITE>& L, uint32_t* w, uint32_t* stk, Tape& tape, int walk_min = 0)
+OA_D int lane_step(const SimParams& P, Lane<R, LITE>& L, uint32_t* w, uint32_t* stk, Tape& tape, bool& scattering,
+                   int walk_min = 0)
 {
-    const float tmin = (L.p.obf & P.eps0_mask) ? P.tmin0 : P.tmin;
     Prd prd;
-    const bool traced = trace<STRIDE, EXT>(P, stk, L.p.pos, L.p.mom, tmin, P.tmax, prd, walk_min);
+    bool traced = true;
+    const bool others = __ballot(scattering) != 0ull;
+    if (!scattering) {
+        const float tmin = (L.p.obf & P.eps0_mask) ? P.tmin0 : P.tmin;
+        traced = trace<STRIDE, EXT>(P, stk, L.p.pos, L.p.mom, tmin, P.tmax, prd, walk_min, others);
+    }
     asm volatile("" ::: "memory");
     unpark<STRIDE>(P, w, L);                      /* by waiting lanes too: their old values need not outlive the trace */
     if (!traced) return STEP_WAITS;
     L.g = parked_g<STRIDE>(w);
-    if constexpr (LITE) { L.lite.lcost = prd.lposcost; L.lite.lx = prd.lx; L.lite.ly = prd.ly; }
-    if (prd.boundary == 0xffffu) return STEP_DONE;
-    prd.normal = normalize(prd.normal);
-    OA_COUNT(OA_ST_STEP);
-    OA_WAVE_COUNT(OA_ST_W_PHYS, OA_ST_L_PHYS);
-    tape.at(P, L.g, L.bounce);
-    const int command = propagate(P, L.rng, L.p, prd, tape);
+    uint32_t flag = 0u;
+    int command = CMD_SCATTER;
+    if (!scattering) {
+        if constexpr (LITE) { L.lite.lcost = prd.lposcost; L.lite.lx = prd.lx; L.lite.ly = prd.ly; }
+        if (prd.boundary == 0xffffu) return STEP_DONE;
+        prd.normal = normalize(prd.normal);
+        OA_COUNT(OA_ST_STEP);
+        OA_WAVE_COUNT(OA_ST_W_PHYS, OA_ST_L_PHYS);
+        tape.at(P, L.g, L.bounce);
+        command = propagate(P, flag, L.rng, L.p, prd, tape);
+    }
+    if (command >= CMD_REEMIT) {
+        scattering = !redirect(P, command, L.trial, flag, L.rng, L.p);
+        if (scattering) {
+            L.trial++;
+            park<STRIDE>(w, L);
+            return STEP_MORE;
+        }
+        L.trial = 0;
+    }
+    set_flag(L.p, flag);
     L.bounce++;
     if constexpr (Tape::keeps_seq) seq_add<STRIDE>(w, (unsigned)L.bounce, ph_flag(L.p), ph_boundary(L.p));
     if (command == CMD_BREAK || !lane_alive(P, L)) return STEP_DONE;
@@ -323,9 +361,9 @@ OA_D void lane_finish(const SimParams& P, const Lane<R, LITE>& L, const uint32_t
 }
 
 /* LDS bytes of a block: parked words and traversal stack of each thread */
-template <class R> inline unsigned block_lds(int block, int stack_depth)
+template <class R> inline unsigned block_lds(int block, int stack_depth, bool lite = false)
 {
-    return (unsigned)(park_words<R>::value + stack_depth) * 4u * (unsigned)block;
+    return (unsigned)(park_words<R>::value + (lite ? OA_LITE_WORDS : 0) + stack_depth) * 4u * (unsigned)block;
 }
 
 } // namespace oa
@@ -338,7 +376,7 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_plain(SimParams P)
     using namespace oa;
     extern __shared__ uint32_t s_lane[];           /* each lane's parked words, then its stack */
     uint32_t* park_w = s_lane + threadIdx.x;
-    uint32_t* stk = park_w + park_words<R>::value * BLOCK;
+    uint32_t* stk = park_w + (park_words<R>::value + ((F & 1) ? OA_LITE_WORDS : 0)) * BLOCK;
     const int64_t g = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     bool hit = false;
     if (g < P.n_photon) {
@@ -346,7 +384,8 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_plain(SimParams P)
         NoTape tape;
         bool more = lane_start<BLOCK, NoTape>(P, L, g, park_w);
         if (more) park<BLOCK>(park_w, L);
-        while (more) more = lane_step<BLOCK, NoTape, (F & 1) != 0, (F & 2) != 0>(P, L, park_w, stk, tape) == STEP_MORE;
+        bool scattering = false;
+        while (more) more = lane_step<BLOCK, NoTape, (F & 1) != 0, (F & 2) != 0>(P, L, park_w, stk, tape, scattering) == STEP_MORE;
         lane_finish<BLOCK>(P, L, park_w);
         hit = (L.p.flagmask & P.hit_mask) != 0u;
     }
@@ -362,11 +401,12 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_wave(SimParams P)
     using namespace oa;
     extern __shared__ uint32_t s_lane[];           /* each lane's parked words, then its stack */
     uint32_t* park_w = s_lane + threadIdx.x;
-    uint32_t* stk = park_w + park_words<R>::value * BLOCK;
+    uint32_t* stk = park_w + (park_words<R>::value + ((F & 1) ? OA_LITE_WORDS : 0)) * BLOCK;
     const int lane = threadIdx.x & 63;
     Lane<R, (F & 1) != 0> L;
     T tape;
     bool active = false;
+    bool scattering = false;
     bool exhausted = false;
     const int period = P.refill_period > 0 ? P.refill_period : 1;
     /* lanes refill together once `batch` of them are idle: photons started in the
@@ -409,7 +449,7 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_wave(SimParams P)
 #endif
         OA_CYC_ADD(OA_ST_C_REFILL, c_iter);
         if (active) {
-            if (lane_step<BLOCK, T, (F & 1) != 0, (F & 2) != 0>(P, L, park_w, stk, tape,
+            if (lane_step<BLOCK, T, (F & 1) != 0, (F & 2) != 0>(P, L, park_w, stk, tape, scattering,
                                                                 exhausted ? OA_WALK_MIN_TAIL : OA_WALK_MIN) == STEP_DONE) {
                 finish(L);
                 active = false;
@@ -564,6 +604,7 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_adjoint_wave(SimParams P, AdjP
     tape.row = S;
     Lane<R, false> L;
     bool active = false;
+    bool scattering = false;
     bool exhausted = n <= 0;
     const int batch = P.refill_batch > 1 ? P.refill_batch : 1;
     for (;;) {
@@ -599,7 +640,7 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_adjoint_wave(SimParams P, AdjP
             continue;
         }
         if (active)
-            active = lane_step<BLOCK, ScoreTape, false, EXT>(P, L, park_w, stk, tape,
+            active = lane_step<BLOCK, ScoreTape, false, EXT>(P, L, park_w, stk, tape, scattering,
                                                              exhausted ? OA_WALK_MIN_TAIL : OA_WALK_MIN) != STEP_DONE;
     }
 }

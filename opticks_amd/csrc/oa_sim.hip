@@ -25,7 +25,7 @@ namespace oa_launch {
 hipError_t OA_SIM_NAME(sim_launch, OA_SIM_BLOCK, OA_SIM_RNG)(const SimParams& P, int kernel, int grid, hipStream_t s)
 {
     constexpr int B = OA_SIM_BLOCK;
-    const unsigned lds = oa::block_lds<OA_SIM_R>(B, P.stack_depth);
+    const unsigned lds = oa::block_lds<OA_SIM_R>(B, P.stack_depth, P.photonlite != nullptr);
     const int f = (P.photonlite ? 1 : 0) | (P.ext_leaves ? 2 : 0);
     if (kernel == 0) {
         const unsigned nb = (unsigned)((P.n_photon + B - 1) / B);
@@ -52,7 +52,7 @@ hipError_t OA_SIM_NAME(sim_launch, OA_SIM_BLOCK, OA_SIM_RNG)(const SimParams& P,
 
 unsigned OA_SIM_NAME(sim_lds, OA_SIM_BLOCK, OA_SIM_RNG)(int stack_depth)
 {
-    return oa::block_lds<OA_SIM_R>(OA_SIM_BLOCK, stack_depth);
+    return oa::block_lds<OA_SIM_R>(OA_SIM_BLOCK, stack_depth, true);
 }
 
 int OA_SIM_NAME(sim_occupancy, OA_SIM_BLOCK, OA_SIM_RNG)(int stack_depth)
