@@ -170,7 +170,7 @@ typedef struct mi_event_out {
     const float*    photon;     /* (n_photon,4,4) or NULL when not in output_mask */
     const uint64_t* seq;        /* (n_photon,2,2) or NULL */
     const float*    hit;        /* (n_hit,4,4)    or NULL */
-    double          device_ms;  /* seeding -> hit compaction, HIP events */
+    double          device_ms;  /* seeding -> hit compaction, device clock */
 } mi_event_out;
 
 void        mi_config_default(mi_config* cfg);
@@ -197,8 +197,8 @@ int  mi_sim_reset(mi_sim* sim, int32_t event_id);
 /*
  * Device-resident form. d_gensteps: (n_gs,6,4) in device memory.
  * n_photon: photons to propagate, at most the gensteps' total (a smaller
- * count propagates that prefix), or -1 for the total; the total is read back
- * (8 bytes) and a larger n_photon fails with MI_ERR_ARG.
+ * count propagates that prefix), or -1 for the total; a larger n_photon fails
+ * with MI_ERR_ARG and propagates nothing.
  * d_photon (n_photon,4,4), d_seq (n_photon,2,2) u64, d_hit (hit_capacity,4,4):
  * caller-owned device buffers; any may be NULL to skip that output.
  * photon_offset: absolute index of the first photon (multi-launch slicing,
@@ -309,7 +309,7 @@ int  mi_sim_simtrace(mi_sim* sim, const float* gensteps, int64_t n_gs,
 /* Replace instance transforms (n_inst,4,4) and refit the TLAS on the GPU. */
 int  mi_sim_refit_instances(mi_sim* sim, const float* inst, int64_t n_inst);
 
-/* Last launch timings in ms (HIP events): [seed, propagate, compact, total]. */
+/* Last launch timings in ms (device clock; HIP events for batches): [seed, propagate, compact, total]. */
 int  mi_sim_last_timing(const mi_sim* sim, double* ms4);
 
 /* Replace the boundary table values (host array, the shape given at create). */

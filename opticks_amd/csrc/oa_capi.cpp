@@ -164,10 +164,15 @@ struct mi_sim {
 
     /* work */
     DBuf<float> gs;
-    DBuf<int64_t> prefix, block_total, evbuf;
+    DBuf<int64_t> prefix, tile_base, evbuf, n_dev;
     DBuf<int32_t> word_prefix, ev_id, gs_event;
     DBuf<uint32_t> seed;                 /* genstep of each photon of the launch */
-    DBuf<unsigned long long> words, next;
+    DBuf<unsigned long long> words;      /* oa_launch::clear_words of the launch */
+    DBuf<unsigned long long> next;       /* photon counter of the adjoint replay */
+    LaunchResult* result = nullptr;      /* pinned: the last launch's counts and clock */
+    double clock_ms = 1e-5;              /* device wall clock tick */
+    int64_t photon_cap = 0;              /* photons the single-event buffers hold (launch_reserve) */
+    int grid_key[3] = { -1, -1, -1 }, grid_blocks = 0;   /* wave_grid's last answer */
     /* outputs of the host-array entry point */
     DBuf<float4> photon, hit;
     DBuf<uint64_t> seq;
@@ -180,7 +185,7 @@ struct mi_sim {
     struct TapeKey {
         bool valid = false;
         int32_t event_id = 0, k = 0;
-        int64_t photon_offset = 0, n_photon = 0, n_gs = 0;
+        int64_t photon_offset = 0, n_photon = 0, stride = 0, n_gs = 0;
         const void* gs = nullptr;
         uint64_t generation = 0;
     } tape_key;
@@ -682,7 +687,12 @@ int mi_sim_create(const mi_geometry* geo, const mi_physics* phys, const mi_confi
     if (!rc) rc = upload_physics(sim, phys);
     if (!rc) rc = apply_config(sim, &c, true);
     if (!rc) {
-        rc = sim->next.reserve(1) == hipSuccess ? MI_OK : fail(MI_ERR_HIP, "alloc counter");
+        int khz = 0;
+        if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, sim->device) == hipSuccess && khz > 0)
+            sim->clock_ms = 1.0 / khz;
+        rc = sim->next.reserve(1) == hipSuccess && sim->n_dev.reserve(2) == hipSuccess &&
+                     hipHostMalloc((void**)&sim->result, sizeof(LaunchResult), hipHostMallocDefault) == hipSuccess
+                 ? MI_OK : fail(MI_ERR_HIP, "alloc counters");
     }
     if (!rc) {
         hipError_t e = oa_launch::noalloc_scratch(sim->device, &sim->scratch);
@@ -703,7 +713,8 @@ void mi_sim_destroy(mi_sim* sim)
     sim->tlas.release(); sim->blas.release(); sim->tlas_items.release(); sim->blas_prims.release();
     sim->inst_box.release(); sim->free_ball.release();
     sim->bnd.release(); sim->optical.release(); sim->icdf.release(); sim->precooked.release();
-    sim->gs.release(); sim->prefix.release(); sim->block_total.release(); sim->evbuf.release();
+    sim->gs.release(); sim->prefix.release(); sim->tile_base.release(); sim->evbuf.release(); sim->n_dev.release();
+    if (sim->result) (void)hipHostFree(sim->result);
     sim->word_prefix.release(); sim->ev_id.release(); sim->words.release(); sim->next.release();
     sim->seed.release(); sim->gs_event.release();
     sim->photon.release(); sim->hit.release(); sim->seq.release();
@@ -770,7 +781,7 @@ static int check_precooked_rows(const mi_sim* sim, int64_t end_index)
 /* xorwow: the jump matrix of each event's skip (offset + event_id * skipahead)
    uploaded into dst (n_event x 800 words); *table stays null for other generators */
 static int xorwow_table(mi_sim* sim, const int32_t* event_ids, int32_t n_event, DBuf<uint32_t>& dst,
-                        const uint32_t** table)
+                        const uint32_t** table, hipStream_t s)
 {
     *table = nullptr;
     if (sim->cfg.rng_kind != MI_RNG_XORWOW) return MI_OK;
@@ -788,7 +799,7 @@ static int xorwow_table(mi_sim* sim, const int32_t* event_ids, int32_t n_event, 
         }
         std::copy(it->second.begin(), it->second.end(), h.begin() + (size_t)e * OA_XORWOW_JUMP_WORDS);
     }
-    HIPCHECK(upload(dst, h.data(), h.size(), sim->stream));
+    HIPCHECK(upload(dst, h.data(), h.size(), s));
     *table = dst.p;
     return MI_OK;
 }
@@ -805,15 +816,22 @@ static int sim_block(const mi_sim* sim)
 
 /* persistent grid: every resident slot of every CU (occupancy API), or the
    configured waves per CU */
-static int wave_grid(const mi_sim* sim)
+static int wave_grid(mi_sim* sim)
 {
     const int block = sim_block(sim);
     const int waves_per_block = block / 64;
     if (sim->cfg.waves_per_cu > 0) return std::max(1, sim->n_cu * sim->cfg.waves_per_cu / waves_per_block);
-    int nb = oa_launch::wave_blocks_per_cu(block, sim->cfg.rng_kind, sim->stack_depth);
-    if (nb <= 0) nb = std::max(1, 8 / waves_per_block);
-    return std::max(1, sim->n_cu * nb);
+    const int key[3] = { block, sim->cfg.rng_kind, sim->stack_depth };
+    if (std::memcmp(key, sim->grid_key, sizeof(key)) != 0) {
+        int nb = oa_launch::wave_blocks_per_cu(block, sim->cfg.rng_kind, sim->stack_depth);
+        if (nb <= 0) nb = std::max(1, 8 / waves_per_block);
+        sim->grid_blocks = std::max(1, sim->n_cu * nb);
+        std::memcpy(sim->grid_key, key, sizeof(key));
+    }
+    return sim->grid_blocks;
 }
+
+static int64_t wave_count(mi_sim* sim) { return (int64_t)wave_grid(sim) * (sim_block(sim) / 64); }
 
 /*
  * One propagation launch over gensteps already on the device with a
@@ -822,34 +840,31 @@ static int wave_grid(const mi_sim* sim)
  */
 static int launch(mi_sim* sim, SimParams& P, hipStream_t s)
 {
-    const int64_t n_words = (P.n_photon + 63) / 64;
-    HIPCHECK(sim->words.reserve((size_t)n_words + 1));
+    HIPCHECK(sim->words.reserve((size_t)oa_launch::clear_words(P.n_photon)));
     P.hitwords = sim->words.p;
+    P.next = sim->words.p + oa_launch::next_offset(P.n_photon);
     HIPCHECK(sim->seed.reserve((size_t)P.n_photon));
     HIPCHECK(sim->gs_event.reserve((size_t)std::max<int64_t>(P.n_gs, 1)));
     HIPCHECK(oa_launch::seed_map(P.gs_prefix, P.n_gs, P.n_photon, sim->seed.p, P.ev_gs_begin, P.n_event,
                                  sim->gs_event.p, s));
     P.seed_map = sim->seed.p;
     P.gs_event = sim->gs_event.p;
-    if (sim->cfg.kernel == MI_KERNEL_WAVEFRONT) {
-        HIPCHECK(oa_launch::zero_u64(sim->words.p, n_words, s));
-        HIPCHECK(oa_launch::zero_u64(sim->next.p, 1, s));
-    }
+    P.wave_width = (int32_t)wave_width(P.n_photon, wave_count(sim));
+    HIPCHECK(oa_launch::clear_launch(sim->words.p, P.n_photon, wave_count(sim), s));
     HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s));
     return MI_OK;
 }
 
-/* stable hit compaction; the hit count lands in block_total[nb], read after the end event */
-static int compact(mi_sim* sim, int64_t n_photon, const float4* d_photon, float4* d_hit, int64_t hit_cap,
-                   int64_t** d_count, hipStream_t s)
+/* buffers of a single-event launch of up to n photons; kept, and grown as events need */
+static int launch_reserve(mi_sim* sim, int64_t n)
 {
-    const int64_t n_words = (n_photon + 63) / 64;
-    const int64_t nb = (n_words + 255) / 256;
-    HIPCHECK(sim->word_prefix.reserve((size_t)n_words + 1));
-    HIPCHECK(sim->block_total.reserve((size_t)nb + 1));
-    HIPCHECK(oa_launch::compact_hits(sim->words.p, n_words, sim->word_prefix.p, sim->block_total.p,
-                                     d_photon, d_hit, hit_cap, s));
-    *d_count = sim->block_total.p + nb;
+    if (n <= sim->photon_cap) return MI_OK;
+    const size_t nw = (size_t)((n + 63) / 64);
+    HIPCHECK(sim->words.reserve((size_t)oa_launch::clear_words(n)));
+    HIPCHECK(sim->seed.reserve((size_t)n));
+    HIPCHECK(sim->word_prefix.reserve(nw + 1));
+    HIPCHECK(sim->tile_base.reserve((size_t)oa_launch::compact_tiles(n) + 1));
+    sim->photon_cap = n;
     return MI_OK;
 }
 
@@ -863,33 +878,38 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
     if (!d_gensteps) return fail(MI_ERR_ARG, "null gensteps");
     if (d_hit && !d_photon) return fail(MI_ERR_ARG, "hits are gathered from the photon array: pass d_photon");
     hipStream_t s = stream ? (hipStream_t)stream : sim->stream;
-    HIPCHECK(hipEventRecord(sim->ev[0], s));
-    HIPCHECK(sim->prefix.reserve((size_t)n_gs + 1));
-    HIPCHECK(oa_launch::gs_prefix((const float*)d_gensteps, n_gs, sim->prefix.p, s));
-    std::vector<int64_t> hprefix;
+    sim->tape_key.valid = false;
+    HIPCHECK(sim->prefix.reserve((size_t)oa_launch::gs_prefix_words(n_gs)));
+    HIPCHECK(sim->evbuf.reserve(4));
+    HIPCHECK(sim->ev_id.reserve(1));
     const int64_t max_slot = sim->cfg.max_slot;
-    int64_t total = 0;
-    if (max_slot > 0) {
+    const auto too_many = [&](int64_t total) {
+        return fail(MI_ERR_ARG, "n_photon " + std::to_string(n_photon) + " exceeds the gensteps' " +
+                                    std::to_string(total) + " photons");
+    };
+    /* The gensteps' photons are counted on the device, and a launch on them does not wait for
+       the host to know: its buffers are sized for the caller's count, or for the largest event
+       so far, and the host sees afterwards whether that held. It waits for the count first
+       where it decides something: slices, rows of precooked uniforms, the plain kernel's grid,
+       and where there was no event so far. */
+    std::vector<int64_t> hprefix;
+    if (max_slot > 0 || (n_photon < 0 && (sim->photon_cap == 0 || sim->cfg.rng_kind == MI_RNG_PRECOOKED ||
+                                           sim->cfg.kernel == MI_KERNEL_PLAIN))) {
+        HIPCHECK(oa_launch::gs_prefix((const float*)d_gensteps, n_gs, sim->prefix.p, s));
         hprefix.resize((size_t)n_gs + 1);
         HIPCHECK(hipMemcpyAsync(hprefix.data(), sim->prefix.p, sizeof(int64_t) * (n_gs + 1), hipMemcpyDeviceToHost, s));
         HIPCHECK(hipStreamSynchronize(s));
-        total = hprefix[n_gs];
-        if (n_photon >= 0 && n_photon != total)
+        const int64_t total = hprefix[n_gs];
+        if (max_slot > 0 && n_photon >= 0 && n_photon != total)
             return fail(MI_ERR_ARG, "with max_slot slicing n_photon must equal the gensteps' photons");
-    } else {
-        HIPCHECK(hipMemcpyAsync(&total, sim->prefix.p + n_gs, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        HIPCHECK(hipStreamSynchronize(s));
-        if (n_photon > total)
-            return fail(MI_ERR_ARG, "n_photon " + std::to_string(n_photon) + " exceeds the gensteps' " +
-                                        std::to_string(total) + " photons");
+        if (n_photon > total) return too_many(total);
+        if (n_photon < 0) n_photon = total;
     }
-    if (n_photon < 0) n_photon = total;
-    HIPCHECK(hipEventRecord(sim->ev[1], s));
     if (n_photon == 0) return fail(MI_NOTHING_TO_DO, "gensteps carry no photons");
-    int prc = check_precooked_rows(sim, photon_offset + n_photon);
+    int prc = n_photon > 0 ? check_precooked_rows(sim, photon_offset + n_photon) : MI_OK;
     if (prc) return prc;
     const uint32_t* xw_table = nullptr;
-    prc = xorwow_table(sim, &event_id, 1, sim->xw_jump, &xw_table);
+    prc = xorwow_table(sim, &event_id, 1, sim->xw_jump, &xw_table, s);
     if (prc) return prc;
     /* slices of whole gensteps with at most max_slot photons (sysrap/SGenstep.h:248) */
     std::vector<std::pair<int64_t, int64_t>> slices;
@@ -906,79 +926,82 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
     } else {
         slices.emplace_back(0, n_gs);
     }
+    const bool sliced = slices.size() > 1;
     /* adjoint tape: wavefront kernel, full photon records (not the lite form) */
     const int32_t K = sim->cfg.adjoint_tape;
     const bool taping = K > 0 && sim->cfg.kernel == MI_KERNEL_WAVEFRONT && !d_lite;
-    sim->tape_key.valid = false;
-    if (taping) {
-        HIPCHECK(sim->tape.reserve((size_t)n_photon * 3 * (size_t)K));
-        HIPCHECK(sim->tape_n.reserve((size_t)n_photon));
-    }
-    int64_t hits = 0;
-    double prop_ms = 0.0, comp_ms = 0.0;
+    int64_t hits = 0, tape_stride = 0;
+    double ms[4] = { 0.0, 0.0, 0.0, 0.0 };
+    const volatile LaunchResult* res = sim->result;
     for (auto& sl : slices) {
         const int64_t g0 = sl.first, g1 = sl.second;
-        const int64_t p0 = hprefix.empty() ? 0 : hprefix[g0];
-        const int64_t np = hprefix.empty() ? n_photon : hprefix[g1] - hprefix[g0];
-        if (slices.size() > 1) {
-            HIPCHECK(oa_launch::gs_prefix((const float*)d_gensteps + 24 * g0, g1 - g0, sim->prefix.p, s));
+        const int64_t p0 = sliced ? hprefix[g0] : 0;
+        const int64_t n_arg = sliced ? hprefix[g1] - hprefix[g0] : n_photon;
+        if (n_arg == 0) continue;
+        for (;;) {
+            int rc = launch_reserve(sim, std::max<int64_t>(n_arg, 1));
+            if (rc) return rc;
+            const int64_t cap = n_arg >= 0 ? n_arg : sim->photon_cap;
+            if (taping) {
+                if (tape_stride == 0 || !sliced) tape_stride = sliced ? n_photon : cap;
+                HIPCHECK(sim->tape.reserve((size_t)tape_stride * 3 * (size_t)K));
+                HIPCHECK(sim->tape_n.reserve((size_t)tape_stride));
+            }
+            const oa_launch::SetupArgs a = { (const float*)d_gensteps + 24 * g0, g1 - g0, n_arg, cap, sim->prefix.p,
+                                             sim->seed.p, sim->words.p, oa_launch::clear_words(cap), sim->evbuf.p,
+                                             sim->ev_id.p, event_id, sim->n_dev.p, sim->result, wave_count(sim) };
+            HIPCHECK(oa_launch::setup(a, s));
+            SimParams P = base_params(sim);
+            P.xw_jump = xw_table;
+            P.gensteps = (const float*)d_gensteps + 24 * g0;
+            P.gs_prefix = sim->prefix.p;
+            P.n_gs = g1 - g0;
+            P.n_event = 1;
+            P.ev_gs_begin = sim->evbuf.p;
+            P.ev_ph_begin = sim->evbuf.p + 2;
+            P.ev_id = sim->ev_id.p;
+            P.n_photon = cap;
+            P.n_dev = sim->n_dev.p;
+            P.seed_map = sim->seed.p;
+            P.photon_offset = photon_offset + p0;
+            P.photon = d_photon ? (float4*)d_photon + 4 * p0 : nullptr;
+            P.seq = d_seq ? (uint64_t*)d_seq + 4 * p0 : nullptr;
+            P.photonlite = d_lite ? (uint4*)d_lite + p0 : nullptr;
+            P.hitwords = sim->words.p;
+            P.next = sim->words.p + oa_launch::next_offset(cap);
+            if (taping) {
+                /* segment-major records with the whole launch's photon count as the stride */
+                P.tape = sim->tape.p + (size_t)p0 * 3;
+                P.tape_n = sim->tape_n.p + p0;
+                P.tape_stride = tape_stride;
+                P.tape_k = K;
+            }
+            HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s));
+            HIPCHECK(oa_launch::compact_hits(sim->words.p, cap, sim->n_dev.p, sim->word_prefix.p, sim->tile_base.p,
+                                             sim->words.p + oa_launch::state_offset(cap), P.photon,
+                                             d_hit ? (float4*)d_hit + 4 * hits : nullptr,
+                                             d_hit ? std::max<int64_t>(0, hit_capacity - hits) : 0, sim->result, s));
+            HIPCHECK(hipStreamSynchronize(s));
+            if (n_arg > res->total) return too_many(res->total);
+            if (n_arg >= 0 || res->total <= cap) break;
+            rc = launch_reserve(sim, res->total);        /* a larger event than any so far: once more */
+            if (rc) return rc;
         }
-        int64_t evh[4] = { 0, g1 - g0, 0, np };
-        int32_t evid = event_id;
-        HIPCHECK(sim->evbuf.reserve(4));
-        HIPCHECK(sim->ev_id.reserve(1));
-        HIPCHECK(hipMemcpyAsync(sim->evbuf.p, evh, sizeof(evh), hipMemcpyHostToDevice, s));
-        HIPCHECK(hipMemcpyAsync(sim->ev_id.p, &evid, sizeof(evid), hipMemcpyHostToDevice, s));
-        SimParams P = base_params(sim);
-        P.xw_jump = xw_table;
-        P.gensteps = (const float*)d_gensteps + 24 * g0;
-        P.gs_prefix = sim->prefix.p;
-        P.n_gs = g1 - g0;
-        P.n_event = 1;
-        P.ev_gs_begin = sim->evbuf.p;
-        P.ev_ph_begin = sim->evbuf.p + 2;
-        P.ev_id = sim->ev_id.p;
-        P.n_photon = np;
-        P.photon_offset = photon_offset + p0;
-        P.photon = d_photon ? (float4*)d_photon + 4 * p0 : nullptr;
-        P.seq = d_seq ? (uint64_t*)d_seq + 4 * p0 : nullptr;
-        P.photonlite = d_lite ? (uint4*)d_lite + p0 : nullptr;
-        if (taping) {
-            /* segment-major records with the whole launch's photon count as the stride */
-            P.tape = sim->tape.p + (size_t)p0 * 3;
-            P.tape_n = sim->tape_n.p + p0;
-            P.tape_stride = n_photon;
-            P.tape_k = K;
+        if (!sliced) {
+            n_photon = res->n_photon;
+            if (n_photon == 0) return fail(MI_NOTHING_TO_DO, "gensteps carry no photons");
         }
-        int rc = launch(sim, P, s);
-        if (rc) return rc;
-        HIPCHECK(hipEventRecord(sim->ev[2], s));
-        int64_t nh = 0;
-        int64_t* d_count = nullptr;
-        rc = compact(sim, np, P.photon, d_hit ? (float4*)d_hit + 4 * hits : nullptr,
-                     d_hit ? std::max<int64_t>(0, hit_capacity - hits) : 0, &d_count, s);
-        if (rc) return rc;
-        HIPCHECK(hipEventRecord(sim->ev[3], s));
-        HIPCHECK(hipMemcpyAsync(&nh, d_count, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        HIPCHECK(hipStreamSynchronize(s));
-        float a = 0.f, b = 0.f;
-        HIPCHECK(hipEventElapsedTime(&a, sim->ev[1], sim->ev[2]));
-        HIPCHECK(hipEventElapsedTime(&b, sim->ev[2], sim->ev[3]));
-        prop_ms += a; comp_ms += b;
-        HIPCHECK(hipEventRecord(sim->ev[1], s));
-        hits += nh;
+        hits += res->n_hit;
+        for (int i = 0; i < 3; ++i) ms[i] += sim->clock_ms * (double)(res->clock[i + 1] - res->clock[i]);
+        ms[3] += sim->clock_ms * (double)(res->clock[3] - res->clock[0]);
     }
     if (taping) {
         mi_sim::TapeKey& tk = sim->tape_key;
         tk.valid = true; tk.event_id = event_id; tk.k = K; tk.photon_offset = photon_offset;
-        tk.n_photon = n_photon; tk.n_gs = n_gs; tk.gs = d_gensteps; tk.generation = sim->generation;
+        tk.n_photon = n_photon; tk.stride = tape_stride; tk.n_gs = n_gs; tk.gs = d_gensteps;
+        tk.generation = sim->generation;
     }
-    sim->last_ms[1] = prop_ms;
-    sim->last_ms[2] = comp_ms;
-    float tot = 0.f;
-    HIPCHECK(hipEventElapsedTime(&tot, sim->ev[0], sim->ev[3]));
-    sim->last_ms[3] = tot;
-    sim->last_ms[0] = std::max(0.0, (double)tot - prop_ms - comp_ms);
+    for (int i = 0; i < 4; ++i) sim->last_ms[i] = ms[i];
     if (n_hit_out) *n_hit_out = hits;
     if (d_hit && hits > hit_capacity) return fail(MI_ERR_CAPACITY, "hit_capacity too small: " + std::to_string(hits) + " hits");
     return MI_OK;
@@ -1017,11 +1040,10 @@ int mi_sim_simulate_device_noalloc(mi_sim* sim, int32_t event_id, const void* d_
     int64_t* prefix = (int64_t*)(base + OA_NOALLOC_OFF_PREFIX);
     int64_t* ev = (int64_t*)(base + OA_NOALLOC_OFF_EV);
     int32_t* ev_id = (int32_t*)(base + OA_NOALLOC_OFF_EVID);
-    unsigned long long* next = (unsigned long long*)(base + OA_NOALLOC_OFF_NEXT);
     uint32_t* xw = (uint32_t*)(base + OA_NOALLOC_OFF_XW);
     unsigned long long* words = (unsigned long long*)(base + OA_NOALLOC_OFF_WORDS);
     int32_t* word_prefix = (int32_t*)(base + OA_NOALLOC_OFF_WPREFIX);
-    int64_t* block_total = (int64_t*)(base + OA_NOALLOC_OFF_BTOTAL);
+    int64_t* tile_base = (int64_t*)(base + OA_NOALLOC_OFF_BTOTAL);
     HIPCHECK(hipEventRecord(sim->ev[0], s));
     HIPCHECK(oa_launch::gs_prefix((const float*)d_gensteps, n_gs, prefix, s));
     int64_t total = 0;
@@ -1041,9 +1063,8 @@ int mi_sim_simulate_device_noalloc(mi_sim* sim, int32_t event_id, const void* d_
                                 hipMemcpyHostToDevice, s));
         xw_table = xw;
     }
-    HIPCHECK(oa_launch::noalloc_setup(ev, ev_id, next, n_gs, n_photon, event_id, s));
+    HIPCHECK(oa_launch::noalloc_setup(ev, ev_id, n_gs, n_photon, event_id, s));
     HIPCHECK(hipEventRecord(sim->ev[1], s));
-    const int64_t n_words = (n_photon + 63) / 64;
     SimParams P = base_params(sim);
     P.xw_jump = xw_table;
     P.gensteps = (const float*)d_gensteps;
@@ -1061,16 +1082,17 @@ int mi_sim_simulate_device_noalloc(mi_sim* sim, int32_t event_id, const void* d_
     P.seq = (uint64_t*)d_seq;
     P.photonlite = nullptr;
     P.hitwords = words;
-    P.next = next;
-    if (sim->cfg.kernel == MI_KERNEL_WAVEFRONT) HIPCHECK(oa_launch::zero_u64(words, n_words, s));
+    P.next = words + oa_launch::next_offset(n_photon);
+    P.wave_width = (int32_t)wave_width(n_photon, wave_count(sim));
+    HIPCHECK(oa_launch::clear_launch(words, n_photon, wave_count(sim), s));
     HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s));
     HIPCHECK(hipEventRecord(sim->ev[2], s));
-    const int64_t nb = (n_words + 255) / 256;
-    HIPCHECK(oa_launch::compact_hits(words, n_words, word_prefix, block_total, (const float4*)d_photon,
-                                     (float4*)d_hit, d_hit ? hit_capacity : 0, s));
+    HIPCHECK(oa_launch::compact_hits(words, n_photon, nullptr, word_prefix, tile_base,
+                                     words + oa_launch::state_offset(n_photon), (const float4*)d_photon,
+                                     (float4*)d_hit, d_hit ? hit_capacity : 0, nullptr, s));
     HIPCHECK(hipEventRecord(sim->ev[3], s));
     int64_t hits = 0;
-    HIPCHECK(hipMemcpyAsync(&hits, block_total + nb, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    HIPCHECK(hipMemcpyAsync(&hits, tile_base + oa_launch::compact_tiles(n_photon), sizeof(int64_t), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
     float a = 0.f, b = 0.f, c = 0.f, t = 0.f;
     HIPCHECK(hipEventElapsedTime(&a, sim->ev[0], sim->ev[1]));
@@ -1103,7 +1125,7 @@ int mi_sim_simulate_batch_device(mi_sim* sim, int32_t n_event, const int32_t* ev
     if (n_gs <= 0) return fail(MI_NOTHING_TO_DO, "zero gensteps");
     hipStream_t s = stream ? (hipStream_t)stream : sim->stream;
     HIPCHECK(hipEventRecord(sim->ev[0], s));
-    HIPCHECK(sim->prefix.reserve((size_t)n_gs + 1));
+    HIPCHECK(sim->prefix.reserve((size_t)oa_launch::gs_prefix_words(n_gs)));
     HIPCHECK(oa_launch::gs_prefix((const float*)d_gensteps, n_gs, sim->prefix.p, s));
     std::vector<int64_t> hp((size_t)n_gs + 1);
     HIPCHECK(hipMemcpyAsync(hp.data(), sim->prefix.p, sizeof(int64_t) * (n_gs + 1), hipMemcpyDeviceToHost, s));
@@ -1121,7 +1143,7 @@ int mi_sim_simulate_batch_device(mi_sim* sim, int32_t n_event, const int32_t* ev
     int prc = check_precooked_rows(sim, max_ev);
     if (prc) return prc;
     const uint32_t* xw_table = nullptr;
-    prc = xorwow_table(sim, event_ids, n_event, sim->xw_jump, &xw_table);
+    prc = xorwow_table(sim, event_ids, n_event, sim->xw_jump, &xw_table, s);
     if (prc) return prc;
     HIPCHECK(sim->evbuf.reserve(evh.size() + n_event + 1));
     HIPCHECK(sim->ev_id.reserve((size_t)n_event));
@@ -1145,14 +1167,14 @@ int mi_sim_simulate_batch_device(mi_sim* sim, int32_t n_event, const int32_t* ev
     if (rc) return rc;
     HIPCHECK(hipEventRecord(sim->ev[2], s));
     const int64_t n_words = (n_photon + 63) / 64;
-    const int64_t nb = (n_words + 255) / 256;
     HIPCHECK(sim->word_prefix.reserve((size_t)n_words + 1));
-    HIPCHECK(sim->block_total.reserve((size_t)nb + 1));
-    HIPCHECK(oa_launch::compact_hits(sim->words.p, n_words, sim->word_prefix.p, sim->block_total.p,
-                                     (const float4*)d_photon, (float4*)d_hit, d_hit ? hit_capacity : 0, s));
+    HIPCHECK(sim->tile_base.reserve((size_t)oa_launch::compact_tiles(n_photon) + 1));
+    HIPCHECK(oa_launch::compact_hits(sim->words.p, n_photon, nullptr, sim->word_prefix.p, sim->tile_base.p,
+                                     sim->words.p + oa_launch::state_offset(n_photon), (const float4*)d_photon,
+                                     (float4*)d_hit, d_hit ? hit_capacity : 0, nullptr, s));
     DBuf<int64_t>& hob = sim->evbuf;   /* reuse tail of evbuf for the offsets */
     int64_t* d_ho = hob.p + evh.size();
-    HIPCHECK(oa_launch::event_hit_offsets(sim->words.p, sim->word_prefix.p, sim->block_total.p,
+    HIPCHECK(oa_launch::event_hit_offsets(sim->words.p, sim->word_prefix.p, sim->tile_base.p,
                                           P.ev_ph_begin, n_event, n_words, d_ho, s));
     HIPCHECK(hipMemcpyAsync(hit_offsets, d_ho, sizeof(int64_t) * (n_event + 1), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipEventRecord(sim->ev[3], s));
@@ -1231,7 +1253,7 @@ int mi_sim_simtrace_device(mi_sim* sim, const void* d_gensteps, int64_t n_gs, in
     if (n_gs <= 0) return fail(MI_NOTHING_TO_DO, "zero gensteps");
     if (!d_gensteps || !d_simtrace) return fail(MI_ERR_ARG, "null simtrace buffers");
     hipStream_t s = stream ? (hipStream_t)stream : sim->stream;
-    HIPCHECK(sim->prefix.reserve((size_t)n_gs + 1));
+    HIPCHECK(sim->prefix.reserve((size_t)oa_launch::gs_prefix_words(n_gs)));
     HIPCHECK(oa_launch::gs_prefix((const float*)d_gensteps, n_gs, sim->prefix.p, s));
     int64_t total = 0;
     HIPCHECK(hipMemcpyAsync(&total, sim->prefix.p + n_gs, sizeof(int64_t), hipMemcpyDeviceToHost, s));
@@ -1375,7 +1397,7 @@ int mi_sim_adjoint_device(mi_sim* sim, int32_t event_id, const void* d_gensteps,
     hipStream_t s = stream ? (hipStream_t)stream : sim->stream;
     HIPCHECK(upload(sim->adj_mat_block, adj->mat_block, (size_t)adj->n_mat + 1, s));
     HIPCHECK(upload(sim->adj_sample_bin, adj->sample_bin, (size_t)sim->n_wl, s));
-    HIPCHECK(sim->prefix.reserve((size_t)n_gs + 1));
+    HIPCHECK(sim->prefix.reserve((size_t)oa_launch::gs_prefix_words(n_gs)));
     HIPCHECK(oa_launch::gs_prefix((const float*)d_gensteps, n_gs, sim->prefix.p, s));
     if (n_photon < 0) {
         HIPCHECK(hipMemcpyAsync(&n_photon, sim->prefix.p + n_gs, sizeof(int64_t), hipMemcpyDeviceToHost, s));
@@ -1384,7 +1406,7 @@ int mi_sim_adjoint_device(mi_sim* sim, int32_t event_id, const void* d_gensteps,
     int prc = check_precooked_rows(sim, photon_offset + n_photon);
     if (prc) return prc;
     const uint32_t* xw_table = nullptr;
-    prc = xorwow_table(sim, &event_id, 1, sim->xw_jump, &xw_table);
+    prc = xorwow_table(sim, &event_id, 1, sim->xw_jump, &xw_table, s);
     if (prc) return prc;
     int64_t evh[4] = { 0, n_gs, 0, n_photon };
     int32_t evid = event_id;
@@ -1408,7 +1430,7 @@ int mi_sim_adjoint_device(mi_sim* sim, int32_t event_id, const void* d_gensteps,
         tk.n_gs == n_gs && tk.gs == d_gensteps && tk.generation == sim->generation &&
         oa_launch::tape_reduce_rows(n_param) > 0) {
         HIPCHECK(sim->tape_flag.reserve(1));
-        P.tape = sim->tape.p; P.tape_n = sim->tape_n.p; P.tape_stride = tk.n_photon; P.tape_k = tk.k;
+        P.tape = sim->tape.p; P.tape_n = sim->tape_n.p; P.tape_stride = tk.stride; P.tape_k = tk.k;
         P.tape_overflow = sim->tape_flag.p;
     }
     const uint32_t n_det = (uint32_t)adj->n_det;
@@ -1531,10 +1553,10 @@ struct mi_batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hipEvent_t ev[2] = { nullptr, nullptr };
-    DBuf<int64_t> prefix, saved_prefix, evbuf, block_total, ho;
+    DBuf<int64_t> prefix, saved_prefix, evbuf, tile_base, ho;
     DBuf<int32_t> ev_id, word_prefix, gs_event;
     DBuf<uint32_t> seed, xw_jump;
-    DBuf<unsigned long long> words, next, flag;
+    DBuf<unsigned long long> words, flag;
     int64_t* h_out = nullptr;   /* pinned: hit offsets (n_event+1), then the prefix-mismatch flag */
     bool launched = false;
     double last_ms = 0.0;
@@ -1565,8 +1587,8 @@ int mi_batch_destroy(mi_batch* b)
     if (b->ev_mid) (void)hipEventDestroy(b->ev_mid);
     if (b->cap) (void)hipStreamDestroy(b->cap);
     if (b->h_out) (void)hipHostFree(b->h_out);
-    b->prefix.release(); b->saved_prefix.release(); b->evbuf.release(); b->block_total.release(); b->ho.release();
-    b->ev_id.release(); b->word_prefix.release(); b->words.release(); b->next.release(); b->flag.release();
+    b->prefix.release(); b->saved_prefix.release(); b->evbuf.release(); b->tile_base.release(); b->ho.release();
+    b->ev_id.release(); b->word_prefix.release(); b->words.release(); b->flag.release();
     b->seed.release(); b->gs_event.release(); b->xw_jump.release();
     b->mat_block.release(); b->sample_bin.release(); b->rows.release(); b->comp.release();
     b->key.release(); b->val.release(); b->key2.release(); b->val2.release(); b->tmp.release(); b->seg.release();
@@ -1576,10 +1598,10 @@ int mi_batch_destroy(mi_batch* b)
 }
 
 /* the work of one batch launch, issued on stream s (recorded when s is capturing) */
-static hipError_t batch_work(mi_batch* b, const SimParams& P, const void* d_gensteps, const void* d_photon, void* d_hit,
+static hipError_t batch_work(mi_batch* b, SimParams P, const void* d_gensteps, const void* d_photon, void* d_hit,
                              hipStream_t s)
 {
-    const mi_sim* sim = b->sim;
+    mi_sim* sim = b->sim;
     hipError_t e;
     if ((e = oa_launch::gs_prefix((const float*)d_gensteps, b->n_gs, b->prefix.p, s)) != hipSuccess) return e;
     if ((e = oa_launch::zero_u64(b->flag.p, 1, s)) != hipSuccess) return e;
@@ -1588,15 +1610,14 @@ static hipError_t batch_work(mi_batch* b, const SimParams& P, const void* d_gens
        replay fails on the host, so its photons are never used */
     if ((e = oa_launch::seed_map(b->saved_prefix.p, b->n_gs, b->n_photon, b->seed.p, P.ev_gs_begin, b->n_event,
                                  b->gs_event.p, s)) != hipSuccess) return e;
-    if (sim->cfg.kernel == MI_KERNEL_WAVEFRONT) {
-        if ((e = oa_launch::zero_u64(b->words.p, b->n_words, s)) != hipSuccess) return e;
-        if ((e = oa_launch::zero_u64(b->next.p, 1, s)) != hipSuccess) return e;
-    }
+    P.wave_width = (int32_t)wave_width(b->n_photon, wave_count(sim));
+    if ((e = oa_launch::clear_launch(b->words.p, b->n_photon, wave_count(sim), s)) != hipSuccess) return e;
     if ((e = oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s)) != hipSuccess) return e;
-    if ((e = oa_launch::compact_hits(b->words.p, b->n_words, b->word_prefix.p, b->block_total.p,
-                                     (const float4*)d_photon, (float4*)d_hit, d_hit ? b->hit_capacity : 0, s)) != hipSuccess)
+    if ((e = oa_launch::compact_hits(b->words.p, b->n_photon, nullptr, b->word_prefix.p, b->tile_base.p,
+                                     b->words.p + oa_launch::state_offset(b->n_photon), (const float4*)d_photon,
+                                     (float4*)d_hit, d_hit ? b->hit_capacity : 0, nullptr, s)) != hipSuccess)
         return e;
-    if ((e = oa_launch::event_hit_offsets(b->words.p, b->word_prefix.p, b->block_total.p, P.ev_ph_begin, b->n_event,
+    if ((e = oa_launch::event_hit_offsets(b->words.p, b->word_prefix.p, b->tile_base.p, P.ev_ph_begin, b->n_event,
                                           b->n_words, b->ho.p, s)) != hipSuccess)
         return e;
     if ((e = hipMemcpyAsync(b->h_out, b->ho.p, sizeof(int64_t) * (b->n_event + 1), hipMemcpyDeviceToHost, s)) != hipSuccess)
@@ -1649,7 +1670,7 @@ static int batch_create(mi_sim* sim, int32_t n_event, const int32_t* event_ids, 
     auto bail = [&](int rc) { mi_batch_destroy(b); return rc; };
 #define BCHECK(expr) do { hipError_t e_ = (expr); if (e_ != hipSuccess) return bail(fail(MI_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_))); } while (0)
     hipStream_t s = sim->stream;
-    BCHECK(b->prefix.reserve((size_t)n_gs + 1));
+    BCHECK(b->prefix.reserve((size_t)oa_launch::gs_prefix_words(n_gs)));
     BCHECK(b->saved_prefix.reserve((size_t)n_gs + 1));
     BCHECK(oa_launch::gs_prefix((const float*)d_gensteps, n_gs, b->prefix.p, s));
     std::vector<int64_t> hp((size_t)n_gs + 1);
@@ -1669,19 +1690,17 @@ static int batch_create(mi_sim* sim, int32_t n_event, const int32_t* event_ids, 
     int prc = check_precooked_rows(sim, max_ev);
     if (prc) return bail(prc);
     const uint32_t* xw_table = nullptr;
-    prc = xorwow_table(sim, event_ids, n_event, b->xw_jump, &xw_table);
+    prc = xorwow_table(sim, event_ids, n_event, b->xw_jump, &xw_table, s);
     if (prc) return bail(prc);
     b->n_words = (b->n_photon + 63) / 64;
-    const int64_t nb = (b->n_words + 255) / 256;
     BCHECK(upload(b->evbuf, evh.data(), evh.size(), s));
     BCHECK(upload(b->ev_id, event_ids, (size_t)n_event, s));
-    BCHECK(b->words.reserve((size_t)b->n_words + 1));
+    BCHECK(b->words.reserve((size_t)oa_launch::clear_words(b->n_photon)));
     BCHECK(b->seed.reserve((size_t)b->n_photon));
     BCHECK(b->gs_event.reserve((size_t)n_gs));
-    BCHECK(b->next.reserve(1));
     BCHECK(b->flag.reserve(1));
     BCHECK(b->word_prefix.reserve((size_t)b->n_words + 1));
-    BCHECK(b->block_total.reserve((size_t)nb + 1));
+    BCHECK(b->tile_base.reserve((size_t)oa_launch::compact_tiles(b->n_photon) + 1));
     BCHECK(b->ho.reserve((size_t)n_event + 1));
     BCHECK(hipHostMalloc((void**)&b->h_out, sizeof(int64_t) * ((size_t)n_event + 2), hipHostMallocDefault));
     for (auto& e : b->ev) BCHECK(hipEventCreate(&e));
@@ -1700,7 +1719,7 @@ static int batch_create(mi_sim* sim, int32_t n_event, const int32_t* event_ids, 
     P.photon = (float4*)d_photon;
     P.seq = (uint64_t*)d_seq;
     P.hitwords = b->words.p;
-    P.next = b->next.p;
+    P.next = b->words.p + oa_launch::next_offset(b->n_photon);
     P.seed_map = b->seed.p;
     P.gs_event = b->gs_event.p;
     if (adj) {

@@ -7,15 +7,40 @@ namespace oa_launch {
 /* genstep of each photon (seed) and, for n_event > 1, event of each genstep */
 hipError_t seed_map(const int64_t* d_prefix, int64_t n_gs, int64_t n_photon, uint32_t* d_seed,
                     const int64_t* d_ev_gs_begin, int32_t n_event, int32_t* d_gs_event, hipStream_t s);
+/* exclusive prefix of the gensteps' photon counts into d_prefix[0..n_gs], which holds
+   gs_prefix_words(n_gs) words (block sums behind it) */
+int64_t gs_prefix_words(int64_t n_gs);
 hipError_t gs_prefix(const float* d_gs, int64_t n_gs, int64_t* d_prefix, hipStream_t s);
+/* start of a single-event launch (k_setup): seeds of up to cap photons, n_clear cleared words,
+   event bounds ev (4) and ev_id (1), the launch's photon count and wave_width n_dev (2) */
+struct SetupArgs {
+    const float* gs; int64_t n_gs, n_arg, cap;
+    int64_t* prefix; uint32_t* seed;
+    unsigned long long* clear; int64_t n_clear;
+    int64_t* ev; int32_t* ev_id; int32_t event_id;
+    int64_t* n_dev; LaunchResult* out;
+    int64_t n_wave;                     /* waves of the propagation grid */
+};
+hipError_t setup(const SetupArgs& a, hipStream_t s);
+/* Cleared words of a launch of n photons: the hit bitmask, then the state of the compaction's
+   tiles (256 bitmask words each) and its ticket, then the propagation's photon counter. */
+inline int64_t compact_tiles(int64_t n_photon) { return ((n_photon + 63) / 64 + 255) / 256; }
+inline int64_t state_offset(int64_t n_photon) { return (n_photon + 63) / 64; }
+inline int64_t next_offset(int64_t n_photon) { return state_offset(n_photon) + compact_tiles(n_photon) + 1; }
+inline int64_t clear_words(int64_t n_photon) { return next_offset(n_photon) + 1; }
 hipError_t simulate(const SimParams& P, int kernel, int block, int grid, hipStream_t s);
 int wave_blocks_per_cu(int block, int rng_kind, int stack_depth);   /* resident blocks of the persistent kernel per CU */
 unsigned sim_lds(int block, int rng_kind, int stack_depth);   /* LDS bytes of a propagation block */
 hipError_t prefix_check(const int64_t* a, const int64_t* b, int64_t n, unsigned long long* flag, hipStream_t s);
 hipError_t zero_u64(unsigned long long* p, int64_t n, hipStream_t s);
-hipError_t compact_hits(const unsigned long long* d_words, int64_t n_words, int32_t* d_word_prefix,
-                        int64_t* d_block_total, const float4* d_photon, float4* d_hit, int64_t hit_cap,
-                        hipStream_t s);
+/* the cleared words of a launch of n photons on n_wave waves, its counter set behind the photons dealt first */
+hipError_t clear_launch(unsigned long long* words, int64_t n_photon, int64_t n_wave, hipStream_t s);
+/* stable compaction of the hits among n_photon photons, or *n_dev of them where it is given;
+   d_state: cleared words from state_offset on; d_tile_base: compact_tiles + 1 words; out (may be
+   null): the hit count and the clock */
+hipError_t compact_hits(const unsigned long long* d_words, int64_t n_photon, const int64_t* n_dev, int32_t* d_word_prefix,
+                        int64_t* d_tile_base, unsigned long long* d_state, const float4* d_photon, float4* d_hit,
+                        int64_t hit_cap, LaunchResult* out, hipStream_t s);
 hipError_t event_hit_offsets(const unsigned long long* d_words, const int32_t* d_word_prefix,
                              const int64_t* d_block_total, const int64_t* d_ev_ph_begin, int32_t n_event,
                              int64_t n_words, int64_t* d_hit_offsets, hipStream_t s);
@@ -55,7 +80,6 @@ int adjoint_blocks_per_cu(int rng_kind, int stack_depth);
 /* no-allocation entry point: the device address of the per-GPU scratch array
    (call with `device` current), and the per-launch event setup kernel */
 hipError_t noalloc_scratch(int device, void** ptr);
-hipError_t noalloc_setup(int64_t* ev, int32_t* ev_id, unsigned long long* next, int64_t n_gs, int64_t n_photon,
-                         int32_t event_id, hipStream_t s);
+hipError_t noalloc_setup(int64_t* ev, int32_t* ev_id, int64_t n_gs, int64_t n_photon, int32_t event_id, hipStream_t s);
 size_t adjoint_sort_bytes(int64_t n_hit, uint32_t n_det);
 }

@@ -4,11 +4,12 @@
  *
  *   k_gs_prefix       exclusive prefix of genstep numphoton (QEvt.cu:181-226 seeding
  *                     reduce)
+ *   k_setup           start of a single-event launch: prefix, seeds and cleared counters
  *   k_seed_fill       the expand: genstep index of every photon, one block per
  *                     genstep writing its photon range (QEvt.cu:181-226 seed
  *                     buffer, sysrap/iexpand.h); k_gs_event the event of every
  *                     genstep for batched launches
- *   k_hit_count/k_hit_scan/k_hit_scatter
+ *   k_compact
  *                     stable stream compaction of flagmask&hit_mask photons via
  *                     a per-64-photon bitmask (QEvt::gatherHit_, SU.cu:145-160)
  *   k_trace           nearest-hit query (simtrace-style)
@@ -46,25 +47,131 @@ __global__ void __launch_bounds__(256) k_gs_event(const int64_t* ev_gs_begin, in
         for (int64_t g = ev_gs_begin[e] + threadIdx.x; g < ev_gs_begin[e + 1]; g += blockDim.x) gs_event[g] = e;
 }
 
-__global__ void __launch_bounds__(1024) k_gs_prefix(const float* gs, int64_t n_gs, int64_t* prefix)
+/* exclusive prefix of the gensteps' photon counts, 1,024 a block: `sums` has each block's
+   total (k_gs_sums) where there is more than one */
+__global__ void __launch_bounds__(1024) k_gs_sums(const float* gs, int64_t n_gs, int64_t* sums)
 {
-    __shared__ int64_t part[1024];
-    const int t = threadIdx.x;
-    const int64_t per = (n_gs + 1023) / 1024;
-    const int64_t b = t * per, e = (b + per < n_gs) ? b + per : n_gs;
-    int64_t s = 0;
-    for (int64_t g = b; g < e; ++g) s += (int64_t)__float_as_uint(gs[24 * g + 3]);
-    part[t] = s;
+    __shared__ int64_t part[16];
+    const int64_t g = (int64_t)blockIdx.x * 1024 + threadIdx.x;
+    int64_t v = g < n_gs ? (int64_t)__float_as_uint(gs[24 * g + 3]) : 0;
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
     __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        int64_t v = t >= off ? part[t - off] : 0;
-        __syncthreads();
-        part[t] += v;
+    if (threadIdx.x == 0) {
+        int64_t t = 0;
+        for (int k = 0; k < 16; ++k) t += part[k];
+        sums[blockIdx.x] = t;
+    }
+}
+
+/* inclusive scan of one value a thread over the block (at most 16 waves); part: 16 words of LDS */
+OA_D int64_t block_scan(int64_t v, int64_t* part)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int64_t u = __shfl_up(v, o);
+        if (lane >= o) v += u;
+    }
+    if (lane == 63) part[wave] = v;
+    __syncthreads();
+    for (int q = 0; q < wave; ++q) v += part[q];
+    return v;
+}
+
+__global__ void __launch_bounds__(1024) k_gs_prefix(const float* gs, int64_t n_gs, const int64_t* sums, int64_t* prefix)
+{
+    __shared__ int64_t part[16], s_before[16];
+    const int t = threadIdx.x;
+    const int64_t g = (int64_t)blockIdx.x * 1024 + t;
+    /* gensteps of the blocks before this one */
+    int64_t b = 0;
+    for (int64_t k = t; k < (int64_t)blockIdx.x; k += 1024) b += sums[k];
+    for (int o = 32; o > 0; o >>= 1) b += __shfl_xor(b, o);
+    if ((t & 63) == 0) s_before[t >> 6] = b;
+    const int64_t v = g < n_gs ? (int64_t)__float_as_uint(gs[24 * g + 3]) : 0;
+    const int64_t incl = block_scan(v, part);
+    int64_t before = 0;
+    for (int k = 0; k < 16; ++k) before += s_before[k];
+    if (g < n_gs) prefix[g] = before + incl - v;
+    if (g == n_gs - 1) prefix[n_gs] = before + incl;
+}
+
+/*
+ * Start of a single-event launch: genstep of every photon (QEvt.cu:181-226), cleared hit
+ * words and counters, event bounds, and the launch's photon count on the device, where the
+ * propagation and the compaction read it: the host need not wait for the gensteps' total
+ * before it launches them. The count is n_arg, or the gensteps' total for n_arg < 0; it is 0,
+ * and nothing is propagated, when that is more than the gensteps have or than the launch's
+ * buffers hold (cap): the host sees the total and reports it or tries again.
+ * SMALL: up to OA_SETUP_GS gensteps; every block forms their prefix in LDS by itself (a few
+ * loads a thread), so one kernel does all of it. Else the prefix is there already.
+ */
+template <bool SMALL>
+__global__ void __launch_bounds__(256) k_setup(const float* gs, int64_t n_gs, int64_t n_arg, int64_t cap, int64_t* prefix,
+                                               uint32_t* seed, unsigned long long* clear, int64_t n_clear, int64_t* ev,
+                                               int32_t* ev_id, int32_t event_id, int64_t* n_dev, LaunchResult* out,
+                                               int64_t n_wave)
+{
+    constexpr int PER = SMALL ? OA_SETUP_GS / 256 : 1;
+    __shared__ int64_t s_prefix[SMALL ? OA_SETUP_GS + 1 : 1];
+    __shared__ int64_t part[16];
+    const int t = threadIdx.x;
+    const bool first = blockIdx.x == 0;
+    if (first && t == 0) out->clock[0] = wall_clock64();
+    if (SMALL) {
+        int64_t c[PER], sum = 0;
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int64_t g = (int64_t)t * PER + k;
+            c[k] = g < n_gs ? (int64_t)__float_as_uint(gs[24 * g + 3]) : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < PER; ++k) sum += c[k];
+        int64_t run = block_scan(sum, part) - sum;
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int64_t g = (int64_t)t * PER + k;
+            if (g <= n_gs) {
+                s_prefix[g] = run;
+                if (first) prefix[g] = run;
+            }
+            run += c[k];
+        }
+        if (t == 255 && n_gs == OA_SETUP_GS) {
+            s_prefix[n_gs] = run;
+            if (first) prefix[n_gs] = run;
+        }
         __syncthreads();
     }
-    int64_t run = part[t] - s;    /* exclusive */
-    for (int64_t g = b; g < e; ++g) { prefix[g] = run; run += (int64_t)__float_as_uint(gs[24 * g + 3]); }
-    if (t == 1023) prefix[n_gs] = part[1023];
+    const int64_t* pre = SMALL ? s_prefix : prefix;
+    const int64_t total = pre[n_gs];
+    int64_t n = n_arg < 0 ? total : n_arg;
+    if (n > total || n > cap) n = 0;
+    const int64_t stride = (int64_t)gridDim.x * 256, id = (int64_t)blockIdx.x * 256 + t;
+    /* the last cleared word is the photon counter: it starts behind the photons dealt first */
+    const int64_t width = wave_width(n, n_wave);
+    for (int64_t i = id; i < n_clear; i += stride) clear[i] = i == n_clear - 1 ? (unsigned long long)(n_wave * width) : 0ull;
+    for (int64_t i = 4 * id; i < n; i += 4 * stride) {
+        int64_t g = upper_index(pre, 0, n_gs, i);
+        uint32_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            while (g + 1 < n_gs && pre[g + 1] <= i + u) ++g;
+            v[u] = (uint32_t)g;
+        }
+        if (i + 4 <= n) *reinterpret_cast<uint4*>(seed + i) = make_uint4(v[0], v[1], v[2], v[3]);
+        else for (int u = 0; i + u < n; ++u) seed[i + u] = v[u];
+    }
+    if (first && t == 0) {
+        ev[0] = 0; ev[1] = n_gs; ev[2] = 0; ev[3] = n;
+        ev_id[0] = event_id;
+        n_dev[0] = n;
+        n_dev[1] = width;
+        out->total = total;
+        out->n_photon = n;
+        out->n_hit = 0;
+        out->clock[1] = wall_clock64();
+    }
 }
 
 /* ------------------------------------------------------------ simtrace */
@@ -117,69 +224,112 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_simtrace(SimParams P, float4* 
 
 /* ---------------------------------------------------- hit compaction */
 
-/* per word popcount -> in-block exclusive prefix; block totals */
-__global__ void __launch_bounds__(256) k_hit_count(const unsigned long long* words, int64_t n_words,
-                                                   int32_t* word_prefix, int64_t* block_total)
+/*
+ * Stable compaction of the hits, one pass: a block takes a tile of 256 bitmask words (16,384
+ * photons), counts them, gets the hits before it by a decoupled look-back over the tiles'
+ * published counts (D. Merrill, M. Garland, "Single-pass parallel prefix scan with decoupled
+ * look-back", NVR-2016-002) and copies its hit records. state[tile] is 0, then count | 1 << 62,
+ * then (hits up to the tile's end) | 2 << 62, one word each, so no ordering with other memory
+ * is needed; state[n_tiles_cap] hands out the tiles, so a tile's predecessors are always
+ * running or done. Both start at zero.
+ * A tile lists its hit photons in LDS first, so that four neighbouring lanes copy one 64 B
+ * record: with a lane per photon and a hit fraction of a tenth, most lanes of a wave only
+ * watched the others copy. Bound by the bytes of the records (read and written once); it
+ * replaces a count, a scan and a scatter kernel (17 us together on small events).
+ * word_prefix (hits of the tile before each word) and tile_base (hits before each tile, then
+ * the total) serve k_hit_event_offsets. out: null, or host-visible words for the total and
+ * the wall clock at the start and end.
+ */
+__global__ void __launch_bounds__(256) k_compact(const unsigned long long* __restrict__ words, int64_t n_photon,
+                                                 const int64_t* n_dev, int64_t tiles_cap, int32_t* word_prefix,
+                                                 int64_t* tile_base, unsigned long long* state,
+                                                 const float4* __restrict__ photon, float4* __restrict__ hit,
+                                                 int64_t hit_cap, LaunchResult* out)
 {
-    __shared__ int32_t s[256];
-    const int t = threadIdx.x;
-    const int64_t w = (int64_t)blockIdx.x * 256 + t;
-    const int32_t c = w < n_words ? __popcll(words[w]) : 0;
-    s[t] = c;
+    __shared__ int32_t s_wave[4];
+    __shared__ int64_t s_tile, s_base;
+    __shared__ uint16_t s_list[256 * 64];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int64_t n = n_dev ? *n_dev : n_photon;
+    const int64_t n_words = (n + 63) / 64, n_tiles = (n_words + 255) / 256;
+    if (t == 0) s_tile = (int64_t)atomicAdd(&state[tiles_cap], 1ull);
     __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-        int32_t v = t >= off ? s[t - off] : 0;
-        __syncthreads();
-        s[t] += v;
-        __syncthreads();
+    const int64_t tile = s_tile;
+    if (tile >= n_tiles) return;
+    if (out && tile == 0 && t == 0) out->clock[2] = wall_clock64();
+    const int64_t w = tile * 256 + t;
+    unsigned long long m = w < n_words ? words[w] : 0ull;
+    const int32_t c = __popcll(m);
+    int32_t incl = c;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int32_t v = __shfl_up(incl, o);
+        if (lane >= o) incl += v;
     }
-    if (w < n_words) word_prefix[w] = s[t] - c;
-    if (t == 255) block_total[blockIdx.x] = s[255];
-}
-
-/* exclusive scan of block totals in place; total into block_total[n_blocks] */
-__global__ void __launch_bounds__(1024) k_hit_scan(int64_t* block_total, int64_t n_blocks)
-{
-    __shared__ int64_t part[1024];
-    const int t = threadIdx.x;
-    const int64_t per = (n_blocks + 1023) / 1024;
-    const int64_t b = t * per, e = (b + per < n_blocks) ? b + per : n_blocks;
-    int64_t s = 0;
-    for (int64_t i = b; i < e; ++i) s += block_total[i];
-    part[t] = s;
+    if (lane == 63) s_wave[wave] = incl;
     __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        int64_t v = t >= off ? part[t - off] : 0;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
+    int32_t before = incl - c;
+    for (int q = 0; q < wave; ++q) before += s_wave[q];
+    const int32_t total = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+    const unsigned long long kCount = 1ull << 62, kDone = 2ull << 62, kValue = kCount - 1ull;
+    if (wave == 0) {
+        int64_t base = 0;
+        if (tile > 0) {
+            if (lane == 0)
+                __hip_atomic_store(&state[tile], kCount | (unsigned long long)total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            /* 64 tiles at a time, the nearest in lane 0 */
+            for (int64_t k = tile - 1;; k -= 64) {
+                const int64_t mine = k - lane;
+                unsigned long long v = kDone;               /* before the first tile: nothing, and the end */
+                do {
+                    if (mine >= 0) v = __hip_atomic_load(&state[mine], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                } while (__ballot(v < kCount) != 0ull);
+                const unsigned long long ends = __ballot(v >= kDone);
+                const int last = ends ? __ffsll((long long)ends) - 1 : 63;
+                int64_t sum = lane <= last ? (int64_t)(v & kValue) : 0;
+                for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+                base += sum;
+                if (ends) break;
+            }
+        }
+        if (lane == 0) {
+            __hip_atomic_store(&state[tile], kDone | (unsigned long long)(base + total), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            s_base = base;
+            tile_base[tile] = base;
+            if (tile == n_tiles - 1) tile_base[n_tiles] = base + total;
+        }
     }
-    int64_t run = part[t] - s;
-    for (int64_t i = b; i < e; ++i) { int64_t v = block_total[i]; block_total[i] = run; run += v; }
-    if (t == 1023) block_total[n_blocks] = part[1023];
-}
-
-/* one wave per bitmask word; lane i copies photon 64*w+i when its bit is set */
-__global__ void __launch_bounds__(256) k_hit_scatter(const unsigned long long* words, int64_t n_words,
-                                                     const int32_t* word_prefix, const int64_t* block_total,
-                                                     const float4* photon, float4* hit, int64_t hit_cap)
-{
-    const int lane = threadIdx.x & 63;
-    const int64_t w = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6;
-    if (w >= n_words) return;
-    const unsigned long long m = words[w];
-    if (!((m >> lane) & 1ull)) return;
-    const int64_t base = block_total[w >> 8] + word_prefix[w];
-    const int64_t r = base + __popcll(m & ((1ull << lane) - 1ull));
-    if (r >= hit_cap) return;
-    const float4* src = photon + 4 * (w * 64 + lane);
-    float4* dst = hit + 4 * r;
-    dst[0] = src[0]; dst[1] = src[1]; dst[2] = src[2]; dst[3] = src[3];
+    if (w < n_words) word_prefix[w] = before;
+    if (hit && photon) {
+        for (int32_t k = before; m; m &= m - 1ull) s_list[k++] = (uint16_t)(t * 64 + __ffsll((long long)m) - 1);
+    }
+    __syncthreads();
+    const int64_t base = s_base;
+    if (hit && photon) {
+        const int64_t room = hit_cap - base;
+        const int32_t n4 = 4 * (int32_t)(room < total ? (room > 0 ? room : 0) : total);
+        const float4* src = photon + 4 * tile * 16384;
+        float4* dst = hit + 4 * base;
+        int32_t i = t;
+        /* four records' quarters in flight a lane */
+        for (; i + 768 < n4; i += 1024) {
+            float4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = src[4 * (int)s_list[(i + 256 * u) >> 2] + (i & 3)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) dst[i + 256 * u] = v[u];
+        }
+        for (; i < n4; i += 256) dst[i] = src[4 * (int)s_list[i >> 2] + (i & 3)];
+    }
+    if (out && tile == n_tiles - 1 && t == 0) {
+        out->n_hit = base + total;
+        out->clock[3] = wall_clock64();
+    }
 }
 
 /* hits among photons [0, ph) for each event boundary ph = ev_ph_begin[e] */
 __global__ void k_hit_event_offsets(const unsigned long long* words, const int32_t* word_prefix,
-                                    const int64_t* block_total, const int64_t* ev_ph_begin, int32_t n_event,
+                                    const int64_t* tile_base, const int64_t* ev_ph_begin, int32_t n_event,
                                     int64_t n_words, int64_t* hit_offsets)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
@@ -187,8 +337,8 @@ __global__ void k_hit_event_offsets(const unsigned long long* words, const int32
     const int64_t ph = ev_ph_begin[e];
     const int64_t w = ph >> 6;
     int64_t r;
-    if (w >= n_words) r = block_total[(n_words + 255) / 256];
-    else r = block_total[w >> 8] + word_prefix[w] + __popcll(words[w] & ((1ull << (ph & 63)) - 1ull));
+    if (w >= n_words) r = tile_base[(n_words + 255) / 256];
+    else r = tile_base[w >> 8] + word_prefix[w] + __popcll(words[w] & ((1ull << (ph & 63)) - 1ull));
     hit_offsets[e] = r;
 }
 
@@ -312,9 +462,30 @@ hipError_t seed_map(const int64_t* d_prefix, int64_t n_gs, int64_t n_photon, uin
     return hipGetLastError();
 }
 
+int64_t gs_prefix_words(int64_t n_gs) { return n_gs + 1 + (n_gs + 1023) / 1024; }
+
 hipError_t gs_prefix(const float* d_gs, int64_t n_gs, int64_t* d_prefix, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_gs_prefix, dim3(1), dim3(1024), 0, s, d_gs, n_gs, d_prefix);
+    const unsigned nb = (unsigned)((n_gs + 1023) / 1024);
+    int64_t* sums = d_prefix + n_gs + 1;
+    if (nb > 1) hipLaunchKernelGGL(k_gs_sums, dim3(nb), dim3(1024), 0, s, d_gs, n_gs, sums);
+    hipLaunchKernelGGL(k_gs_prefix, dim3(nb), dim3(1024), 0, s, d_gs, n_gs, sums, d_prefix);
+    return hipGetLastError();
+}
+
+hipError_t setup(const SetupArgs& a, hipStream_t s)
+{
+    const int64_t work = std::max<int64_t>(a.cap / 8, a.n_clear);
+    const unsigned nb = (unsigned)std::min<int64_t>(1024, (work + 255) / 256 + 1);
+    if (a.n_gs <= OA_SETUP_GS) {
+        hipLaunchKernelGGL(k_setup<true>, dim3(nb), dim3(256), 0, s, a.gs, a.n_gs, a.n_arg, a.cap, a.prefix, a.seed, a.clear,
+                           a.n_clear, a.ev, a.ev_id, a.event_id, a.n_dev, a.out, a.n_wave);
+    } else {
+        const hipError_t e = gs_prefix(a.gs, a.n_gs, a.prefix, s);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_setup<false>, dim3(nb), dim3(256), 0, s, a.gs, a.n_gs, a.n_arg, a.cap, a.prefix, a.seed, a.clear,
+                           a.n_clear, a.ev, a.ev_id, a.event_id, a.n_dev, a.out, a.n_wave);
+    }
     return hipGetLastError();
 }
 
@@ -351,18 +522,14 @@ hipError_t simulate(const SimParams& P, int kernel, int block, int grid, hipStre
     }
 }
 
-hipError_t compact_hits(const unsigned long long* d_words, int64_t n_words, int32_t* d_word_prefix,
-                        int64_t* d_block_total, const float4* d_photon, float4* d_hit, int64_t hit_cap,
-                        hipStream_t s)
+hipError_t compact_hits(const unsigned long long* d_words, int64_t n_photon, const int64_t* n_dev, int32_t* d_word_prefix,
+                        int64_t* d_tile_base, unsigned long long* d_state, const float4* d_photon, float4* d_hit,
+                        int64_t hit_cap, LaunchResult* out, hipStream_t s)
 {
-    const int64_t nb = (n_words + 255) / 256;
-    if (nb > 0) hipLaunchKernelGGL(k_hit_count, dim3((unsigned)nb), dim3(256), 0, s, d_words, n_words, d_word_prefix, d_block_total);
-    hipLaunchKernelGGL(k_hit_scan, dim3(1), dim3(1024), 0, s, d_block_total, nb);
-    if (d_hit && d_photon && n_words > 0) {
-        const int64_t nt = n_words * 64;
-        hipLaunchKernelGGL(k_hit_scatter, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s,
-                           d_words, n_words, d_word_prefix, d_block_total, d_photon, d_hit, hit_cap);
-    }
+    const int64_t nt = compact_tiles(n_photon);
+    if (nt > 0)
+        hipLaunchKernelGGL(k_compact, dim3((unsigned)nt), dim3(256), 0, s, d_words, n_photon, n_dev, nt, d_word_prefix,
+                           d_tile_base, d_state, d_photon, d_hit, hit_cap, out);
     return hipGetLastError();
 }
 
@@ -396,6 +563,20 @@ __global__ void k_prefix_check(const int64_t* a, const int64_t* b, int64_t n, un
 hipError_t prefix_check(const int64_t* a, const int64_t* b, int64_t n, unsigned long long* flag, hipStream_t s)
 {
     if (n > 0) hipLaunchKernelGGL(k_prefix_check, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, b, n, flag);
+    return hipGetLastError();
+}
+
+__global__ void k_clear_launch(unsigned long long* p, int64_t n, unsigned long long last)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = i == n - 1 ? last : 0ull;
+}
+
+hipError_t clear_launch(unsigned long long* words, int64_t n_photon, int64_t n_wave, hipStream_t s)
+{
+    const int64_t n = clear_words(n_photon);
+    hipLaunchKernelGGL(k_clear_launch, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, words, n,
+                       (unsigned long long)(n_wave * wave_width(n_photon, n_wave)));
     return hipGetLastError();
 }
 
@@ -848,15 +1029,12 @@ size_t adjoint_sort_bytes(int64_t n_hit, uint32_t n_det)
    the process; every handle on a GPU shares it. */
 static __device__ __align__(256) unsigned char scratch[OA_NOALLOC_SCRATCH_BYTES];
 
-/* event bounds {0, n_gs, 0, n_photon}, event id and refill counter of one
-   no-allocation launch, written by a kernel (no host staging) */
-__global__ void k_noalloc_setup(int64_t* ev, int32_t* ev_id, unsigned long long* next, int64_t n_gs,
-                                int64_t n_photon, int32_t event_id)
+/* event bounds {0, n_gs, 0, n_photon} and event id of one no-allocation launch, written by a kernel (no host staging) */
+__global__ void k_noalloc_setup(int64_t* ev, int32_t* ev_id, int64_t n_gs, int64_t n_photon, int32_t event_id)
 {
     if (threadIdx.x == 0) {
         ev[0] = 0; ev[1] = n_gs; ev[2] = 0; ev[3] = n_photon;
         ev_id[0] = event_id;
-        next[0] = 0ull;
     }
 }
 
@@ -883,10 +1061,9 @@ hipError_t noalloc_scratch(int device, void** ptr)
     return hipSuccess;
 }
 
-hipError_t noalloc_setup(int64_t* ev, int32_t* ev_id, unsigned long long* next, int64_t n_gs, int64_t n_photon,
-                         int32_t event_id, hipStream_t s)
+hipError_t noalloc_setup(int64_t* ev, int32_t* ev_id, int64_t n_gs, int64_t n_photon, int32_t event_id, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_noalloc_setup, dim3(1), dim3(64), 0, s, ev, ev_id, next, n_gs, n_photon, event_id);
+    hipLaunchKernelGGL(k_noalloc_setup, dim3(1), dim3(64), 0, s, ev, ev_id, n_gs, n_photon, event_id);
     return hipGetLastError();
 }
 

@@ -37,13 +37,13 @@
 #define OA_ALIGN256(x)         ((((long long)(x)) + 255ll) & ~255ll)
 #define OA_NOALLOC_WORDS       (OA_NOALLOC_MAX_PHOTON / 64 + 1)                 /* hit bitmask words */
 #define OA_NOALLOC_BLOCKS      ((OA_NOALLOC_WORDS + 255) / 256 + 1)             /* compaction block totals */
-#define OA_NOALLOC_OFF_PREFIX  0ll                                              /* (MAX_GS+1) int64 */
-#define OA_NOALLOC_OFF_EV      (OA_NOALLOC_OFF_PREFIX + OA_ALIGN256(8 * (OA_NOALLOC_MAX_GS + 1)))
+#define OA_NOALLOC_OFF_PREFIX  0ll                                              /* (MAX_GS+1) int64, a block sum each 1,024 */
+#define OA_NOALLOC_OFF_EV      (OA_NOALLOC_OFF_PREFIX + OA_ALIGN256(8 * (OA_NOALLOC_MAX_GS + 1 + OA_NOALLOC_MAX_GS / 1024)))
 #define OA_NOALLOC_OFF_EVID    (OA_NOALLOC_OFF_EV + 256ll)                      /* 4 int64 event bounds */
-#define OA_NOALLOC_OFF_NEXT    (OA_NOALLOC_OFF_EVID + 256ll)                    /* 1 int32 event id */
-#define OA_NOALLOC_OFF_XW      (OA_NOALLOC_OFF_NEXT + 256ll)                    /* 1 u64 refill counter */
+#define OA_NOALLOC_OFF_XW      (OA_NOALLOC_OFF_EVID + 256ll)                    /* 1 int32 event id */
 #define OA_NOALLOC_OFF_WORDS   (OA_NOALLOC_OFF_XW + OA_ALIGN256(4 * 800))       /* xorwow jump matrix */
-#define OA_NOALLOC_OFF_WPREFIX (OA_NOALLOC_OFF_WORDS + OA_ALIGN256(8 * OA_NOALLOC_WORDS))
+/* the hit words, then the compaction's tile states and ticket and the photon counter */
+#define OA_NOALLOC_OFF_WPREFIX (OA_NOALLOC_OFF_WORDS + OA_ALIGN256(8 * (OA_NOALLOC_WORDS + OA_NOALLOC_BLOCKS + 2)))
 #define OA_NOALLOC_OFF_BTOTAL  (OA_NOALLOC_OFF_WPREFIX + OA_ALIGN256(4 * OA_NOALLOC_WORDS))
 #define OA_NOALLOC_SCRATCH_BYTES (OA_NOALLOC_OFF_BTOTAL + OA_ALIGN256(8 * OA_NOALLOC_BLOCKS))
 
@@ -87,6 +87,35 @@ struct PrimRec {
     uint32_t global_prim;
     uint32_t index;               /* the prim's index (in the BLAS-ordered copy) */
 };
+
+/* what a launch tells the host, in host-visible memory */
+struct LaunchResult {
+    int64_t total;                /* photons of the gensteps */
+    int64_t n_photon;             /* photons propagated (0: the count was refused, see k_setup) */
+    int64_t n_hit;
+    uint64_t clock[4];            /* device wall clock: setup begins, ends, compaction begins, ends */
+};
+
+/*
+ * Photons dealt to each of the n_wave waves of the propagation grid at its start: 64, or an
+ * equal share of an event too small for that. With fewer lanes a wave runs fewer of the
+ * physics' branches, but more waves start: at least OA_MIN_WIDTH (8 against 64: 199 / 219 us on
+ * 1,000 photons in the water sphere, 286 / 309 us on 12,000 in a detector; 1: 209 / 281 us).
+ */
+#ifndef OA_MIN_WIDTH
+#define OA_MIN_WIDTH 8
+#endif
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline int64_t wave_width(int64_t n_photon, int64_t n_wave)
+{
+    if (n_photon > 64 * n_wave - n_wave) return 64;
+    const int64_t share = (n_photon + n_wave - 1) / n_wave;
+    return share < OA_MIN_WIDTH ? OA_MIN_WIDTH : share;
+}
+
+#define OA_SETUP_GS 2048          /* gensteps whose prefix every block of k_setup forms by itself */
 
 struct SimParams {
     /* geometry */
@@ -132,7 +161,9 @@ struct SimParams {
     const int64_t* ev_gs_begin;   /* (n_event+1) genstep index boundaries */
     const int64_t* ev_ph_begin;   /* (n_event+1) global photon boundaries */
     const int32_t* ev_id;         /* (n_event) event index for skipahead */
-    int64_t        n_photon;      /* total photons of the launch */
+    int64_t        n_photon;      /* total photons of the launch (with n_dev: at most) */
+    const int64_t* n_dev;         /* null, or on the device (k_setup): their number, and wave_width */
+    int32_t        wave_width;    /* without n_dev: photons each wave is dealt first (wave_width) */
     int64_t        photon_offset; /* added to the in-event index (single-event slicing) */
     /* outputs */
     float4*        photon;        /* (n_photon,4) float4 or null */
@@ -140,7 +171,7 @@ struct SimParams {
     uint4*         photonlite;    /* (n_photon) sphotonlite or null (lite kernel instantiation) */
     unsigned long long* hitwords; /* (n_photon+63)/64 bitmask, zeroed before launch */
     /* persistent kernel */
-    unsigned long long* next;     /* global photon counter */
+    unsigned long long* next;     /* global photon counter, behind the photons dealt first */
     int32_t refill_period;
     int32_t refill_batch;         /* refill once this many lanes are idle (or all are) */
     int32_t regroup_pct;          /* trace: leaf phase once fewer than this % of the walking lanes still walk */

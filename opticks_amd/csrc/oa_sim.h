@@ -378,8 +378,9 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_plain(SimParams P)
     uint32_t* park_w = s_lane + threadIdx.x;
     uint32_t* stk = park_w + (park_words<R>::value + ((F & 1) ? OA_LITE_WORDS : 0)) * BLOCK;
     const int64_t g = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    const int64_t n_photon = P.n_dev ? *P.n_dev : P.n_photon;
     bool hit = false;
-    if (g < P.n_photon) {
+    if (g < n_photon) {
         Lane<R, (F & 1) != 0> L;
         NoTape tape;
         bool more = lane_start<BLOCK, NoTape>(P, L, g, park_w);
@@ -390,7 +391,7 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_plain(SimParams P)
         hit = (L.p.flagmask & P.hit_mask) != 0u;
     }
     const unsigned long long m = __ballot(hit);
-    if ((threadIdx.x & 63) == 0 && g < P.n_photon) P.hitwords[g >> 6] = m;
+    if ((threadIdx.x & 63) == 0 && g < n_photon) P.hitwords[g >> 6] = m;
 }
 
 /* ------------------------------------------------ persistent kernel */
@@ -418,6 +419,7 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_wave(SimParams P)
         tape.finish(P, L.g, L.bounce);
         if ((L.p.flagmask & P.hit_mask) != 0u) atomicOr(P.hitwords + (L.g >> 6), 1ull << (L.g & 63));
     };
+    const int64_t n_photon = P.n_dev ? P.n_dev[0] : P.n_photon;
     for (int iter = 0;; ++iter) {
         OA_CYC_MARK(c_iter);
         const unsigned long long idle = __ballot(!active);
@@ -425,19 +427,29 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_wave(SimParams P)
         if (!exhausted && idle != 0ull && (idle == all || ((iter % period) == 0 && __popcll(idle) >= batch))) {
             const int n_idle = __popcll(idle);
             const int leader = __ffsll((long long)idle) - 1;
+            /* the first photons are dealt out by position, `width` to a wave (wave_width);
+               the counter starts behind them */
             unsigned long long base = 0ull;
-            if (lane == leader) base = atomicAdd(P.next, (unsigned long long)n_idle);
-            base = __shfl(base, leader);
+            int take = n_idle;
+            if (iter == 0) {
+                take = P.n_dev ? (int)P.n_dev[1] : P.wave_width;
+                base = ((unsigned long long)blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6)) * (unsigned)take;
+            } else {
+                if (lane == leader) base = atomicAdd(P.next, (unsigned long long)n_idle);
+                base = __shfl(base, leader);
+            }
             if (!active) {
                 const unsigned long long below = idle & ((1ull << lane) - 1ull);
-                const int64_t g = (int64_t)(base + (unsigned long long)__popcll(below));
-                if (g < P.n_photon) {
+                const int rank = __popcll(below);
+                const int64_t g = (int64_t)base + rank;
+                if (rank < take && g < n_photon) {
                     active = lane_start<BLOCK, T>(P, L, g, park_w);
                     if (active) park<BLOCK>(park_w, L);
                     else finish(L);
                 }
             }
-            if ((int64_t)(base + (unsigned long long)n_idle) >= P.n_photon) exhausted = true;
+            if (take < 64 && iter == 0) exhausted = true;         /* a small event: all of it is dealt */
+            else if ((int64_t)base + n_idle >= n_photon) exhausted = true;
         }
         const unsigned long long act = __ballot(active);
         if (act == 0ull) {

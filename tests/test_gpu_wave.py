@@ -114,3 +114,48 @@ def test_waiting_lanes_keep_results(n, batch):
     assert np.array_equal(sim.seq, seq)
     assert np.array_equal(sim.photon.view(np.uint32), photon.view(np.uint32))
     sim.close()
+
+
+# gensteps on either side of what one block prefixes by itself, some without photons; photon
+# counts around a compaction tile (16,384 photons)
+@pytest.mark.parametrize("n_gs, total", [(1, 16384), (2047, 16385), (2048, 32767), (2049, 32768), (5000, 40001)])
+def test_event_setup_and_compaction_match_checker(n_gs, total):
+    g = np.random.default_rng(n_gs)
+    counts = np.zeros(n_gs, np.int64)
+    some = g.choice(n_gs, max(1, n_gs // 2), replace=False)
+    counts[some] = g.multinomial(total, np.full(len(some), 1.0 / len(some)))
+    w = configs.config0(num_photon=100)
+    one = configs.torch_genstep(1, configs.T_POINT_ISO, wavelength=300.0, weight=200.0)
+    gs = np.repeat(one[None], n_gs, 0).astype(np.float32)
+    gs[:, 1, :3] = g.uniform(-300, 300, (n_gs, 3))
+    gs.view(np.uint32)[:, 0, 3] = counts
+    photon, seq = po.World(w.geometry, w.physics).simulate(gs, event_idx=2, seed=5)
+    want = photon[(photon[:, 3, 3].view(np.uint32) & 0x40) != 0]
+    sim = QSim(w.geometry, w.physics, SEventConfig(seed=5))
+    dev = torch.device("cuda:0")
+    small = torch.from_numpy(w.gensteps).to(dev)
+    gs_t = torch.from_numpy(gs).to(dev)
+    photon_t = torch.zeros((total, 4, 4), dtype=torch.float32, device=dev)
+    seq_t = torch.zeros((total, 2, 2), dtype=torch.int64, device=dev)
+    hit_t = torch.zeros((total, 4, 4), dtype=torch.float32, device=dev)
+    # a first event smaller than the one that follows: its buffers have to grow
+    assert sim.simulate_device(small, photon_t, seq_t, hit_t) <= 100
+    for n_photon in (-1, total):
+        photon_t.zero_()
+        hit_t.zero_()
+        m = sim.simulate_device(gs_t, photon_t, seq_t, hit_t, eventID=2, n_photon=n_photon)
+        assert m == len(want)
+        assert np.array_equal(photon_t.cpu().numpy().view(np.uint32), photon.view(np.uint32))
+        assert np.array_equal(seq_t.cpu().numpy().view(np.uint64), seq)
+        assert np.array_equal(hit_t.cpu().numpy()[:m].view(np.uint32), want.view(np.uint32))
+    # refused on the device: nothing is written, and the next event is not disturbed
+    photon_t.zero_()
+    with pytest.raises(RuntimeError):
+        sim.simulate_device(gs_t, photon_t, seq_t, hit_t, eventID=2, n_photon=total + 1)
+    assert not photon_t.any()
+    assert sim.simulate_device(gs_t, photon_t, seq_t, hit_t, eventID=2) == len(want)
+    # a short hit buffer: the count is still reported, the hits that fit are in it
+    with pytest.raises(RuntimeError):
+        sim.simulate_device(gs_t, photon_t, seq_t, hit_t[:7], eventID=2)
+    assert np.array_equal(hit_t.cpu().numpy()[:7].view(np.uint32), want[:7].view(np.uint32))
+    sim.close()
