@@ -195,6 +195,18 @@ int  mi_sim_simulate(mi_sim* sim, int32_t event_id, const float* gensteps,
 int  mi_sim_reset(mi_sim* sim, int32_t event_id);
 
 /*
+ * mi_sim_simulate in two parts, for callers that own the result arrays: mi_sim_run
+ * propagates and reports the counts (its array pointers stay NULL), mi_sim_fetch copies
+ * that run's photon (n_photon,4,4), seq (n_photon,2,2) and hit (n_hit,4,4) arrays into the
+ * caller's host memory (NULL: not wanted) until the handle's next host call or reset.
+ * mi_host_alloc gives pinned memory, into which the copies run at the link's full rate.
+ */
+int  mi_sim_run(mi_sim* sim, int32_t event_id, const float* gensteps, int64_t n_gs, mi_event_out* out);
+int  mi_sim_fetch(mi_sim* sim, float* photon, uint64_t* seq, float* hit);
+int  mi_host_alloc(size_t bytes, void** ptr);
+void mi_host_free(void* ptr);
+
+/*
  * Device-resident form. d_gensteps: (n_gs,6,4) in device memory.
  * n_photon: photons to propagate, at most the gensteps' total (a smaller
  * count propagates that prefix), or -1 for the total; a larger n_photon fails

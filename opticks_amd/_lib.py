@@ -75,7 +75,8 @@ SYMBOLS = ["mi_config_default", "mi_last_error", "mi_version", "mi_sim_create", 
            "mi_sim_last_adjoint_timing", "mi_batch_create", "mi_batch_launch", "mi_batch_wait",
            "mi_batch_num_photon", "mi_batch_destroy", "mi_sim_autotune", "mi_batch_create_adjoint",
            "mi_batch_last_timing", "mi_sim_merge_hits_device", "mi_sim_simulate_lite_device",
-           "mi_sim_simtrace_device", "mi_sim_simtrace", "mi_sim_simulate_device_noalloc"]
+           "mi_sim_simtrace_device", "mi_sim_simtrace", "mi_sim_simulate_device_noalloc", "mi_sim_run",
+           "mi_sim_fetch", "mi_host_alloc", "mi_host_free"]
 
 _lib = None
 
@@ -96,6 +97,11 @@ def lib():
     L.mi_sim_set_config.argtypes = [C.c_void_p, C.POINTER(MiConfig)]
     L.mi_sim_get_config.argtypes = [C.c_void_p, C.POINTER(MiConfig)]
     L.mi_sim_simulate.argtypes = [C.c_void_p, C.c_int32, C.c_void_p, C.c_int64, C.POINTER(MiEventOut)]
+    L.mi_sim_run.argtypes = L.mi_sim_simulate.argtypes
+    L.mi_sim_fetch.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
+    L.mi_host_alloc.argtypes = [C.c_size_t, C.POINTER(C.c_void_p)]
+    L.mi_host_free.argtypes = [C.c_void_p]
+    L.mi_host_free.restype = None
     L.mi_sim_reset.argtypes = [C.c_void_p, C.c_int32]
     L.mi_sim_simulate_device.argtypes = [C.c_void_p, C.c_int32, C.c_void_p, C.c_int64, C.c_int64, C.c_int64,
                                          C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64,
@@ -134,7 +140,7 @@ def lib():
                                   C.c_void_p, C.c_void_p, C.c_int64, C.c_int32, C.POINTER(MiTuneResult),
                                   C.c_int32, C.POINTER(C.c_int32)]
     for name in SYMBOLS:
-        if name not in ("mi_last_error", "mi_version", "mi_config_default", "mi_sim_destroy"):
+        if name not in ("mi_last_error", "mi_version", "mi_config_default", "mi_sim_destroy", "mi_host_free"):
             getattr(L, name).restype = C.c_int
     _lib = L
     return L

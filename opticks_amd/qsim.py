@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import threading
 from dataclasses import dataclass, field, fields
 
 import numpy as np
@@ -137,11 +138,75 @@ def _ptr(a):
     return a.ctypes.data if a is not None and len(a) else None
 
 
+class _HostBuffer:
+    """Pinned host memory behind result arrays; goes back to its pool, or is freed, when the
+    last array over it is gone."""
+
+    def __init__(self, pool, ptr, size):
+        self.pool, self.ptr, self.size = pool, ptr, size
+
+    def array(self, dtype, shape):
+        a = np.frombuffer(_view(self), dtype=dtype, count=int(np.prod(shape)))
+        return a.reshape(shape)
+
+    def __del__(self):
+        try:
+            if not self.pool.put(self.ptr, self.size):
+                L.lib().mi_host_free(self.ptr)
+        except Exception:               # the interpreter is ending
+            pass
+
+
+def _view(buffer):
+    """a writable ctypes view of the buffer that keeps it alive"""
+    v = (C.c_char * buffer.size).from_address(buffer.ptr)
+    v.buffer = buffer
+    return v
+
+
+class _HostPool:
+    """Pinned memory of dropped result arrays, kept for the next event's: at most `most`
+    buffers, given back on close. Arrays may be dropped by any thread."""
+
+    most = 6
+
+    def __init__(self):
+        self._lock = threading.RLock()       # a drop may run inside take() (garbage collection)
+        self._spare = []
+        self._open = True
+
+    def take(self, size):
+        with self._lock:
+            fit = [b for b in self._spare if size <= b[1] <= 2 * size + (1 << 20)]
+            if fit:
+                b = min(fit, key=lambda b: b[1])
+                self._spare.remove(b)
+                return _HostBuffer(self, *b)
+        p = C.c_void_p()
+        L.check(L.lib().mi_host_alloc(size, C.byref(p)), "mi_host_alloc")
+        return _HostBuffer(self, p.value, size)
+
+    def put(self, ptr, size):
+        with self._lock:
+            if not self._open or len(self._spare) >= self.most:
+                return False
+            self._spare.append((ptr, size))
+            return True
+
+    def close(self, final=True):
+        with self._lock:
+            spare, self._spare = self._spare, []
+            self._open = self._open and not final
+        for ptr, _ in spare:
+            L.lib().mi_host_free(ptr)
+
+
 class QSim:
     """One geometry + physics upload; events simulated against it."""
 
     def __init__(self, geometry: dict, physics: dict, config: SEventConfig | None = None):
         self.config = config or SEventConfig()
+        self._host = _HostPool()
         g = {k: np.ascontiguousarray(v) for k, v in geometry.items()}
         self._g = g
         itra = g.get("itra")
@@ -178,6 +243,7 @@ class QSim:
         if getattr(self, "handle", None):
             L.lib().mi_sim_destroy(self.handle)
             self.handle = None
+            self._host.close()
 
     def __del__(self):
         try:
@@ -203,26 +269,29 @@ class QSim:
         """gensteps (G,6,4) -> hits (M,4,4); photon/seq/hit kept on self."""
         gs = np.ascontiguousarray(gs, np.float32).reshape(-1, 6, 4)
         out = L.MiEventOut()
-        rc = L.lib().mi_sim_simulate(self.handle, eventID, gs.ctypes.data if len(gs) else None, len(gs),
-                                     C.byref(out))
+        rc = L.lib().mi_sim_run(self.handle, eventID, gs.ctypes.data if len(gs) else None, len(gs), C.byref(out))
         if rc == L.MI_NOTHING_TO_DO:
             self.photon = self.seq = self.hit = None
             return None
-        L.check(rc, "mi_sim_simulate")
+        L.check(rc, "mi_sim_run")
         n, m = out.n_photon, out.n_hit
         om = self.config.output_mask
-        self.photon = (np.ctypeslib.as_array((C.c_float * (16 * n)).from_address(out.photon)).reshape(n, 4, 4).copy()
-                       if out.photon else None)
-        self.seq = (np.ctypeslib.as_array((C.c_uint64 * (4 * n)).from_address(out.seq)).reshape(n, 2, 2).copy()
-                    if out.seq else None)
-        self.hit = (np.ctypeslib.as_array((C.c_float * (16 * max(m, 1))).from_address(out.hit))
-                    .reshape(-1, 4, 4)[:m].copy() if (out.hit and om & L.MI_OUT_HIT) else None)
+        # arrays of their own for every event, over pinned memory that the copies fill directly
+        new = {b: self._host.take(max(64, size)) if om & b else None
+               for b, size in ((L.MI_OUT_PHOTON, 64 * n), (L.MI_OUT_SEQ, 32 * n), (L.MI_OUT_HIT, 64 * m))}
+        photon, seq, hit = (new[b] for b in (L.MI_OUT_PHOTON, L.MI_OUT_SEQ, L.MI_OUT_HIT))
+        L.check(L.lib().mi_sim_fetch(self.handle, *(None if b is None else b.ptr for b in (photon, seq, hit))),
+                "mi_sim_fetch")
+        self.photon = None if photon is None else photon.array(np.float32, (n, 4, 4))
+        self.seq = None if seq is None else seq.array(np.uint64, (n, 2, 2))
+        self.hit = None if hit is None else hit.array(np.float32, (m, 4, 4))
         self.device_ms = out.device_ms
         return self.hit
 
     def reset(self, eventID: int = 0):
         L.check(L.lib().mi_sim_reset(self.handle, eventID), "mi_sim_reset")
         self.photon = self.seq = self.hit = None
+        self._host.close(final=False)
 
     def last_timing(self):
         t = (C.c_double * 4)()

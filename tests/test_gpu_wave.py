@@ -159,3 +159,26 @@ def test_event_setup_and_compaction_match_checker(n_gs, total):
         sim.simulate_device(gs_t, photon_t, seq_t, hit_t[:7], eventID=2)
     assert np.array_equal(hit_t.cpu().numpy()[:7].view(np.uint32), want[:7].view(np.uint32))
     sim.close()
+
+
+def test_event_arrays_are_their_own():
+    """Result arrays keep their values over later events, a reset and the handle's end, and
+    memory of dropped ones is used again, a bounded number of buffers of it."""
+    w = configs.config0(num_photon=1000)
+    sim = QSim(w.geometry, w.physics, SEventConfig(seed=1))
+    kept = []
+    for e in range(5):
+        hit = sim.simulate(w.gensteps, e)
+        kept.append((hit, sim.photon, sim.seq, hit.copy(), sim.photon.copy(), sim.seq.copy()))
+    sim.photon[0] = 0.0                                    # writable, and nobody else's
+    kept[-1][4][0] = 0.0
+    sim.reset()
+    for e in range(20):
+        sim.simulate(w.gensteps, 100 + e)                  # the arrays of the event before are dropped
+    assert len(sim._host._spare) <= sim._host.most
+    sim.close()
+    assert not sim._host._spare
+    for hit, photon, seq, hit0, photon0, seq0 in kept:
+        assert np.array_equal(hit.view(np.uint32), hit0.view(np.uint32))
+        assert np.array_equal(photon.view(np.uint32), photon0.view(np.uint32))
+        assert np.array_equal(seq, seq0)
