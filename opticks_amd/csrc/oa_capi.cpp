@@ -214,11 +214,11 @@ struct mi_sim {
     DBuf<unsigned char> adj_tmp;
     DBuf<int64_t> adj_seg;
     /* hit merging */
-    DBuf<uint8_t> m_flags;
-    DBuf<uint32_t> m_sel, m_vals, m_vals2;
-    DBuf<uint64_t> m_keys, m_keys2;
-    DBuf<int32_t> m_len, m_off, m_counts;
-    DBuf<unsigned char> m_tmp;
+    DBuf<uint4> m_sel;
+    DBuf<uint32_t> m_order, m_order2;
+    DBuf<unsigned char> m_keys, m_keys2, m_tmp;
+    DBuf<unsigned long long> m_state;
+    oa_merge::Result* m_result = nullptr;           /* pinned */
 };
 
 extern "C" {
@@ -740,9 +740,9 @@ void mi_sim_destroy(mi_sim* sim)
     sim->tape.release(); sim->tape_n.release(); sim->tape_flag.release();
     sim->adj_key.release(); sim->adj_val.release(); sim->adj_key2.release(); sim->adj_val2.release();
     sim->adj_tmp.release(); sim->adj_seg.release();
-    sim->m_flags.release(); sim->m_sel.release(); sim->m_vals.release(); sim->m_vals2.release();
-    sim->m_keys.release(); sim->m_keys2.release(); sim->m_len.release(); sim->m_off.release();
-    sim->m_counts.release(); sim->m_tmp.release();
+    sim->m_sel.release(); sim->m_order.release(); sim->m_order2.release(); sim->m_keys.release(); sim->m_keys2.release();
+    sim->m_tmp.release(); sim->m_state.release();
+    if (sim->m_result) (void)hipHostFree(sim->m_result);
     sim->h_photon.release(); sim->h_seq.release(); sim->h_hit.release(); sim->h_simtrace.release();
     for (auto& e : sim->ev) if (e) (void)hipEventDestroy(e);
     if (sim->stream) (void)hipStreamDestroy(sim->stream);
@@ -1552,43 +1552,49 @@ int mi_sim_merge_hits_device(mi_sim* sim, int32_t record, const void* d_in, int6
     if (out_capacity < 0 || (out_capacity > 0 && !d_out)) return fail(MI_ERR_ARG, "bad output buffer");
     if (n_in == 0) return MI_OK;
     hipStream_t s = stream ? (hipStream_t)stream : sim->stream;
-    const size_t n = (size_t)n_in;
-    HIPCHECK(sim->m_flags.reserve(n));
-    HIPCHECK(sim->m_sel.reserve(n));
-    HIPCHECK(sim->m_vals.reserve(n));
-    HIPCHECK(sim->m_vals2.reserve(n));
-    HIPCHECK(sim->m_keys.reserve(n));
-    HIPCHECK(sim->m_keys2.reserve(n));
-    HIPCHECK(sim->m_len.reserve(n));
-    HIPCHECK(sim->m_off.reserve(n));
-    HIPCHECK(sim->m_counts.reserve(2));
-    const size_t tmp_bytes = std::max<size_t>(1, oa_merge::scratch_bytes(n_in));
-    HIPCHECK(sim->m_tmp.reserve(tmp_bytes));
-    oa_merge::Scratch S{ sim->m_flags.p, sim->m_sel.p, sim->m_vals.p, sim->m_vals2.p, sim->m_keys.p, sim->m_keys2.p,
-                         sim->m_len.p, sim->m_off.p, sim->m_counts.p, sim->m_tmp.p, tmp_bytes };
+    if (!sim->m_result) HIPCHECK(hipHostMalloc((void**)&sim->m_result, sizeof(oa_merge::Result), hipHostMallocDefault));
+    HIPCHECK(sim->m_sel.reserve((size_t)n_in));
+    HIPCHECK(sim->m_state.reserve((size_t)oa_merge::state_words(n_in)));
     const int rec = record == MI_RECORD_PHOTON ? OA_MERGE_PHOTON : OA_MERGE_PHOTONLITE;
-    HIPCHECK(oa_merge::select(S, rec, d_in, n_in, select_mask, s));
-    int32_t cnt[2] = { 0, 0 };
-    HIPCHECK(hipMemcpyAsync(cnt, sim->m_counts.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    const volatile oa_merge::Result* res = sim->m_result;
+    /* the window decides the largest bucket; without one there are no keys */
+    HIPCHECK(oa_merge::select(rec, d_in, n_in, select_mask, time_window > 0.f ? time_window : 1.f, sim->m_state.p,
+                              sim->m_sel.p, sim->m_result, s));
     HIPCHECK(hipStreamSynchronize(s));
-    const int64_t n_sel = cnt[0];
+    const int64_t n_sel = res->n_sel;
     if (n_sel == 0) return MI_OK;
     if (time_window == 0.f) {
         /* selection only, input order (SPM::NOMERGE_TIME_WINDOW) */
         *n_out = n_sel;
         if (n_sel > out_capacity) return fail(MI_ERR_CAPACITY, "out_capacity too small: " + std::to_string(n_sel) + " records");
-        HIPCHECK(oa_merge::gather_selected(S, rec, d_in, d_out, n_sel, s));
+        HIPCHECK(oa_merge::gather_selected(rec, d_in, sim->m_sel.p, n_sel, d_out, s));
         HIPCHECK(hipStreamSynchronize(s));
         return MI_OK;
     }
-    HIPCHECK(oa_merge::sort_runs(S, rec, d_in, n_sel, time_window, s));
-    HIPCHECK(hipMemcpyAsync(cnt + 1, sim->m_counts.p + 1, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIPCHECK(hipStreamSynchronize(s));
-    const int64_t n_runs = cnt[1];
+    const uint32_t max_bucket = res->max_bucket;
+    const int bits = oa_merge::key_bits(res->max_id, max_bucket);
+    const size_t key_bytes = (size_t)n_sel * (bits <= 32 ? 4 : 8);
+    const size_t tmp_bytes = std::max<size_t>(1, oa_merge::sort_bytes(n_sel, bits));
+    HIPCHECK(sim->m_keys.reserve(key_bytes));
+    HIPCHECK(sim->m_keys2.reserve(key_bytes));
+    HIPCHECK(sim->m_order.reserve((size_t)n_sel));
+    HIPCHECK(sim->m_order2.reserve((size_t)n_sel));
+    HIPCHECK(sim->m_tmp.reserve(tmp_bytes));
+    HIPCHECK(oa_merge::sort_runs(sim->m_sel.p, n_sel, time_window, max_bucket, bits, sim->m_keys.p, sim->m_keys2.p,
+                                 sim->m_order.p, sim->m_order2.p, sim->m_tmp.p, tmp_bytes, s));
+    const auto reduce = [&](int64_t cap) -> int {
+        HIPCHECK(oa_merge::reduce_runs(rec, d_in, sim->m_sel.p, n_sel, bits, sim->m_keys2.p, sim->m_order2.p,
+                                       sim->m_state.p, d_out, cap, sim->m_result, s));
+        HIPCHECK(hipStreamSynchronize(s));
+        return MI_OK;
+    };
+    /* a buffer that may be too small is left as it is unless the runs, counted first, fit */
+    const bool sure = n_sel <= out_capacity;
+    if (const int rc = reduce(sure ? out_capacity : 0)) return rc;
+    const int64_t n_runs = res->n_runs;
     *n_out = n_runs;
     if (n_runs > out_capacity) return fail(MI_ERR_CAPACITY, "out_capacity too small: " + std::to_string(n_runs) + " records");
-    HIPCHECK(oa_merge::reduce_runs(S, rec, d_in, d_out, n_runs, s));
-    HIPCHECK(hipStreamSynchronize(s));
+    if (!sure) return reduce(out_capacity);
     return MI_OK;
 }
 

@@ -130,3 +130,40 @@ def test_photonlite_output_matches_checker_and_merges():
         assert np.array_equal(out, ref)
     assert np.array_equal(out, spm.merge_lites(G, SD, 1.0))
     sim.close()
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 4095, 4096, 4097, 3 * 4096 + 17, 300_001])
+def test_merge_tiles_and_key_widths(sim_and_photons, n):
+    """Sizes around the 4096-record tiles; keys of few bits, of more than 32, of one value, of
+    buckets up to 32 bits; long and single-record runs."""
+    sim, _ = sim_and_photons
+    rng = np.random.default_rng(n)
+    late = np.array([0.0, 1.0, 2.1e9], np.float32)
+    for kind in ("narrow", "wide", "one", "late"):
+        P = synthetic(n, n + 1)
+        u = P.view(np.uint32)
+        if kind == "wide":
+            P[:, 0, 3] = rng.random(n).astype(np.float32) * 4.0e6
+            u[:, 3, 1] = rng.integers(0, 65536, n).astype(np.uint32)
+        if kind == "one":
+            P[:, 0, 3], u[:, 3, 1] = 0.0, 0
+        if kind == "late":
+            P[:, 0, 3] = rng.choice(late, n)
+        lt = np.stack([(u[:, 1, 3] & 0xFFFF0000) | (u[:, 3, 1] & 0xFFFF), u[:, 0, 3], np.arange(n, dtype=np.uint32),
+                       u[:, 3, 3]], axis=1).astype(np.uint32)
+        t, tl = torch.from_numpy(P).to(DEV), torch.from_numpy(lt.view(np.int32)).to(DEV)
+        for tw in (0.5, 0.0):
+            ref, refl = spm.merge_photons(P, SD, tw), spm.merge_lites(lt, SD, tw)
+            for rows, merged, ref_bits in ((t, sim.merge_hits_device(t, SD, tw), ref.view(np.uint32)),
+                                           (tl, sim.merge_hits_device(tl, SD, tw), refl)):
+                got = merged.cpu().numpy().view(np.uint32)
+                assert got.shape == ref_bits.shape and np.array_equal(got, ref_bits), (kind, tw)
+                tight = torch.full((len(ref_bits),) + tuple(rows.shape[1:]), 0, dtype=rows.dtype, device=DEV)
+                if len(ref_bits):                  # a buffer of just the merged size, then one short of it
+                    sim.merge_hits_device(rows, SD, tw, out_t=tight)
+                    assert np.array_equal(tight.cpu().numpy().view(np.uint32), ref_bits), (kind, tw)
+                if len(ref_bits) > 1:
+                    short = torch.zeros_like(tight)[:-1].contiguous()
+                    with pytest.raises(RuntimeError, match="out_capacity"):
+                        sim.merge_hits_device(rows, SD, tw, out_t=short)
+                    assert not short.cpu().numpy().any()
