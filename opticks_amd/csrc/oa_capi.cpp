@@ -217,7 +217,8 @@ struct mi_sim {
     DBuf<uint4> m_sel;
     DBuf<uint32_t> m_order, m_order2;
     DBuf<unsigned char> m_keys, m_keys2, m_tmp;
-    DBuf<unsigned long long> m_state;
+    DBuf<int32_t> m_count;
+    DBuf<uint2> m_most;
     oa_merge::Result* m_result = nullptr;           /* pinned */
 };
 
@@ -741,7 +742,7 @@ void mi_sim_destroy(mi_sim* sim)
     sim->adj_key.release(); sim->adj_val.release(); sim->adj_key2.release(); sim->adj_val2.release();
     sim->adj_tmp.release(); sim->adj_seg.release();
     sim->m_sel.release(); sim->m_order.release(); sim->m_order2.release(); sim->m_keys.release(); sim->m_keys2.release();
-    sim->m_tmp.release(); sim->m_state.release();
+    sim->m_tmp.release(); sim->m_count.release(); sim->m_most.release();
     if (sim->m_result) (void)hipHostFree(sim->m_result);
     sim->h_photon.release(); sim->h_seq.release(); sim->h_hit.release(); sim->h_simtrace.release();
     for (auto& e : sim->ev) if (e) (void)hipEventDestroy(e);
@@ -1554,12 +1555,13 @@ int mi_sim_merge_hits_device(mi_sim* sim, int32_t record, const void* d_in, int6
     hipStream_t s = stream ? (hipStream_t)stream : sim->stream;
     if (!sim->m_result) HIPCHECK(hipHostMalloc((void**)&sim->m_result, sizeof(oa_merge::Result), hipHostMallocDefault));
     HIPCHECK(sim->m_sel.reserve((size_t)n_in));
-    HIPCHECK(sim->m_state.reserve((size_t)oa_merge::state_words(n_in)));
+    HIPCHECK(sim->m_count.reserve(oa_merge::count_words(n_in)));
+    HIPCHECK(sim->m_most.reserve(oa_merge::most_words(n_in)));
     const int rec = record == MI_RECORD_PHOTON ? OA_MERGE_PHOTON : OA_MERGE_PHOTONLITE;
     const volatile oa_merge::Result* res = sim->m_result;
     /* the window decides the largest bucket; without one there are no keys */
-    HIPCHECK(oa_merge::select(rec, d_in, n_in, select_mask, time_window > 0.f ? time_window : 1.f, sim->m_state.p,
-                              sim->m_sel.p, sim->m_result, s));
+    HIPCHECK(oa_merge::select(rec, d_in, n_in, select_mask, time_window > 0.f ? time_window : 1.f, sim->m_count.p,
+                              sim->m_most.p, sim->m_sel.p, sim->m_result, s));
     HIPCHECK(hipStreamSynchronize(s));
     const int64_t n_sel = res->n_sel;
     if (n_sel == 0) return MI_OK;
@@ -1567,7 +1569,7 @@ int mi_sim_merge_hits_device(mi_sim* sim, int32_t record, const void* d_in, int6
         /* selection only, input order (SPM::NOMERGE_TIME_WINDOW) */
         *n_out = n_sel;
         if (n_sel > out_capacity) return fail(MI_ERR_CAPACITY, "out_capacity too small: " + std::to_string(n_sel) + " records");
-        HIPCHECK(oa_merge::gather_selected(rec, d_in, sim->m_sel.p, n_sel, d_out, s));
+        HIPCHECK(oa_merge::gather_selected(rec, d_in, n_in, sim->m_count.p, sim->m_sel.p, d_out, s));
         HIPCHECK(hipStreamSynchronize(s));
         return MI_OK;
     }
@@ -1580,21 +1582,20 @@ int mi_sim_merge_hits_device(mi_sim* sim, int32_t record, const void* d_in, int6
     HIPCHECK(sim->m_order.reserve((size_t)n_sel));
     HIPCHECK(sim->m_order2.reserve((size_t)n_sel));
     HIPCHECK(sim->m_tmp.reserve(tmp_bytes));
-    HIPCHECK(oa_merge::sort_runs(sim->m_sel.p, n_sel, time_window, max_bucket, bits, sim->m_keys.p, sim->m_keys2.p,
-                                 sim->m_order.p, sim->m_order2.p, sim->m_tmp.p, tmp_bytes, s));
-    const auto reduce = [&](int64_t cap) -> int {
-        HIPCHECK(oa_merge::reduce_runs(rec, d_in, sim->m_sel.p, n_sel, bits, sim->m_keys2.p, sim->m_order2.p,
-                                       sim->m_state.p, d_out, cap, sim->m_result, s));
-        HIPCHECK(hipStreamSynchronize(s));
-        return MI_OK;
-    };
-    /* a buffer that may be too small is left as it is unless the runs, counted first, fit */
+    HIPCHECK(oa_merge::sort_runs(n_in, sim->m_count.p, sim->m_sel.p, n_sel, time_window, max_bucket, bits, sim->m_keys.p,
+                                 sim->m_keys2.p, sim->m_order.p, sim->m_order2.p, sim->m_tmp.p, tmp_bytes, s));
+    HIPCHECK(oa_merge::count_runs(n_in, sim->m_count.p, n_sel, bits, sim->m_keys2.p, sim->m_result, s));
+    /* a buffer that may be too small is left as it is unless the runs fit */
     const bool sure = n_sel <= out_capacity;
-    if (const int rc = reduce(sure ? out_capacity : 0)) return rc;
+    if (!sure) HIPCHECK(hipStreamSynchronize(s));
+    if (sure || res->n_runs <= out_capacity) {
+        HIPCHECK(oa_merge::reduce_runs(rec, d_in, n_in, sim->m_count.p, sim->m_sel.p, n_sel, bits, sim->m_keys2.p,
+                                       sim->m_order2.p, d_out, out_capacity, s));
+        HIPCHECK(hipStreamSynchronize(s));
+    }
     const int64_t n_runs = res->n_runs;
     *n_out = n_runs;
     if (n_runs > out_capacity) return fail(MI_ERR_CAPACITY, "out_capacity too small: " + std::to_string(n_runs) + " records");
-    if (!sure) return reduce(out_capacity);
     return MI_OK;
 }
 

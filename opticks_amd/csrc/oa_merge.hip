@@ -16,14 +16,19 @@
  *   sphotonlite 16 B  key/reduce/select  sysrap/sphotonlite.h:68-97
  *
  * One pass reads the records (k_select) and keeps of each selected one the 16 bytes that the
- * merge needs; bound by the lines it has to fetch, 64 B a photon record for any word of it
- * (640 MB for 10M records, 113 us at 5.7 TB/s). The keys are as wide as the selection's largest
- * identity and bucket need, 20 bits for 2,000 sensors and 400 buckets instead of 48: three
- * radix passes over 8-byte pairs instead of six over 12. k_reduce finds the runs and folds
- * each from the kept words, left to right in sorted order, so ties in time keep the earliest
- * record in input order; only the record that a run keeps is fetched.
- * 10M records, 2M selected, 0.7M merged: 662 us before (flag pass, flagged select, key pass,
- * 48-bit sort, run-length encode, scan, reduce over the records themselves).
+ * merge needs, tile by tile, with a count per tile; one block sums the counts (k_tile_offsets)
+ * and the keys go to their places by them. Bound by the lines k_select has to fetch, 64 B a
+ * photon record for any word of it. The keys are as wide as the selection's largest identity
+ * and bucket need, 20 bits for 2,000 sensors and 400 buckets instead of 48: three radix passes
+ * over 8-byte pairs instead of six over 12. k_reduce finds the runs again tile by tile and
+ * folds each from the kept words, left to right in sorted order, so ties in time keep the
+ * earliest record in input order; only the record that a run keeps is fetched.
+ * The tiles' offsets come from a small kernel between two passes: a look-back across the tiles
+ * needs a ticket each, and tickets, one atomic on one word, come at 40-60 ns apiece over eight
+ * L2s (k_select 180 us with 2,441 tiles, 665 with 4,883 and two atomics a tile).
+ * 10M records, 2M selected, 0.7M merged: 662 -> 384 us (select 139, keys 11, sort 115 with its
+ * fills, reduce 64; the rest gaps). Before, a flag pass, flagged select, key pass, 48-bit sort,
+ * run-length encode and scan, and a reduce over the records themselves.
  */
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
@@ -56,171 +61,209 @@ typedef uint32_t quad __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ inline uint32_t bucket_of(uint32_t time, float tw) { return (uint32_t)(__uint_as_float(time) / tw); }
 
-/* 16 rounds of 256 records or sorted keys make a tile */
-#define OA_TILE_ROUNDS 16
-#define OA_TILE (256 * OA_TILE_ROUNDS)
+/* rounds of 256 items that make a tile: records of the selection (their loads are all in
+   flight at once), and sorted keys */
+#define OA_SELECT_ROUNDS 8
+#define OA_REDUCE_ROUNDS 4
 
 /*
- * Items of the tiles before `tile`, by a decoupled look-back over state[tile]: 0, then
- * count | 1 << 62, then (items up to its end) | 2 << 62 (as the hit compaction does it). Run by
- * one wave; the tiles are handed out by ticket, so those before it are running or done.
+ * Ranks of a tile's items, of which thread t marks item 256 k + t by bit k of `marked`: s_pre
+ * gets the items before each of the 4 x ROUNDS ballots, rank_in_tile the item's own.
  */
-__device__ int64_t look_back(unsigned long long* state, int64_t tile, int64_t total, int lane)
+template <int ROUNDS>
+__device__ int32_t tile_ranks(uint32_t marked, unsigned long long* s_mask, int32_t* s_pre)
 {
-    const unsigned long long kCount = 1ull << 62, kDone = 2ull << 62, kValue = kCount - 1ull;
-    int64_t base = 0;
-    if (tile > 0) {
-        if (lane == 0)
-            __hip_atomic_store(&state[tile], kCount | (unsigned long long)total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (int64_t k = tile - 1;; k -= 64) {
-            const int64_t mine = k - lane;
-            unsigned long long v = kDone;
-            do {
-                if (mine >= 0) v = __hip_atomic_load(&state[mine], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } while (__ballot(v < kCount) != 0ull);
-            const unsigned long long ends = __ballot(v >= kDone);
-            const int last = ends ? __ffsll((long long)ends) - 1 : 63;
-            int64_t sum = lane <= last ? (int64_t)(v & kValue) : 0;
-            for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-            base += sum;
-            if (ends) break;
-        }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < ROUNDS; ++k) {
+        const unsigned long long m = __ballot(marked >> k & 1u);
+        if (lane == 0) s_mask[4 * k + wave] = m;
     }
-    if (lane == 0)
-        __hip_atomic_store(&state[tile], kDone | (unsigned long long)(base + total), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    return base;
-}
-
-/* The tile's 64 ballot words (4 waves x 16 rounds, in item order) to the items before each word
-   (s_pre) and before the tile (returned to every thread); total: the tile's items */
-__device__ int64_t tile_prefix(const unsigned long long* s_mask, int32_t* s_pre, int64_t* s_base, unsigned long long* state,
-                               int64_t tile, int32_t& total)
-{
     __syncthreads();
-    if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        const int32_t c = __popcll(s_mask[lane]);
+    if (wave == 0) {
+        const int32_t c = lane < 4 * ROUNDS ? __popcll(s_mask[lane]) : 0;
         int32_t incl = c;
         for (int o = 1; o < 64; o <<= 1) {
             const int32_t v = __shfl_up(incl, o);
             if (lane >= o) incl += v;
         }
-        s_pre[lane] = incl - c;
-        const int32_t all = __shfl(incl, 63);
-        if (lane == 63) s_pre[64] = all;
-        const int64_t base = look_back(state, tile, all, lane);
-        if (lane == 0) *s_base = base;
+        if (lane < 4 * ROUNDS) s_pre[lane] = incl - c;
+        if (lane == 63) s_pre[4 * ROUNDS] = incl;
     }
     __syncthreads();
-    total = s_pre[64];
-    return *s_base;
+    return s_pre[4 * ROUNDS];
 }
 
+__device__ inline int32_t rank_in_tile(int k, const unsigned long long* s_mask, const int32_t* s_pre)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    return s_pre[4 * k + wave] + __popcll(s_mask[4 * k + wave] & ((1ull << lane) - 1ull));
+}
+
+/* a tile's selected, in input order, at the tile's own place in sel; count[tile] of them, and
+   the largest identity and bucket */
 template <class Acc>
 __global__ void __launch_bounds__(256) k_select(const uint32_t* __restrict__ in, int64_t n, uint32_t mask, float tw,
-                                                int64_t n_tiles, unsigned long long* state, uint4* __restrict__ sel,
-                                                oa_merge::Result* out)
+                                                int32_t* count, uint2* most, uint4* __restrict__ sel)
 {
-    __shared__ unsigned long long s_mask[64];
-    __shared__ int32_t s_pre[65];
-    __shared__ int64_t s_tile, s_base;
+    constexpr int ROUNDS = OA_SELECT_ROUNDS;
+    __shared__ unsigned long long s_mask[4 * ROUNDS];
+    __shared__ int32_t s_pre[4 * ROUNDS + 1];
     __shared__ uint32_t s_max[2];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    if (t == 0) { s_tile = (int64_t)atomicAdd(&state[n_tiles], 1ull); s_max[0] = s_max[1] = 0u; }
-    __syncthreads();
-    const int64_t tile = s_tile;
-    if (tile >= n_tiles) return;
-    uint4 v[OA_TILE_ROUNDS];
+    if (threadIdx.x < 2) s_max[threadIdx.x] = 0u;
+    const int64_t tile = (int64_t)blockIdx.x * (256 * ROUNDS), first = tile + threadIdx.x;
+    uint4 v[ROUNDS];
     uint32_t taken = 0, max_id = 0, max_bucket = 0;
 #pragma unroll
-    for (int k = 0; k < OA_TILE_ROUNDS; ++k) {
-        const int64_t i = tile * OA_TILE + k * 256 + t;
-        const uint32_t* r = in + i * Acc::WORDS;
-        const uint32_t fm = i < n ? Acc::flagmask(r) : 0u;
-        const bool take = i < n && (mask == OA_MERGE_ALREADY_SELECTED || (fm & mask) != 0u);
-        if (take) {
-            v[k] = make_uint4((uint32_t)i, Acc::time(r), Acc::identity(r) | (Acc::hitcount(r) << 16), fm);
-            taken |= 1u << k;
-        }
-        const unsigned long long m = __ballot(take);
-        if (lane == 0) s_mask[4 * k + wave] = m;
+    for (int k = 0; k < ROUNDS; ++k) {
+        const int64_t i = first + k * 256;
+        const uint32_t* r = in + (i < n ? i : n - 1) * Acc::WORDS;
+        v[k] = make_uint4((uint32_t)i, Acc::time(r), Acc::identity(r) | (Acc::hitcount(r) << 16), Acc::flagmask(r));
     }
 #pragma unroll
-    for (int k = 0; k < OA_TILE_ROUNDS; ++k) {
-        if (!(taken >> k & 1u)) continue;
-        max_id = max(max_id, v[k].z & 0xffffu);
-        max_bucket = max(max_bucket, bucket_of(v[k].y, tw));
+    for (int k = 0; k < ROUNDS; ++k) {
+        const bool take = first + k * 256 < n && (mask == OA_MERGE_ALREADY_SELECTED || (v[k].w & mask) != 0u);
+        taken |= (uint32_t)take << k;
+        max_id = max(max_id, take ? v[k].z & 0xffffu : 0u);
+        max_bucket = max(max_bucket, take ? bucket_of(v[k].y, tw) : 0u);
+    }
+    const int32_t total = tile_ranks<ROUNDS>(taken, s_mask, s_pre);
+#pragma unroll
+    for (int k = 0; k < ROUNDS; ++k)
+        if (taken >> k & 1u) sel[tile + rank_in_tile(k, s_mask, s_pre)] = v[k];
+    for (int o = 32; o > 0; o >>= 1) {
+        max_id = max(max_id, (uint32_t)__shfl_xor((int)max_id, o));
+        max_bucket = max(max_bucket, (uint32_t)__shfl_xor((int)max_bucket, o));
+    }
+    if ((threadIdx.x & 63) == 0) { atomicMax(&s_max[0], max_id); atomicMax(&s_max[1], max_bucket); }
+    __syncthreads();
+    if (threadIdx.x == 0) { count[blockIdx.x] = total; most[blockIdx.x] = make_uint2(s_max[0], s_max[1]); }
+}
+
+/* count[0..n) to the items before each tile, in place, and their total into count[n]; that and
+   the largest of `most` (null: none) into the host-visible out. One block: 8,192 tiles a step. */
+__global__ void __launch_bounds__(1024) k_tile_offsets(int32_t* count, const uint2* most, int64_t n, int64_t* total_out,
+                                                       oa_merge::Result* out)
+{
+    constexpr int EACH = 8;
+    __shared__ int32_t s_wave[16];
+    __shared__ uint32_t s_max[2];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    if (t < 2) s_max[t] = 0u;
+    int32_t base = 0;
+    uint32_t max_id = 0, max_bucket = 0;
+    for (int64_t i0 = 0; i0 < n; i0 += 1024 * EACH) {
+        const int64_t i = i0 + (int64_t)t * EACH;
+        int32_t c[EACH], sum = 0;
+#pragma unroll
+        for (int u = 0; u < EACH; ++u) c[u] = i + u < n ? count[i + u] : 0;
+        if (most) {
+#pragma unroll
+            for (int u = 0; u < EACH; ++u) {
+                const uint2 m = most[i + u < n ? i + u : n - 1];
+                max_id = max(max_id, m.x);
+                max_bucket = max(max_bucket, m.y);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < EACH; ++u) sum += c[u];
+        int32_t incl = sum;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int32_t v = __shfl_up(incl, o);
+            if (lane >= o) incl += v;
+        }
+        __syncthreads();
+        if (lane == 63) s_wave[wave] = incl;
+        __syncthreads();
+        int32_t before = base + incl - sum;
+        for (int w = 0; w < 16; ++w) {
+            if (w < wave) before += s_wave[w];
+            base += s_wave[w];
+        }
+#pragma unroll
+        for (int u = 0; u < EACH; ++u) {
+            if (i + u < n) count[i + u] = before;
+            before += c[u];
+        }
     }
     for (int o = 32; o > 0; o >>= 1) {
         max_id = max(max_id, (uint32_t)__shfl_xor((int)max_id, o));
         max_bucket = max(max_bucket, (uint32_t)__shfl_xor((int)max_bucket, o));
     }
+    __syncthreads();
     if (lane == 0) { atomicMax(&s_max[0], max_id); atomicMax(&s_max[1], max_bucket); }
-    int32_t total;
-    const int64_t base = tile_prefix(s_mask, s_pre, &s_base, state, tile, total);
-    /* the running maxima: both in one word each, touched only by tiles that raise them */
-    unsigned long long* maxima = state + n_tiles + 1;
-    if (t < 2 && (unsigned long long)s_max[t] > __hip_atomic_load(&maxima[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(&maxima[t], (unsigned long long)s_max[t]);
-#pragma unroll
-    for (int k = 0; k < OA_TILE_ROUNDS; ++k) {
-        if (!(taken >> k & 1u)) continue;
-        const unsigned long long m = s_mask[4 * k + wave];
-        sel[base + s_pre[4 * k + wave] + __popcll(m & ((1ull << lane) - 1ull))] = v[k];
-    }
-    if (tile == n_tiles - 1 && t == 0) out->n_sel = base + total;
+    __syncthreads();
+    if (t > 0) return;
+    count[n] = base;
+    *total_out = base;
+    if (most) { out->max_id = s_max[0]; out->max_bucket = s_max[1]; }
 }
 
-/* the maxima are complete when k_select is */
-__global__ void k_maxima(const unsigned long long* maxima, oa_merge::Result* out)
-{
-    out->max_id = (uint32_t)maxima[0];
-    out->max_bucket = (uint32_t)maxima[1];
-}
-
-__global__ void k_clear(unsigned long long* p, int64_t n)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0ull;
-}
-
-/* QUADS lanes copy a record */
+/* a tile's selected records to their places, QUADS lanes copying each */
 template <int QUADS>
-__global__ void __launch_bounds__(256) k_gather(const quad* __restrict__ in, const uint4* __restrict__ sel, int64_t n,
-                                                quad* __restrict__ out)
+__global__ void __launch_bounds__(256) k_gather(const quad* __restrict__ in, const uint4* __restrict__ sel,
+                                                const int32_t* __restrict__ offset, quad* __restrict__ out)
 {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= n * QUADS) return;
-    out[t] = in[(int64_t)sel[t / QUADS].x * QUADS + t % QUADS];
+    const int64_t tile = (int64_t)blockIdx.x * (256 * OA_SELECT_ROUNDS), o = offset[blockIdx.x];
+    const int32_t c = (int32_t)(offset[blockIdx.x + 1] - o);
+    for (int32_t i = threadIdx.x; i < c * QUADS; i += 256)
+        out[o * QUADS + i] = in[(int64_t)sel[tile + i / QUADS].x * QUADS + i % QUADS];
+}
+
+/* a tile's keys, and the places in sel that they belong to, to their places */
+template <class Key>
+__global__ void __launch_bounds__(256) k_keys(const uint4* __restrict__ sel, const int32_t* __restrict__ offset, float tw,
+                                              int bucket_bits, Key* __restrict__ keys, uint32_t* __restrict__ order)
+{
+    const int64_t tile = (int64_t)blockIdx.x * (256 * OA_SELECT_ROUNDS), o = offset[blockIdx.x];
+    const int32_t c = (int32_t)(offset[blockIdx.x + 1] - o);
+    for (int32_t i = threadIdx.x; i < c; i += 256) {
+        const uint4 v = sel[tile + i];
+        keys[o + i] = (Key)(v.z & 0xffffu) << bucket_bits | (Key)bucket_of(v.y, tw);
+        order[o + i] = (uint32_t)(tile + i);
+    }
+}
+
+/* the sorted keys of a tile at which a run starts, one bit a round */
+template <class Key>
+__device__ uint32_t run_heads(const Key* keys, int64_t n, int64_t first)
+{
+    uint32_t heads = 0;
+#pragma unroll
+    for (int k = 0; k < OA_REDUCE_ROUNDS; ++k) {
+        const int64_t i = first + k * 256;
+        const bool head = i < n && (i == 0 || keys[i] != keys[i - 1]);
+        heads |= (uint32_t)head << k;
+    }
+    return heads;
 }
 
 template <class Key>
-__global__ void __launch_bounds__(256) k_keys(const uint4* __restrict__ sel, int64_t n, float tw, int bucket_bits,
-                                              Key* __restrict__ keys, uint32_t* __restrict__ order)
+__global__ void __launch_bounds__(256) k_count_runs(const Key* __restrict__ keys, int64_t n, int32_t* count)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const uint4 v = sel[i];
-    keys[i] = (Key)(v.z & 0xffffu) << bucket_bits | (Key)bucket_of(v.y, tw);
-    order[i] = (uint32_t)i;
+    __shared__ int32_t s_n[4];
+    int32_t c = __popc(run_heads(keys, n, (int64_t)blockIdx.x * (256 * OA_REDUCE_ROUNDS) + threadIdx.x));
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+    if ((threadIdx.x & 63) == 0) s_n[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) count[blockIdx.x] = s_n[0] + s_n[1] + s_n[2] + s_n[3];
 }
 
 /*
- * The merged record of the run of equal keys that starts at sorted position o, folded left to
- * right with the record type's reduce_op, four records' words in flight a step:
+ * The merged record of the run of `len` equal keys at sorted position o (of at least len when
+ * `open`: it goes on as long as the keys do), folded left to right with the record type's
+ * reduce_op, four records' words in flight a step:
  *   sphoton      r = (fminf(a.time, b.time) == a.time) ? a : b; flagmasks OR-ed, 16-bit
  *                hitcounts added
  *   sphotonlite  r = a; r.time = fminf(a.time, b.time); likewise (first: a's input index)
  * x: input index of the kept record, y: time, z: hitcount, w: flagmask
  */
 template <bool LITE, class Key>
-__device__ uint4 fold_run(const uint4* sel, const Key* keys, const uint32_t* order, int64_t n, int64_t o)
+__device__ uint4 fold_run(const uint4* sel, const Key* keys, const uint32_t* order, int64_t n, int64_t o, int32_t len,
+                          bool open)
 {
-    const Key key = keys[o];
-    const uint4 a = sel[order[o]];
-    uint32_t best = a.x, fm = a.w, hc = a.z >> 16;
-    float bt = __uint_as_float(a.y);
+    uint32_t best = 0, fm = 0, hc = 0;
+    float bt = 0.f;
     const auto fold = [&](const uint4& b) {
         const float t = __uint_as_float(b.y);
         if (LITE) bt = fminf(bt, t);
@@ -228,18 +271,27 @@ __device__ uint4 fold_run(const uint4* sel, const Key* keys, const uint32_t* ord
         fm |= b.w;
         hc = (hc + (b.z >> 16)) & 0xffffu;
     };
-    int64_t j = o + 1;
-    while (j < n && keys[j] == key) {
-        if (j + 4 <= n && keys[j + 3] == key) {
-            uint4 b[4];
+    const auto four = [&](int64_t j, int32_t c) {
+        uint32_t w[4];
+        uint4 b[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) b[u] = sel[order[j + u]];
+        for (int u = 0; u < 4; ++u) w[u] = order[u < c ? j + u : j];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) fold(b[u]);
-            j += 4;
-        } else {
-            fold(sel[order[j]]);
-            j += 1;
+        for (int u = 0; u < 4; ++u) b[u] = sel[w[u]];
+        if (j == o) { best = b[0].x; bt = __uint_as_float(b[0].y); hc = b[0].z >> 16; fm = b[0].w; }
+        else fold(b[0]);
+#pragma unroll
+        for (int u = 1; u < 4; ++u)
+            if (u < c) fold(b[u]);
+    };
+    for (int32_t j = 0; j < len; j += 4) four(o + j, len - j);
+    if (open) {
+        const Key key = keys[o];
+        for (int64_t j = o + len; j < n && keys[j] == key;) {
+            int32_t c = 1;
+            while (c < 4 && j + c < n && keys[j + c] == key) ++c;
+            four(j, c);
+            j += c;
         }
     }
     return make_uint4(best, __float_as_uint(bt), hc, fm);
@@ -248,36 +300,22 @@ __device__ uint4 fold_run(const uint4* sel, const Key* keys, const uint32_t* ord
 template <bool LITE, class Key>
 __global__ void __launch_bounds__(256) k_reduce(const uint32_t* __restrict__ in, const uint4* __restrict__ sel,
                                                 const Key* __restrict__ keys, const uint32_t* __restrict__ order, int64_t n,
-                                                int64_t n_tiles, unsigned long long* state, uint32_t* __restrict__ out,
-                                                int64_t out_cap, oa_merge::Result* res)
+                                                const int32_t* __restrict__ offset, uint32_t* __restrict__ out,
+                                                int64_t out_cap)
 {
-    __shared__ unsigned long long s_mask[64];
-    __shared__ int32_t s_pre[65];
-    __shared__ int64_t s_tile, s_base;
-    __shared__ uint16_t s_head[OA_TILE];
+    constexpr int ROUNDS = OA_REDUCE_ROUNDS;
+    __shared__ unsigned long long s_mask[4 * ROUNDS];
+    __shared__ int32_t s_pre[4 * ROUNDS + 1];
+    __shared__ uint16_t s_head[256 * ROUNDS + 1];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    if (t == 0) s_tile = (int64_t)atomicAdd(&state[n_tiles], 1ull);
-    __syncthreads();
-    const int64_t tile = s_tile;
-    if (tile >= n_tiles) return;
-    const int64_t first = tile * OA_TILE;
-    uint32_t heads = 0;
+    const int64_t first = (int64_t)blockIdx.x * (256 * ROUNDS), base = offset[blockIdx.x];
+    const int32_t here = (int32_t)(n - first < 256 * ROUNDS ? n - first : 256 * ROUNDS);
+    const uint32_t heads = run_heads(keys, n, first + t);
+    const int32_t total = tile_ranks<ROUNDS>(heads, s_mask, s_pre);
 #pragma unroll
-    for (int k = 0; k < OA_TILE_ROUNDS; ++k) {
-        const int64_t i = first + k * 256 + t;
-        const bool head = i < n && (i == 0 || keys[i] != keys[i - 1]);
-        if (head) heads |= 1u << k;
-        const unsigned long long m = __ballot(head);
-        if (lane == 0) s_mask[4 * k + wave] = m;
-    }
-    int32_t total;
-    const int64_t base = tile_prefix(s_mask, s_pre, &s_base, state, tile, total);
-#pragma unroll
-    for (int k = 0; k < OA_TILE_ROUNDS; ++k) {
-        if (!(heads >> k & 1u)) continue;
-        const unsigned long long m = s_mask[4 * k + wave];
-        s_head[s_pre[4 * k + wave] + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)(k * 256 + t);
-    }
+    for (int k = 0; k < ROUNDS; ++k)
+        if (heads >> k & 1u) s_head[rank_in_tile(k, s_mask, s_pre)] = (uint16_t)(k * 256 + t);
+    if (t == 0) s_head[total] = (uint16_t)here;
     __syncthreads();
     const int64_t room = out_cap - base;
     const int32_t fit = (int32_t)(room < total ? (room > 0 ? room : 0) : total);
@@ -285,7 +323,7 @@ __global__ void __launch_bounds__(256) k_reduce(const uint32_t* __restrict__ in,
     for (int32_t h0 = 0; h0 < fit; h0 += 256) {
         const int32_t h = h0 + t;
         uint4 r = make_uint4(0u, 0u, 0u, 0u);
-        if (h < fit) r = fold_run<LITE>(sel, keys, order, n, first + s_head[h]);
+        if (h < fit) r = fold_run<LITE>(sel, keys, order, n, first + s_head[h], s_head[h + 1] - s_head[h], h == total - 1);
         if (LITE) {
             if (h < fit) {
                 const quad a = reinterpret_cast<const quad*>(in)[r.x];
@@ -307,10 +345,8 @@ __global__ void __launch_bounds__(256) k_reduce(const uint32_t* __restrict__ in,
             reinterpret_cast<quad*>(out)[(base + hq) * 4 + part] = w;
         }
     }
-    if (tile == n_tiles - 1 && t == 0) res->n_runs = base + total;
 }
 
-inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 inline int bits_of(uint32_t v) { return v ? 32 - __builtin_clz(v) : 0; }
 
 template <class Key>
@@ -323,41 +359,57 @@ size_t sort_bytes_t(int64_t n, int bits)
 }
 
 template <class Key>
-hipError_t sort_t(const uint4* sel, int64_t n, float tw, int bucket_bits, int bits, Key* keys, Key* keys2, uint32_t* order,
-                  uint32_t* order2, void* tmp, size_t tmp_bytes, hipStream_t s)
+hipError_t sort_t(const uint4* sel, int64_t n_tiles, const int32_t* offset, int64_t n, float tw, int bucket_bits, int bits,
+                  Key* keys, Key* keys2, uint32_t* order, uint32_t* order2, void* tmp, size_t tmp_bytes, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_keys<Key>, dim3(nblk(n, 256)), dim3(256), 0, s, sel, n, tw, bucket_bits, keys, order);
+    hipLaunchKernelGGL(k_keys<Key>, dim3((unsigned)n_tiles), dim3(256), 0, s, sel, offset, tw, bucket_bits, keys, order);
     return hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, keys, keys2, order, order2, (int)n, 0, bits, s);
+}
+
+template <class Key>
+void reduce_t(int record, const void* d_in, const uint4* sel, int64_t n, int64_t n_tiles, const Key* keys,
+              const uint32_t* order, int32_t* offset, void* d_out, int64_t out_cap, hipStream_t s)
+{
+    const dim3 grid((unsigned)n_tiles), block(256);
+    if (record == OA_MERGE_PHOTON)
+        hipLaunchKernelGGL((k_reduce<false, Key>), grid, block, 0, s, (const uint32_t*)d_in, sel, keys, order, n, offset,
+                           (uint32_t*)d_out, out_cap);
+    else
+        hipLaunchKernelGGL((k_reduce<true, Key>), grid, block, 0, s, (const uint32_t*)d_in, sel, keys, order, n, offset,
+                           (uint32_t*)d_out, out_cap);
 }
 
 } // namespace
 
 namespace oa_merge {
 
-static int64_t tiles(int64_t n) { return (n + OA_TILE - 1) / OA_TILE; }
-int64_t state_words(int64_t n) { return tiles(n) + 3; }
+static int64_t tiles(int64_t n, int rounds) { return (n + 256 * rounds - 1) / (256 * rounds); }
+/* counts of the selection's tiles and of the runs', each with a total behind it */
+size_t count_words(int64_t n) { return (size_t)(tiles(n, OA_SELECT_ROUNDS) + tiles(n, OA_REDUCE_ROUNDS) + 2); }
+size_t most_words(int64_t n) { return (size_t)tiles(n, OA_SELECT_ROUNDS); }
 
-hipError_t select(int record, const void* d_in, int64_t n, uint32_t mask, float tw, unsigned long long* state, uint4* sel,
+hipError_t select(int record, const void* d_in, int64_t n, uint32_t mask, float tw, int32_t* count, uint2* most, uint4* sel,
                   Result* out, hipStream_t s)
 {
-    const int64_t nt = tiles(n);
-    hipLaunchKernelGGL(k_clear, dim3(nblk(nt + 3, 256)), dim3(256), 0, s, state, nt + 3);
+    const int64_t nt = tiles(n, OA_SELECT_ROUNDS);
     if (record == OA_MERGE_PHOTON)
-        hipLaunchKernelGGL(k_select<PhotonAcc>, dim3((unsigned)nt), dim3(256), 0, s, (const uint32_t*)d_in, n, mask, tw, nt,
-                           state, sel, out);
+        hipLaunchKernelGGL(k_select<PhotonAcc>, dim3((unsigned)nt), dim3(256), 0, s, (const uint32_t*)d_in, n, mask, tw,
+                           count, most, sel);
     else
-        hipLaunchKernelGGL(k_select<LiteAcc>, dim3((unsigned)nt), dim3(256), 0, s, (const uint32_t*)d_in, n, mask, tw, nt,
-                           state, sel, out);
-    hipLaunchKernelGGL(k_maxima, dim3(1), dim3(1), 0, s, state + nt + 1, out);
+        hipLaunchKernelGGL(k_select<LiteAcc>, dim3((unsigned)nt), dim3(256), 0, s, (const uint32_t*)d_in, n, mask, tw,
+                           count, most, sel);
+    hipLaunchKernelGGL(k_tile_offsets, dim3(1), dim3(1024), 0, s, count, most, nt, &out->n_sel, out);
     return hipGetLastError();
 }
 
-hipError_t gather_selected(int record, const void* d_in, const uint4* sel, int64_t n, void* d_out, hipStream_t s)
+hipError_t gather_selected(int record, const void* d_in, int64_t n, const int32_t* count, const uint4* sel, void* d_out,
+                           hipStream_t s)
 {
+    const dim3 grid((unsigned)tiles(n, OA_SELECT_ROUNDS)), block(256);
     if (record == OA_MERGE_PHOTON)
-        hipLaunchKernelGGL(k_gather<4>, dim3(nblk(4 * n, 256)), dim3(256), 0, s, (const quad*)d_in, sel, n, (quad*)d_out);
+        hipLaunchKernelGGL(k_gather<4>, grid, block, 0, s, (const quad*)d_in, sel, count, (quad*)d_out);
     else
-        hipLaunchKernelGGL(k_gather<1>, dim3(nblk(n, 256)), dim3(256), 0, s, (const quad*)d_in, sel, n, (quad*)d_out);
+        hipLaunchKernelGGL(k_gather<1>, grid, block, 0, s, (const quad*)d_in, sel, count, (quad*)d_out);
     return hipGetLastError();
 }
 
@@ -367,29 +419,41 @@ int key_bits(uint32_t max_id, uint32_t max_bucket)
     return b > 0 ? b : 1;
 }
 
-size_t sort_bytes(int64_t n, int bits) { return bits <= 32 ? sort_bytes_t<uint32_t>(n, bits) : sort_bytes_t<uint64_t>(n, bits); }
-
-hipError_t sort_runs(const uint4* sel, int64_t n, float tw, uint32_t max_bucket, int bits, void* keys, void* keys2,
-                     uint32_t* order, uint32_t* order2, void* tmp, size_t tmp_bytes, hipStream_t s)
+size_t sort_bytes(int64_t n_sel, int bits)
 {
-    const int bb = bits_of(max_bucket);
-    return bits <= 32
-        ? sort_t(sel, n, tw, bb, bits, (uint32_t*)keys, (uint32_t*)keys2, order, order2, tmp, tmp_bytes, s)
-        : sort_t(sel, n, tw, bb, bits, (uint64_t*)keys, (uint64_t*)keys2, order, order2, tmp, tmp_bytes, s);
+    return bits <= 32 ? sort_bytes_t<uint32_t>(n_sel, bits) : sort_bytes_t<uint64_t>(n_sel, bits);
 }
 
-hipError_t reduce_runs(int record, const void* d_in, const uint4* sel, int64_t n, int bits, const void* keys2,
-                       const uint32_t* order2, unsigned long long* state, void* d_out, int64_t out_cap, Result* out,
-                       hipStream_t s)
+hipError_t sort_runs(int64_t n, const int32_t* count, const uint4* sel, int64_t n_sel, float tw, uint32_t max_bucket,
+                     int bits, void* keys, void* keys2, uint32_t* order, uint32_t* order2, void* tmp, size_t tmp_bytes,
+                     hipStream_t s)
 {
-    const int64_t nt = tiles(n);
-    hipLaunchKernelGGL(k_clear, dim3(nblk(nt + 1, 256)), dim3(256), 0, s, state, nt + 1);
-#define OA_REDUCE(LITE, Key)                                                                                            \
-    hipLaunchKernelGGL((k_reduce<LITE, Key>), dim3((unsigned)nt), dim3(256), 0, s, (const uint32_t*)d_in, sel,          \
-                       (const Key*)keys2, order2, n, nt, state, (uint32_t*)d_out, out_cap, out)
-    if (record == OA_MERGE_PHOTON) { if (bits <= 32) OA_REDUCE(false, uint32_t); else OA_REDUCE(false, uint64_t); }
-    else { if (bits <= 32) OA_REDUCE(true, uint32_t); else OA_REDUCE(true, uint64_t); }
-#undef OA_REDUCE
+    const int bb = bits_of(max_bucket);
+    const int64_t nt = tiles(n, OA_SELECT_ROUNDS);
+    return bits <= 32
+        ? sort_t(sel, nt, count, n_sel, tw, bb, bits, (uint32_t*)keys, (uint32_t*)keys2, order, order2, tmp, tmp_bytes, s)
+        : sort_t(sel, nt, count, n_sel, tw, bb, bits, (uint64_t*)keys, (uint64_t*)keys2, order, order2, tmp, tmp_bytes, s);
+}
+
+hipError_t count_runs(int64_t n, int32_t* count, int64_t n_sel, int bits, const void* keys2, Result* out, hipStream_t s)
+{
+    int32_t* runs = count + tiles(n, OA_SELECT_ROUNDS) + 1;
+    const int64_t nt = tiles(n_sel, OA_REDUCE_ROUNDS);
+    if (bits <= 32)
+        hipLaunchKernelGGL(k_count_runs<uint32_t>, dim3((unsigned)nt), dim3(256), 0, s, (const uint32_t*)keys2, n_sel, runs);
+    else
+        hipLaunchKernelGGL(k_count_runs<uint64_t>, dim3((unsigned)nt), dim3(256), 0, s, (const uint64_t*)keys2, n_sel, runs);
+    hipLaunchKernelGGL(k_tile_offsets, dim3(1), dim3(1024), 0, s, runs, (const uint2*)nullptr, nt, &out->n_runs, out);
+    return hipGetLastError();
+}
+
+hipError_t reduce_runs(int record, const void* d_in, int64_t n, int32_t* count, const uint4* sel, int64_t n_sel, int bits,
+                       const void* keys2, const uint32_t* order2, void* d_out, int64_t out_cap, hipStream_t s)
+{
+    int32_t* runs = count + tiles(n, OA_SELECT_ROUNDS) + 1;
+    const int64_t nt = tiles(n_sel, OA_REDUCE_ROUNDS);
+    if (bits <= 32) reduce_t(record, d_in, sel, n_sel, nt, (const uint32_t*)keys2, order2, runs, d_out, out_cap, s);
+    else reduce_t(record, d_in, sel, n_sel, nt, (const uint64_t*)keys2, order2, runs, d_out, out_cap, s);
     return hipGetLastError();
 }
 
