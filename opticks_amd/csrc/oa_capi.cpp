@@ -1322,6 +1322,9 @@ int mi_sim_simtrace_device(mi_sim* sim, const void* d_gensteps, int64_t n_gs, in
     P.gs_prefix = sim->prefix.p;
     P.n_gs = n_gs;
     P.n_photon = total;
+    HIPCHECK(sim->words.reserve(1));
+    HIPCHECK(oa_launch::zero_u64(sim->words.p, 1, s));
+    P.next = sim->words.p;
     HIPCHECK(oa_launch::simtrace(P, (float4*)d_simtrace, s));
     HIPCHECK(hipStreamSynchronize(s));
     return MI_OK;

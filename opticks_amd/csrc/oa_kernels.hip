@@ -176,19 +176,25 @@ __global__ void __launch_bounds__(256) k_setup(const float* gs, int64_t n_gs, in
 
 /* ------------------------------------------------------------ simtrace */
 
-/* CSGOptiX7.cu:563-604 simtrace: one ray per photon of OpticksGenstep_FRAME
-   gensteps, generated by qsim::generate_photon_simtrace_frame
-   (qudarap/qsim.h:2460-2522) on RNG stream (event 0, photon index), recorded as
-   sevent::add_simtrace (sysrap/sevent.h:670-696); a miss writes q0 = (0.6,0.6,0.6,1),
-   the miss program's midgrey background (CSGOptiX7.cu:683-700, CSGOptiX/SBT.cc:185-191) */
-template <int BLOCK, bool EXT>
-__global__ void __launch_bounds__(BLOCK) OA_OCC k_simtrace(SimParams P, float4* out)
+/* largest k in [0, n) with a[k] <= v, the same v on every lane of a wave: 64 ways a step,
+   three dependent loads for 40,000 gensteps where halving takes sixteen */
+__device__ int64_t wave_upper_index(const int64_t* a, int64_t n, int64_t v, int lane)
 {
-    __shared__ uint32_t s_stack[OA_STACK_DEPTH * BLOCK];
-    const int64_t idx = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if (idx >= P.n_photon) return;
-    const int64_t gsi = upper_index(P.gs_prefix, 0, P.n_gs, idx);
-    const float4* gq = reinterpret_cast<const float4*>(P.gensteps + 24 * gsi);
+    int64_t lo = 0;
+    for (int64_t len = n; len > 1;) {
+        const int64_t step = (len + 63) / 64, probe = lane * step;
+        const unsigned long long m = __ballot(probe < len && a[lo + probe] <= v);
+        const int64_t k = m ? 63 - __clzll((long long)m) : 0;
+        lo += k * step;
+        len = len - k * step < step ? len - k * step : step;
+    }
+    return lo;
+}
+
+/* the ray of photon idx of genstep gq: qsim::generate_photon_simtrace_frame
+   (qudarap/qsim.h:2460-2522) on RNG stream (event 0, photon index) */
+__device__ void simtrace_ray(const SimParams& P, const float4* gq, int64_t idx, v3& pos, v3& dir)
+{
     PhiloxRng rng;
     rng.key = P.seed;
     rng.photon = (uint64_t)idx;
@@ -202,24 +208,168 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_simtrace(SimParams P, float4* 
     const float u1 = u[1];
     const float cosTheta = 2.f * u1 - 1.f;
     const float sinTheta = sqrtf(1.f - cosTheta * cosTheta);
-    v3 dir = gridaxes == 1u ? mk(0.f, cosPhi, sinPhi)
-           : gridaxes == 2u ? mk(cosPhi, 0.f, sinPhi)
-           : gridaxes == 3u ? mk(cosPhi, sinPhi, 0.f)
-           : mk(sinTheta * cosPhi, sinTheta * sinPhi, cosTheta);
+    dir = gridaxes == 1u ? mk(0.f, cosPhi, sinPhi)
+        : gridaxes == 2u ? mk(cosPhi, 0.f, sinPhi)
+        : gridaxes == 3u ? mk(cosPhi, sinPhi, 0.f)
+        : mk(sinTheta * cosPhi, sinTheta * sinPhi, cosTheta);
     const float4 q1 = gq[1];
-    const v3 pos = q_right(gq + 2, mk(q1.x, q1.y, q1.z), 1.f);
+    pos = q_right(gq + 2, mk(q1.x, q1.y, q1.z), 1.f);
     dir = q_right(gq + 2, dir, 0.f);
-    Prd prd;
-    trace<BLOCK, EXT>(P, s_stack + threadIdx.x, pos, dir, P.tmin, P.tmax, prd);
+}
+
+/* sevent::add_simtrace (sysrap/sevent.h:670-696); a miss writes q0 = (0.6,0.6,0.6,1), the
+   miss program's midgrey background (CSGOptiX7.cu:683-700, CSGOptiX/SBT.cc:185-191) */
+__device__ void simtrace_record(const SimParams& P, float4* o, v3 pos, v3 dir, const Prd& prd)
+{
     const bool miss = prd.boundary == 0xffffu;
     const float t = miss ? 1.f : prd.t;
     const uint32_t gpb = miss ? 0xffffffffu : (((prd.gprim & 0xffffu) << 16) | (prd.boundary & 0xffffu));
     const uint32_t ii = miss ? 0xffffffffu : prd.iindex_identity;
-    float4* o = out + 4 * idx;
     o[0] = miss ? make_float4(0.6f, 0.6f, 0.6f, t) : make_float4(prd.normal.x, prd.normal.y, prd.normal.z, t);
     o[1] = make_float4(pos.x + t * dir.x, pos.y + t * dir.y, pos.z + t * dir.z, P.tmin);
     o[2] = make_float4(pos.x, pos.y, pos.z, __uint_as_float(gpb));
     o[3] = make_float4(dir.x, dir.y, dir.z, __uint_as_float(ii));
+}
+
+/* words of a ray in a wave's queue */
+#define OA_RAY_WORDS 16
+
+/*
+ * CSGOptiX7.cu:563-604 simtrace: one ray per photon of OpticksGenstep_FRAME gensteps, the
+ * nearest hit that oa::trace finds. A ray is all that a lane carries, so a wave need not
+ * follow 64 of them from start to end. Rays are made and tested against the front instances
+ * 64 at a time, and those not settled by them go to a queue in LDS. Lanes are persistent, each
+ * at its own point of its own walk (trace's two phases), and the wave does next what enough
+ * of them want: lanes that hold an instance leaf wait until OA_RAY_LEAVES do, lanes whose ray
+ * is settled until OA_RAY_REFILL are, and record and refill together; the others walk nodes
+ * meanwhile. Bound by instruction issue, most of it the CSG trees of the leaf phase: with 64
+ * rays from start to end a tree ran on 15 lanes, since a third of a grid's rays meet an
+ * instance at all. 10.1M rays among 2,000 detectors: 1.72 ms before, 1.45 ms. OA_RAY_LEAVES 32 /
+ * 40 / 48 / 56: 1.55 / 1.47 / 1.45 / 1.47 ms; OA_RAY_REFILL 8 / 12 / 16 / 24: 1.48 / 1.45 / 1.47 / 1.47.
+ * Waves claim rays from a counter (P.next, zero at the start), since those among the detectors
+ * take longest: dealt out in advance, 2.40 ms. A claim is 256 rays, the counter being one word
+ * (64: 2.18 ms, 128: 1.52, 256: 1.45), and down to 64 where that leaves a wave fewer than eight.
+ */
+#define OA_RAY_LEAVES 48
+#define OA_RAY_REFILL 12
+#define OA_RAY_QUEUE (OA_RAY_REFILL + 64)
+template <bool EXT>
+__global__ void __launch_bounds__(64) OA_OCC k_simtrace(SimParams P, int claim, float4* out)
+{
+    extern __shared__ uint32_t s_lane[];             /* the queue, then each lane's stack */
+    uint32_t* stk = s_lane + OA_RAY_WORDS * OA_RAY_QUEUE + threadIdx.x;
+    const int lane = threadIdx.x;
+    const float4 fb = const_load(const_ptr(P.free_ball));
+    int64_t next = 0, end = 0;                       /* what is left of the claimed rays */
+    bool more = true;
+    int queued = 0;
+    int64_t idx = -1;                                /* this lane's ray; it is settled when `done` */
+    bool done = true;
+    v3 o = mk(0.f, 0.f, 0.f), d = o;
+    float tlo = 0.f;
+    Nearest best;
+    nearest_none(best, P.tmax);
+    int sp = 0;
+    uint32_t cur = OA_BVH_EMPTY, leaf = OA_BVH_EMPTY;
+    for (;;) {
+        const unsigned long long free_lanes = __ballot(done);
+        const int n_free = __popcll(free_lanes);
+        if (n_free == 64 || (n_free >= OA_RAY_REFILL && more)) {
+            if (done && idx >= 0) {
+                Prd prd;
+                hit_record(P, best, o, d, prd);
+                simtrace_record(P, out + 4 * idx, o, d, prd);
+                idx = -1;
+            }
+            while (queued < OA_RAY_REFILL) {
+                if (next == end) {
+                    unsigned long long c = 0ull;
+                    if (lane == 0) c = atomicAdd(P.next, (unsigned long long)claim);
+                    next = (int64_t)__shfl(c, 0);
+                    end = next + claim < P.n_photon ? next + claim : P.n_photon;
+                    if (next >= P.n_photon) { next = end; break; }
+                }
+                const int64_t last = (next + 64 < end ? next + 64 : end) - 1, i = next + lane;
+                const int64_t g0 = wave_upper_index(P.gs_prefix, P.n_gs, next, lane);
+                const int64_t g1 = g0 + wave_upper_index(P.gs_prefix + g0, P.n_gs - g0, last, lane);
+                bool walks = i <= last;
+                v3 ro = mk(0.f, 0.f, 0.f), rd = ro;
+                Nearest rb;
+                nearest_none(rb, P.tmax);
+                float rlo = P.tmin;
+                if (walks) {
+                    const int64_t gsi = upper_index(P.gs_prefix, g0, g1 + 1, i);
+                    simtrace_ray(P, reinterpret_cast<const float4*>(P.gensteps + 24 * gsi), i, ro, rd);
+                    if (P.front_plain) {
+                        trace_front(P, ro, rd, P.tmin, rb);
+                        walks = !P.tlas_empty && beyond_free_ball(fb, ro, rd, P.tmin, rb.t, rlo);
+                    }
+                    if (!walks) {
+                        Prd prd;
+                        hit_record(P, rb, ro, rd, prd);
+                        simtrace_record(P, out + 4 * i, ro, rd, prd);
+                    }
+                }
+                const unsigned long long m = __ballot(walks);
+                if (walks) {
+                    uint32_t* w = s_lane + queued + __popcll(m & ((1ull << lane) - 1ull));
+                    const uint32_t v[OA_RAY_WORDS] = {
+                        (uint32_t)i, (uint32_t)((uint64_t)i >> 32), fbits(ro.x), fbits(ro.y), fbits(ro.z), fbits(rd.x),
+                        fbits(rd.y), fbits(rd.z), fbits(rb.t), rb.inst, rb.prim, fbits(rb.is.x), fbits(rb.is.y),
+                        fbits(rb.is.z), fbits(rb.is.w), fbits(rlo) };
+#pragma unroll
+                    for (int q = 0; q < OA_RAY_WORDS; ++q) w[q * OA_RAY_QUEUE] = v[q];
+                }
+                queued += __popcll(m);
+                next = last + 1;
+            }
+            more = queued > 0;
+            /* one wave to a block: the queue's stores are in before it is read */
+            __syncthreads();
+            const int take = n_free < queued ? n_free : queued;
+            if (take == 0 && n_free == 64) break;
+            queued -= take;
+            const int rank = __popcll(free_lanes & ((1ull << lane) - 1ull));
+            if (done && rank < take) {
+                uint32_t v[OA_RAY_WORDS];
+#pragma unroll
+                for (int q = 0; q < OA_RAY_WORDS; ++q) v[q] = s_lane[queued + rank + q * OA_RAY_QUEUE];
+                idx = (int64_t)((uint64_t)v[0] | ((uint64_t)v[1] << 32));
+                o = mk(__uint_as_float(v[2]), __uint_as_float(v[3]), __uint_as_float(v[4]));
+                d = mk(__uint_as_float(v[5]), __uint_as_float(v[6]), __uint_as_float(v[7]));
+                best.t = __uint_as_float(v[8]);
+                best.inst = v[9];
+                best.prim = v[10];
+                best.key = best.inst == 0xffffffffu ? ~0ull : ((uint64_t)best.inst << 32) | best.prim;
+                best.is.x = __uint_as_float(v[11]); best.is.y = __uint_as_float(v[12]);
+                best.is.z = __uint_as_float(v[13]); best.is.w = __uint_as_float(v[14]);
+                tlo = __uint_as_float(v[15]);
+                sp = 0;
+                cur = P.tlas_empty ? OA_BVH_EMPTY : 0u;
+                leaf = P.front_plain ? OA_BVH_EMPTY : P.front_leaf;
+                done = false;
+            }
+            __syncthreads();
+        }
+        v3 inv, oi;
+        slab_ray(o, d, inv, oi);
+        unsigned long long walking, holding;
+        for (;;) {
+            holding = __ballot(!done && leaf != OA_BVH_EMPTY);
+            walking = __ballot(!done && leaf == OA_BVH_EMPTY);
+            if (walking == 0ull || __popcll(holding) >= OA_RAY_LEAVES) break;
+            if (more && __popcll(~(holding | walking)) >= OA_RAY_REFILL) break;
+            if (!done && leaf == OA_BVH_EMPTY) done = walk_nodes<64>(P, inv, oi, tlo, best, stk, sp, cur, leaf);
+        }
+        if (__popcll(holding) < OA_RAY_LEAVES && more && __popcll(~(holding | walking)) >= OA_RAY_REFILL) continue;
+        if (!done && leaf != OA_BVH_EMPTY) {
+            const uint32_t at = leaf;
+            leaf = OA_BVH_EMPTY;
+            test_leaf<64, EXT>(P, at, o, d, P.tmin, tlo, best, stk, sp);
+            /* after a front leaf (the TLAS walk not begun: cur is still the root) */
+            if (cur == 0u && !beyond_free_ball(fb, o, d, P.tmin, best.t, tlo)) cur = OA_BVH_EMPTY;
+        }
+    }
 }
 
 /* ---------------------------------------------------- hit compaction */
@@ -586,16 +736,22 @@ hipError_t zero_u64(unsigned long long* p, int64_t n, hipStream_t s)
     return hipGetLastError();
 }
 
-#ifndef OA_SIMTRACE_BLOCK
-#define OA_SIMTRACE_BLOCK 64   /* 64: 3.55 ms, 128: 3.71, 256: 3.87 on a 10.1M-ray grid */
-#endif
-
 hipError_t simtrace(const SimParams& P, float4* out, hipStream_t s)
 {
-    constexpr int B = OA_SIMTRACE_BLOCK;
-    const unsigned nb = (unsigned)((P.n_photon + B - 1) / B);
-    if (P.ext_leaves) hipLaunchKernelGGL((k_simtrace<B, true>), dim3(nb), dim3(B), 0, s, P, out);
-    else hipLaunchKernelGGL((k_simtrace<B, false>), dim3(nb), dim3(B), 0, s, P, out);
+    const unsigned lds = (unsigned)(OA_RAY_WORDS * OA_RAY_QUEUE + 64 * P.stack_depth) * 4u;
+    int dev = 0, n_cu = 0, per_cu = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e == hipSuccess)
+        e = P.ext_leaves ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_simtrace<true>, 64, lds)
+                         : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_simtrace<false>, 64, lds);
+    if (e != hipSuccess) return e;
+    const int64_t need = (P.n_photon + 63) / 64, slots = (int64_t)n_cu * (per_cu > 0 ? per_cu : 8);
+    const unsigned nb = (unsigned)(need < slots ? need : slots);
+    const int64_t share = P.n_photon / (8 * (int64_t)nb) / 64;
+    const int claim = 64 * (int)(share < 1 ? 1 : share > 4 ? 4 : share);
+    if (P.ext_leaves) hipLaunchKernelGGL(k_simtrace<true>, dim3(nb), dim3(64), lds, s, P, claim, out);
+    else hipLaunchKernelGGL(k_simtrace<false>, dim3(nb), dim3(64), lds, s, P, claim, out);
     return hipGetLastError();
 }
 

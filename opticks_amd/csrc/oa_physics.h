@@ -710,11 +710,23 @@ OA_D void inst_ray_rows(float4 r0, float4 r1, float4 r2, float4 r3, v3 o, v3 d, 
 }
 OA_D void inst_ray(const float4* m, v3 o, v3 d, v3& oo, v3& od) { inst_ray_rows(m[0], m[1], m[2], m[3], o, d, oo, od); }
 
+/* a ray's nearest hit so far (exact ties: the smaller (instance, prim) key) */
+struct Nearest {
+    float t;
+    uint64_t key;
+    uint32_t inst, prim;
+    Isect is;
+};
+OA_D void nearest_none(Nearest& best, float tmax)
+{
+    best.t = tmax; best.key = ~0ull; best.inst = 0xffffffffu; best.prim = 0u;
+    best.is.x = best.is.y = best.is.z = best.is.w = 0.f;
+}
+
 /* one prim of one instance (entry k of the BLAS-ordered prim records) against the
    nearest hit so far (t, then the (instance, prim) key) */
 template <bool EXT>
-OA_D void consider_prim(const SimParams& P, uint32_t ii, uint32_t k, v3 oo, v3 od, float tmin, float& best_t,
-                        uint64_t& best_key, uint32_t& best_inst, uint32_t& best_prim, Isect& best_is)
+OA_D void consider_prim(const SimParams& P, uint32_t ii, uint32_t k, v3 oo, v3 od, float tmin, Nearest& best)
 {
     const PrimRec pr = P.blas_prims[k];
     const uint32_t pi = pr.index;
@@ -724,8 +736,8 @@ OA_D void consider_prim(const SimParams& P, uint32_t ii, uint32_t k, v3 oo, v3 o
        (a convex polyhedron behind the ray reports valid with t = 0) */
     if (!(is.w >= tmin)) return;
     const uint64_t key = ((uint64_t)ii << 32) | (uint64_t)pi;
-    if (is.w < best_t || (is.w == best_t && key < best_key)) {
-        best_t = is.w; best_key = key; best_inst = ii; best_prim = pi; best_is = is;
+    if (is.w < best.t || (is.w == best.t && key < best.key)) {
+        best.t = is.w; best.key = key; best.inst = ii; best.prim = pi; best.is = is;
     }
 }
 
@@ -763,8 +775,7 @@ OA_D float4 const_load(cptr4 p) { const cf4 v = *p; return make_float4(v.x, v.y,
  * records come by scalar loads and the leaf type is a scalar branch, where the leaf phase
  * below chains vector loads (item, instance, prim record, node) with a switch per lane.
  */
-OA_D void trace_front(const SimParams& P, v3 o, v3 d, float tmin, float& best_t, uint64_t& best_key, uint32_t& best_inst,
-                      uint32_t& best_prim, Isect& best_is)
+OA_D void trace_front(const SimParams& P, v3 o, v3 d, float tmin, Nearest& best)
 {
     const uint32_t first = P.front_leaf & 0x00ffffffu, count = (P.front_leaf >> 24) & 0x7fu;
     for (uint32_t k = 0; k < count; ++k) {
@@ -789,11 +800,118 @@ OA_D void trace_front(const SimParams& P, v3 o, v3 d, float tmin, float& best_t,
                 continue;
             if (!(is.w >= tmin)) continue;
             const uint64_t key = ((uint64_t)ii << 32) | (uint64_t)pi;
-            if (is.w < best_t || (is.w == best_t && key < best_key)) {
-                best_t = is.w; best_key = key; best_inst = ii; best_prim = pi; best_is = is;
+            if (is.w < best.t || (is.w == best.t && key < best.key)) {
+                best.t = is.w; best.key = key; best.inst = ii; best.prim = pi; best.is = is;
             }
         }
     }
+}
+
+/* One iteration of the node walk: pop when the lane holds nothing, visit a node, and take a
+   leaf (popped or the visit's nearest child) at once. True: nothing is left. */
+template <int STRIDE>
+OA_D bool walk_nodes(const SimParams& P, v3 inv, v3 oi, float tlo, const Nearest& best, uint32_t* stk, int& sp, uint32_t& cur,
+                     uint32_t& leaf)
+{
+    if (cur == OA_BVH_EMPTY) {
+        if (sp == 0) return true;
+        sp--;
+        cur = stk[sp * STRIDE];
+    }
+    if (!(cur & OA_BVH_LEAF_BIT)) {
+        OA_COUNT(OA_ST_TLAS);
+#ifdef OA_STATS
+        const int sp0 = sp;
+#endif
+        cur = visit<STRIDE>(P.tlas, cur, inv, oi, tlo, best.t, stk, sp);
+#ifdef OA_STATS
+        if (cur == OA_BVH_EMPTY && sp == sp0) OA_COUNT(OA_ST_TLAS_DEAD);
+#endif
+    }
+    if (cur != OA_BVH_EMPTY && (cur & OA_BVH_LEAF_BIT)) {
+        leaf = cur;
+        cur = OA_BVH_EMPTY;
+    }
+    return false;
+}
+
+/* the instances of a leaf link: ray into each frame, BLAS walk, prim tests. Returns the
+   iterations this took. */
+template <int STRIDE, bool EXT>
+OA_D uint32_t test_leaf(const SimParams& P, uint32_t leaf, v3 o, v3 d, float tmin, float tlo, Nearest& best, uint32_t* stk,
+                    int& sp)
+{
+    uint32_t iterations = 0;
+    const uint32_t first = leaf & 0x00ffffffu, count = (leaf >> 24) & 0x7fu;
+    for (uint32_t k = 0; k < count; ++k) {
+        const uint32_t ii = P.tlas_items[first + k];
+        OA_COUNT(OA_ST_INST);
+        const float4* m = reinterpret_cast<const float4*>(P.inst + ii);
+        v3 oo, od;
+        inst_ray(m, o, d, oo, od);
+        v3 inv2, oi2;
+        slab_ray(oo, od, inv2, oi2);
+        const int sp_base = sp;
+        uint32_t bc = __float_as_uint(m[2].w);     /* BLAS root of this solid (front instances: one leaf of all its prims) */
+        for (;;) {
+            OA_WAVE_COUNT(OA_ST_W_P2, OA_ST_L_P2);
+            iterations++;
+            /* as in the node walk: pop, visit, and test a leaf's prims in one iteration */
+            if (bc == OA_BVH_EMPTY) {
+                if (sp == sp_base) break;
+                sp--;
+                bc = stk[sp * STRIDE];
+            }
+            if (!(bc & OA_BVH_LEAF_BIT)) {
+                OA_COUNT(OA_ST_BLAS);
+#ifdef OA_STATS
+                const int sp0 = sp;
+#endif
+                bc = visit<STRIDE, true>(P.blas, bc, inv2, oi2, tlo, best.t, stk, sp);
+#ifdef OA_STATS
+                if (bc == OA_BVH_EMPTY && sp == sp0) OA_COUNT(OA_ST_BLAS_DEAD);
+#endif
+                if (bc == OA_BVH_EMPTY || !(bc & OA_BVH_LEAF_BIT)) continue;
+            }
+            const uint32_t bf = bc & 0x00ffffffu, bn = (bc >> 24) & 0x7fu;
+            OA_CYC_MARK(c_prim);
+            for (uint32_t j = 0; j < bn; ++j) {
+                OA_COUNT(OA_ST_PRIM);
+                OA_WAVE_COUNT(OA_ST_W_PRIM, OA_ST_L_PRIM);
+                consider_prim<EXT>(P, ii, bf + j, oo, od, tmin, best);
+            }
+            OA_CYC_ADD(OA_ST_C_PRIM, c_prim);
+            bc = OA_BVH_EMPTY;
+        }
+    }
+    return iterations;
+}
+
+/* what a trace reports of its nearest hit */
+OA_D void hit_record(const SimParams& P, const Nearest& best, v3 o, v3 d, Prd& prd)
+{
+    if (best.inst == 0xffffffffu) {
+        prd.normal = mk(0.f, 0.f, 0.f); prd.t = 0.f; prd.lposcost = 0.f;
+        prd.lx = 0.f; prd.ly = __uint_as_float(0x7fc00000u); prd.gprim = 0xffffu;
+        prd.iindex_identity = 0xffffffffu; prd.boundary = 0xffffu;
+        return;
+    }
+    const float4* m = reinterpret_cast<const float4*>(P.inst + best.inst);
+    const float4 r0 = m[0], r1 = m[1], r2 = m[2];
+    prd.normal = mk(r0.x * best.is.x + r0.y * best.is.y + r0.z * best.is.z,
+                    r1.x * best.is.x + r1.y * best.is.y + r1.z * best.is.z,
+                    r2.x * best.is.x + r2.y * best.is.y + r2.z * best.is.z);
+    prd.t = best.t;
+    v3 oo, od;
+    inst_ray(m, o, d, oo, od);
+    const v3 lpos = oo + best.t * od;
+    prd.lposcost = lpos.z / sqrtf(dot(lpos, lpos));
+    prd.lx = lpos.x;
+    prd.ly = lpos.y;
+    const uint32_t ident = __float_as_uint(r1.w);
+    prd.iindex_identity = ((best.inst & 0xffffu) << 16) | (ident & 0xffffu);
+    prd.boundary = P.prim[best.prim].boundary & 0xffffu;
+    prd.gprim = P.prim[best.prim].global_prim;
 }
 
 /*
@@ -821,10 +939,8 @@ OA_D bool trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float
     OA_CYC_MARK(c_trace);
     v3 inv, oi;
     slab_ray(o, d, inv, oi);
-    float best_t = tmax;
-    uint64_t best_key = ~0ull;
-    uint32_t best_inst = 0xffffffffu, best_prim = 0u;
-    Isect best_is; best_is.x = best_is.y = best_is.z = best_is.w = 0.f;
+    Nearest best;
+    nearest_none(best, tmax);
     int sp = 0;
     uint32_t cur = P.tlas_empty ? OA_BVH_EMPTY : 0u;    /* TLAS root node */
     /* the front instances (world-sized boxes kept out of the TLAS) are tested on every
@@ -835,8 +951,8 @@ OA_D bool trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float
     float tlo = tmin;
     bool done = false;
     if (P.front_plain) {
-        trace_front(P, o, d, tmin, best_t, best_key, best_inst, best_prim, best_is);
-        done = !(cur == 0u && beyond_free_ball(const_load(const_ptr(P.free_ball)), o, d, tmin, best_t, tlo));
+        trace_front(P, o, d, tmin, best);
+        done = !(cur == 0u && beyond_free_ball(const_load(const_ptr(P.free_ball)), o, d, tmin, best.t, tlo));
         /* the TLAS walk and the CSG trees behind it run for as long as their slowest lane:
            lanes that need them wait for company while others of the wave have a step to do */
         const unsigned long long walkers = __ballot(!done);
@@ -862,27 +978,7 @@ OA_D bool trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float
 #ifdef OA_STATS
             n1++;
 #endif
-            /* one iteration: pop when the lane holds nothing, visit a node, and
-               take a leaf (popped or the visit's nearest child) at once */
-            if (cur == OA_BVH_EMPTY) {
-                if (sp == 0) { done = true; break; }
-                sp--;
-                cur = stk[sp * STRIDE];
-            }
-            if (!(cur & OA_BVH_LEAF_BIT)) {
-                OA_COUNT(OA_ST_TLAS);
-#ifdef OA_STATS
-                const int sp0 = sp;
-#endif
-                cur = visit<STRIDE>(P.tlas, cur, inv, oi, tlo, best_t, stk, sp);
-#ifdef OA_STATS
-                if (cur == OA_BVH_EMPTY && sp == sp0) OA_COUNT(OA_ST_TLAS_DEAD);
-#endif
-            }
-            if (cur != OA_BVH_EMPTY && (cur & OA_BVH_LEAF_BIT)) {
-                leaf = cur;
-                cur = OA_BVH_EMPTY;
-            }
+            if (walk_nodes<STRIDE>(P, inv, oi, tlo, best, stk, sp, cur, leaf)) done = true;
         }
         OA_CYC_ADD(OA_ST_C_P1, c_p1);
         if (leaf == OA_BVH_EMPTY) continue;
@@ -892,55 +988,17 @@ OA_D bool trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float
            record, CSG nodes): waves in it issue first, so their next load starts sooner
            (0.6% on the 64 events against no priority; raising the walk instead lost 1%) */
         __builtin_amdgcn_s_setprio(2);
-        const uint32_t first = leaf & 0x00ffffffu, count = (leaf >> 24) & 0x7fu;
+        const uint32_t at = leaf;
         leaf = OA_BVH_EMPTY;
-        for (uint32_t k = 0; k < count; ++k) {
-            const uint32_t ii = P.tlas_items[first + k];
-            OA_COUNT(OA_ST_INST);
-            const float4* m = reinterpret_cast<const float4*>(P.inst + ii);
-            v3 oo, od;
-            inst_ray(m, o, d, oo, od);
-            v3 inv2, oi2;
-            slab_ray(oo, od, inv2, oi2);
-            const int sp_base = sp;
-            uint32_t bc = __float_as_uint(m[2].w);     /* BLAS root of this solid (front instances: one leaf of all its prims) */
-            for (;;) {
-                OA_WAVE_COUNT(OA_ST_W_P2, OA_ST_L_P2);
+        const uint32_t iterations = test_leaf<STRIDE, EXT>(P, at, o, d, tmin, tlo, best, stk, sp);
 #ifdef OA_STATS
-                n2++;
+        n2 += iterations;
 #endif
-                /* as in the node walk: pop, visit, and test a leaf's prims in one iteration */
-                if (bc == OA_BVH_EMPTY) {
-                    if (sp == sp_base) break;
-                    sp--;
-                    bc = stk[sp * STRIDE];
-                }
-                if (!(bc & OA_BVH_LEAF_BIT)) {
-                    OA_COUNT(OA_ST_BLAS);
-#ifdef OA_STATS
-                    const int sp0 = sp;
-#endif
-                    bc = visit<STRIDE, true>(P.blas, bc, inv2, oi2, tlo, best_t, stk, sp);
-#ifdef OA_STATS
-                    if (bc == OA_BVH_EMPTY && sp == sp0) OA_COUNT(OA_ST_BLAS_DEAD);
-#endif
-                    if (bc == OA_BVH_EMPTY || !(bc & OA_BVH_LEAF_BIT)) continue;
-                }
-                const uint32_t bf = bc & 0x00ffffffu, bn = (bc >> 24) & 0x7fu;
-                OA_CYC_MARK(c_prim);
-                for (uint32_t j = 0; j < bn; ++j) {
-                    OA_COUNT(OA_ST_PRIM);
-                    OA_WAVE_COUNT(OA_ST_W_PRIM, OA_ST_L_PRIM);
-                    consider_prim<EXT>(P, ii, bf + j, oo, od, tmin, best_t, best_key, best_inst, best_prim, best_is);
-                }
-                OA_CYC_ADD(OA_ST_C_PRIM, c_prim);
-                bc = OA_BVH_EMPTY;
-            }
-        }
+        (void)iterations;
         OA_CYC_ADD(OA_ST_C_P2, c_p2);
         __builtin_amdgcn_s_setprio(0);
         /* after a front leaf phase (the TLAS walk not begun: cur is still the root) */
-        if (cur == 0u && !beyond_free_ball(*P.free_ball, o, d, tmin, best_t, tlo)) cur = OA_BVH_EMPTY;
+        if (cur == 0u && !beyond_free_ball(*P.free_ball, o, d, tmin, best.t, tlo)) cur = OA_BVH_EMPTY;
     }
     OA_CYC_ADD(OA_ST_C_TRACE, c_trace);
 #ifdef OA_STATS
@@ -951,32 +1009,11 @@ OA_D bool trace(const SimParams& P, uint32_t* stk, v3 o, v3 d, float tmin, float
         if (k < OA_SLOW_MAX) {
             oa_slow[3 * k + 0] = make_float4(o.x, o.y, o.z, tmin);
             oa_slow[3 * k + 1] = make_float4(d.x, d.y, d.z, tmax);
-            oa_slow[3 * k + 2] = make_float4(best_t, (float)n1, (float)n2, __uint_as_float(best_inst));
+            oa_slow[3 * k + 2] = make_float4(best.t, (float)n1, (float)n2, __uint_as_float(best.inst));
         }
     }
 #endif
-    if (best_inst == 0xffffffffu) {
-        prd.normal = mk(0.f, 0.f, 0.f); prd.t = 0.f; prd.lposcost = 0.f;
-        prd.lx = 0.f; prd.ly = __uint_as_float(0x7fc00000u); prd.gprim = 0xffffu;
-        prd.iindex_identity = 0xffffffffu; prd.boundary = 0xffffu;
-        return true;
-    }
-    const float4* m = reinterpret_cast<const float4*>(P.inst + best_inst);
-    const float4 r0 = m[0], r1 = m[1], r2 = m[2];
-    prd.normal = mk(r0.x * best_is.x + r0.y * best_is.y + r0.z * best_is.z,
-                    r1.x * best_is.x + r1.y * best_is.y + r1.z * best_is.z,
-                    r2.x * best_is.x + r2.y * best_is.y + r2.z * best_is.z);
-    prd.t = best_t;
-    v3 oo, od;
-    inst_ray(m, o, d, oo, od);
-    const v3 lpos = oo + best_t * od;
-    prd.lposcost = lpos.z / sqrtf(dot(lpos, lpos));
-    prd.lx = lpos.x;
-    prd.ly = lpos.y;
-    const uint32_t ident = __float_as_uint(r1.w);
-    prd.iindex_identity = ((best_inst & 0xffffu) << 16) | (ident & 0xffffu);
-    prd.boundary = P.prim[best_prim].boundary & 0xffffu;
-    prd.gprim = P.prim[best_prim].global_prim;
+    hit_record(P, best, o, d, prd);
     return true;
 }
 

@@ -182,3 +182,32 @@ def test_event_arrays_are_their_own():
         assert np.array_equal(hit.view(np.uint32), hit0.view(np.uint32))
         assert np.array_equal(photon.view(np.uint32), photon0.view(np.uint32))
         assert np.array_equal(seq, seq0)
+
+
+# fewer rays than lanes, around a wave and a claim of rays, more than the waves hold at once
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 4099, 700_001])
+@pytest.mark.parametrize("world", ["shell", "plain", "tree", "onions", "zoo"])
+def test_simtrace_queue_matches_checker(world, n):
+    """Rays that the front instances settle, that wait for the walk and for the leaf phase, and
+    that miss everything, with gensteps of uneven size, some without rays."""
+    w = {"shell": lambda: configs.config1(num_gs=1, per_gs=10), "plain": lambda: front_world("plain", 10),
+         "tree": lambda: front_world("tree", 10), "onions": lambda: onions(12, 10),
+         "zoo": lambda: configs.leaf_zoo(num_photon=10)}[world]()
+    g = np.random.default_rng(n)
+    n_gs = 5 if n < 1000 else 301
+    counts = np.zeros(n_gs, np.int64)
+    some = g.choice(n_gs, n_gs // 2, replace=False)
+    counts[some] = g.multinomial(n, np.full(len(some), 1.0 / len(some)))
+    extent = 20000.0 if world == "shell" else 1000.0
+    gs = np.repeat(configs.frame_gensteps((0, 0, 0, extent), (0, 0, 0, 0, 0, 0, 1, 1), gridscale=1.0), n_gs, 0)
+    gs[:, 5, :3] = g.uniform(-extent, extent, (n_gs, 3))
+    gs.view(np.uint32)[:, 0, 1] = g.integers(0, 4, n_gs)
+    gs.view(np.uint32)[:, 0, 3] = counts
+    ref = po.World(w.geometry, w.physics).simtrace(gs, seed=9)
+    sim = QSim(w.geometry, w.physics, SEventConfig(seed=9))
+    gs_t = torch.from_numpy(gs).to("cuda:0")
+    for _ in range(2):
+        out = sim.simtrace_device(gs_t).cpu().numpy()
+        assert out.shape == ref.shape == (n, 4, 4)
+        assert np.array_equal(out.view(np.uint32), ref.view(np.uint32))
+    sim.close()
