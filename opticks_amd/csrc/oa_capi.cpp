@@ -211,12 +211,13 @@ struct mi_sim {
     DBuf<int32_t> adj_mat_block, adj_sample_bin;
     DBuf<float> adj_rows, adj_comp;
     DBuf<uint32_t> adj_key, adj_val, adj_key2, adj_val2;
-    DBuf<unsigned char> adj_tmp;
+    DBuf<uint32_t> adj_tmp;
     DBuf<int64_t> adj_seg;
     /* hit merging */
     DBuf<uint4> m_sel;
     DBuf<uint32_t> m_order, m_order2;
-    DBuf<unsigned char> m_keys, m_keys2, m_tmp;
+    DBuf<unsigned char> m_keys, m_keys2;
+    DBuf<uint32_t> m_tmp;
     DBuf<int32_t> m_count;
     DBuf<uint2> m_most;
     oa_merge::Result* m_result = nullptr;           /* pinned */
@@ -1506,7 +1507,6 @@ int mi_sim_adjoint_device(mi_sim* sim, int32_t event_id, const void* d_gensteps,
     const int64_t chunk = (tape_only && adj->max_row_floats <= 0)
                               ? std::max<int64_t>(n_hit, 1)
                               : std::max<int64_t>(1, std::min<int64_t>(std::max<int64_t>(n_hit, 1), rows_max / n_param));
-    const size_t tmp_bytes = std::max<size_t>(1, oa_launch::adjoint_sort_bytes(chunk, n_det));
     if (sim->adj_rows.reserve((size_t)((tape_only ? 1 : chunk) * n_param)) != hipSuccess)
         return fail(MI_ERR_CAPACITY, "adjoint: cannot allocate " + std::to_string(chunk * n_param * 4) + " bytes of score rows");
     HIPCHECK(sim->adj_comp.reserve((size_t)n_det * n_param));
@@ -1514,7 +1514,7 @@ int mi_sim_adjoint_device(mi_sim* sim, int32_t event_id, const void* d_gensteps,
     HIPCHECK(sim->adj_val.reserve((size_t)chunk));
     HIPCHECK(sim->adj_key2.reserve((size_t)chunk));
     HIPCHECK(sim->adj_val2.reserve((size_t)chunk));
-    HIPCHECK(sim->adj_tmp.reserve(tmp_bytes));
+    HIPCHECK(sim->adj_tmp.reserve(oa_launch::adjoint_sort_words(chunk, n_det)));
     HIPCHECK(sim->adj_seg.reserve((size_t)n_det + 1));
     /* persistent replay over every resident block slot */
     const int replay_grid = sim->n_cu * std::max(1, oa_launch::adjoint_blocks_per_cu(sim->cfg.rng_kind, sim->stack_depth));
@@ -1525,7 +1525,7 @@ int mi_sim_adjoint_device(mi_sim* sim, int32_t event_id, const void* d_gensteps,
     ab.hit = (const float4*)d_hit; ab.hit_off = nullptr; ab.n_ev = 0; ab.hit_cap = 0;
     ab.n_det = n_det; ab.S = sim->adj_rows.p;
     ab.key = sim->adj_key.p; ab.val = sim->adj_val.p; ab.key2 = sim->adj_key2.p; ab.val2 = sim->adj_val2.p;
-    ab.tmp = sim->adj_tmp.p; ab.tmp_bytes = tmp_bytes; ab.seg = sim->adj_seg.p;
+    ab.tmp = sim->adj_tmp.p; ab.seg = sim->adj_seg.p;
     ab.G = (float*)d_grad; ab.C = sim->adj_comp.p;
     int64_t h0 = 0;
     do {
@@ -1579,14 +1579,13 @@ int mi_sim_merge_hits_device(mi_sim* sim, int32_t record, const void* d_in, int6
     const uint32_t max_bucket = res->max_bucket;
     const int bits = oa_merge::key_bits(res->max_id, max_bucket);
     const size_t key_bytes = (size_t)n_sel * (bits <= 32 ? 4 : 8);
-    const size_t tmp_bytes = std::max<size_t>(1, oa_merge::sort_bytes(n_sel, bits));
     HIPCHECK(sim->m_keys.reserve(key_bytes));
     HIPCHECK(sim->m_keys2.reserve(key_bytes));
     HIPCHECK(sim->m_order.reserve((size_t)n_sel));
     HIPCHECK(sim->m_order2.reserve((size_t)n_sel));
-    HIPCHECK(sim->m_tmp.reserve(tmp_bytes));
+    HIPCHECK(sim->m_tmp.reserve(oa_merge::sort_words(n_sel, bits)));
     HIPCHECK(oa_merge::sort_runs(n_in, sim->m_count.p, sim->m_sel.p, n_sel, time_window, max_bucket, bits, sim->m_keys.p,
-                                 sim->m_keys2.p, sim->m_order.p, sim->m_order2.p, sim->m_tmp.p, tmp_bytes, s));
+                                 sim->m_keys2.p, sim->m_order.p, sim->m_order2.p, sim->m_tmp.p, s));
     HIPCHECK(oa_merge::count_runs(n_in, sim->m_count.p, n_sel, bits, sim->m_keys2.p, sim->m_result, s));
     /* a buffer that may be too small is left as it is unless the runs fit */
     const bool sure = n_sel <= out_capacity;
@@ -1632,12 +1631,11 @@ struct mi_batch {
     bool has_adj = false;
     int32_t n_mat = 0, n_bin = 0, n_param = 0, n_det = 0;
     int64_t chunk = 0, n_chunk = 0;
-    size_t tmp_bytes = 0;
     float* d_grad = nullptr;
     DBuf<int32_t> mat_block, sample_bin;
     DBuf<float> rows, comp;
     DBuf<uint32_t> key, val, key2, val2;
-    DBuf<unsigned char> tmp;
+    DBuf<uint32_t> tmp;
     DBuf<int64_t> seg;
     DBuf<uint32_t> tape, tape_flag;     /* segment records of the forward (mi_config.adjoint_tape) */
     DBuf<uint8_t> tape_n;
@@ -1706,7 +1704,7 @@ static hipError_t batch_adjoint_work(mi_batch* b, SimParams P, const void* d_hit
     ab.hit = (const float4*)d_hit; ab.hit_off = b->ho.p; ab.n_ev = b->n_event; ab.hit_cap = b->hit_capacity;
     ab.n_det = (uint32_t)b->n_det; ab.S = b->rows.p;
     ab.key = b->key.p; ab.val = b->val.p; ab.key2 = b->key2.p; ab.val2 = b->val2.p;
-    ab.tmp = b->tmp.p; ab.tmp_bytes = b->tmp_bytes; ab.seg = b->seg.p;
+    ab.tmp = b->tmp.p; ab.seg = b->seg.p;
     ab.G = b->d_grad; ab.C = b->comp.p;
     for (int64_t c = 0; c < b->n_chunk; ++c) {
         const int64_t begin = c * b->chunk;
@@ -1809,7 +1807,6 @@ static int batch_create(mi_sim* sim, int32_t n_event, const int32_t* event_ids, 
                        ? std::max<int64_t>(1, std::min<int64_t>(hit_capacity, (int64_t)1 << 30))
                        : std::max<int64_t>(1, std::min<int64_t>(hit_capacity, rows_max / b->n_param));
         b->n_chunk = (hit_capacity + b->chunk - 1) / b->chunk;
-        b->tmp_bytes = std::max<size_t>(1, oa_launch::adjoint_sort_bytes(b->chunk, (uint32_t)b->n_det));
         BCHECK(upload(b->mat_block, adj->mat_block, (size_t)adj->n_mat + 1, s));
         BCHECK(upload(b->sample_bin, adj->sample_bin, (size_t)sim->n_wl, s));
         if (b->rows.reserve((size_t)((tape_only ? 1 : b->chunk) * b->n_param)) != hipSuccess)
@@ -1820,7 +1817,7 @@ static int batch_create(mi_sim* sim, int32_t n_event, const int32_t* event_ids, 
         BCHECK(b->val.reserve((size_t)b->chunk));
         BCHECK(b->key2.reserve((size_t)b->chunk));
         BCHECK(b->val2.reserve((size_t)b->chunk));
-        BCHECK(b->tmp.reserve(b->tmp_bytes));
+        BCHECK(b->tmp.reserve(oa_launch::adjoint_sort_words(b->chunk, (uint32_t)b->n_det)));
         BCHECK(b->seg.reserve((size_t)b->n_det + 1));
         BCHECK(hipEventCreate(&b->ev_mid));
         if (taping) {

@@ -60,7 +60,7 @@ struct AdjBufs {
     uint32_t n_det;
     float* S;
     uint32_t *key, *val, *key2, *val2;
-    void* tmp; size_t tmp_bytes;
+    uint32_t* tmp;
     int64_t* seg;
     float *G, *C;
 };
@@ -81,5 +81,5 @@ int adjoint_blocks_per_cu(int rng_kind, int stack_depth);
    (call with `device` current), and the per-launch event setup kernel */
 hipError_t noalloc_scratch(int device, void** ptr);
 hipError_t noalloc_setup(int64_t* ev, int32_t* ev_id, int64_t n_gs, int64_t n_photon, int32_t event_id, hipStream_t s);
-size_t adjoint_sort_bytes(int64_t n_hit, uint32_t n_det);
+size_t adjoint_sort_words(int64_t n_hit, uint32_t n_det);
 }

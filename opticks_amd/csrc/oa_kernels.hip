@@ -1071,7 +1071,7 @@ __global__ void __launch_bounds__(256) k_tape_det_reduce(SimParams P, AdjParams 
     }
 }
 
-#include <hipcub/hipcub.hpp>
+#include "oa_radix.h"
 
 namespace oa_launch {
 
@@ -1122,11 +1122,14 @@ hipError_t adjoint_chunk(const SimParams& P, const AdjBufs& a, int64_t begin, in
     auto order = [&]() -> hipError_t {
         if (P.tape) hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, P.tape_overflow, (int64_t)1);
         if (n_max > 0) {
+            /* the keys are made where an odd or even number of passes ends them in key2, val2 */
+            const int bits = det_key_bits(a.n_det);
+            const bool even = oa_radix::passes(bits) % 2 == 0;
+            uint32_t* k0 = even ? a.key2 : a.key;
+            uint32_t* v0 = even ? a.val2 : a.val;
             hipLaunchKernelGGL(k_hit_det, dim3((unsigned)((n_max + 255) / 256)), dim3(256), 0, s, P, a.hit, begin,
-                               n_max, a.hit_off, a.n_ev, a.hit_cap, a.n_det, a.key, a.val);
-            size_t tmp_bytes = a.tmp_bytes;
-            hipError_t e = hipcub::DeviceRadixSort::SortPairs(a.tmp, tmp_bytes, a.key, a.key2, a.val, a.val2,
-                                                              (int)n_max, 0, det_key_bits(a.n_det), s);
+                               n_max, a.hit_off, a.n_ev, a.hit_cap, a.n_det, k0, v0);
+            hipError_t e = oa_radix::sort(k0, even ? a.key : a.key2, v0, even ? a.val : a.val2, n_max, bits, a.tmp, s);
             if (e != hipSuccess) return e;
         }
         hipLaunchKernelGGL(k_det_segments, dim3((a.n_det + 1 + 255) / 256), dim3(256), 0, s, a.key2, n_max, a.n_det,
@@ -1167,13 +1170,7 @@ hipError_t adjoint_chunk(const SimParams& P, const AdjBufs& a, int64_t begin, in
     return hipGetLastError();
 }
 
-size_t adjoint_sort_bytes(int64_t n_hit, uint32_t n_det)
-{
-    size_t bytes = 0;
-    (void)hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, (uint32_t*)nullptr, (uint32_t*)nullptr,
-                                             (uint32_t*)nullptr, (uint32_t*)nullptr, (int)n_hit, 0, det_key_bits(n_det));
-    return bytes;
-}
+size_t adjoint_sort_words(int64_t n_hit, uint32_t n_det) { return oa_radix::words(n_hit, det_key_bits(n_det)); }
 
 } // namespace oa_launch
 

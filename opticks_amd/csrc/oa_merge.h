@@ -33,13 +33,12 @@ hipError_t gather_selected(int record, const void* d_in, int64_t n, const int32_
 
 /* significant key bits: (identity, bucket) as one integer */
 int key_bits(uint32_t max_id, uint32_t max_bucket);
-/* hipCUB temporary storage for n_sel pairs of such keys */
-size_t sort_bytes(int64_t n_sel, int bits);
+/* words of temporary storage for n_sel pairs of such keys */
+size_t sort_words(int64_t n_sel, int bits);
 /* stable sort of the n_sel selected by key: keys, keys2 hold n_sel words of 4 bytes (bits <= 32)
    or 8, order, order2 n_sel words; the sorted keys and their places in sel end in keys2, order2 */
 hipError_t sort_runs(int64_t n, const int32_t* count, const uint4* sel, int64_t n_sel, float tw, uint32_t max_bucket,
-                     int bits, void* keys, void* keys2, uint32_t* order, uint32_t* order2, void* tmp, size_t tmp_bytes,
-                     hipStream_t s);
+                     int bits, void* keys, void* keys2, uint32_t* order, uint32_t* order2, uint32_t* tmp, hipStream_t s);
 /* number of runs of equal keys into out, their tiles' offsets behind the selection's in count */
 hipError_t count_runs(int64_t n, int32_t* count, int64_t n_sel, int bits, const void* keys2, Result* out, hipStream_t s);
 /* one merged record per run, in key order, as many as fit out_cap */

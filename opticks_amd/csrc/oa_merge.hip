@@ -6,7 +6,7 @@
  *      selected" mask), stable;
  *   1. time window 0: return the selection in input order;
  *   2-4. key = (identity << 48) | (unsigned)(time / window) as a 64-bit
- *      integer, then a stable sort of the selected records by key; here the
+ *      integer, then a stable sort of the selected records by key (oa_radix.h); here the
  *      same order is sorted as identity << b | bucket, with b the bits of the
  *      largest bucket selected and identity its low 16 bits (the shift by 48
  *      keeps the same ones);
@@ -26,14 +26,15 @@
  * The tiles' offsets come from a small kernel between two passes: a look-back across the tiles
  * needs a ticket each, and tickets, one atomic on one word, come at 40-60 ns apiece over eight
  * L2s (k_select 180 us with 2,441 tiles, 665 with 4,883 and two atomics a tile).
- * 10M records, 2M selected, 0.7M merged: 662 -> 384 us (select 139, keys 11, sort 115 with its
- * fills, reduce 64; the rest gaps). Before, a flag pass, flagged select, key pass, 48-bit sort,
+ * 10M records, 2M selected, 0.7M merged: 662 -> 347 us (select 139, keys 11, sort 110, reduce 50;
+ * the rest launches and gaps). Before, a flag pass, flagged select, key pass, 48-bit sort,
  * run-length encode and scan, and a reduce over the records themselves.
  */
 #include <hip/hip_runtime.h>
-#include <hipcub/hipcub.hpp>
 #include <stdint.h>
+#include <utility>
 #include "oa_merge.h"
+#include "oa_radix.h"
 
 namespace {
 
@@ -249,53 +250,90 @@ __global__ void __launch_bounds__(256) k_count_runs(const Key* __restrict__ keys
     if (threadIdx.x == 0) count[blockIdx.x] = s_n[0] + s_n[1] + s_n[2] + s_n[3];
 }
 
+/* the merged record of a run so far. index: input index of the kept record (photon) or the
+   first (lite) */
+struct Folded {
+    uint32_t index;
+    float time;
+    uint32_t hitcount, flagmask;
+};
+
 /*
- * The merged record of the run of `len` equal keys at sorted position o (of at least len when
- * `open`: it goes on as long as the keys do), folded left to right with the record type's
- * reduce_op, four records' words in flight a step:
+ * The record types' reduce_op, a before b in sorted order:
  *   sphoton      r = (fminf(a.time, b.time) == a.time) ? a : b; flagmasks OR-ed, 16-bit
  *                hitcounts added
- *   sphotonlite  r = a; r.time = fminf(a.time, b.time); likewise (first: a's input index)
- * x: input index of the kept record, y: time, z: hitcount, w: flagmask
+ *   sphotonlite  r = a; r.time = fminf(a.time, b.time); likewise
+ * Associative, times that are not numbers included (such an a gives way to any b, such a b to
+ * any other a), so a run may be folded in pieces kept in order.
  */
-template <bool LITE, class Key>
-__device__ uint4 fold_run(const uint4* sel, const Key* keys, const uint32_t* order, int64_t n, int64_t o, int32_t len,
-                          bool open)
+template <bool LITE>
+__device__ inline Folded fold(const Folded& a, const Folded& b)
 {
-    uint32_t best = 0, fm = 0, hc = 0;
-    float bt = 0.f;
-    const auto fold = [&](const uint4& b) {
-        const float t = __uint_as_float(b.y);
-        if (LITE) bt = fminf(bt, t);
-        else if (!(fminf(bt, t) == bt)) { best = b.x; bt = t; }
-        fm |= b.w;
-        hc = (hc + (b.z >> 16)) & 0xffffu;
-    };
-    const auto four = [&](int64_t j, int32_t c) {
+    const float m = fminf(a.time, b.time);
+    const bool first = LITE || m == a.time;
+    return Folded{ first ? a.index : b.index, LITE ? m : first ? a.time : b.time, (a.hitcount + b.hitcount) & 0xffffu,
+                   a.flagmask | b.flagmask };
+}
+
+/* sorted positions [o, o + len), len > 0, left to right, four records' words in flight a step */
+template <bool LITE>
+__device__ Folded fold_range(const uint4* sel, const uint32_t* order, int64_t o, int64_t len)
+{
+    const auto one = [](const uint4& v) { return Folded{ v.x, __uint_as_float(v.y), v.z >> 16, v.w }; };
+    Folded r = one(sel[order[o]]);
+    for (int64_t j = 1; j < len; j += 4) {
         uint32_t w[4];
         uint4 b[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) w[u] = order[u < c ? j + u : j];
+        for (int u = 0; u < 4; ++u) w[u] = order[j + u < len ? o + j + u : o];
 #pragma unroll
         for (int u = 0; u < 4; ++u) b[u] = sel[w[u]];
-        if (j == o) { best = b[0].x; bt = __uint_as_float(b[0].y); hc = b[0].z >> 16; fm = b[0].w; }
-        else fold(b[0]);
 #pragma unroll
-        for (int u = 1; u < 4; ++u)
-            if (u < c) fold(b[u]);
-    };
-    for (int32_t j = 0; j < len; j += 4) four(o + j, len - j);
-    if (open) {
-        const Key key = keys[o];
-        for (int64_t j = o + len; j < n && keys[j] == key;) {
-            int32_t c = 1;
-            while (c < 4 && j + c < n && keys[j + c] == key) ++c;
-            four(j, c);
-            j += c;
-        }
+        for (int u = 0; u < 4; ++u)
+            if (j + u < len) r = fold<LITE>(r, one(b[u]));
     }
-    return make_uint4(best, __float_as_uint(bt), hc, fm);
+    return r;
 }
+
+/* the same by a wave: a piece to a lane, then the pieces pairwise */
+template <bool LITE>
+__device__ Folded fold_range_wave(const uint4* sel, const uint32_t* order, int64_t o, int64_t len, int lane)
+{
+    const int64_t each = (len + 63) / 64, b = lane * each < len ? lane * each : len;
+    const int64_t mine = len - b < each ? len - b : each;
+    Folded r{ 0u, 0.f, 0u, 0u };
+    if (mine > 0) r = fold_range<LITE>(sel, order, o + b, mine);
+    const int pieces = (int)((len + each - 1) / each);
+    for (int step = 1; step < 64; step <<= 1) {
+        const Folded q{ (uint32_t)__shfl_down((int)r.index, step), __shfl_down(r.time, step),
+                        (uint32_t)__shfl_down((int)r.hitcount, step), (uint32_t)__shfl_down((int)r.flagmask, step) };
+        if ((lane & (2 * step - 1)) == 0 && lane + step < pieces) r = fold<LITE>(r, q);
+    }
+    return r;                                        /* lane 0's */
+}
+
+/* end of the run of keys[o], which reaches `from` at least */
+template <class Key>
+__device__ int64_t run_end(const Key* keys, int64_t n, int64_t o, int64_t from)
+{
+    const Key key = keys[o];
+    int64_t lo = from, hi = n;                       /* first position in [lo, hi] with another key */
+    for (int64_t step = 1; lo < hi; step *= 2) {     /* most runs end close by */
+        const int64_t p = lo + step - 1;
+        if (p >= hi) break;
+        if (keys[p] != key) { hi = p; break; }
+        lo = p + 1;
+    }
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (keys[mid] == key) lo = mid + 1; else hi = mid;
+    }
+    return lo;
+}
+
+/* runs of more records than this are folded by a wave: the slowest of 64 lanes sets a wave's
+   pace (3M photons' lite records have runs of several hundred: k_reduce 213 us, and 25 so) */
+#define OA_LONG_RUN 32
 
 template <bool LITE, class Key>
 __global__ void __launch_bounds__(256) k_reduce(const uint32_t* __restrict__ in, const uint4* __restrict__ sel,
@@ -307,6 +345,9 @@ __global__ void __launch_bounds__(256) k_reduce(const uint32_t* __restrict__ in,
     __shared__ unsigned long long s_mask[4 * ROUNDS];
     __shared__ int32_t s_pre[4 * ROUNDS + 1];
     __shared__ uint16_t s_head[256 * ROUNDS + 1];
+    __shared__ uint16_t s_long[256 * ROUNDS / OA_LONG_RUN + 1];
+    __shared__ int32_t s_n_long;
+    __shared__ int64_t s_end;                        /* of the last run, which may go on past the tile */
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int64_t first = (int64_t)blockIdx.x * (256 * ROUNDS), base = offset[blockIdx.x];
     const int32_t here = (int32_t)(n - first < 256 * ROUNDS ? n - first : 256 * ROUNDS);
@@ -315,55 +356,65 @@ __global__ void __launch_bounds__(256) k_reduce(const uint32_t* __restrict__ in,
 #pragma unroll
     for (int k = 0; k < ROUNDS; ++k)
         if (heads >> k & 1u) s_head[rank_in_tile(k, s_mask, s_pre)] = (uint16_t)(k * 256 + t);
-    if (t == 0) s_head[total] = (uint16_t)here;
+    if (t == 0) { s_head[total] = (uint16_t)here; s_n_long = 0; }
+    __syncthreads();
+    if (t == 0 && total > 0) s_end = run_end(keys, n, first + s_head[total - 1], first + here);
     __syncthreads();
     const int64_t room = out_cap - base;
     const int32_t fit = (int32_t)(room < total ? (room > 0 ? room : 0) : total);
-    /* a run to a lane, then, of photon records, four lanes to a record */
-    for (int32_t h0 = 0; h0 < fit; h0 += 256) {
-        const int32_t h = h0 + t;
-        uint4 r = make_uint4(0u, 0u, 0u, 0u);
-        if (h < fit) r = fold_run<LITE>(sel, keys, order, n, first + s_head[h], s_head[h + 1] - s_head[h], h == total - 1);
+    const auto run_len = [&](int32_t h) { return (h == total - 1 ? s_end - first : (int64_t)s_head[h + 1]) - s_head[h]; };
+    /* the record that h0 + 64 wave + lane's run is merged into; photon records are copied by
+       four lanes each */
+    const auto write = [&](int32_t h, bool have, const Folded& r) {
         if (LITE) {
-            if (h < fit) {
-                const quad a = reinterpret_cast<const quad*>(in)[r.x];
-                reinterpret_cast<quad*>(out)[base + h] = quad{ r.z << 16 | (a.x & 0xffffu), r.y, a.z, r.w };
+            if (have) {
+                const quad a = reinterpret_cast<const quad*>(in)[r.index];
+                reinterpret_cast<quad*>(out)[base + h] = quad{ r.hitcount << 16 | (a.x & 0xffffu), __float_as_uint(r.time),
+                                                               a.z, r.flagmask };
             }
-            continue;
+            return;
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int src = 16 * q + (lane >> 2);              /* the wave's record this lane copies a quarter of */
-            const uint32_t best = (uint32_t)__shfl((int)r.x, src), hc = (uint32_t)__shfl((int)r.z, src),
-                           fm = (uint32_t)__shfl((int)r.w, src);
-            const int32_t hq = h0 + 64 * wave + src;
-            if (hq >= fit) continue;
-            const int part = lane & 3;
+            const int src = 16 * q + (lane >> 2), part = lane & 3;
+            const bool on = __shfl((int)have, src) != 0;
+            const uint32_t best = (uint32_t)__shfl((int)r.index, src), hc = (uint32_t)__shfl((int)r.hitcount, src),
+                           fm = (uint32_t)__shfl((int)r.flagmask, src);
+            const int32_t hq = __shfl(h, src);
+            if (!on) continue;
             quad w = reinterpret_cast<const quad*>(in)[(int64_t)best * 4 + part];
             if (part == 1) w.w = (w.w & 0x0000ffffu) | (hc << 16);
             if (part == 3) w.w = fm;
             reinterpret_cast<quad*>(out)[(base + hq) * 4 + part] = w;
         }
+    };
+    for (int32_t h0 = 0; h0 < fit; h0 += 256) {
+        const int32_t h = h0 + t;
+        const int64_t len = h < fit ? run_len(h) : 0;
+        const bool own = len > 0 && len <= OA_LONG_RUN;
+        Folded r{ 0u, 0.f, 0u, 0u };
+        if (own) r = fold_range<LITE>(sel, order, first + s_head[h], len);
+        if (len > OA_LONG_RUN) s_long[atomicAdd(&s_n_long, 1)] = (uint16_t)h;
+        write(h, own, r);
+    }
+    __syncthreads();
+    for (int32_t k = wave; k < s_n_long; k += 4) {
+        const int32_t h = s_long[k];
+        const Folded r = fold_range_wave<LITE>(sel, order, first + s_head[h], run_len(h), lane);
+        write(h, lane == 0, r);
     }
 }
 
 inline int bits_of(uint32_t v) { return v ? 32 - __builtin_clz(v) : 0; }
 
-template <class Key>
-size_t sort_bytes_t(int64_t n, int bits)
-{
-    size_t b = 0;
-    (void)hipcub::DeviceRadixSort::SortPairs(nullptr, b, (Key*)nullptr, (Key*)nullptr, (uint32_t*)nullptr,
-                                             (uint32_t*)nullptr, (int)n, 0, bits);
-    return b;
-}
-
+/* the keys are made where an odd or even number of sort passes ends them in keys2, order2 */
 template <class Key>
 hipError_t sort_t(const uint4* sel, int64_t n_tiles, const int32_t* offset, int64_t n, float tw, int bucket_bits, int bits,
-                  Key* keys, Key* keys2, uint32_t* order, uint32_t* order2, void* tmp, size_t tmp_bytes, hipStream_t s)
+                  Key* keys, Key* keys2, uint32_t* order, uint32_t* order2, uint32_t* tmp, hipStream_t s)
 {
+    if (oa_radix::passes(bits) % 2 == 0) { std::swap(keys, keys2); std::swap(order, order2); }
     hipLaunchKernelGGL(k_keys<Key>, dim3((unsigned)n_tiles), dim3(256), 0, s, sel, offset, tw, bucket_bits, keys, order);
-    return hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, keys, keys2, order, order2, (int)n, 0, bits, s);
+    return oa_radix::sort(keys, keys2, order, order2, n, bits, tmp, s);
 }
 
 template <class Key>
@@ -419,20 +470,16 @@ int key_bits(uint32_t max_id, uint32_t max_bucket)
     return b > 0 ? b : 1;
 }
 
-size_t sort_bytes(int64_t n_sel, int bits)
-{
-    return bits <= 32 ? sort_bytes_t<uint32_t>(n_sel, bits) : sort_bytes_t<uint64_t>(n_sel, bits);
-}
+size_t sort_words(int64_t n_sel, int bits) { return oa_radix::words(n_sel, bits); }
 
 hipError_t sort_runs(int64_t n, const int32_t* count, const uint4* sel, int64_t n_sel, float tw, uint32_t max_bucket,
-                     int bits, void* keys, void* keys2, uint32_t* order, uint32_t* order2, void* tmp, size_t tmp_bytes,
-                     hipStream_t s)
+                     int bits, void* keys, void* keys2, uint32_t* order, uint32_t* order2, uint32_t* tmp, hipStream_t s)
 {
     const int bb = bits_of(max_bucket);
     const int64_t nt = tiles(n, OA_SELECT_ROUNDS);
     return bits <= 32
-        ? sort_t(sel, nt, count, n_sel, tw, bb, bits, (uint32_t*)keys, (uint32_t*)keys2, order, order2, tmp, tmp_bytes, s)
-        : sort_t(sel, nt, count, n_sel, tw, bb, bits, (uint64_t*)keys, (uint64_t*)keys2, order, order2, tmp, tmp_bytes, s);
+        ? sort_t(sel, nt, count, n_sel, tw, bb, bits, (uint32_t*)keys, (uint32_t*)keys2, order, order2, tmp, s)
+        : sort_t(sel, nt, count, n_sel, tw, bb, bits, (uint64_t*)keys, (uint64_t*)keys2, order, order2, tmp, s);
 }
 
 hipError_t count_runs(int64_t n, int32_t* count, int64_t n_sel, int bits, const void* keys2, Result* out, hipStream_t s)
