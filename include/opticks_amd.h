@@ -396,6 +396,10 @@ int  mi_sim_merge_hits_device(mi_sim* sim, int32_t record, const void* d_in, int
                               uint32_t select_mask, float time_window,
                               void* d_out, int64_t out_capacity, int64_t* n_out, void* stream);
 
+/* Hits per detector: counts of the n_hit sphoton records whose sensor identifier (low 16 bits
+ * of identity) is 1..n_det, as n_det floats on the device. Asynchronous on the stream. */
+int  mi_hit_counts_device(const void* d_hit, int64_t n_hit, int32_t n_det, void* d_count, void* stream);
+
 /*
  * Captured batch (no counterpart in the reference): the batched form's
  * launch sequence -- genstep prefix, persistent propagation, hit compaction,

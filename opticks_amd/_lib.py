@@ -76,7 +76,7 @@ SYMBOLS = ["mi_config_default", "mi_last_error", "mi_version", "mi_sim_create", 
            "mi_batch_num_photon", "mi_batch_destroy", "mi_sim_autotune", "mi_batch_create_adjoint",
            "mi_batch_last_timing", "mi_sim_merge_hits_device", "mi_sim_simulate_lite_device",
            "mi_sim_simtrace_device", "mi_sim_simtrace", "mi_sim_simulate_device_noalloc", "mi_sim_run",
-           "mi_sim_fetch", "mi_host_alloc", "mi_host_free"]
+           "mi_sim_fetch", "mi_host_alloc", "mi_host_free", "mi_hit_counts_device"]
 
 _lib = None
 
@@ -102,6 +102,7 @@ def lib():
     L.mi_host_alloc.argtypes = [C.c_size_t, C.POINTER(C.c_void_p)]
     L.mi_host_free.argtypes = [C.c_void_p]
     L.mi_host_free.restype = None
+    L.mi_hit_counts_device.argtypes = [C.c_void_p, C.c_int64, C.c_int32, C.c_void_p, C.c_void_p]
     L.mi_sim_reset.argtypes = [C.c_void_p, C.c_int32]
     L.mi_sim_simulate_device.argtypes = [C.c_void_p, C.c_int32, C.c_void_p, C.c_int64, C.c_int64, C.c_int64,
                                          C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64,

@@ -121,6 +121,15 @@ def perturbed_theta(params: LengthParams, base: dict, seed=42, frac=0.2):
 def hits_per_detector(hit_t, n_hit, n_det):
     """Counts of hits per detector (sensor identifier 1..n_det) from a (M,4,4) hit tensor."""
     import torch
+    hits = hit_t[:n_hit]
+    if (hits.is_cuda and hits.dtype == torch.float32 and hits.dim() == 3 and hits.shape[1:] == (4, 4)
+            and hits.is_contiguous() and 1 <= n_det <= 0x7fffffff):
+        with torch.cuda.device(hits.device):
+            counts = torch.empty(n_det, dtype=torch.float32, device=hits.device)
+            L.check(L.lib().mi_hit_counts_device(hits.data_ptr() if len(hits) else None, len(hits), int(n_det),
+                                                 counts.data_ptr(), torch.cuda.current_stream().cuda_stream),
+                    "mi_hit_counts_device")
+        return counts
     if n_hit == 0:
         return torch.zeros(n_det, dtype=torch.float32, device=hit_t.device)
     ident = hit_t[:n_hit, 3, 1].contiguous().view(torch.int32) & 0xffff

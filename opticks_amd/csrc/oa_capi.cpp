@@ -1601,6 +1601,15 @@ int mi_sim_merge_hits_device(mi_sim* sim, int32_t record, const void* d_in, int6
     return MI_OK;
 }
 
+int mi_hit_counts_device(const void* d_hit, int64_t n_hit, int32_t n_det, void* d_count, void* stream)
+{
+    if (n_hit < 0 || (n_hit > 0 && !d_hit)) return fail(MI_ERR_ARG, "bad hit records");
+    if (n_det < 1 || !d_count) return fail(MI_ERR_ARG, "bad detector counts");
+    if ((n_hit + 255) / 256 > (int64_t)INT32_MAX) return fail(MI_ERR_CAPACITY, "too many hits in one count");
+    HIPCHECK(oa_launch::hit_counts(d_hit, n_hit, (uint32_t)n_det, (float*)d_count, (hipStream_t)stream));
+    return MI_OK;
+}
+
 int mi_sim_last_adjoint_timing(const mi_sim* sim, double* ms3)
 {
     if (!sim || !ms3) return fail(MI_ERR_ARG, "null argument");

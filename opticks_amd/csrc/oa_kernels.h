@@ -81,5 +81,7 @@ int adjoint_blocks_per_cu(int rng_kind, int stack_depth);
    (call with `device` current), and the per-launch event setup kernel */
 hipError_t noalloc_scratch(int device, void** ptr);
 hipError_t noalloc_setup(int64_t* ev, int32_t* ev_id, int64_t n_gs, int64_t n_photon, int32_t event_id, hipStream_t s);
+/* hits per detector 1..n_det of n sphoton records into n_det floats */
+hipError_t hit_counts(const void* d_hit, int64_t n, uint32_t n_det, float* d_count, hipStream_t s);
 size_t adjoint_sort_words(int64_t n_hit, uint32_t n_det);
 }

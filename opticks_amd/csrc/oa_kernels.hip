@@ -807,6 +807,23 @@ __global__ void k_hit_det(SimParams P, const float4* hits, int64_t begin, int64_
     val[i] = (uint32_t)i;
 }
 
+/* hits per detector (sensor identifier 1..n_det in an sphoton's low 16 identity bits): whole
+   numbers, turned to float in place at the end. 0.1M hits of 2,000 detectors: 9 us, where a
+   dozen tensor operations with two host waits between them took 300. */
+__global__ void k_hit_counts(const uint32_t* __restrict__ hits, int64_t n, uint32_t n_det, uint32_t* count)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t id = hits[16 * i + 13] & 0xffffu;
+    if (id >= 1u && id <= n_det) atomicAdd(count + (id - 1u), 1u);
+}
+
+__global__ void k_count_floats(uint32_t* count, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) count[i] = __float_as_uint((float)count[i]);
+}
+
 /* start of each detector's run in the sorted keys */
 __global__ void k_det_segments(const uint32_t* key, int64_t n, uint32_t n_det, int64_t* seg)
 {
@@ -1167,6 +1184,17 @@ hipError_t adjoint_chunk(const SimParams& P, const AdjBufs& a, int64_t begin, in
     else if (nj <= 2) OA_TAPE_REDUCE(2);
     else OA_TAPE_REDUCE(4);
 #undef OA_TAPE_REDUCE
+    return hipGetLastError();
+}
+
+hipError_t hit_counts(const void* d_hit, int64_t n, uint32_t n_det, float* d_count, hipStream_t s)
+{
+    uint32_t* c = reinterpret_cast<uint32_t*>(d_count);
+    const dim3 det((n_det + 255u) / 256u);
+    hipLaunchKernelGGL(k_zero_u32, det, dim3(256), 0, s, c, (int64_t)n_det);
+    if (n > 0)
+        hipLaunchKernelGGL(k_hit_counts, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (const uint32_t*)d_hit, n, n_det, c);
+    hipLaunchKernelGGL(k_count_floats, det, dim3(256), 0, s, c, (int64_t)n_det);
     return hipGetLastError();
 }
 

@@ -323,3 +323,21 @@ def test_tape_batch_adjoint_equals_replay_bitwise():
     for k in (1, 2):
         for a, b_ in zip(out[0], out[k]):
             assert np.array_equal(a.view(np.uint32), b_.view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [0, 1, 255, 257, 100_003])
+@pytest.mark.parametrize("n_det", [1, 300, 65535])
+def test_hit_counts_match_cpu(n, n_det):
+    """Counts on the device against the CPU path, with identifiers of 0, past n_det and with bits
+    above the 16, from a whole buffer and from a strided one."""
+    from opticks_amd.adjoint import hits_per_detector
+    rng = np.random.default_rng(n + n_det)
+    hit = np.zeros((n + 5, 4, 4), np.float32)
+    hit.view(np.uint32)[:, 3, 1] = rng.integers(0, min(n_det + 20, 65536), n + 5) | (rng.integers(0, 256, n + 5) << 24)
+    want = hits_per_detector(torch.from_numpy(hit), n, n_det)
+    hit_t = torch.from_numpy(hit).to("cuda:0")
+    got = hits_per_detector(hit_t, n, n_det)
+    assert got.dtype == want.dtype and torch.equal(got.cpu(), want)
+    wide = torch.zeros((n + 5, 4, 5), dtype=torch.float32, device="cuda:0")
+    wide[:, :, :4] = hit_t
+    assert torch.equal(hits_per_detector(wide[:, :, :4], n, n_det).cpu(), want)
