@@ -12,9 +12,8 @@ compiled in parallel, then linked.
 Flags: -ffp-contract=off keeps a*b+c unfused so results match the CPU checker
 bit for bit; packed FP32 instructions are disabled (-packed-fp32-ops); the
 AMDGPU machine scheduler runs its iterative ILP strategy, which leaves the
-propagation kernel fewer register spills under its 168-VGPR budget (56 instead
-of 85 spilled VGPRs) and measures 2% faster; instruction order only, the
-arithmetic and so the results are the same.
+propagation kernel fewer register spills under its 168-VGPR budget and measured
+2% faster; instruction order only, the arithmetic and so the results are the same.
 """
 from __future__ import annotations
 

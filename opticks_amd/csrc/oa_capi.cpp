@@ -219,6 +219,7 @@ struct mi_sim {
     DBuf<unsigned char> m_keys, m_keys2;
     DBuf<uint32_t> m_tmp;
     DBuf<int32_t> m_count;
+    DBuf<unsigned long long> ray_next;              /* simtrace's counter of claimed rays */
     DBuf<uint2> m_most;
     oa_merge::Result* m_result = nullptr;           /* pinned */
 };
@@ -743,7 +744,7 @@ void mi_sim_destroy(mi_sim* sim)
     sim->adj_key.release(); sim->adj_val.release(); sim->adj_key2.release(); sim->adj_val2.release();
     sim->adj_tmp.release(); sim->adj_seg.release();
     sim->m_sel.release(); sim->m_order.release(); sim->m_order2.release(); sim->m_keys.release(); sim->m_keys2.release();
-    sim->m_tmp.release(); sim->m_count.release(); sim->m_most.release();
+    sim->m_tmp.release(); sim->m_count.release(); sim->m_most.release(); sim->ray_next.release();
     if (sim->m_result) (void)hipHostFree(sim->m_result);
     sim->h_photon.release(); sim->h_seq.release(); sim->h_hit.release(); sim->h_simtrace.release();
     for (auto& e : sim->ev) if (e) (void)hipEventDestroy(e);
@@ -1323,9 +1324,9 @@ int mi_sim_simtrace_device(mi_sim* sim, const void* d_gensteps, int64_t n_gs, in
     P.gs_prefix = sim->prefix.p;
     P.n_gs = n_gs;
     P.n_photon = total;
-    HIPCHECK(sim->words.reserve(1));
-    HIPCHECK(oa_launch::zero_u64(sim->words.p, 1, s));
-    P.next = sim->words.p;
+    HIPCHECK(sim->ray_next.reserve(1));
+    HIPCHECK(oa_launch::zero_u64(sim->ray_next.p, 1, s));
+    P.next = sim->ray_next.p;
     HIPCHECK(oa_launch::simtrace(P, (float4*)d_simtrace, s));
     HIPCHECK(hipStreamSynchronize(s));
     return MI_OK;

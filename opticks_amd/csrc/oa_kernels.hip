@@ -9,11 +9,12 @@
  *                     genstep writing its photon range (QEvt.cu:181-226 seed
  *                     buffer, sysrap/iexpand.h); k_gs_event the event of every
  *                     genstep for batched launches
- *   k_compact
- *                     stable stream compaction of flagmask&hit_mask photons via
+ *   k_simtrace        frame-genstep rays, nearest hit
+ *   k_hit_counts      hits per detector
+ *   k_compact         stable stream compaction of flagmask&hit_mask photons via
  *                     a per-64-photon bitmask (QEvt::gatherHit_, SU.cu:145-160)
  *   k_trace           nearest-hit query (simtrace-style)
- *   k_refit_level               GPU refit of the TLAS levels after instance moves
+ *   k_refit_level     GPU refit of the TLAS levels after instance moves
  */
 #include <hip/hip_runtime.h>
 #include <mutex>

@@ -51,7 +51,7 @@ struct Lane {
  * and it is what needs the registers (node tests, CSG trees). Everything else a
  * photon carries is kept in LDS while it runs: stored by park() at the end of a
  * step, read back by unpark() after the trace. Left to the compiler these values
- * were spilled to scratch memory, whose slots (152 B a lane, 3.7 MB of the resident
+ * were spilled to scratch memory, whose slots (152 B a lane then, 3.7 MB of the resident
  * waves of an XCD, nearly its whole L2) missed the vector L1: a lone wave spent half
  * of a step waiting on memory. Word i of a lane is at base[i * STRIDE], so the lanes
  * of a wave are in different banks and pairs of words move in one instruction.
