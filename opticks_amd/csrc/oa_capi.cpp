@@ -1325,7 +1325,6 @@ int mi_sim_simtrace_device(mi_sim* sim, const void* d_gensteps, int64_t n_gs, in
     P.n_gs = n_gs;
     P.n_photon = total;
     HIPCHECK(sim->ray_next.reserve(1));
-    HIPCHECK(oa_launch::zero_u64(sim->ray_next.p, 1, s));
     P.next = sim->ray_next.p;
     HIPCHECK(oa_launch::simtrace(P, (float4*)d_simtrace, s));
     HIPCHECK(hipStreamSynchronize(s));

@@ -9,7 +9,7 @@
  *                     genstep writing its photon range (QEvt.cu:181-226 seed
  *                     buffer, sysrap/iexpand.h); k_gs_event the event of every
  *                     genstep for batched launches
- *   k_simtrace        frame-genstep rays, nearest hit
+ *   k_simtrace, k_simtrace_few   frame-genstep rays, nearest hit
  *   k_hit_counts      hits per detector
  *   k_compact         stable stream compaction of flagmask&hit_mask photons via
  *                     a per-64-photon bitmask (QEvt::gatherHit_, SU.cu:145-160)
@@ -232,6 +232,25 @@ __device__ void simtrace_record(const SimParams& P, float4* o, v3 pos, v3 dir, c
     o[3] = make_float4(dir.x, dir.y, dir.z, __uint_as_float(ii));
 }
 
+/* CSGOptiX7.cu:563-604 simtrace, a ray to a lane from start to end (see simtrace below) */
+template <bool EXT>
+__global__ void __launch_bounds__(64) OA_OCC k_simtrace_few(SimParams P, float4* out)
+{
+    extern __shared__ uint32_t s_lane[];             /* each lane's stack */
+    const int lane = threadIdx.x;
+    const int64_t first = (int64_t)blockIdx.x * 64, i = first + lane;
+    const int64_t last = first + 63 < P.n_photon ? first + 63 : P.n_photon - 1;
+    const int64_t g0 = wave_upper_index(P.gs_prefix, P.n_gs, first, lane);
+    const int64_t g1 = g0 + wave_upper_index(P.gs_prefix + g0, P.n_gs - g0, last, lane);
+    if (i > last) return;
+    const int64_t gsi = upper_index(P.gs_prefix, g0, g1 + 1, i);
+    v3 o, d;
+    simtrace_ray(P, reinterpret_cast<const float4*>(P.gensteps + 24 * gsi), i, o, d);
+    Prd prd;
+    trace<64, EXT>(P, s_lane + lane, o, d, P.tmin, P.tmax, prd);
+    simtrace_record(P, out + 4 * i, o, d, prd);
+}
+
 /* words of a ray in a wave's queue */
 #define OA_RAY_WORDS 16
 
@@ -249,13 +268,14 @@ __device__ void simtrace_record(const SimParams& P, float4* o, v3 pos, v3 dir, c
  * 40 / 48 / 56: 1.55 / 1.47 / 1.45 / 1.47 ms; OA_RAY_REFILL 8 / 12 / 16 / 24: 1.48 / 1.45 / 1.47 / 1.47.
  * Waves claim rays from a counter (P.next, zero at the start), since those among the detectors
  * take longest: dealt out in advance, 2.40 ms. A claim is 256 rays, the counter being one word
- * (64: 2.18 ms, 128: 1.52, 256: 1.45), and down to 64 where that leaves a wave fewer than eight.
+ * (64: 2.18 ms, 128: 1.52, 256: 1.45).
  */
 #define OA_RAY_LEAVES 48
 #define OA_RAY_REFILL 12
+#define OA_RAY_CLAIM 256
 #define OA_RAY_QUEUE (OA_RAY_REFILL + 64)
 template <bool EXT>
-__global__ void __launch_bounds__(64) OA_OCC k_simtrace(SimParams P, int claim, float4* out)
+__global__ void __launch_bounds__(64) OA_OCC k_simtrace(SimParams P, float4* out)
 {
     extern __shared__ uint32_t s_lane[];             /* the queue, then each lane's stack */
     uint32_t* stk = s_lane + OA_RAY_WORDS * OA_RAY_QUEUE + threadIdx.x;
@@ -285,9 +305,9 @@ __global__ void __launch_bounds__(64) OA_OCC k_simtrace(SimParams P, int claim, 
             while (queued < OA_RAY_REFILL) {
                 if (next == end) {
                     unsigned long long c = 0ull;
-                    if (lane == 0) c = atomicAdd(P.next, (unsigned long long)claim);
+                    if (lane == 0) c = atomicAdd(P.next, (unsigned long long)OA_RAY_CLAIM);
                     next = (int64_t)__shfl(c, 0);
-                    end = next + claim < P.n_photon ? next + claim : P.n_photon;
+                    end = next + OA_RAY_CLAIM < P.n_photon ? next + OA_RAY_CLAIM : P.n_photon;
                     if (next >= P.n_photon) { next = end; break; }
                 }
                 const int64_t last = (next + 64 < end ? next + 64 : end) - 1, i = next + lane;
@@ -737,8 +757,25 @@ hipError_t zero_u64(unsigned long long* p, int64_t n, hipStream_t s)
     return hipGetLastError();
 }
 
+/*
+ * Persistent waves pay where they hold many rays each and the rays walk: every claim of rays is
+ * an atomic on one word, and the last rays of a wave run alone. A ray to a lane / persistent /
+ * a ray to a lane with sixteen-step genstep lookups, as it was, in us, 2,000 detectors: 0.4M rays
+ * 162 / 269 / 186, 1M 273 / 398 / 394, 2M 420 / 591 / 556, 4M 731 / 721 / 901, 10M
+ * 1,653 / 1,442 / 1,944. Without a TLAS (a water sphere) every ray is settled by the front
+ * instances: 10M 392 / 612 / 690.
+ */
+#define OA_RAY_MANY 4000000
 hipError_t simtrace(const SimParams& P, float4* out, hipStream_t s)
 {
+    if (P.n_photon < OA_RAY_MANY || P.tlas_empty) {
+        const dim3 grid((unsigned)((P.n_photon + 63) / 64));
+        const unsigned stacks = 64u * (unsigned)P.stack_depth * 4u;
+        if (P.ext_leaves) hipLaunchKernelGGL(k_simtrace_few<true>, grid, dim3(64), stacks, s, P, out);
+        else hipLaunchKernelGGL(k_simtrace_few<false>, grid, dim3(64), stacks, s, P, out);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, P.next, (int64_t)1);
     const unsigned lds = (unsigned)(OA_RAY_WORDS * OA_RAY_QUEUE + 64 * P.stack_depth) * 4u;
     int dev = 0, n_cu = 0, per_cu = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -749,10 +786,8 @@ hipError_t simtrace(const SimParams& P, float4* out, hipStream_t s)
     if (e != hipSuccess) return e;
     const int64_t need = (P.n_photon + 63) / 64, slots = (int64_t)n_cu * (per_cu > 0 ? per_cu : 8);
     const unsigned nb = (unsigned)(need < slots ? need : slots);
-    const int64_t share = P.n_photon / (8 * (int64_t)nb) / 64;
-    const int claim = 64 * (int)(share < 1 ? 1 : share > 4 ? 4 : share);
-    if (P.ext_leaves) hipLaunchKernelGGL(k_simtrace<true>, dim3(nb), dim3(64), lds, s, P, claim, out);
-    else hipLaunchKernelGGL(k_simtrace<false>, dim3(nb), dim3(64), lds, s, P, claim, out);
+    if (P.ext_leaves) hipLaunchKernelGGL(k_simtrace<true>, dim3(nb), dim3(64), lds, s, P, out);
+    else hipLaunchKernelGGL(k_simtrace<false>, dim3(nb), dim3(64), lds, s, P, out);
     return hipGetLastError();
 }
 

@@ -184,8 +184,9 @@ def test_event_arrays_are_their_own():
         assert np.array_equal(seq, seq0)
 
 
-# fewer rays than lanes, around a wave and a claim of rays, more than the waves hold at once
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 4099, 700_001])
+# fewer rays than lanes, around a wave, and enough for the persistent kernel, with and without a
+# whole number of its claims of 256
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 4099, 700_001, 3_999_999, 4_000_000, 4_000_037])
 @pytest.mark.parametrize("world", ["shell", "plain", "tree", "onions", "zoo"])
 def test_simtrace_queue_matches_checker(world, n):
     """Rays that the front instances settle, that wait for the walk and for the leaf phase, and
