@@ -275,7 +275,10 @@ class QSim:
             return None
         L.check(rc, "mi_sim_run")
         n, m = out.n_photon, out.n_hit
-        om = self.config.output_mask
+        # the handle's outputs: self.config may have been changed since, without set_config
+        om = self.get_config_c().output_mask
+        if not self.config.output_mask & L.MI_OUT_HIT:
+            om &= ~L.MI_OUT_HIT
         # arrays of their own for every event, over pinned memory that the copies fill directly
         new = {b: self._host.take(max(64, size)) if om & b else None
                for b, size in ((L.MI_OUT_PHOTON, 64 * n), (L.MI_OUT_SEQ, 32 * n), (L.MI_OUT_HIT, 64 * m))}
