@@ -56,6 +56,7 @@ struct DBuf {
         size_t bytes = std::max<size_t>(want, 1) * sizeof(T);
         hipError_t e = hipMalloc((void**)&p, bytes);
         if (e == hipSuccess) n = std::max<size_t>(want, 1);
+        else { p = nullptr; (void)hipGetLastError(); }   /* reported here, not by the next launch */
         return e;
     }
     void release() { if (p) (void)hipFree(p); p = nullptr; n = 0; }
@@ -188,7 +189,6 @@ struct mi_sim {
     DBuf<unsigned long long> next;       /* photon counter of the adjoint replay */
     LaunchResult* result = nullptr;      /* pinned: the last launch's counts and clock */
     double clock_ms = 1e-5;              /* device wall clock tick */
-    int64_t photon_cap = 0;              /* photons the single-event buffers hold (launch_reserve) */
     int grid_key[3] = { -1, -1, -1 }, grid_blocks = 0;   /* wave_grid's last answer */
     /* outputs of the host-array entry point */
     DBuf<float4> photon, hit;
@@ -877,17 +877,25 @@ static int launch(mi_sim* sim, SimParams& P, hipStream_t s)
     return MI_OK;
 }
 
-/* buffers of a single-event launch of up to n photons; kept, and grown as events need */
+/* buffers of a launch of up to n photons; kept, and grown as events and batches need */
 static int launch_reserve(mi_sim* sim, int64_t n)
 {
-    if (n <= sim->photon_cap) return MI_OK;
-    const size_t nw = (size_t)((n + 63) / 64);
     HIPCHECK(sim->words.reserve((size_t)oa_launch::clear_words(n)));
     HIPCHECK(sim->seed.reserve((size_t)n));
-    HIPCHECK(sim->word_prefix.reserve(nw + 1));
+    HIPCHECK(sim->word_prefix.reserve((size_t)((n + 63) / 64) + 1));
     HIPCHECK(sim->tile_base.reserve((size_t)oa_launch::compact_tiles(n) + 1));
-    sim->photon_cap = n;
     return MI_OK;
+}
+
+/* photons that those buffers hold, read off the buffers themselves: a failed allocation leaves
+   one of them empty */
+static int64_t photons_held(const mi_sim* sim)
+{
+    const int64_t words = (int64_t)sim->words.n, seeds = (int64_t)sim->seed.n, prefixes = (int64_t)sim->word_prefix.n,
+                  tiles = (int64_t)sim->tile_base.n;
+    /* w bitmask words take w + ceil(w / 256) + 2 cleared ones */
+    const int64_t w = std::min({ 256 * std::max<int64_t>(words - 2, 0) / 257, prefixes - 1, 256 * (tiles - 1) });
+    return std::max<int64_t>(0, std::min(64 * w, seeds));
 }
 
 static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gensteps, int64_t n_gs, int64_t n_photon,
@@ -915,7 +923,7 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
        where it decides something: slices, rows of precooked uniforms, the plain kernel's grid,
        and where there was no event so far. */
     std::vector<int64_t> hprefix;
-    if (max_slot > 0 || (n_photon < 0 && (sim->photon_cap == 0 || sim->cfg.rng_kind == MI_RNG_PRECOOKED ||
+    if (max_slot > 0 || (n_photon < 0 && (photons_held(sim) == 0 || sim->cfg.rng_kind == MI_RNG_PRECOOKED ||
                                            sim->cfg.kernel == MI_KERNEL_PLAIN))) {
         HIPCHECK(oa_launch::gs_prefix((const float*)d_gensteps, n_gs, sim->prefix.p, s));
         hprefix.resize((size_t)n_gs + 1);
@@ -961,9 +969,9 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
         const int64_t n_arg = sliced ? hprefix[g1] - hprefix[g0] : n_photon;
         if (n_arg == 0) continue;
         for (;;) {
-            int rc = launch_reserve(sim, std::max<int64_t>(n_arg, 1));
+            int rc = n_arg >= 0 ? launch_reserve(sim, n_arg) : MI_OK;
             if (rc) return rc;
-            const int64_t cap = n_arg >= 0 ? n_arg : sim->photon_cap;
+            const int64_t cap = n_arg >= 0 ? n_arg : photons_held(sim);
             if (taping) {
                 if (tape_stride == 0 || !sliced) tape_stride = sliced ? n_photon : cap;
                 HIPCHECK(sim->tape.reserve((size_t)tape_stride * 3 * (size_t)K));

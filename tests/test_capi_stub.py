@@ -65,3 +65,39 @@ def test_outputs_follow_the_handles_mask(stub):
     sim.config.output_mask = L.MI_OUT_PHOTON
     assert sim.simulate(event(100)) is None
     sim.close()
+
+
+def run_device(lib, sim, gs, n_photon=-1, n_alloc=None):
+    """mi_sim_simulate_device over host arrays: (return code, hits)"""
+    n = int(gs[:, 0, 3].view(np.int32).sum()) if n_alloc is None else n_alloc
+    photon = np.zeros((n, 4, 4), np.float32)
+    hit = np.zeros((n, 4, 4), np.float32)
+    m = L.C.c_int64(-1)
+    rc = lib.mi_sim_simulate_device(sim.handle, 0, gs.ctypes.data, len(gs), n_photon, 0, photon.ctypes.data, None,
+                                    hit.ctypes.data, n, L.C.byref(m), None)
+    return rc, m.value
+
+
+@pytest.mark.parametrize("grow", ["event", "batch"])
+@pytest.mark.parametrize("known", [True, False])
+def test_event_after_a_failed_allocation(stub, grow, known):
+    """An event or a batch too large for the memory fails with an error; the events after it get
+    buffers that hold them."""
+    sim = sim_of()
+    small, large = event(1000), event(1_000_000)
+    assert run_device(stub, sim, small) == (0, 500)
+    for limit in (100_000, 1_000_000, 3_900_000):
+        stub.stub_limit(limit)                         # the first, second, ... buffer cannot grow
+        if grow == "event":
+            rc, _ = run_device(stub, sim, large, n_photon=1_000_000)
+        else:
+            ev, off, po, ho = (np.array(a, t) for a, t in (([0], np.int32), ([0, 1], np.int64), ([0, 0], np.int64),
+                                                           ([0, 0], np.int64)))
+            rc = stub.mi_sim_simulate_batch_device(sim.handle, 1, ev.ctypes.data, off.ctypes.data, large.ctypes.data,
+                                                   po.ctypes.data, None, None, None, 0, ho.ctypes.data, None)
+        assert rc < 0 and "stub" in L.last_error()
+        assert run_device(stub, sim, small, n_photon=1000 if known else -1) == (0, 500)
+        assert stub.stub_bad() == 0
+    stub.stub_reset()
+    assert run_device(stub, sim, large) == (0, 500_000)
+    sim.close()
