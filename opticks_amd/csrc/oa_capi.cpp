@@ -918,13 +918,14 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
                                     std::to_string(total) + " photons");
     };
     /* The gensteps' photons are counted on the device, and a launch on them does not wait for
-       the host to know: its buffers are sized for the caller's count, or for the largest event
-       so far, and the host sees afterwards whether that held. It waits for the count first
-       where it decides something: slices, rows of precooked uniforms, the plain kernel's grid,
-       and where there was no event so far. */
+       the host to know: the buffers of earlier events are used as they are, and the host sees
+       afterwards whether they held the event. It waits for the count first where it decides
+       something: slices, rows of precooked uniforms, the plain kernel's grid, and where the
+       buffers are too small for the caller's count, which may be more than the gensteps have. */
     std::vector<int64_t> hprefix;
-    if (max_slot > 0 || (n_photon < 0 && (photons_held(sim) == 0 || sim->cfg.rng_kind == MI_RNG_PRECOOKED ||
-                                           sim->cfg.kernel == MI_KERNEL_PLAIN))) {
+    const int64_t held = photons_held(sim);
+    if (max_slot > 0 || held == 0 || n_photon > held ||
+        (n_photon < 0 && (sim->cfg.rng_kind == MI_RNG_PRECOOKED || sim->cfg.kernel == MI_KERNEL_PLAIN))) {
         HIPCHECK(oa_launch::gs_prefix((const float*)d_gensteps, n_gs, sim->prefix.p, s));
         hprefix.resize((size_t)n_gs + 1);
         HIPCHECK(hipMemcpyAsync(hprefix.data(), sim->prefix.p, sizeof(int64_t) * (n_gs + 1), hipMemcpyDeviceToHost, s));

@@ -101,3 +101,16 @@ def test_event_after_a_failed_allocation(stub, grow, known):
     stub.stub_reset()
     assert run_device(stub, sim, large) == (0, 500_000)
     sim.close()
+
+
+@pytest.mark.parametrize("n_photon", [1001, 10 ** 6, 10 ** 12])
+@pytest.mark.parametrize("tape", [0, 32])
+def test_too_many_photons_are_refused_without_buffers_for_them(stub, n_photon, tape):
+    sim = sim_of(adjoint_tape=tape)
+    for first in (False, True):
+        stub.stub_reset()
+        rc, m = run_device(stub, sim, event(1000), n_photon=n_photon, n_alloc=1000)
+        assert rc == -1 and m == 0 and f"n_photon {n_photon} exceeds the gensteps' 1000 photons" in L.last_error()
+        assert stub.stub_largest() < 1001 * 12 * max(tape, 1) + 4096
+        assert run_device(stub, sim, event(1000)) == (0, 500)
+    sim.close()
