@@ -203,7 +203,7 @@ struct mi_sim {
     struct TapeKey {
         bool valid = false;
         int32_t event_id = 0, k = 0;
-        int64_t photon_offset = 0, n_photon = 0, stride = 0, n_gs = 0;
+        int64_t photon_offset = 0, n_photon = 0, n_gs = 0;
         const void* gs = nullptr;
         uint64_t generation = 0;
     } tape_key;
@@ -887,15 +887,26 @@ static int launch_reserve(mi_sim* sim, int64_t n)
     return MI_OK;
 }
 
-/* photons that those buffers hold, read off the buffers themselves: a failed allocation leaves
-   one of them empty */
-static int64_t photons_held(const mi_sim* sim)
+/* the adjoint tape of an event of n photons, K records each; none for K = 0 */
+static int tape_reserve(mi_sim* sim, int64_t n, int32_t K)
+{
+    if (K == 0) return MI_OK;
+    HIPCHECK(sim->tape.reserve((size_t)n * 3 * (size_t)K));
+    HIPCHECK(sim->tape_n.reserve((size_t)n));
+    return MI_OK;
+}
+
+/* photons that these buffers, and for K > 0 the tape, hold, read off the buffers
+   themselves: a failed allocation leaves one of them empty */
+static int64_t photons_held(const mi_sim* sim, int32_t K)
 {
     const int64_t words = (int64_t)sim->words.n, seeds = (int64_t)sim->seed.n, prefixes = (int64_t)sim->word_prefix.n,
                   tiles = (int64_t)sim->tile_base.n;
     /* w bitmask words take w + ceil(w / 256) + 2 cleared ones */
     const int64_t w = std::min({ 256 * std::max<int64_t>(words - 2, 0) / 257, prefixes - 1, 256 * (tiles - 1) });
-    return std::max<int64_t>(0, std::min(64 * w, seeds));
+    int64_t n = std::max<int64_t>(0, std::min(64 * w, seeds));
+    if (K > 0) n = std::min(n, std::min((int64_t)(sim->tape.n / (3 * (size_t)K)), (int64_t)sim->tape_n.n));
+    return n;
 }
 
 static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gensteps, int64_t n_gs, int64_t n_photon,
@@ -923,7 +934,10 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
        something: slices, rows of precooked uniforms, the plain kernel's grid, and where the
        buffers are too small for the caller's count, which may be more than the gensteps have. */
     std::vector<int64_t> hprefix;
-    const int64_t held = photons_held(sim);
+    /* adjoint tape: wavefront kernel, full photon records (not the lite form) */
+    const int32_t K = sim->cfg.kernel == MI_KERNEL_WAVEFRONT && !d_lite ? sim->cfg.adjoint_tape : 0;
+    const bool taping = K > 0;
+    const int64_t held = photons_held(sim, K);
     if (max_slot > 0 || held == 0 || n_photon > held ||
         (n_photon < 0 && (sim->cfg.rng_kind == MI_RNG_PRECOOKED || sim->cfg.kernel == MI_KERNEL_PLAIN))) {
         HIPCHECK(oa_launch::gs_prefix((const float*)d_gensteps, n_gs, sim->prefix.p, s));
@@ -958,10 +972,11 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
         slices.emplace_back(0, n_gs);
     }
     const bool sliced = slices.size() > 1;
-    /* adjoint tape: wavefront kernel, full photon records (not the lite form) */
-    const int32_t K = sim->cfg.adjoint_tape;
-    const bool taping = K > 0 && sim->cfg.kernel == MI_KERNEL_WAVEFRONT && !d_lite;
-    int64_t hits = 0, tape_stride = 0;
+    if (n_photon >= 0) {                 /* a sliced event has one tape */
+        const int rc = tape_reserve(sim, n_photon, K);
+        if (rc) return rc;
+    }
+    int64_t hits = 0;
     double ms[4] = { 0.0, 0.0, 0.0, 0.0 };
     const volatile LaunchResult* res = sim->result;
     for (auto& sl : slices) {
@@ -972,12 +987,7 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
         for (;;) {
             int rc = n_arg >= 0 ? launch_reserve(sim, n_arg) : MI_OK;
             if (rc) return rc;
-            const int64_t cap = n_arg >= 0 ? n_arg : photons_held(sim);
-            if (taping) {
-                if (tape_stride == 0 || !sliced) tape_stride = sliced ? n_photon : cap;
-                HIPCHECK(sim->tape.reserve((size_t)tape_stride * 3 * (size_t)K));
-                HIPCHECK(sim->tape_n.reserve((size_t)tape_stride));
-            }
+            const int64_t cap = n_arg >= 0 ? n_arg : photons_held(sim, K);
             const oa_launch::SetupArgs a = { (const float*)d_gensteps + 24 * g0, g1 - g0, n_arg, cap, sim->prefix.p,
                                              sim->seed.p, sim->words.p, oa_launch::clear_words(cap), sim->evbuf.p,
                                              sim->ev_id.p, event_id, sim->n_dev.p, sim->result, wave_count(sim) };
@@ -1001,10 +1011,10 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
             P.hitwords = sim->words.p;
             P.next = sim->words.p + oa_launch::next_offset(cap);
             if (taping) {
-                /* segment-major records with the whole launch's photon count as the stride */
+                /* segment-major records with the event's photon count as the stride */
                 P.tape = sim->tape.p + (size_t)p0 * 3;
                 P.tape_n = sim->tape_n.p + p0;
-                P.tape_stride = tape_stride;
+                P.tape_stride = sliced ? n_photon : 0;
                 P.tape_k = K;
             }
             HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s));
@@ -1016,6 +1026,7 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
             if (n_arg > res->total) return too_many(res->total);
             if (n_arg >= 0 || res->total <= cap) break;
             rc = launch_reserve(sim, res->total);        /* a larger event than any so far: once more */
+            if (!rc) rc = tape_reserve(sim, res->total, K);
             if (rc) return rc;
         }
         if (!sliced) {
@@ -1029,7 +1040,7 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
     if (taping) {
         mi_sim::TapeKey& tk = sim->tape_key;
         tk.valid = true; tk.event_id = event_id; tk.k = K; tk.photon_offset = photon_offset;
-        tk.n_photon = n_photon; tk.stride = tape_stride; tk.n_gs = n_gs; tk.gs = d_gensteps;
+        tk.n_photon = n_photon; tk.n_gs = n_gs; tk.gs = d_gensteps;
         tk.generation = sim->generation;
     }
     for (int i = 0; i < 4; ++i) sim->last_ms[i] = ms[i];
@@ -1502,7 +1513,7 @@ int mi_sim_adjoint_device(mi_sim* sim, int32_t event_id, const void* d_gensteps,
         tk.n_gs == n_gs && tk.gs == d_gensteps && tk.generation == sim->generation &&
         oa_launch::tape_reduce_rows(n_param) > 0) {
         HIPCHECK(sim->tape_flag.reserve(1));
-        P.tape = sim->tape.p; P.tape_n = sim->tape_n.p; P.tape_stride = tk.stride; P.tape_k = tk.k;
+        P.tape = sim->tape.p; P.tape_n = sim->tape_n.p; P.tape_stride = tk.n_photon; P.tape_k = tk.k;
         P.tape_overflow = sim->tape_flag.p;
     }
     const uint32_t n_det = (uint32_t)adj->n_det;

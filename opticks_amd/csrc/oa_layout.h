@@ -182,7 +182,7 @@ struct SimParams {
        segments the photon had (above tape_k: the records stop at tape_k) */
     uint32_t* tape;
     uint8_t*  tape_n;
-    int64_t   tape_stride;
+    int64_t   tape_stride;        /* 0 (forward kernels): the launch's photon count */
     int32_t   tape_k;
     uint32_t* tape_overflow;      /* set when a hit's photon had more segments than the tape holds */
 };

@@ -65,6 +65,7 @@ enum : int { SEG_SAIL = 0, SEG_ABSORB = 1, SEG_SCATTER = 2 };
    segment number: `at` names it before the step, `finish` gets the count. */
 struct NoTape {
     static constexpr bool keeps_seq = true;
+    __device__ inline __attribute__((always_inline)) void begin(const SimParams&, int64_t) {}
     __device__ inline __attribute__((always_inline)) void at(const SimParams&, int64_t, int) {}
     __device__ inline __attribute__((always_inline)) void seg(const SimParams&, int, float, float, float, float, int) {}
     __device__ inline __attribute__((always_inline)) void finish(const SimParams&, int64_t, int) {}
@@ -77,11 +78,15 @@ struct NoTape {
    and the number it had. The adjoint then scores a hit from its records instead
    of replaying the photon. It adds no per-lane state: it holds the photon index
    and step number the lane keeps anyway, and forms the record address from them
-   and the launch fields only at the store. */
+   and the launch's fields only at the store. */
 struct RecordTape {
     static constexpr bool keeps_seq = true;
-    int64_t g;
+    int64_t g, stride;
     int32_t step;
+    __device__ inline __attribute__((always_inline)) void begin(const SimParams& P, int64_t n_photon)
+    {
+        stride = P.tape_stride ? P.tape_stride : n_photon;
+    }
     __device__ inline __attribute__((always_inline)) void at(const SimParams&, int64_t g_, int step_)
     {
         g = g_; step = step_;
@@ -92,7 +97,7 @@ struct RecordTape {
         if (step < P.tape_k) {
             /* streaming stores: the records are read back only by the adjoint, after the
                launch (0.38 -> 0.31 ms of taping on 10M photons against cached stores) */
-            uint32_t* r = P.tape + 3 * ((int64_t)step * P.tape_stride + g);
+            uint32_t* r = P.tape + 3 * ((int64_t)step * stride + g);
             __builtin_nontemporal_store((uint32_t)line | ((uint32_t)ev << 30), &r[0]);
             __builtin_nontemporal_store(__float_as_uint(wl), &r[1]);
             __builtin_nontemporal_store(__float_as_uint(ell), &r[2]);

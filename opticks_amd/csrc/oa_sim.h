@@ -420,6 +420,7 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_wave(SimParams P)
         if ((L.p.flagmask & P.hit_mask) != 0u) atomicOr(P.hitwords + (L.g >> 6), 1ull << (L.g & 63));
     };
     const int64_t n_photon = P.n_dev ? P.n_dev[0] : P.n_photon;
+    tape.begin(P, n_photon);
     for (int iter = 0;; ++iter) {
         OA_CYC_MARK(c_iter);
         const unsigned long long idle = __ballot(!active);

@@ -23,7 +23,7 @@ std::map<const char*, size_t> g_alloc;         /* live allocations */
 size_t g_limit = (size_t)1 << 40, g_largest = 0;
 std::atomic<int> g_bad{0}, g_inside{0}, g_overlap{0};
 int g_fail_trace = 0, g_resident = 4, g_waves_dealt = 0, g_grid = 0;
-int64_t g_n = 0;
+int64_t g_n = 0, g_stride = 0;
 
 hipError_t alloc(void** p, size_t n)
 {
@@ -66,6 +66,7 @@ void stub_fail_trace(int f) { g_fail_trace = f; }
 size_t stub_largest() { return g_largest; }
 int stub_bad() { return g_bad; }
 int stub_overlap() { return g_overlap; }
+int stub_tape_stride() { return (int)g_stride; }
 int stub_waves_dealt() { return g_waves_dealt; }
 int stub_grid() { return g_grid; }
 int stub_resident() { return g_resident; }
@@ -149,7 +150,8 @@ hipError_t simulate(const SimParams& P, int, int, int grid, hipStream_t)
     holds(P.hitwords, 8 * (size_t)((n + 63) / 64));
     holds(P.next, 8);
     if (P.tape) {
-        holds(P.tape, 12 * (size_t)(P.tape_k - 1) * (size_t)P.tape_stride + 12 * (size_t)n);
+        g_stride = P.tape_stride;
+        holds(P.tape, 12 * (size_t)(P.tape_k - 1) * (size_t)(P.tape_stride ? P.tape_stride : n) + 12 * (size_t)n);
         holds(P.tape_n, (size_t)n);
     }
     if (P.photon)

@@ -114,3 +114,26 @@ def test_too_many_photons_are_refused_without_buffers_for_them(stub, n_photon, t
         assert stub.stub_largest() < 1001 * 12 * max(tape, 1) + 4096
         assert run_device(stub, sim, event(1000)) == (0, 500)
     sim.close()
+
+
+def test_tape_of_an_event_of_unknown_size_is_its_own(stub):
+    """The adjoint tape of a small event after a large one without a tape is as large as the
+    small event needs."""
+    sim = sim_of()
+    assert run_device(stub, sim, event(1_000_000)) == (0, 500_000)
+    sim.config.adjoint_tape = 32
+    sim.set_config(sim.config)
+    stub.stub_reset()
+    for n in (1000, 3000, 500, 3000):
+        assert run_device(stub, sim, event(n)) == (0, n // 2)
+        assert stub.stub_bad() == 0 and stub.stub_largest() <= 3000 * 32 * 12
+        assert stub.stub_tape_stride() in (0, n)           # 0: the launch's own photon count
+    sim.config.adjoint_tape = 64                           # records of the same tape, more of them
+    sim.set_config(sim.config)
+    assert run_device(stub, sim, event(3000)) == (0, 1500)
+    sim.config.max_slot = 2000                             # slices of one event: the event's count
+    sim.set_config(sim.config)
+    gs = np.concatenate([event(1500), event(1000), event(700)])
+    assert run_device(stub, sim, gs) == (0, 750 + 500 + 350)
+    assert stub.stub_tape_stride() == 3200
+    sim.close()

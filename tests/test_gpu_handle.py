@@ -1,0 +1,70 @@
+"""One handle that sees events of very different sizes and kinds: each event's results and what it
+costs are those of a handle of its own (MI355X only)."""
+import gc
+
+import numpy as np
+import pytest
+
+import pyoracle as po
+from opticks_amd import configs
+from opticks_amd import _lib as L
+from opticks_amd.adjoint import yield_jacobian
+from opticks_amd.qsim import QSim, SEventConfig
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+if not torch.cuda.is_available():
+    pytest.skip("no GPU", allow_module_level=True)
+
+DEV = torch.device("cuda:0")
+
+
+class Device:
+    """An event's gensteps and output buffers on the GPU."""
+
+    def __init__(self, gensteps):
+        self.gs = torch.from_numpy(np.ascontiguousarray(gensteps, np.float32)).to(DEV)
+        self.n = int(np.ascontiguousarray(gensteps, np.float32).view(np.int32)[:, 0, 3].sum())
+        self.photon = torch.zeros((self.n, 4, 4), dtype=torch.float32, device=DEV)
+        self.seq = torch.zeros((self.n, 2, 2), dtype=torch.int64, device=DEV)
+        self.hit = torch.zeros((self.n, 4, 4), dtype=torch.float32, device=DEV)
+
+    def run(self, sim, n_photon=-1, eventID=0):
+        for t in (self.photon, self.seq, self.hit):
+            t.zero_()
+        m = sim.simulate_device(self.gs, self.photon, self.seq, self.hit, eventID=eventID, n_photon=n_photon)
+        return [t.cpu().numpy().view(np.uint32).copy() for t in (self.photon, self.seq, self.hit[:m])]
+
+
+def test_tape_after_a_larger_event():
+    """Taped events of unknown size after a larger one without a tape, after a larger taped one and
+    in slices: photons and adjoint of a handle that saw nothing else."""
+    w = configs.config3(num_gs=6, per_gs=500)
+    params = w.meta["params"]
+    cfg = dict(seed=w.seed, adjoint_tape=16)
+    small, mid = Device(w.gensteps[:2]), Device(w.gensteps)
+
+    def taped(sim, ev, n_photon):
+        out = ev.run(sim, n_photon)
+        G = yield_jacobian(sim, params, ev.gs, ev.hit, len(out[2]), 2000, n_photon=ev.n)
+        return out + [G.cpu().numpy().view(np.uint32)]
+
+    want = {}
+    for ev in (small, mid):
+        fresh = QSim(w.geometry, w.physics, SEventConfig(**cfg))
+        want[ev.n] = taped(fresh, ev, ev.n)
+        fresh.close()
+    assert want[mid.n][3].any()
+    sim = QSim(w.geometry, w.physics, SEventConfig(seed=w.seed))
+    Device(configs.config3(num_gs=4, per_gs=100_000).gensteps).run(sim)
+    free = torch.cuda.mem_get_info()[0]
+    sim.set_config(SEventConfig(**cfg))
+    for ev, n_photon in ((small, -1), (mid, -1), (small, -1), (small, small.n), (mid, mid.n)):
+        for got, ref in zip(taped(sim, ev, n_photon), want[ev.n]):
+            assert np.array_equal(got, ref)
+    assert free - torch.cuda.mem_get_info()[0] < 400_000 * 12 * 16 // 2
+    sim.set_config(SEventConfig(max_slot=1000, **cfg))
+    for got, ref in zip(taped(sim, mid, -1), want[mid.n]):
+        assert np.array_equal(got, ref)
+    sim.close()
