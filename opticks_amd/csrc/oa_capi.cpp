@@ -863,8 +863,8 @@ static int64_t wave_count(mi_sim* sim) { return (int64_t)wave_grid(sim) * (sim_b
 static int launch(mi_sim* sim, SimParams& P, hipStream_t s)
 {
     HIPCHECK(sim->words.reserve((size_t)oa_launch::clear_words(P.n_photon)));
-    P.hitwords = sim->words.p;
-    P.next = sim->words.p + oa_launch::next_offset(P.n_photon);
+    P.hitwords = sim->words.p + oa_launch::bitmask_offset(P.n_photon);
+    P.next = sim->words.p;
     HIPCHECK(sim->seed.reserve((size_t)P.n_photon));
     HIPCHECK(sim->gs_event.reserve((size_t)std::max<int64_t>(P.n_gs, 1)));
     HIPCHECK(oa_launch::seed_map(P.gs_prefix, P.n_gs, P.n_photon, sim->seed.p, P.ev_gs_begin, P.n_event,
@@ -989,7 +989,7 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
             if (rc) return rc;
             const int64_t cap = n_arg >= 0 ? n_arg : photons_held(sim, K);
             const oa_launch::SetupArgs a = { (const float*)d_gensteps + 24 * g0, g1 - g0, n_arg, cap, sim->prefix.p,
-                                             sim->seed.p, sim->words.p, oa_launch::clear_words(cap), sim->evbuf.p,
+                                             sim->seed.p, sim->words.p, sim->evbuf.p,
                                              sim->ev_id.p, event_id, sim->n_dev.p, sim->result, wave_count(sim) };
             HIPCHECK(oa_launch::setup(a, s));
             SimParams P = base_params(sim);
@@ -1008,8 +1008,8 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
             P.photon = d_photon ? (float4*)d_photon + 4 * p0 : nullptr;
             P.seq = d_seq ? (uint64_t*)d_seq + 4 * p0 : nullptr;
             P.photonlite = d_lite ? (uint4*)d_lite + p0 : nullptr;
-            P.hitwords = sim->words.p;
-            P.next = sim->words.p + oa_launch::next_offset(cap);
+            P.hitwords = sim->words.p + oa_launch::bitmask_offset(cap);
+            P.next = sim->words.p;
             if (taping) {
                 /* segment-major records with the event's photon count as the stride */
                 P.tape = sim->tape.p + (size_t)p0 * 3;
@@ -1019,8 +1019,7 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
             }
             HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s));
             HIPCHECK(oa_launch::compact_hits(sim->words.p, cap, sim->n_dev.p, sim->word_prefix.p, sim->tile_base.p,
-                                             sim->words.p + oa_launch::state_offset(cap), P.photon,
-                                             d_hit ? (float4*)d_hit + 4 * hits : nullptr,
+                                             P.photon, d_hit ? (float4*)d_hit + 4 * hits : nullptr,
                                              d_hit ? std::max<int64_t>(0, hit_capacity - hits) : 0, sim->result, s));
             HIPCHECK(hipStreamSynchronize(s));
             if (n_arg > res->total) return too_many(res->total);
@@ -1123,15 +1122,14 @@ int mi_sim_simulate_device_noalloc(mi_sim* sim, int32_t event_id, const void* d_
     P.photon = (float4*)d_photon;
     P.seq = (uint64_t*)d_seq;
     P.photonlite = nullptr;
-    P.hitwords = words;
-    P.next = words + oa_launch::next_offset(n_photon);
+    P.hitwords = words + oa_launch::bitmask_offset(n_photon);
+    P.next = words;
     P.wave_width = (int32_t)wave_width(n_photon, wave_count(sim));
     HIPCHECK(oa_launch::clear_launch(words, n_photon, wave_count(sim), s));
     HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s));
     HIPCHECK(hipEventRecord(sim->ev[2], s));
     HIPCHECK(oa_launch::compact_hits(words, n_photon, nullptr, word_prefix, tile_base,
-                                     words + oa_launch::state_offset(n_photon), (const float4*)d_photon,
-                                     (float4*)d_hit, d_hit ? hit_capacity : 0, nullptr, s));
+                                     (const float4*)d_photon, (float4*)d_hit, d_hit ? hit_capacity : 0, nullptr, s));
     HIPCHECK(hipEventRecord(sim->ev[3], s));
     int64_t hits = 0;
     HIPCHECK(hipMemcpyAsync(&hits, tile_base + oa_launch::compact_tiles(n_photon), sizeof(int64_t), hipMemcpyDeviceToHost, s));
@@ -1212,11 +1210,10 @@ int mi_sim_simulate_batch_device(mi_sim* sim, int32_t n_event, const int32_t* ev
     HIPCHECK(sim->word_prefix.reserve((size_t)n_words + 1));
     HIPCHECK(sim->tile_base.reserve((size_t)oa_launch::compact_tiles(n_photon) + 1));
     HIPCHECK(oa_launch::compact_hits(sim->words.p, n_photon, nullptr, sim->word_prefix.p, sim->tile_base.p,
-                                     sim->words.p + oa_launch::state_offset(n_photon), (const float4*)d_photon,
-                                     (float4*)d_hit, d_hit ? hit_capacity : 0, nullptr, s));
+                                     (const float4*)d_photon, (float4*)d_hit, d_hit ? hit_capacity : 0, nullptr, s));
     DBuf<int64_t>& hob = sim->evbuf;   /* reuse tail of evbuf for the offsets */
     int64_t* d_ho = hob.p + evh.size();
-    HIPCHECK(oa_launch::event_hit_offsets(sim->words.p, sim->word_prefix.p, sim->tile_base.p,
+    HIPCHECK(oa_launch::event_hit_offsets(P.hitwords, sim->word_prefix.p, sim->tile_base.p,
                                           P.ev_ph_begin, n_event, n_words, d_ho, s));
     HIPCHECK(hipMemcpyAsync(hit_offsets, d_ho, sizeof(int64_t) * (n_event + 1), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipEventRecord(sim->ev[3], s));
@@ -1709,10 +1706,9 @@ static hipError_t batch_work(mi_batch* b, SimParams P, const void* d_gensteps, c
     if ((e = oa_launch::clear_launch(b->words.p, b->n_photon, wave_count(sim), s)) != hipSuccess) return e;
     if ((e = oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s)) != hipSuccess) return e;
     if ((e = oa_launch::compact_hits(b->words.p, b->n_photon, nullptr, b->word_prefix.p, b->tile_base.p,
-                                     b->words.p + oa_launch::state_offset(b->n_photon), (const float4*)d_photon,
-                                     (float4*)d_hit, d_hit ? b->hit_capacity : 0, nullptr, s)) != hipSuccess)
+                                     (const float4*)d_photon, (float4*)d_hit, d_hit ? b->hit_capacity : 0, nullptr, s)) != hipSuccess)
         return e;
-    if ((e = oa_launch::event_hit_offsets(b->words.p, b->word_prefix.p, b->tile_base.p, P.ev_ph_begin, b->n_event,
+    if ((e = oa_launch::event_hit_offsets(P.hitwords, b->word_prefix.p, b->tile_base.p, P.ev_ph_begin, b->n_event,
                                           b->n_words, b->ho.p, s)) != hipSuccess)
         return e;
     if ((e = hipMemcpyAsync(b->h_out, b->ho.p, sizeof(int64_t) * (b->n_event + 1), hipMemcpyDeviceToHost, s)) != hipSuccess)
@@ -1813,8 +1809,8 @@ static int batch_create(mi_sim* sim, int32_t n_event, const int32_t* event_ids, 
     P.photon_offset = 0;
     P.photon = (float4*)d_photon;
     P.seq = (uint64_t*)d_seq;
-    P.hitwords = b->words.p;
-    P.next = b->words.p + oa_launch::next_offset(b->n_photon);
+    P.hitwords = b->words.p + oa_launch::bitmask_offset(b->n_photon);
+    P.next = b->words.p;
     P.seed_map = b->seed.p;
     P.gs_event = b->gs_event.p;
     if (adj) {

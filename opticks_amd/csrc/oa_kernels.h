@@ -11,23 +11,26 @@ hipError_t seed_map(const int64_t* d_prefix, int64_t n_gs, int64_t n_photon, uin
    gs_prefix_words(n_gs) words (block sums behind it) */
 int64_t gs_prefix_words(int64_t n_gs);
 hipError_t gs_prefix(const float* d_gs, int64_t n_gs, int64_t* d_prefix, hipStream_t s);
-/* start of a single-event launch (k_setup): seeds of up to cap photons, n_clear cleared words,
-   event bounds ev (4) and ev_id (1), the launch's photon count and wave_width n_dev (2) */
+/* start of a single-event launch (k_setup): seeds of up to cap photons, its cleared words (words:
+   clear_words(cap)), event bounds ev (4) and ev_id (1), the launch's photon count and wave_width
+   n_dev (2) */
 struct SetupArgs {
     const float* gs; int64_t n_gs, n_arg, cap;
     int64_t* prefix; uint32_t* seed;
-    unsigned long long* clear; int64_t n_clear;
+    unsigned long long* words;
     int64_t* ev; int32_t* ev_id; int32_t event_id;
     int64_t* n_dev; LaunchResult* out;
     int64_t n_wave;                     /* waves of the propagation grid */
 };
 hipError_t setup(const SetupArgs& a, hipStream_t s);
-/* Cleared words of a launch of n photons: the hit bitmask, then the state of the compaction's
-   tiles (256 bitmask words each) and its ticket, then the propagation's photon counter. */
+/* Cleared words of a launch of up to n photons: the propagation's photon counter, the compaction's
+   ticket and the state of its tiles (256 bitmask words each), then the hit bitmask. The counters
+   are in front, so that an event of fewer photons clears and reads what it needs alone. */
+#define OA_WORDS_TICKET 1
+#define OA_WORDS_STATE 2
 inline int64_t compact_tiles(int64_t n_photon) { return ((n_photon + 63) / 64 + 255) / 256; }
-inline int64_t state_offset(int64_t n_photon) { return (n_photon + 63) / 64; }
-inline int64_t next_offset(int64_t n_photon) { return state_offset(n_photon) + compact_tiles(n_photon) + 1; }
-inline int64_t clear_words(int64_t n_photon) { return next_offset(n_photon) + 1; }
+inline int64_t bitmask_offset(int64_t n_photon) { return OA_WORDS_STATE + compact_tiles(n_photon); }
+inline int64_t clear_words(int64_t n_photon) { return bitmask_offset(n_photon) + (n_photon + 63) / 64; }
 hipError_t simulate(const SimParams& P, int kernel, int block, int grid, hipStream_t s);
 int wave_blocks_per_cu(int block, int rng_kind, int stack_depth);   /* resident blocks of the persistent kernel per CU */
 unsigned sim_lds(int block, int rng_kind, int stack_depth);   /* LDS bytes of a propagation block */
@@ -36,12 +39,12 @@ hipError_t zero_u64(unsigned long long* p, int64_t n, hipStream_t s);
 /* the cleared words of a launch of n photons on n_wave waves, its counter set behind the photons dealt first */
 hipError_t clear_launch(unsigned long long* words, int64_t n_photon, int64_t n_wave, hipStream_t s);
 /* stable compaction of the hits among n_photon photons, or *n_dev of them where it is given;
-   d_state: cleared words from state_offset on; d_tile_base: compact_tiles + 1 words; out (may be
-   null): the hit count and the clock */
-hipError_t compact_hits(const unsigned long long* d_words, int64_t n_photon, const int64_t* n_dev, int32_t* d_word_prefix,
-                        int64_t* d_tile_base, unsigned long long* d_state, const float4* d_photon, float4* d_hit,
-                        int64_t hit_cap, LaunchResult* out, hipStream_t s);
-hipError_t event_hit_offsets(const unsigned long long* d_words, const int32_t* d_word_prefix,
+   d_words: the launch's cleared words; d_tile_base: compact_tiles + 1 words; out (may be null): the
+   hit count and the clock */
+hipError_t compact_hits(unsigned long long* d_words, int64_t n_photon, const int64_t* n_dev, int32_t* d_word_prefix,
+                        int64_t* d_tile_base, const float4* d_photon, float4* d_hit, int64_t hit_cap, LaunchResult* out,
+                        hipStream_t s);
+hipError_t event_hit_offsets(const unsigned long long* d_bitmask, const int32_t* d_word_prefix,
                              const int64_t* d_block_total, const int64_t* d_ev_ph_begin, int32_t n_event,
                              int64_t n_words, int64_t* d_hit_offsets, hipStream_t s);
 hipError_t simtrace(const SimParams& P, float4* out, hipStream_t s);

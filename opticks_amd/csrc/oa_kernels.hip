@@ -109,7 +109,7 @@ __global__ void __launch_bounds__(1024) k_gs_prefix(const float* gs, int64_t n_g
  */
 template <bool SMALL>
 __global__ void __launch_bounds__(256) k_setup(const float* gs, int64_t n_gs, int64_t n_arg, int64_t cap, int64_t* prefix,
-                                               uint32_t* seed, unsigned long long* clear, int64_t n_clear, int64_t* ev,
+                                               uint32_t* seed, unsigned long long* words, int64_t bitmask, int64_t* ev,
                                                int32_t* ev_id, int32_t event_id, int64_t* n_dev, LaunchResult* out,
                                                int64_t n_wave)
 {
@@ -149,9 +149,11 @@ __global__ void __launch_bounds__(256) k_setup(const float* gs, int64_t n_gs, in
     int64_t n = n_arg < 0 ? total : n_arg;
     if (n > total || n > cap) n = 0;
     const int64_t stride = (int64_t)gridDim.x * 256, id = (int64_t)blockIdx.x * 256 + t;
-    /* the last cleared word is the photon counter: it starts behind the photons dealt first */
-    const int64_t width = wave_width(n, n_wave);
-    for (int64_t i = id; i < n_clear; i += stride) clear[i] = i == n_clear - 1 ? (unsigned long long)(n_wave * width) : 0ull;
+    /* the photon counter starts behind the photons dealt first; of the bitmask and the tiles, what
+       n photons use */
+    const int64_t width = wave_width(n, n_wave), n_words = (n + 63) / 64, n_tiles = (n_words + 255) / 256;
+    for (int64_t i = id; i < OA_WORDS_STATE + n_tiles; i += stride) words[i] = i == 0 ? (unsigned long long)(n_wave * width) : 0ull;
+    for (int64_t i = id; i < n_words; i += stride) words[bitmask + i] = 0ull;
     for (int64_t i = 4 * id; i < n; i += 4 * stride) {
         int64_t g = upper_index(pre, 0, n_gs, i);
         uint32_t v[4];
@@ -401,8 +403,9 @@ __global__ void __launch_bounds__(64) OA_OCC k_simtrace(SimParams P, float4* out
  * published counts (D. Merrill, M. Garland, "Single-pass parallel prefix scan with decoupled
  * look-back", NVR-2016-002) and copies its hit records. state[tile] is 0, then count | 1 << 62,
  * then (hits up to the tile's end) | 2 << 62, one word each, so no ordering with other memory
- * is needed; state[n_tiles_cap] hands out the tiles, so a tile's predecessors are always
- * running or done. Both start at zero.
+ * is needed; the ticket hands out the tiles, so a tile's predecessors are always running or
+ * done. Both start at zero. Where the count is the device's (n_dev), the blocks beyond its tiles
+ * leave without a ticket: they are as many as the largest event's tiles.
  * A tile lists its hit photons in LDS first, so that four neighbouring lanes copy one 64 B
  * record: with a lane per photon and a hit fraction of a tenth, most lanes of a wave only
  * watched the others copy. Bound by the bytes of the records (read and written once); it
@@ -412,8 +415,8 @@ __global__ void __launch_bounds__(64) OA_OCC k_simtrace(SimParams P, float4* out
  * the wall clock at the start and end.
  */
 __global__ void __launch_bounds__(256) k_compact(const unsigned long long* __restrict__ words, int64_t n_photon,
-                                                 const int64_t* n_dev, int64_t tiles_cap, int32_t* word_prefix,
-                                                 int64_t* tile_base, unsigned long long* state,
+                                                 const int64_t* n_dev, int32_t* word_prefix, int64_t* tile_base,
+                                                 unsigned long long* ticket, unsigned long long* state,
                                                  const float4* __restrict__ photon, float4* __restrict__ hit,
                                                  int64_t hit_cap, LaunchResult* out)
 {
@@ -423,10 +426,10 @@ __global__ void __launch_bounds__(256) k_compact(const unsigned long long* __res
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int64_t n = n_dev ? *n_dev : n_photon;
     const int64_t n_words = (n + 63) / 64, n_tiles = (n_words + 255) / 256;
-    if (t == 0) s_tile = (int64_t)atomicAdd(&state[tiles_cap], 1ull);
+    if ((int64_t)blockIdx.x >= n_tiles) return;
+    if (t == 0) s_tile = (int64_t)atomicAdd(ticket, 1ull);
     __syncthreads();
     const int64_t tile = s_tile;
-    if (tile >= n_tiles) return;
     if (out && tile == 0 && t == 0) out->clock[2] = wall_clock64();
     const int64_t w = tile * 256 + t;
     unsigned long long m = w < n_words ? words[w] : 0ull;
@@ -646,16 +649,16 @@ hipError_t gs_prefix(const float* d_gs, int64_t n_gs, int64_t* d_prefix, hipStre
 
 hipError_t setup(const SetupArgs& a, hipStream_t s)
 {
-    const int64_t work = std::max<int64_t>(a.cap / 8, a.n_clear);
+    const int64_t work = std::max<int64_t>(a.cap / 8, clear_words(a.cap));
     const unsigned nb = (unsigned)std::min<int64_t>(1024, (work + 255) / 256 + 1);
     if (a.n_gs <= OA_SETUP_GS) {
-        hipLaunchKernelGGL(k_setup<true>, dim3(nb), dim3(256), 0, s, a.gs, a.n_gs, a.n_arg, a.cap, a.prefix, a.seed, a.clear,
-                           a.n_clear, a.ev, a.ev_id, a.event_id, a.n_dev, a.out, a.n_wave);
+        hipLaunchKernelGGL(k_setup<true>, dim3(nb), dim3(256), 0, s, a.gs, a.n_gs, a.n_arg, a.cap, a.prefix, a.seed, a.words,
+                           bitmask_offset(a.cap), a.ev, a.ev_id, a.event_id, a.n_dev, a.out, a.n_wave);
     } else {
         const hipError_t e = gs_prefix(a.gs, a.n_gs, a.prefix, s);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_setup<false>, dim3(nb), dim3(256), 0, s, a.gs, a.n_gs, a.n_arg, a.cap, a.prefix, a.seed, a.clear,
-                           a.n_clear, a.ev, a.ev_id, a.event_id, a.n_dev, a.out, a.n_wave);
+        hipLaunchKernelGGL(k_setup<false>, dim3(nb), dim3(256), 0, s, a.gs, a.n_gs, a.n_arg, a.cap, a.prefix, a.seed, a.words,
+                           bitmask_offset(a.cap), a.ev, a.ev_id, a.event_id, a.n_dev, a.out, a.n_wave);
     }
     return hipGetLastError();
 }
@@ -693,14 +696,15 @@ hipError_t simulate(const SimParams& P, int kernel, int block, int grid, hipStre
     }
 }
 
-hipError_t compact_hits(const unsigned long long* d_words, int64_t n_photon, const int64_t* n_dev, int32_t* d_word_prefix,
-                        int64_t* d_tile_base, unsigned long long* d_state, const float4* d_photon, float4* d_hit,
-                        int64_t hit_cap, LaunchResult* out, hipStream_t s)
+hipError_t compact_hits(unsigned long long* d_words, int64_t n_photon, const int64_t* n_dev, int32_t* d_word_prefix,
+                        int64_t* d_tile_base, const float4* d_photon, float4* d_hit, int64_t hit_cap, LaunchResult* out,
+                        hipStream_t s)
 {
     const int64_t nt = compact_tiles(n_photon);
     if (nt > 0)
-        hipLaunchKernelGGL(k_compact, dim3((unsigned)nt), dim3(256), 0, s, d_words, n_photon, n_dev, nt, d_word_prefix,
-                           d_tile_base, d_state, d_photon, d_hit, hit_cap, out);
+        hipLaunchKernelGGL(k_compact, dim3((unsigned)nt), dim3(256), 0, s, d_words + bitmask_offset(n_photon), n_photon,
+                           n_dev, d_word_prefix, d_tile_base, d_words + OA_WORDS_TICKET, d_words + OA_WORDS_STATE, d_photon,
+                           d_hit, hit_cap, out);
     return hipGetLastError();
 }
 
@@ -737,10 +741,10 @@ hipError_t prefix_check(const int64_t* a, const int64_t* b, int64_t n, unsigned 
     return hipGetLastError();
 }
 
-__global__ void k_clear_launch(unsigned long long* p, int64_t n, unsigned long long last)
+__global__ void k_clear_launch(unsigned long long* p, int64_t n, unsigned long long next)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = i == n - 1 ? last : 0ull;
+    if (i < n) p[i] = i == 0 ? next : 0ull;
 }
 
 hipError_t clear_launch(unsigned long long* words, int64_t n_photon, int64_t n_wave, hipStream_t s)

@@ -42,7 +42,7 @@
 #define OA_NOALLOC_OFF_EVID    (OA_NOALLOC_OFF_EV + 256ll)                      /* 4 int64 event bounds */
 #define OA_NOALLOC_OFF_XW      (OA_NOALLOC_OFF_EVID + 256ll)                    /* 1 int32 event id */
 #define OA_NOALLOC_OFF_WORDS   (OA_NOALLOC_OFF_XW + OA_ALIGN256(4 * 800))       /* xorwow jump matrix */
-/* the hit words, then the compaction's tile states and ticket and the photon counter */
+/* the photon counter, the compaction's ticket and tile states, then the hit words */
 #define OA_NOALLOC_OFF_WPREFIX (OA_NOALLOC_OFF_WORDS + OA_ALIGN256(8 * (OA_NOALLOC_WORDS + OA_NOALLOC_BLOCKS + 2)))
 #define OA_NOALLOC_OFF_BTOTAL  (OA_NOALLOC_OFF_WPREFIX + OA_ALIGN256(4 * OA_NOALLOC_WORDS))
 #define OA_NOALLOC_SCRATCH_BYTES (OA_NOALLOC_OFF_BTOTAL + OA_ALIGN256(8 * OA_NOALLOC_BLOCKS))

@@ -135,7 +135,7 @@ hipError_t setup(const SetupArgs& a, hipStream_t)
     g_n = n;
     g_waves_dealt = (int)a.n_wave;
     holds(a.seed, 4 * (size_t)a.cap);
-    holds(a.clear, 8 * (size_t)clear_words(a.cap));
+    holds(a.words, 8 * (size_t)clear_words(a.cap));
     if (holds(a.n_dev, 16)) { a.n_dev[0] = n; a.n_dev[1] = 64; }
     a.out->total = total;
     a.out->n_photon = n;
@@ -161,10 +161,10 @@ hipError_t simulate(const SimParams& P, int, int, int grid, hipStream_t)
     return hipSuccess;
 }
 /* every second photon is a hit */
-hipError_t compact_hits(const unsigned long long*, int64_t cap, const int64_t* n_dev, int32_t* wp, int64_t* tb,
-                        unsigned long long*, const float4* photon, float4* hit, int64_t hit_cap, LaunchResult* out, hipStream_t)
+hipError_t compact_hits(unsigned long long* words, int64_t cap, const int64_t* n_dev, int32_t* wp, int64_t* tb, const float4* photon, float4* hit, int64_t hit_cap, LaunchResult* out, hipStream_t)
 {
     const int64_t n = n_dev ? *n_dev : cap, m = n / 2;
+    holds(words, 8 * (size_t)clear_words(cap));
     holds(wp, 4 * (size_t)((cap + 63) / 64));
     if (holds(tb, 8 * (size_t)(compact_tiles(cap) + 1))) tb[compact_tiles(n)] = m;
     for (int64_t i = 0; hit && i < m && i < hit_cap; ++i) std::memcpy(hit + 4 * i, photon + 4 * (2 * i + 1), 64);
