@@ -148,7 +148,7 @@ typedef struct mi_config {
     int32_t  block_size;       /* threads per block: 64 (default), 128 or 256 */
     int32_t  refill_period;    /* wavefront kernel: bounces between lane refills */
     int32_t  bvh_leaf_size;    /* instances per TLAS leaf (1..8)  */
-    int32_t  waves_per_cu;     /* wavefront kernel: resident waves per CU (0 = auto) */
+    int32_t  waves_per_cu;     /* wavefront kernel: resident waves per CU (0 = as many as fit, which is the most) */
     int32_t  trace_regroup_pct; /* trace: a wave's node walk hands over to the leaf phase once
                                    fewer than this percent of its walking lanes still walk
                                    (0 = once none do; 0..100; results do not depend on it) */

@@ -189,7 +189,7 @@ struct mi_sim {
     DBuf<unsigned long long> next;       /* photon counter of the adjoint replay */
     LaunchResult* result = nullptr;      /* pinned: the last launch's counts and clock */
     double clock_ms = 1e-5;              /* device wall clock tick */
-    int grid_key[3] = { -1, -1, -1 }, grid_blocks = 0;   /* wave_grid's last answer */
+    int shape_key[5] = { -1, -1, -1, -1, -1 }, resident_blocks = 0;   /* wave_shape's last answer */
     /* outputs of the host-array entry point */
     DBuf<float4> photon, hit;
     DBuf<uint64_t> seq;
@@ -836,24 +836,27 @@ static int sim_block(const mi_sim* sim)
     return b;
 }
 
-/* persistent grid: every resident slot of every CU (occupancy API), or the
-   configured waves per CU */
-static int wave_grid(mi_sim* sim)
+/* persistent grid: every resident slot of every CU, for the kernel that the launch runs (occupancy
+   API), or the configured waves per CU where those are fewer; a larger grid has waves that wait for
+   others to end with the photons they are dealt (3M photons, 2,000 detectors: 1.80 ms with 12 waves a
+   CU resident, 2.13 with 48 asked for; lite output of 20,000 detectors 1.96 with the 11 that fit,
+   2.03 with 12) */
+struct WaveShape { int block, grid; int64_t waves; };
+static WaveShape wave_shape(mi_sim* sim, bool lite, bool tape)
 {
-    const int block = sim_block(sim);
-    const int waves_per_block = block / 64;
-    if (sim->cfg.waves_per_cu > 0) return std::max(1, sim->n_cu * sim->cfg.waves_per_cu / waves_per_block);
-    const int key[3] = { block, sim->cfg.rng_kind, sim->stack_depth };
-    if (std::memcmp(key, sim->grid_key, sizeof(key)) != 0) {
-        int nb = oa_launch::wave_blocks_per_cu(block, sim->cfg.rng_kind, sim->stack_depth);
+    const int block = sim_block(sim), waves_per_block = block / 64;
+    const int key[5] = { block, sim->cfg.rng_kind, sim->stack_depth, lite, tape };
+    if (std::memcmp(key, sim->shape_key, sizeof(key)) != 0) {
+        int nb = oa_launch::wave_blocks_per_cu(block, sim->cfg.rng_kind, sim->stack_depth, lite, sim->ext_leaves, tape);
         if (nb <= 0) nb = std::max(1, 8 / waves_per_block);
-        sim->grid_blocks = std::max(1, sim->n_cu * nb);
-        std::memcpy(sim->grid_key, key, sizeof(key));
+        sim->resident_blocks = std::max(1, sim->n_cu * nb);
+        std::memcpy(sim->shape_key, key, sizeof(key));
     }
-    return sim->grid_blocks;
+    int grid = sim->resident_blocks;
+    if (sim->cfg.waves_per_cu > 0)
+        grid = (int)std::max<int64_t>(1, std::min<int64_t>(grid, (int64_t)sim->n_cu * sim->cfg.waves_per_cu / waves_per_block));
+    return { block, grid, (int64_t)grid * waves_per_block };
 }
-
-static int64_t wave_count(mi_sim* sim) { return (int64_t)wave_grid(sim) * (sim_block(sim) / 64); }
 
 /*
  * One propagation launch over gensteps already on the device with a
@@ -871,9 +874,10 @@ static int launch(mi_sim* sim, SimParams& P, hipStream_t s)
                                  sim->gs_event.p, s));
     P.seed_map = sim->seed.p;
     P.gs_event = sim->gs_event.p;
-    P.wave_width = (int32_t)wave_width(P.n_photon, wave_count(sim));
-    HIPCHECK(oa_launch::clear_launch(sim->words.p, P.n_photon, wave_count(sim), s));
-    HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s));
+    const WaveShape shape = wave_shape(sim, false, P.tape != nullptr);
+    P.wave_width = (int32_t)wave_width(P.n_photon, shape.waves);
+    HIPCHECK(oa_launch::clear_launch(sim->words.p, P.n_photon, shape.waves, s));
+    HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, shape.block, shape.grid, s));
     return MI_OK;
 }
 
@@ -976,6 +980,7 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
         const int rc = tape_reserve(sim, n_photon, K);
         if (rc) return rc;
     }
+    const WaveShape shape = wave_shape(sim, d_lite != nullptr, taping);
     int64_t hits = 0;
     double ms[4] = { 0.0, 0.0, 0.0, 0.0 };
     const volatile LaunchResult* res = sim->result;
@@ -990,7 +995,7 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
             const int64_t cap = n_arg >= 0 ? n_arg : photons_held(sim, K);
             const oa_launch::SetupArgs a = { (const float*)d_gensteps + 24 * g0, g1 - g0, n_arg, cap, sim->prefix.p,
                                              sim->seed.p, sim->words.p, sim->evbuf.p,
-                                             sim->ev_id.p, event_id, sim->n_dev.p, sim->result, wave_count(sim) };
+                                             sim->ev_id.p, event_id, sim->n_dev.p, sim->result, shape.waves };
             HIPCHECK(oa_launch::setup(a, s));
             SimParams P = base_params(sim);
             P.xw_jump = xw_table;
@@ -1017,7 +1022,7 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
                 P.tape_stride = sliced ? n_photon : 0;
                 P.tape_k = K;
             }
-            HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s));
+            HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, shape.block, shape.grid, s));
             HIPCHECK(oa_launch::compact_hits(sim->words.p, cap, sim->n_dev.p, sim->word_prefix.p, sim->tile_base.p,
                                              P.photon, d_hit ? (float4*)d_hit + 4 * hits : nullptr,
                                              d_hit ? std::max<int64_t>(0, hit_capacity - hits) : 0, sim->result, s));
@@ -1124,9 +1129,10 @@ int mi_sim_simulate_device_noalloc(mi_sim* sim, int32_t event_id, const void* d_
     P.photonlite = nullptr;
     P.hitwords = words + oa_launch::bitmask_offset(n_photon);
     P.next = words;
-    P.wave_width = (int32_t)wave_width(n_photon, wave_count(sim));
-    HIPCHECK(oa_launch::clear_launch(words, n_photon, wave_count(sim), s));
-    HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s));
+    const WaveShape shape = wave_shape(sim, false, false);
+    P.wave_width = (int32_t)wave_width(n_photon, shape.waves);
+    HIPCHECK(oa_launch::clear_launch(words, n_photon, shape.waves, s));
+    HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, shape.block, shape.grid, s));
     HIPCHECK(hipEventRecord(sim->ev[2], s));
     HIPCHECK(oa_launch::compact_hits(words, n_photon, nullptr, word_prefix, tile_base,
                                      (const float4*)d_photon, (float4*)d_hit, d_hit ? hit_capacity : 0, nullptr, s));
@@ -1702,9 +1708,10 @@ static hipError_t batch_work(mi_batch* b, SimParams P, const void* d_gensteps, c
        replay fails on the host, so its photons are never used */
     if ((e = oa_launch::seed_map(b->saved_prefix.p, b->n_gs, b->n_photon, b->seed.p, P.ev_gs_begin, b->n_event,
                                  b->gs_event.p, s)) != hipSuccess) return e;
-    P.wave_width = (int32_t)wave_width(b->n_photon, wave_count(sim));
-    if ((e = oa_launch::clear_launch(b->words.p, b->n_photon, wave_count(sim), s)) != hipSuccess) return e;
-    if ((e = oa_launch::simulate(P, sim->cfg.kernel, sim_block(sim), wave_grid(sim), s)) != hipSuccess) return e;
+    const WaveShape shape = wave_shape(sim, false, P.tape != nullptr);
+    P.wave_width = (int32_t)wave_width(b->n_photon, shape.waves);
+    if ((e = oa_launch::clear_launch(b->words.p, b->n_photon, shape.waves, s)) != hipSuccess) return e;
+    if ((e = oa_launch::simulate(P, sim->cfg.kernel, shape.block, shape.grid, s)) != hipSuccess) return e;
     if ((e = oa_launch::compact_hits(b->words.p, b->n_photon, nullptr, b->word_prefix.p, b->tile_base.p,
                                      (const float4*)d_photon, (float4*)d_hit, d_hit ? b->hit_capacity : 0, nullptr, s)) != hipSuccess)
         return e;

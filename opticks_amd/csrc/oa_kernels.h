@@ -32,7 +32,8 @@ inline int64_t compact_tiles(int64_t n_photon) { return ((n_photon + 63) / 64 + 
 inline int64_t bitmask_offset(int64_t n_photon) { return OA_WORDS_STATE + compact_tiles(n_photon); }
 inline int64_t clear_words(int64_t n_photon) { return bitmask_offset(n_photon) + (n_photon + 63) / 64; }
 hipError_t simulate(const SimParams& P, int kernel, int block, int grid, hipStream_t s);
-int wave_blocks_per_cu(int block, int rng_kind, int stack_depth);   /* resident blocks of the persistent kernel per CU */
+/* blocks of the persistent kernel that are resident on a CU, of the instantiation that a launch runs */
+int wave_blocks_per_cu(int block, int rng_kind, int stack_depth, bool lite, bool ext, bool tape);
 unsigned sim_lds(int block, int rng_kind, int stack_depth);   /* LDS bytes of a propagation block */
 hipError_t prefix_check(const int64_t* a, const int64_t* b, int64_t n, unsigned long long* flag, hipStream_t s);
 hipError_t zero_u64(unsigned long long* p, int64_t n, hipStream_t s);

@@ -668,15 +668,19 @@ hipError_t setup(const SetupArgs& a, hipStream_t s)
     (P.rng_kind == 1 ? fn##_##B##_1(__VA_ARGS__) : P.rng_kind == 2 ? fn##_##B##_2(__VA_ARGS__) \
                                                  : fn##_##B##_0(__VA_ARGS__))
 
-int wave_blocks_per_cu(int block, int rng_kind, int stack_depth)
+int wave_blocks_per_cu(int block, int rng_kind, int stack_depth, bool lite, bool ext, bool tape)
 {
-    const int k = rng_kind;
+#define OA_OCCUPANCY(B)                                                                   \
+    (rng_kind == 1 ? sim_occupancy_##B##_1(stack_depth, f, tape)                          \
+     : rng_kind == 2 ? sim_occupancy_##B##_2(stack_depth, f, tape) : sim_occupancy_##B##_0(stack_depth, f, tape))
+    const int f = (lite ? 1 : 0) | (ext ? 2 : 0);
     switch (block) {
-        case 64: return k == 1 ? sim_occupancy_64_1(stack_depth) : k == 2 ? sim_occupancy_64_2(stack_depth) : sim_occupancy_64_0(stack_depth);
-        case 128: return k == 1 ? sim_occupancy_128_1(stack_depth) : k == 2 ? sim_occupancy_128_2(stack_depth) : sim_occupancy_128_0(stack_depth);
-        case 256: return k == 1 ? sim_occupancy_256_1(stack_depth) : k == 2 ? sim_occupancy_256_2(stack_depth) : sim_occupancy_256_0(stack_depth);
+        case 64: return OA_OCCUPANCY(64);
+        case 128: return OA_OCCUPANCY(128);
+        case 256: return OA_OCCUPANCY(256);
         default: return 0;
     }
+#undef OA_OCCUPANCY
 }
 
 unsigned sim_lds(int block, int rng_kind, int stack_depth)

@@ -428,8 +428,10 @@ __global__ void __launch_bounds__(BLOCK) OA_OCC k_sim_wave(SimParams P)
         if (!exhausted && idle != 0ull && (idle == all || ((iter % period) == 0 && __popcll(idle) >= batch))) {
             const int n_idle = __popcll(idle);
             const int leader = __ffsll((long long)idle) - 1;
-            /* the first photons are dealt out by position, `width` to a wave (wave_width);
-               the counter starts behind them */
+            /* the first photons are dealt out by position, `width` to a wave (wave_width); the
+               counter starts behind them. The grid is no larger than what is resident: photons of
+               a wave that can start only when another has ended would begin a history at the
+               end of the event. */
             unsigned long long base = 0ull;
             int take = n_idle;
             if (iter == 0) {

@@ -22,6 +22,20 @@
 
 namespace oa_launch {
 
+/* the persistent kernel of a launch: features F (1: lite output, 2: extended leaves), and whether
+   it keeps segment records for a following adjoint (which has no lite output) */
+static void (*OA_SIM_NAME(wave_kernel, OA_SIM_BLOCK, OA_SIM_RNG)(int f, bool tape))(SimParams)
+{
+    constexpr int B = OA_SIM_BLOCK;
+    if (tape) return (f & 2) ? k_sim_wave<B, 2, OA_SIM_R, oa::RecordTape> : k_sim_wave<B, 0, OA_SIM_R, oa::RecordTape>;
+    switch (f) {
+        case 0: return k_sim_wave<B, 0, OA_SIM_R>;
+        case 1: return k_sim_wave<B, 1, OA_SIM_R>;
+        case 2: return k_sim_wave<B, 2, OA_SIM_R>;
+        default: return k_sim_wave<B, 3, OA_SIM_R>;
+    }
+}
+
 hipError_t OA_SIM_NAME(sim_launch, OA_SIM_BLOCK, OA_SIM_RNG)(const SimParams& P, int kernel, int grid, hipStream_t s)
 {
     constexpr int B = OA_SIM_BLOCK;
@@ -35,17 +49,8 @@ hipError_t OA_SIM_NAME(sim_launch, OA_SIM_BLOCK, OA_SIM_RNG)(const SimParams& P,
             case 2: hipLaunchKernelGGL((k_sim_plain<B, 2, OA_SIM_R>), dim3(nb), dim3(B), lds, s, P); break;
             default: hipLaunchKernelGGL((k_sim_plain<B, 3, OA_SIM_R>), dim3(nb), dim3(B), lds, s, P); break;
         }
-    } else if (P.tape) {
-        /* a forward for a following adjoint: segment records on the tape (no lite output) */
-        if (f & 2) hipLaunchKernelGGL((k_sim_wave<B, 2, OA_SIM_R, oa::RecordTape>), dim3((unsigned)grid), dim3(B), lds, s, P);
-        else hipLaunchKernelGGL((k_sim_wave<B, 0, OA_SIM_R, oa::RecordTape>), dim3((unsigned)grid), dim3(B), lds, s, P);
     } else {
-        switch (f) {
-            case 0: hipLaunchKernelGGL((k_sim_wave<B, 0, OA_SIM_R>), dim3((unsigned)grid), dim3(B), lds, s, P); break;
-            case 1: hipLaunchKernelGGL((k_sim_wave<B, 1, OA_SIM_R>), dim3((unsigned)grid), dim3(B), lds, s, P); break;
-            case 2: hipLaunchKernelGGL((k_sim_wave<B, 2, OA_SIM_R>), dim3((unsigned)grid), dim3(B), lds, s, P); break;
-            default: hipLaunchKernelGGL((k_sim_wave<B, 3, OA_SIM_R>), dim3((unsigned)grid), dim3(B), lds, s, P); break;
-        }
+        hipLaunchKernelGGL(OA_SIM_NAME(wave_kernel, OA_SIM_BLOCK, OA_SIM_RNG)(f, P.tape != nullptr), dim3((unsigned)grid), dim3(B), lds, s, P);
     }
     return hipGetLastError();
 }
@@ -55,11 +60,14 @@ unsigned OA_SIM_NAME(sim_lds, OA_SIM_BLOCK, OA_SIM_RNG)(int stack_depth)
     return oa::block_lds<OA_SIM_R>(OA_SIM_BLOCK, stack_depth, true);
 }
 
-int OA_SIM_NAME(sim_occupancy, OA_SIM_BLOCK, OA_SIM_RNG)(int stack_depth)
+/* LDS is given to blocks in units of 1,280 B, which the occupancy query does not count: blocks of
+   12,804 to 14,080 B fit a CU 11 times, where it answers 12 up to 13,653 B (measured) */
+int OA_SIM_NAME(sim_occupancy, OA_SIM_BLOCK, OA_SIM_RNG)(int stack_depth, int f, bool tape)
 {
+    const unsigned lds = oa::block_lds<OA_SIM_R>(OA_SIM_BLOCK, stack_depth, (f & 1) != 0);
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sim_wave<OA_SIM_BLOCK, 0, OA_SIM_R>, OA_SIM_BLOCK,
-                                                     oa::block_lds<OA_SIM_R>(OA_SIM_BLOCK, stack_depth)) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (const void*)OA_SIM_NAME(wave_kernel, OA_SIM_BLOCK, OA_SIM_RNG)(f, tape), OA_SIM_BLOCK,
+                                                     (lds + 1279u) / 1280u * 1280u) != hipSuccess)
         return 0;
     return nb;
 }

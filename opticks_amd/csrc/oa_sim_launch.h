@@ -12,7 +12,7 @@ struct AdjParams;
 #define OA_SIM_DECLARE(B, K)                                                                   \
     hipError_t sim_launch_##B##_##K(const SimParams& P, int kernel, int grid, hipStream_t s); \
     unsigned sim_lds_##B##_##K(int stack_depth);                                               \
-    int sim_occupancy_##B##_##K(int stack_depth);
+    int sim_occupancy_##B##_##K(int stack_depth, int f, bool tape);
 
 namespace oa_launch {
 OA_SIM_DECLARE(64, 0)

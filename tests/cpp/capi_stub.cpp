@@ -70,6 +70,7 @@ int stub_tape_stride() { return (int)g_stride; }
 int stub_waves_dealt() { return g_waves_dealt; }
 int stub_grid() { return g_grid; }
 int stub_resident() { return g_resident; }
+int stub_resident_lite() { return g_resident - 1; }
 
 hipError_t hipMalloc(void** p, size_t n) { return alloc(p, n); }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return alloc(p, n); }
@@ -171,7 +172,7 @@ hipError_t compact_hits(unsigned long long* words, int64_t cap, const int64_t* n
     if (out) out->n_hit = m;
     return hipSuccess;
 }
-int wave_blocks_per_cu(int, int, int) { return g_resident; }
+int wave_blocks_per_cu(int, int, int, bool lite, bool, bool) { return g_resident - (lite ? 1 : 0); }
 unsigned sim_lds(int, int, int) { return 1024; }
 hipError_t prefix_check(const int64_t*, const int64_t*, int64_t, unsigned long long*, hipStream_t) { return hipSuccess; }
 hipError_t zero_u64(unsigned long long*, int64_t, hipStream_t) { return hipSuccess; }

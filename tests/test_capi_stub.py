@@ -137,3 +137,21 @@ def test_tape_of_an_event_of_unknown_size_is_its_own(stub):
     assert run_device(stub, sim, gs) == (0, 750 + 500 + 350)
     assert stub.stub_tape_stride() == 3200
     sim.close()
+
+
+@pytest.mark.parametrize("waves_per_cu", [0, 3, 8, 64])
+def test_first_photons_are_dealt_to_resident_waves(stub, waves_per_cu):
+    """Photons dealt out by position go to waves that start at once: the grid has no more waves
+    than fit the GPU (2 CUs of stub_resident() one-wave blocks, one fewer with lite output)."""
+    sim = sim_of(waves_per_cu=waves_per_cu)
+    gs = event(1000)
+    lite = np.zeros((1000, 4), np.uint32)
+    m = L.C.c_int64(0)
+    for is_lite, fit in ((False, stub.stub_resident()), (True, stub.stub_resident_lite())):
+        if is_lite:
+            assert stub.mi_sim_simulate_lite_device(sim.handle, 0, gs.ctypes.data, 1, -1, 0, lite.ctypes.data, None, None,
+                                                    None, 0, L.C.byref(m), None) == 0
+        else:
+            assert run_device(stub, sim, gs) == (0, 500)
+        assert stub.stub_grid() == stub.stub_waves_dealt() == 2 * min(waves_per_cu or fit, fit)
+    sim.close()

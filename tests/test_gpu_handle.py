@@ -108,3 +108,40 @@ def test_small_events_after_a_large_one():
         assert np.array_equal(got[0], photon.view(np.uint32)) and np.array_equal(got[2], want.view(np.uint32))
         assert np.array_equal(got[1].view(np.uint64).reshape(seq.shape), seq)
     sim.close()
+
+
+# events smaller and larger than the resident waves hold, on grids of fewer and of more waves
+@pytest.mark.parametrize("n", [1, 65, 9001, 200_003, 600_001])
+@pytest.mark.parametrize("waves_per_cu", [1, 13, 48])
+def test_grids_beyond_residency_keep_results(n, waves_per_cu):
+    w = configs.config1(num_gs=1, per_gs=n)
+    photon, seq = po.World(w.geometry, w.physics).simulate(w.gensteps, event_idx=2, seed=7)
+    ev = Device(w.gensteps)
+    for kw in (dict(), dict(block_size=256), dict(adjoint_tape=8)):
+        sim = QSim(w.geometry, w.physics, SEventConfig(seed=7, waves_per_cu=waves_per_cu, **kw))
+        got = ev.run(sim, eventID=2)
+        assert np.array_equal(got[0], photon.view(np.uint32))
+        assert np.array_equal(got[1].view(np.uint64).reshape(seq.shape), seq)
+        sim.close()
+
+
+@pytest.mark.parametrize("num_det, n", [(2000, 30_000), (20_000, 30_000), (20_000, 900_000)])
+def test_lite_output_of_deep_detectors(num_det, n):
+    """Lite records of detectors whose traversal stack leaves a CU fewer blocks with lite output
+    than without: time and flags of the photon records, the checker's among them."""
+    w = configs.detector_shell(num_det=num_det, num_gs=6, per_gs=n // 6)
+    ev = Device(w.gensteps)
+    sim = QSim(w.geometry, w.physics, SEventConfig(seed=w.seed))
+    photon = ev.run(sim)[0]
+    lite = torch.zeros((ev.n, 4), dtype=torch.int32, device=DEV)
+    seq = torch.zeros_like(ev.seq)
+    sim.simulate_lite_device(ev.gs, lite, None, seq, None)
+    got = lite.cpu().numpy().view(np.uint32)
+    assert np.array_equal(got[:, 1], photon[:, 0, 3]) and np.array_equal(got[:, 3], photon[:, 3, 3])
+    assert np.array_equal(got[:, 0] & 0xffff, photon[:, 3, 1] & 0xffff)
+    assert torch.equal(seq, ev.seq)
+    few = w.gensteps[:1].copy()
+    few.view(np.uint32)[:, 0, 3] = min(5000, n // 6)
+    ref, _ = po.World(w.geometry, w.physics).simulate(few, seed=w.seed)
+    assert np.array_equal(photon[:len(ref)], ref.view(np.uint32))
+    sim.close()
