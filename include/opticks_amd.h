@@ -199,7 +199,8 @@ int  mi_sim_reset(mi_sim* sim, int32_t event_id);
  * propagates and reports the counts (its array pointers stay NULL), mi_sim_fetch copies
  * that run's photon (n_photon,4,4), seq (n_photon,2,2) and hit (n_hit,4,4) arrays into the
  * caller's host memory (NULL: not wanted) until the handle's next host call or reset.
- * mi_host_alloc gives pinned memory, into which the copies run at the link's full rate.
+ * Ordinary memory is filled by way of a pinned ring of the handle (16 MB, with up to five threads
+ * for the length of the call); into pinned memory (mi_host_alloc) the GPU copies directly.
  */
 int  mi_sim_run(mi_sim* sim, int32_t event_id, const float* gensteps, int64_t n_gs, mi_event_out* out);
 int  mi_sim_fetch(mi_sim* sim, float* photon, uint64_t* seq, float* hit);

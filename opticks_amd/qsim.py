@@ -139,11 +139,14 @@ def _ptr(a):
 
 
 class _HostBuffer:
-    """Pinned host memory behind result arrays; goes back to its pool, or is freed, when the
-    last array over it is gone."""
+    """Memory behind a result array; goes back to its pool when the last array over it is gone."""
 
-    def __init__(self, pool, ptr, size):
-        self.pool, self.ptr, self.size = pool, ptr, size
+    def __init__(self, pool, memory):
+        self.pool, self.memory = pool, memory
+
+    @property
+    def ptr(self):
+        return self.memory.ctypes.data
 
     def array(self, dtype, shape):
         a = np.frombuffer(_view(self), dtype=dtype, count=int(np.prod(shape)))
@@ -151,22 +154,22 @@ class _HostBuffer:
 
     def __del__(self):
         try:
-            if not self.pool.put(self.ptr, self.size):
-                L.lib().mi_host_free(self.ptr)
+            self.pool.put(self.memory)
         except Exception:               # the interpreter is ending
             pass
 
 
 def _view(buffer):
     """a writable ctypes view of the buffer that keeps it alive"""
-    v = (C.c_char * buffer.size).from_address(buffer.ptr)
+    v = (C.c_char * buffer.memory.nbytes).from_address(buffer.ptr)
     v.buffer = buffer
     return v
 
 
 class _HostPool:
-    """Pinned memory of dropped result arrays, kept for the next event's: at most `most`
-    buffers, given back on close. Arrays may be dropped by any thread."""
+    """Memory of dropped result arrays, kept for the next event's: at most `most` buffers, given
+    back on close. It is ordinary memory, whose pages are there already the second time (new pages
+    take the host longer than the copy from the GPU). Arrays may be dropped by any thread."""
 
     most = 6
 
@@ -177,28 +180,21 @@ class _HostPool:
 
     def take(self, size):
         with self._lock:
-            fit = [b for b in self._spare if size <= b[1] <= 2 * size + (1 << 20)]
+            fit = [m for m in self._spare if size <= m.nbytes <= 2 * size + (1 << 20)]
             if fit:
-                b = min(fit, key=lambda b: b[1])
-                self._spare.remove(b)
-                return _HostBuffer(self, *b)
-        p = C.c_void_p()
-        L.check(L.lib().mi_host_alloc(size, C.byref(p)), "mi_host_alloc")
-        return _HostBuffer(self, p.value, size)
+                k = min(range(len(self._spare)), key=lambda k: (self._spare[k].nbytes < size, self._spare[k].nbytes))
+                return _HostBuffer(self, self._spare.pop(k))
+        return _HostBuffer(self, np.empty(size, np.uint8))
 
-    def put(self, ptr, size):
+    def put(self, memory):
         with self._lock:
-            if not self._open or len(self._spare) >= self.most:
-                return False
-            self._spare.append((ptr, size))
-            return True
+            if self._open and len(self._spare) < self.most:
+                self._spare.append(memory)
 
     def close(self, final=True):
         with self._lock:
-            spare, self._spare = self._spare, []
+            self._spare = []
             self._open = self._open and not final
-        for ptr, _ in spare:
-            L.lib().mi_host_free(ptr)
 
 
 class QSim:
@@ -279,7 +275,7 @@ class QSim:
         om = self.get_config_c().output_mask
         if not self.config.output_mask & L.MI_OUT_HIT:
             om &= ~L.MI_OUT_HIT
-        # arrays of their own for every event, over pinned memory that the copies fill directly
+        # arrays of their own for every event
         new = {b: self._host.take(max(64, size)) if om & b else None
                for b, size in ((L.MI_OUT_PHOTON, 64 * n), (L.MI_OUT_SEQ, 32 * n), (L.MI_OUT_HIT, 64 * m))}
         photon, seq, hit = (new[b] for b in (L.MI_OUT_PHOTON, L.MI_OUT_SEQ, L.MI_OUT_HIT))

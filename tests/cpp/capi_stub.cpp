@@ -66,6 +66,13 @@ void stub_fail_trace(int f) { g_fail_trace = f; }
 size_t stub_largest() { return g_largest; }
 int stub_bad() { return g_bad; }
 int stub_overlap() { return g_overlap; }
+/* whether the HIP runtime knows the address: device or pinned memory */
+int stub_known(const void* p)
+{
+    std::lock_guard<std::mutex> l(g_m);
+    auto it = g_alloc.upper_bound((const char*)p);
+    return it != g_alloc.begin() && (--it, (const char*)p < it->first + it->second);
+}
 int stub_tape_stride() { return (int)g_stride; }
 int stub_waves_dealt() { return g_waves_dealt; }
 int stub_grid() { return g_grid; }
@@ -86,9 +93,7 @@ hipError_t hipGetLastError() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "stub"; }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
 {
-    std::lock_guard<std::mutex> l(g_m);
-    auto it = g_alloc.upper_bound((const char*)p);
-    const bool known = it != g_alloc.begin() && (--it, (const char*)p < it->first + it->second);
+    const bool known = stub_known(p);
     std::memset(a, 0, sizeof(*a));
     a->type = known ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
     return known ? hipSuccess : hipErrorInvalidValue;

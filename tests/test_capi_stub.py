@@ -155,3 +155,44 @@ def test_first_photons_are_dealt_to_resident_waves(stub, waves_per_cu):
             assert run_device(stub, sim, gs) == (0, 500)
         assert stub.stub_grid() == stub.stub_waves_dealt() == 2 * min(waves_per_cu or fit, fit)
     sim.close()
+
+
+@pytest.mark.parametrize("n", [1, 4096, 30_011, 120_000])
+def test_results_are_ordinary_memory(stub, n):
+    """Results that outlive a call are not in memory of the HIP runtime, whose mappings a forked
+    child does not have and which cannot be freed during a graph capture; copied in pieces of all
+    sizes, also where the pieces' pinned memory cannot be had."""
+    stub.stub_known.argtypes = [L.C.c_void_p]
+    sim = sim_of()
+    gs = event(n)
+    for limited in (False, True):
+        hit = sim.simulate(gs)
+        for a in (sim.photon, sim.seq) + ((hit,) if len(hit) else ()):
+            assert not stub.stub_known(a.ctypes.data)
+        assert np.array_equal(sim.photon[:, 0, 0], np.arange(n)) and np.array_equal(sim.seq[:, 0, 0], np.arange(n))
+        assert np.array_equal(hit[:, 0, 0], 2 * np.arange(n // 2) + 1)
+        out = L.MiEventOut()
+        assert stub.mi_sim_simulate(sim.handle, 0, gs.ctypes.data, len(gs), L.C.byref(out)) == 0
+        assert not any(stub.stub_known(p) for p in (out.photon, out.seq, out.hit))
+        got = np.ctypeslib.as_array((L.C.c_float * (16 * n)).from_address(out.photon)).reshape(n, 4, 4)
+        assert np.array_equal(got, sim.photon)
+        sim.close()
+        sim = sim_of()
+        stub.stub_limit(max(64 * n, 3 << 20))                  # too little for the ring, but for the last n
+    sim.close()
+
+
+def test_fetch_into_pinned_and_ordinary_memory(stub):
+    n = 50_000
+    sim = sim_of()
+    gs = event(n)
+    out = L.MiEventOut()
+    assert stub.mi_sim_run(sim.handle, 0, gs.ctypes.data, len(gs), L.C.byref(out)) == 0
+    p = L.C.c_void_p()
+    assert stub.mi_host_alloc(64 * n, L.C.byref(p)) == 0 and stub.stub_known(p)
+    seq = np.zeros((n, 2, 2), np.uint64)
+    assert stub.mi_sim_fetch(sim.handle, p, seq.ctypes.data, None) == 0
+    got = np.ctypeslib.as_array((L.C.c_float * (16 * n)).from_address(p.value)).reshape(n, 4, 4)
+    assert np.array_equal(got[:, 0, 0], np.arange(n)) and np.array_equal(seq[:, 0, 0], np.arange(n))
+    stub.mi_host_free(p)
+    sim.close()

@@ -145,3 +145,51 @@ def test_lite_output_of_deep_detectors(num_det, n):
     ref, _ = po.World(w.geometry, w.physics).simulate(few, seed=w.seed)
     assert np.array_equal(photon[:len(ref)], ref.view(np.uint32))
     sim.close()
+
+
+def mapping_flags(address):
+    """VmFlags of the mapping that holds the address"""
+    inside = False
+    for line in open("/proc/self/smaps"):
+        head = line.split()[0]
+        if "-" in head and not head.endswith(":"):
+            lo, hi = (int(x, 16) for x in head.split("-"))
+            inside = lo <= address < hi
+        elif inside and line.startswith("VmFlags:"):
+            return line.split()[1:]
+    raise AssertionError("no such mapping")
+
+
+@pytest.mark.parametrize("n", [1000, 300_000])
+def test_results_are_ordinary_memory(n):
+    """Result arrays can be used like any other: a forked child has them (its mappings are not
+    those of the GPU's driver), and dropping them during a graph capture leaves it valid."""
+    w = configs.config0(num_photon=n)
+    photon, seq = po.World(w.geometry, w.physics).simulate(w.gensteps, seed=w.seed)
+    sim = QSim(w.geometry, w.physics, SEventConfig(seed=w.seed))
+    kept = []
+    for _ in range(3):
+        sim.simulate(w.gensteps)
+        kept.append((sim.photon, sim.seq, sim.hit))
+    for arrays in kept:
+        assert np.array_equal(arrays[0].view(np.uint32), photon.view(np.uint32)) and np.array_equal(arrays[1], seq)
+        for a in arrays:
+            assert a.flags.writeable and not {"dc", "io", "pf"} & set(mapping_flags(a.ctypes.data))
+    frame = configs.frame_gensteps((0, 0, 0, 500.0), (0, 0, 0, 0, 0, 0, n, 1), gridscale=0.1)
+    rays = po.World(w.geometry, w.physics).simtrace(frame, seed=w.seed)
+    assert np.array_equal(sim.simtrace(frame).view(np.uint32), rays.view(np.uint32))
+    x = torch.zeros(1024, device=DEV)
+    sim.photon = sim.seq = sim.hit = None
+    del arrays, a
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        y = x + 1
+        kept.clear()                                           # nine arrays, more than a handle keeps
+        gc.collect()
+        z = y + 1
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert z[0].item() == 2.0
+    sim.close()
