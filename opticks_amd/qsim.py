@@ -167,29 +167,46 @@ def _view(buffer):
 
 
 class _HostPool:
-    """Memory of dropped result arrays, kept for the next event's: at most `most` buffers, given
-    back on close. It is ordinary memory, whose pages are there already the second time (new pages
-    take the host longer than the copy from the GPU). Arrays may be dropped by any thread."""
+    """Memory of dropped result arrays, kept for the next events': the `most` buffers dropped last,
+    of `most_bytes` together and each for `age` arrays handed out, given back on close. It is ordinary
+    memory, whose pages are there already the second time (new pages take the host longer than the
+    copy from the GPU). Arrays may be dropped by any thread."""
 
     most = 6
+    most_bytes = 1 << 30
+    age = 32
 
     def __init__(self):
         self._lock = threading.RLock()       # a drop may run inside take() (garbage collection)
-        self._spare = []
+        self._spare = []                     # (arrays handed out when it was dropped, memory), oldest first
+        self._taken = 0
         self._open = True
 
     def take(self, size):
         with self._lock:
-            fit = [m for m in self._spare if size <= m.nbytes <= 2 * size + (1 << 20)]
+            self._taken += 1
+            fit = [k for k, (_, m) in enumerate(self._spare) if size <= m.nbytes <= 2 * size + (1 << 20)]
             if fit:
-                k = min(range(len(self._spare)), key=lambda k: (self._spare[k].nbytes < size, self._spare[k].nbytes))
-                return _HostBuffer(self, self._spare.pop(k))
-        return _HostBuffer(self, np.empty(size, np.uint8))
+                return _HostBuffer(self, self._spare.pop(min(fit, key=lambda k: self._spare[k][1].nbytes))[1])
+        try:
+            memory = np.empty(size, np.uint8)
+        except MemoryError:
+            self.close(final=False)
+            memory = np.empty(size, np.uint8)
+        return _HostBuffer(self, memory)
 
     def put(self, memory):
-        with self._lock:
-            if self._open and len(self._spare) < self.most:
-                self._spare.append(memory)
+        # a drop does not wait: a forked child may have been made while a thread held the lock
+        if not self._lock.acquire(blocking=False):
+            return
+        try:
+            if self._open:
+                self._spare.append((self._taken, memory))
+            while self._spare and (len(self._spare) > self.most or self._taken - self._spare[0][0] > self.age
+                                   or sum(m.nbytes for _, m in self._spare) > self.most_bytes):
+                self._spare.pop(0)
+        finally:
+            self._lock.release()
 
     def close(self, final=True):
         with self._lock:

@@ -196,3 +196,42 @@ def test_fetch_into_pinned_and_ordinary_memory(stub):
     assert np.array_equal(got[:, 0, 0], np.arange(n)) and np.array_equal(seq[:, 0, 0], np.arange(n))
     stub.mi_host_free(p)
     sim.close()
+
+
+def test_spare_memory_follows_the_events(stub, monkeypatch):
+    """Memory kept for later events is bounded in buffers and bytes, and after large events many
+    small ones find theirs in it; where memory is short it is given up for the arrays asked for."""
+    sim = sim_of()
+    pool = sim._host
+    kept = []
+    for _ in range(4):
+        sim.simulate(event(100_000))
+        kept.append((sim.photon, sim.seq, sim.hit))
+    kept.clear()
+    sim.simulate(event(100_000))
+    assert 0 < len(pool._spare) <= pool.most
+    for _ in range(20):
+        sim.simulate(event(1000))
+    sizes = lambda: [m.nbytes for _, m in pool._spare]
+    assert 0 < len(pool._spare) <= pool.most and max(sizes()) <= 64 * 1000
+    before = {m.ctypes.data for _, m in pool._spare}
+    sim.simulate(event(1000))
+    assert {a.ctypes.data for a in (sim.photon, sim.seq, sim.hit)} <= before
+    sim.simulate(event(100_000))
+    monkeypatch.setattr(type(pool), "most_bytes", 64 * 100_000 - 1)
+    sim.simulate(event(1000))
+    assert sum(sizes()) < 64 * 100_000
+    empty, failures = np.empty, []
+
+    def short_of_memory(size, dtype):
+        if pool._spare:
+            failures.append(size)
+            raise MemoryError
+        return empty(size, dtype)
+
+    monkeypatch.setattr("opticks_amd.qsim.np.empty", short_of_memory)
+    assert len(sim.simulate(event(400_000))) == 200_000 and failures
+    monkeypatch.undo()
+    sim.photon = sim.seq = sim.hit = None
+    stub.mi_sim_destroy(sim.handle)
+    sim.handle = None
