@@ -1539,6 +1539,7 @@ int mi_sim_simtrace(mi_sim* sim, const float* gensteps, int64_t n_gs, const floa
     if (n == 0) return fail(MI_NOTHING_TO_DO, "gensteps carry no photons");
     hipStream_t s = sim->stream;
     HIPCHECK(upload(sim->gs, gensteps, (size_t)n_gs * 24, s));
+    sim->run_mask = 0;                              /* the photon buffer is for the records now */
     HIPCHECK(sim->photon.reserve((size_t)n * 4));
     HIPCHECK(hipEventRecord(sim->ev[0], s));
     int rc = mi_sim_simtrace_device(sim, sim->gs.p, n_gs, n, sim->photon.p, s);
@@ -1547,7 +1548,6 @@ int mi_sim_simtrace(mi_sim* sim, const float* gensteps, int64_t n_gs, const floa
     HIPCHECK(hipEventSynchronize(sim->ev[3]));
     float ms = 0.f;
     HIPCHECK(hipEventElapsedTime(&ms, sim->ev[0], sim->ev[3]));
-    sim->run_mask = 0;                              /* the photon buffer holds the records now */
     HIPCHECK(sim->h_simtrace.reserve(64 * (size_t)n));
     rc = fetch(sim, { { sim->h_simtrace.p, sim->photon.p, 64 * (size_t)n } }, s);
     if (rc) return rc;

@@ -235,3 +235,25 @@ def test_spare_memory_follows_the_events(stub, monkeypatch):
     sim.photon = sim.seq = sim.hit = None
     stub.mi_sim_destroy(sim.handle)
     sim.handle = None
+
+
+def test_fetch_after_a_failed_simtrace(stub):
+    """A simtrace that fails has used the photon buffer of the run before it: that run's outputs
+    cannot be fetched any more, as after one that succeeds."""
+    sim = sim_of()
+    gs = event(1000)
+    out = L.MiEventOut()
+    photon = np.zeros((1000, 4, 4), np.float32)
+    frame = configs.frame_gensteps((0, 0, 0, 100.0), (0, 0, 0, 0, 0, 0, 1000, 1))
+    for fails in (True, False):
+        assert stub.mi_sim_run(sim.handle, 0, gs.ctypes.data, 1, L.C.byref(out)) == 0
+        assert stub.mi_sim_fetch(sim.handle, photon.ctypes.data, None, None) == 0
+        stub.stub_fail_trace(int(fails))
+        if fails:
+            with pytest.raises(RuntimeError):
+                sim.simtrace(frame)
+        else:
+            assert len(sim.simtrace(frame)) == 1000
+        assert stub.mi_sim_fetch(sim.handle, photon.ctypes.data, None, None) == -1
+        assert "no such output" in L.last_error()
+    sim.close()
