@@ -236,8 +236,7 @@ int  mi_sim_simulate_device(mi_sim* sim, int32_t event_id,
  * device or host allocation on its success path. Limits: at most
  * MI_NOALLOC_MAX_GENSTEPS gensteps and MI_NOALLOC_MAX_PHOTONS photons per call
  * (MI_ERR_CAPACITY beyond); no max_slot slicing. All handles and calls on one
- * GPU share that scratch: calls that overlap on one GPU (other threads or
- * streams) race and must be serialized by the caller.
+ * GPU share that scratch: calls from several threads of a process take turns.
  */
 #define MI_NOALLOC_MAX_GENSTEPS (1ll << 20)
 #define MI_NOALLOC_MAX_PHOTONS  (1ll << 26)

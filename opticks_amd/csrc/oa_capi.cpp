@@ -23,6 +23,7 @@
 #include <initializer_list>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <thread>
 #include <utility>
 
@@ -1211,7 +1212,15 @@ int mi_sim_simulate_device(mi_sim* sim, int32_t event_id, const void* d_gensteps
  * allocation. Differences from mi_sim_simulate_device: no max_slot slicing,
  * photons find their genstep by binary search of the prefix (same results),
  * limits of OA_NOALLOC_MAX_GS gensteps and OA_NOALLOC_MAX_PHOTON photons.
+ * Calls on one GPU take turns: where one clears the scratch under another, whose
+ * compaction waits for counts of its own, that wait would not end.
  */
+static std::mutex& noalloc_turn(int device)
+{
+    static std::mutex m[64];
+    return m[device & 63];
+}
+
 int mi_sim_simulate_device_noalloc(mi_sim* sim, int32_t event_id, const void* d_gensteps, int64_t n_gs,
                                    int64_t n_photon, int64_t photon_offset, void* d_photon, void* d_seq, void* d_hit,
                                    int64_t hit_capacity, int64_t* n_hit_out, void* stream)
@@ -1225,6 +1234,7 @@ int mi_sim_simulate_device_noalloc(mi_sim* sim, int32_t event_id, const void* d_
     if (n_photon > OA_NOALLOC_MAX_PHOTON) return fail(MI_ERR_CAPACITY, "no-allocation simulate: more than 2^26 photons");
     if (!sim->scratch) return fail(MI_ERR_HIP, "no-allocation simulate: no scratch address");
     hipStream_t s = stream ? (hipStream_t)stream : sim->stream;
+    std::lock_guard<std::mutex> turn(noalloc_turn(sim->device));
     char* base = (char*)sim->scratch;
     int64_t* prefix = (int64_t*)(base + OA_NOALLOC_OFF_PREFIX);
     int64_t* ev = (int64_t*)(base + OA_NOALLOC_OFF_EV);

@@ -257,3 +257,27 @@ def test_fetch_after_a_failed_simtrace(stub):
         assert stub.mi_sim_fetch(sim.handle, photon.ctypes.data, None, None) == -1
         assert "no such output" in L.last_error()
     sim.close()
+
+
+def test_calls_sharing_the_noalloc_scratch_take_turns(stub):
+    """All no-allocation calls on a GPU share its scratch, in which the compaction of one waits for
+    counts that the clearing of another would take away: they run one after the other."""
+    import threading
+    gs = event(1000)
+    rcs = []
+
+    def calls():
+        sim = sim_of()
+        m = L.C.c_int64(0)
+        for _ in range(3):
+            rcs.append(stub.mi_sim_simulate_device_noalloc(sim.handle, 0, gs.ctypes.data, 1, -1, 0, None, None, None, 0,
+                                                           L.C.byref(m), None))
+            assert m.value == 500
+        sim.close()
+
+    threads = [threading.Thread(target=calls) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert rcs == [0] * 12 and stub.stub_overlap() == 0
