@@ -329,7 +329,7 @@ struct mi_sim {
     DBuf<uint32_t> seed;                 /* genstep of each photon of the launch */
     DBuf<unsigned long long> words;      /* oa_launch::clear_words of the launch */
     DBuf<unsigned long long> next;       /* photon counter of the adjoint replay */
-    LaunchResult* result = nullptr;      /* pinned: the last launch's counts and clock */
+    PinnedBuf result;                    /* LaunchResult: the last launch's counts and clock */
     double clock_ms = 1e-5;              /* device wall clock tick */
     int shape_key[5] = { -1, -1, -1, -1, -1 }, resident_blocks = 0;   /* wave_shape's last answer */
     /* outputs of the host-array entry point */
@@ -855,8 +855,7 @@ int mi_sim_create(const mi_geometry* geo, const mi_physics* phys, const mi_confi
         if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, sim->device) == hipSuccess && khz > 0)
             sim->clock_ms = 1.0 / khz;
         rc = sim->next.reserve(1) == hipSuccess && sim->n_dev.reserve(2) == hipSuccess &&
-                     hipHostMalloc((void**)&sim->result, sizeof(LaunchResult), hipHostMallocDefault) == hipSuccess
-                 ? MI_OK : fail(MI_ERR_HIP, "alloc counters");
+                     sim->result.reserve(oa_launch::result_bytes((int64_t)1 << 24)) == hipSuccess ? MI_OK : fail(MI_ERR_HIP, "alloc counters");
     }
     if (!rc) {
         hipError_t e = oa_launch::noalloc_scratch(sim->device, &sim->scratch);
@@ -878,7 +877,7 @@ void mi_sim_destroy(mi_sim* sim)
     sim->inst_box.release(); sim->free_ball.release();
     sim->bnd.release(); sim->optical.release(); sim->icdf.release(); sim->precooked.release();
     sim->gs.release(); sim->prefix.release(); sim->tile_base.release(); sim->evbuf.release(); sim->n_dev.release();
-    if (sim->result) (void)hipHostFree(sim->result);
+    sim->result.release();
     sim->word_prefix.release(); sim->ev_id.release(); sim->words.release(); sim->next.release();
     sim->seed.release(); sim->gs_event.release();
     sim->photon.release(); sim->hit.release(); sim->seq.release();
@@ -1032,6 +1031,7 @@ static int launch_reserve(mi_sim* sim, int64_t n)
     HIPCHECK(sim->seed.reserve((size_t)n));
     HIPCHECK(sim->word_prefix.reserve((size_t)((n + 63) / 64) + 1));
     HIPCHECK(sim->tile_base.reserve((size_t)oa_launch::compact_tiles(n) + 1));
+    HIPCHECK(sim->result.reserve(oa_launch::result_bytes(n)));
     return MI_OK;
 }
 
@@ -1049,9 +1049,9 @@ static int tape_reserve(mi_sim* sim, int64_t n, int32_t K)
 static int64_t photons_held(const mi_sim* sim, int32_t K)
 {
     const int64_t words = (int64_t)sim->words.n, seeds = (int64_t)sim->seed.n, prefixes = (int64_t)sim->word_prefix.n,
-                  tiles = (int64_t)sim->tile_base.n;
+                  tiles = (int64_t)sim->tile_base.n - 1, ends = ((int64_t)sim->result.bytes - (int64_t)oa_launch::result_bytes(0)) / 8;
     /* w bitmask words take w + ceil(w / 256) + 2 cleared ones */
-    const int64_t w = std::min({ 256 * std::max<int64_t>(words - 2, 0) / 257, prefixes - 1, 256 * (tiles - 1) });
+    const int64_t w = std::min({ 256 * std::max<int64_t>(words - 2, 0) / 257, prefixes - 1, 256 * tiles, 256 * ends });
     int64_t n = std::max<int64_t>(0, std::min(64 * w, seeds));
     if (K > 0) n = std::min(n, std::min((int64_t)(sim->tape.n / (3 * (size_t)K)), (int64_t)sim->tape_n.n));
     return n;
@@ -1127,7 +1127,8 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
     const WaveShape shape = wave_shape(sim, d_lite != nullptr, taping);
     int64_t hits = 0;
     double ms[4] = { 0.0, 0.0, 0.0, 0.0 };
-    const volatile LaunchResult* res = sim->result;
+    const volatile LaunchResult* res = nullptr;
+    int n_setup = 0;
     for (auto& sl : slices) {
         const int64_t g0 = sl.first, g1 = sl.second;
         const int64_t p0 = sliced ? hprefix[g0] : 0;
@@ -1137,9 +1138,12 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
             int rc = n_arg >= 0 ? launch_reserve(sim, n_arg) : MI_OK;
             if (rc) return rc;
             const int64_t cap = n_arg >= 0 ? n_arg : photons_held(sim, K);
+            LaunchResult* const out = (LaunchResult*)sim->result.p;
+            res = out;
+            n_setup = oa_launch::setup_blocks(cap);
             const oa_launch::SetupArgs a = { (const float*)d_gensteps + 24 * g0, g1 - g0, n_arg, cap, sim->prefix.p,
                                              sim->seed.p, sim->words.p, sim->evbuf.p,
-                                             sim->ev_id.p, event_id, sim->n_dev.p, sim->result, shape.waves };
+                                             sim->ev_id.p, event_id, sim->n_dev.p, out, shape.waves };
             HIPCHECK(oa_launch::setup(a, s));
             SimParams P = base_params(sim);
             P.xw_jump = xw_table;
@@ -1169,12 +1173,13 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
             HIPCHECK(oa_launch::simulate(P, sim->cfg.kernel, shape.block, shape.grid, s));
             HIPCHECK(oa_launch::compact_hits(sim->words.p, cap, sim->n_dev.p, sim->word_prefix.p, sim->tile_base.p,
                                              P.photon, d_hit ? (float4*)d_hit + 4 * hits : nullptr,
-                                             d_hit ? std::max<int64_t>(0, hit_capacity - hits) : 0, sim->result, s));
+                                             d_hit ? std::max<int64_t>(0, hit_capacity - hits) : 0, out, s));
             HIPCHECK(hipStreamSynchronize(s));
-            if (n_arg > res->total) return too_many(res->total);
-            if (n_arg >= 0 || res->total <= cap) break;
-            rc = launch_reserve(sim, res->total);        /* a larger event than any so far: once more */
-            if (!rc) rc = tape_reserve(sim, res->total, K);
+            const int64_t total = res->total;
+            if (n_arg > total) return too_many(total);
+            if (n_arg >= 0 || total <= cap) break;
+            rc = launch_reserve(sim, total);             /* a larger event than any so far: once more (*res moves) */
+            if (!rc) rc = tape_reserve(sim, total, K);
             if (rc) return rc;
         }
         if (!sliced) {
@@ -1182,8 +1187,12 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
             if (n_photon == 0) return fail(MI_NOTHING_TO_DO, "gensteps carry no photons");
         }
         hits += res->n_hit;
-        for (int i = 0; i < 3; ++i) ms[i] += sim->clock_ms * (double)(res->clock[i + 1] - res->clock[i]);
-        ms[3] += sim->clock_ms * (double)(res->clock[3] - res->clock[0]);
+        const uint64_t* ends = result_ends((LaunchResult*)sim->result.p);
+        const uint64_t clock[4] = { res->setup_begins, *std::max_element(ends, ends + n_setup), res->compaction_begins,
+                                    *std::max_element(ends + OA_SETUP_BLOCKS,
+                                                      ends + OA_SETUP_BLOCKS + oa_launch::compact_tiles(res->n_photon)) };
+        for (int i = 0; i < 3; ++i) ms[i] += sim->clock_ms * (double)(clock[i + 1] - clock[i]);
+        ms[3] += sim->clock_ms * (double)(clock[3] - clock[0]);
     }
     if (taping) {
         mi_sim::TapeKey& tk = sim->tape_key;

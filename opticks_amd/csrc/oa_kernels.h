@@ -10,7 +10,8 @@ hipError_t seed_map(const int64_t* d_prefix, int64_t n_gs, int64_t n_photon, uin
 /* exclusive prefix of the gensteps' photon counts into d_prefix[0..n_gs], which holds
    gs_prefix_words(n_gs) words (block sums behind it) */
 int64_t gs_prefix_words(int64_t n_gs);
-hipError_t gs_prefix(const float* d_gs, int64_t n_gs, int64_t* d_prefix, hipStream_t s);
+/* out (may be null): setup_begins is set where the prefix takes several blocks */
+hipError_t gs_prefix(const float* d_gs, int64_t n_gs, int64_t* d_prefix, hipStream_t s, LaunchResult* out = nullptr);
 /* start of a single-event launch (k_setup): seeds of up to cap photons, its cleared words (words:
    clear_words(cap)), event bounds ev (4) and ev_id (1), the launch's photon count and wave_width
    n_dev (2) */
@@ -19,16 +20,18 @@ struct SetupArgs {
     int64_t* prefix; uint32_t* seed;
     unsigned long long* words;
     int64_t* ev; int32_t* ev_id; int32_t event_id;
-    int64_t* n_dev; LaunchResult* out;
+    int64_t* n_dev; LaunchResult* out;  /* out: result_bytes(cap) */
     int64_t n_wave;                     /* waves of the propagation grid */
 };
 hipError_t setup(const SetupArgs& a, hipStream_t s);
+int setup_blocks(int64_t cap);
 /* Cleared words of a launch of up to n photons: the propagation's photon counter, the compaction's
    ticket and the state of its tiles (256 bitmask words each), then the hit bitmask. The counters
    are in front, so that an event of fewer photons clears and reads what it needs alone. */
 #define OA_WORDS_TICKET 1
 #define OA_WORDS_STATE 2
 inline int64_t compact_tiles(int64_t n_photon) { return ((n_photon + 63) / 64 + 255) / 256; }
+inline size_t result_bytes(int64_t n_photon) { return sizeof(LaunchResult) + 8 * (size_t)(OA_SETUP_BLOCKS + compact_tiles(n_photon)); }
 inline int64_t bitmask_offset(int64_t n_photon) { return OA_WORDS_STATE + compact_tiles(n_photon); }
 inline int64_t clear_words(int64_t n_photon) { return bitmask_offset(n_photon) + (n_photon + 63) / 64; }
 hipError_t simulate(const SimParams& P, int kernel, int block, int grid, hipStream_t s);

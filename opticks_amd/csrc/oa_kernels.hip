@@ -50,9 +50,10 @@ __global__ void __launch_bounds__(256) k_gs_event(const int64_t* ev_gs_begin, in
 
 /* exclusive prefix of the gensteps' photon counts, 1,024 a block: `sums` has each block's
    total (k_gs_sums) where there is more than one */
-__global__ void __launch_bounds__(1024) k_gs_sums(const float* gs, int64_t n_gs, int64_t* sums)
+__global__ void __launch_bounds__(1024) k_gs_sums(const float* gs, int64_t n_gs, int64_t* sums, LaunchResult* out)
 {
     __shared__ int64_t part[16];
+    if (out && blockIdx.x == 0 && threadIdx.x == 0) out->setup_begins = wall_clock64();
     const int64_t g = (int64_t)blockIdx.x * 1024 + threadIdx.x;
     int64_t v = g < n_gs ? (int64_t)__float_as_uint(gs[24 * g + 3]) : 0;
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
@@ -105,7 +106,8 @@ __global__ void __launch_bounds__(1024) k_gs_prefix(const float* gs, int64_t n_g
  * and nothing is propagated, when that is more than the gensteps have or than the launch's
  * buffers hold (cap): the host sees the total and reports it or tries again.
  * SMALL: up to OA_SETUP_GS gensteps; every block forms their prefix in LDS by itself (a few
- * loads a thread), so one kernel does all of it. Else the prefix is there already.
+ * loads a thread), so one kernel does all of it. Else the prefix is there already (k_gs_sums has
+ * stamped the begin).
  */
 template <bool SMALL>
 __global__ void __launch_bounds__(256) k_setup(const float* gs, int64_t n_gs, int64_t n_arg, int64_t cap, int64_t* prefix,
@@ -118,7 +120,7 @@ __global__ void __launch_bounds__(256) k_setup(const float* gs, int64_t n_gs, in
     __shared__ int64_t part[16];
     const int t = threadIdx.x;
     const bool first = blockIdx.x == 0;
-    if (first && t == 0) out->clock[0] = wall_clock64();
+    if (SMALL && first && t == 0) out->setup_begins = wall_clock64();
     if (SMALL) {
         int64_t c[PER], sum = 0;
 #pragma unroll
@@ -173,8 +175,9 @@ __global__ void __launch_bounds__(256) k_setup(const float* gs, int64_t n_gs, in
         out->total = total;
         out->n_photon = n;
         out->n_hit = 0;
-        out->clock[1] = wall_clock64();
     }
+    __syncthreads();
+    if (t == 0) result_ends(out)[blockIdx.x] = wall_clock64();
 }
 
 /* ------------------------------------------------------------ simtrace */
@@ -430,7 +433,7 @@ __global__ void __launch_bounds__(256) k_compact(const unsigned long long* __res
     if (t == 0) s_tile = (int64_t)atomicAdd(ticket, 1ull);
     __syncthreads();
     const int64_t tile = s_tile;
-    if (out && tile == 0 && t == 0) out->clock[2] = wall_clock64();
+    if (out && tile == 0 && t == 0) out->compaction_begins = wall_clock64();
     const int64_t w = tile * 256 + t;
     unsigned long long m = w < n_words ? words[w] : 0ull;
     const int32_t c = __popcll(m);
@@ -495,10 +498,10 @@ __global__ void __launch_bounds__(256) k_compact(const unsigned long long* __res
         }
         for (; i < n4; i += 256) dst[i] = src[4 * (int)s_list[i >> 2] + (i & 3)];
     }
-    if (out && tile == n_tiles - 1 && t == 0) {
-        out->n_hit = base + total;
-        out->clock[3] = wall_clock64();
-    }
+    if (!out) return;
+    if (tile == n_tiles - 1 && t == 0) out->n_hit = base + total;
+    __syncthreads();
+    if (t == 0) result_ends(out)[OA_SETUP_BLOCKS + tile] = wall_clock64();
 }
 
 /* hits among photons [0, ph) for each event boundary ph = ev_ph_begin[e] */
@@ -638,24 +641,29 @@ hipError_t seed_map(const int64_t* d_prefix, int64_t n_gs, int64_t n_photon, uin
 
 int64_t gs_prefix_words(int64_t n_gs) { return n_gs + 1 + (n_gs + 1023) / 1024; }
 
-hipError_t gs_prefix(const float* d_gs, int64_t n_gs, int64_t* d_prefix, hipStream_t s)
+hipError_t gs_prefix(const float* d_gs, int64_t n_gs, int64_t* d_prefix, hipStream_t s, LaunchResult* out)
 {
     const unsigned nb = (unsigned)((n_gs + 1023) / 1024);
     int64_t* sums = d_prefix + n_gs + 1;
-    if (nb > 1) hipLaunchKernelGGL(k_gs_sums, dim3(nb), dim3(1024), 0, s, d_gs, n_gs, sums);
+    if (nb > 1) hipLaunchKernelGGL(k_gs_sums, dim3(nb), dim3(1024), 0, s, d_gs, n_gs, sums, out);
     hipLaunchKernelGGL(k_gs_prefix, dim3(nb), dim3(1024), 0, s, d_gs, n_gs, sums, d_prefix);
     return hipGetLastError();
 }
 
+int setup_blocks(int64_t cap)
+{
+    const int64_t work = std::max<int64_t>(cap / 8, clear_words(cap));
+    return (int)std::min<int64_t>(OA_SETUP_BLOCKS, (work + 255) / 256 + 1);
+}
+
 hipError_t setup(const SetupArgs& a, hipStream_t s)
 {
-    const int64_t work = std::max<int64_t>(a.cap / 8, clear_words(a.cap));
-    const unsigned nb = (unsigned)std::min<int64_t>(1024, (work + 255) / 256 + 1);
+    const unsigned nb = (unsigned)setup_blocks(a.cap);
     if (a.n_gs <= OA_SETUP_GS) {
         hipLaunchKernelGGL(k_setup<true>, dim3(nb), dim3(256), 0, s, a.gs, a.n_gs, a.n_arg, a.cap, a.prefix, a.seed, a.words,
                            bitmask_offset(a.cap), a.ev, a.ev_id, a.event_id, a.n_dev, a.out, a.n_wave);
     } else {
-        const hipError_t e = gs_prefix(a.gs, a.n_gs, a.prefix, s);
+        const hipError_t e = gs_prefix(a.gs, a.n_gs, a.prefix, s, a.out);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(k_setup<false>, dim3(nb), dim3(256), 0, s, a.gs, a.n_gs, a.n_arg, a.cap, a.prefix, a.seed, a.words,
                            bitmask_offset(a.cap), a.ev, a.ev_id, a.event_id, a.n_dev, a.out, a.n_wave);

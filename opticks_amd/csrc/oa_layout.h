@@ -93,8 +93,16 @@ struct LaunchResult {
     int64_t total;                /* photons of the gensteps */
     int64_t n_photon;             /* photons propagated (0: the count was refused, see k_setup) */
     int64_t n_hit;
-    uint64_t clock[4];            /* device wall clock: setup begins, ends, compaction begins, ends */
+    uint64_t setup_begins, compaction_begins;     /* device wall clock */
 };
+
+/* Behind it in the same memory, the clock where each block of k_setup and each tile of k_compact
+   ended (the largest is the kernel's end): OA_SETUP_BLOCKS words, then one a tile. */
+#define OA_SETUP_BLOCKS 1024
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline uint64_t* result_ends(LaunchResult* r) { return reinterpret_cast<uint64_t*>(r + 1); }
 
 /*
  * Photons dealt to each of the n_wave waves of the propagation grid at its start: 64, or an

@@ -131,6 +131,7 @@ def test_tape_of_an_event_of_unknown_size_is_its_own(stub):
     sim.config.adjoint_tape = 64                           # records of the same tape, more of them
     sim.set_config(sim.config)
     assert run_device(stub, sim, event(3000)) == (0, 1500)
+    assert run_device(stub, sim, event(1_300_000)) == (0, 650_000)    # buffers, and what the host reads, move
     sim.config.max_slot = 2000                             # slices of one event: the event's count
     sim.set_config(sim.config)
     gs = np.concatenate([event(1500), event(1000), event(700)])

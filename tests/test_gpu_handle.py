@@ -193,3 +193,30 @@ def test_results_are_ordinary_memory(n):
         torch.cuda.synchronize()
         assert z[0].item() == 2.0
     sim.close()
+
+
+def test_device_times_cover_the_work():
+    """The parts of last_timing reach from the first genstep read to the last hit written: the
+    compaction takes no less than its records' bytes at the card's nominal 8 TB/s (15 us here; 6.4
+    where the tile that ended first but one gave the time), and the total is what events around
+    the call see, but for launching and waiting."""
+    w = configs.config0(num_photon=1, sensor=True)
+    gs = np.repeat(w.gensteps, 40_000, 0)
+    gs.view(np.uint32)[:, 0, 3] = 25
+    ev = Device(gs)
+    sim = QSim(w.geometry, w.physics, SEventConfig(seed=w.seed))
+    stream = torch.cuda.Stream()
+    parts, rest = [], []
+    for i in range(12):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        torch.cuda.synchronize()
+        a.record(stream)
+        m = sim.simulate_device(ev.gs, ev.photon, ev.seq, ev.hit, eventID=i, stream=stream)
+        b.record(stream)
+        b.synchronize()
+        t = sim.last_timing()
+        assert m > 900_000 and 128 * m / 8e9 < t["compact_ms"] < t["total_ms"] < a.elapsed_time(b)
+        assert abs(t["seed_ms"] + t["propagate_ms"] + t["compact_ms"] - t["total_ms"]) < 1e-6
+        rest.append(a.elapsed_time(b) - t["total_ms"])
+    assert sorted(rest)[6] < 0.1
+    sim.close()
