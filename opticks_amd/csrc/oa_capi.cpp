@@ -1067,7 +1067,6 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
     if (!d_gensteps) return fail(MI_ERR_ARG, "null gensteps");
     if (d_hit && !d_photon) return fail(MI_ERR_ARG, "hits are gathered from the photon array: pass d_photon");
     hipStream_t s = stream ? (hipStream_t)stream : sim->stream;
-    sim->tape_key.valid = false;
     HIPCHECK(sim->prefix.reserve((size_t)oa_launch::gs_prefix_words(n_gs)));
     HIPCHECK(sim->evbuf.reserve(4));
     HIPCHECK(sim->ev_id.reserve(1));
@@ -1120,6 +1119,9 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
         slices.emplace_back(0, n_gs);
     }
     const bool sliced = slices.size() > 1;
+    /* from here on the tape is this event's, unless its count is refused or 0: then nothing is written */
+    const bool had_tape = sim->tape_key.valid;
+    sim->tape_key.valid = false;
     if (n_photon >= 0) {                 /* a sliced event has one tape */
         const int rc = tape_reserve(sim, n_photon, K);
         if (rc) return rc;
@@ -1176,7 +1178,10 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
                                              d_hit ? std::max<int64_t>(0, hit_capacity - hits) : 0, out, s));
             HIPCHECK(hipStreamSynchronize(s));
             const int64_t total = res->total;
-            if (n_arg > total) return too_many(total);
+            if (n_arg > total) {
+                sim->tape_key.valid = had_tape;
+                return too_many(total);
+            }
             if (n_arg >= 0 || total <= cap) break;
             rc = launch_reserve(sim, total);             /* a larger event than any so far: once more (*res moves) */
             if (!rc) rc = tape_reserve(sim, total, K);
@@ -1184,7 +1189,10 @@ static int simulate_device_impl(mi_sim* sim, int32_t event_id, const void* d_gen
         }
         if (!sliced) {
             n_photon = res->n_photon;
-            if (n_photon == 0) return fail(MI_NOTHING_TO_DO, "gensteps carry no photons");
+            if (n_photon == 0) {
+                sim->tape_key.valid = had_tape;
+                return fail(MI_NOTHING_TO_DO, "gensteps carry no photons");
+            }
         }
         hits += res->n_hit;
         const uint64_t* ends = result_ends((LaunchResult*)sim->result.p);

@@ -22,7 +22,7 @@ std::mutex g_m;
 std::map<const char*, size_t> g_alloc;         /* live allocations */
 size_t g_limit = (size_t)1 << 40, g_largest = 0;
 std::atomic<int> g_bad{0}, g_inside{0}, g_overlap{0};
-int g_fail_trace = 0, g_resident = 4, g_waves_dealt = 0, g_grid = 0;
+int g_adjoint_tape = 0, g_fail_trace = 0, g_resident = 4, g_waves_dealt = 0, g_grid = 0;
 int64_t g_n = 0, g_stride = 0;
 
 hipError_t alloc(void** p, size_t n)
@@ -81,6 +81,7 @@ int stub_known(const void* p)
     auto it = g_alloc.upper_bound((const char*)p);
     return it != g_alloc.begin() && (--it, (const char*)p < it->first + it->second);
 }
+int stub_adjoint_tape() { return g_adjoint_tape; }
 int stub_tape_stride() { return (int)g_stride; }
 int stub_waves_dealt() { return g_waves_dealt; }
 int stub_grid() { return g_grid; }
@@ -209,7 +210,11 @@ hipError_t simtrace(const SimParams& P, float4* out, hipStream_t)
 }
 hipError_t trace(const SimParams&, const float4*, int64_t, float4*, hipStream_t) { return hipSuccess; }
 hipError_t refit(BvhNode*, int64_t, uint32_t, const uint32_t*, const float*, hipStream_t) { return hipSuccess; }
-hipError_t adjoint_chunk(const SimParams&, const AdjBufs&, int64_t, int64_t, int, int, hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t adjoint_chunk(const SimParams& P, const AdjBufs&, int64_t, int64_t, int, int, hipEvent_t, hipStream_t)
+{
+    g_adjoint_tape = P.tape != nullptr;
+    return hipSuccess;
+}
 int tape_reduce_rows(int32_t) { return 32; }
 int adjoint_blocks_per_cu(int, int) { return 1; }
 hipError_t noalloc_scratch(int, void** p)

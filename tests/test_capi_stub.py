@@ -282,3 +282,29 @@ def test_calls_sharing_the_noalloc_scratch_take_turns(stub):
     for t in threads:
         t.join()
     assert rcs == [0] * 12 and stub.stub_overlap() == 0
+
+
+def test_a_refused_call_keeps_the_tape(stub):
+    """A call refused for its photon count has propagated nothing: the adjoint of the event before
+    it still finds that event's tape."""
+    from opticks_amd.adjoint import LengthParams
+    w = configs.config0(num_photon=1)
+    params = LengthParams(w.physics, ("Water",), n_bin=4)
+    adj = params.c_struct(1)
+    grad = np.zeros((1, params.n_param), np.float32)
+    sim = sim_of(adjoint_tape=4)
+    gs, other = event(2000), event(1500)
+
+    def adjoint_has_tape():
+        assert stub.mi_sim_adjoint_device(sim.handle, 0, gs.ctypes.data, 1, 2000, 0, None, 0, L.C.byref(adj), grad.ctypes.data,
+                                          None) == 0
+        return stub.stub_adjoint_tape()
+
+    assert run_device(stub, sim, gs) == (0, 1000) and adjoint_has_tape()
+    for n_photon, g in ((2001, gs), (1600, other), (10 ** 9, other)):
+        rc, _ = run_device(stub, sim, g, n_photon=n_photon, n_alloc=2000)
+        assert rc == -1 and adjoint_has_tape()
+    assert run_device(stub, sim, event(0), n_alloc=1) == (1, 0) and adjoint_has_tape()
+    assert run_device(stub, sim, other) == (0, 750) and not adjoint_has_tape()
+    assert run_device(stub, sim, gs) == (0, 1000) and adjoint_has_tape()
+    sim.close()
