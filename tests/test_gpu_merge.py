@@ -167,3 +167,113 @@ def test_merge_tiles_and_key_widths(sim_and_photons, n):
                     with pytest.raises(RuntimeError, match="out_capacity"):
                         sim.merge_hits_device(rows, SD, tw, out_t=short)
                     assert not short.cpu().numpy().any()
+
+
+def bucket(time, tw):
+    """(unsigned)(time / window) as the GPU converts: towards zero, clamped to 32 bits, not-a-number 0"""
+    q = np.float32(time) / np.float32(tw)
+    return 0 if not q > 0 else min(int(min(float(q), 2.0 ** 33)), 0xffffffff)
+
+
+def smaller(a, b):
+    """fminf: a number rather than not-a-number"""
+    return b if np.isnan(a) else a if np.isnan(b) else min(a, b)
+
+
+@pytest.mark.parametrize("kind", ["mixed", "one run", "nan runs"])
+def test_merge_times_that_are_no_ordinary_numbers(sim_and_photons, kind):
+    """NaN, infinite, negative and zero times of both signs in short runs and in runs that a wave
+    folds in pieces: the record types' reduce_op applied left to right in the sorted order."""
+    sim, _ = sim_and_photons
+    rng = np.random.default_rng(len(kind))
+    n, tw = 9001, 1.0
+    P = synthetic(n, 5)
+    u = P.view(np.uint32)
+    special = np.array([np.nan, np.inf, -np.inf, -3.5, -0.25, 0.0, -0.0, 0.25, 0.75, 1.5, 5.0e9, 1e-40], np.float32)
+    P[:, 0, 3] = rng.choice(special, n)
+    u[:, 3, 1] = rng.integers(1, 4, n).astype(np.uint32)
+    u[:, 3, 3] = SD | (rng.integers(0, 8, n).astype(np.uint32) << 8)
+    if kind == "one run":
+        P[:, 0, 3] = rng.choice(np.array([np.nan, -3.5, -0.0, 0.0, 0.25, 0.75], np.float32), n)
+        u[:, 3, 1] = 7
+    if kind == "nan runs":
+        P[:, 0, 3] = np.nan
+        u[:, 3, 1] = rng.integers(0, 400, n).astype(np.uint32)
+    t = P[:, 0, 3]
+    lt = np.stack([(u[:, 1, 3] & 0xFFFF0000) | (u[:, 3, 1] & 0xFFFF), u[:, 0, 3], np.arange(n, dtype=np.uint32), u[:, 3, 3]],
+                  axis=1).astype(np.uint32)
+    runs = {}
+    for i in range(n):
+        runs.setdefault((int(u[i, 3, 1]) & 0xffff, bucket(t[i], tw)), []).append(i)
+    want, wantl = [], []
+    for key in sorted(runs):
+        best = first = runs[key][0]
+        hc, fm, tt = int(u[best, 1, 3]) >> 16, int(u[best, 3, 3]), t[best]
+        for b in runs[key][1:]:
+            if not smaller(t[best], t[b]) == t[best]:
+                best = b
+            tt = smaller(tt, t[b])
+            hc, fm = (hc + (int(u[b, 1, 3]) >> 16)) & 0xffff, fm | int(u[b, 3, 3])
+        r = u[best].copy()
+        r[1, 3] = (int(r[1, 3]) & 0xffff) | (hc << 16)
+        r[3, 3] = fm
+        want.append(r)
+        wantl.append((hc << 16 | int(lt[first, 0]) & 0xffff, tt, int(lt[first, 2]), fm))
+    got = sim.merge_hits_device(torch.from_numpy(P).to(DEV), SD, tw).cpu().numpy().view(np.uint32)
+    assert np.array_equal(got, np.array(want))
+    gl = sim.merge_hits_device(torch.from_numpy(lt.view(np.int32)).to(DEV), SD, tw).cpu().numpy().view(np.uint32)
+    assert len(gl) == len(wantl)
+    for col in (0, 2, 3):
+        assert np.array_equal(gl[:, col], np.array([w[col] for w in wantl], np.uint32))
+    # the smaller of two zeros, or of two that are no numbers, is either
+    assert np.array_equal(gl[:, 1].copy().view(np.float32), np.array([w[1] for w in wantl], np.float32), equal_nan=True)
+
+
+def merged_lites(lt, tw):
+    """spm.merge_lites of selected records with ordinary times >= 0, by whole arrays"""
+    t = lt[:, 1].view(np.float32)
+    keys = ((lt[:, 0] & 0xffff).astype(np.uint64) << 32) | (t / np.float32(tw)).astype(np.float32).astype(np.uint64)
+    order = np.argsort(keys, kind="stable")
+    ks = keys[order]
+    start = np.flatnonzero(np.r_[True, ks[1:] != ks[:-1]])
+    hc = np.add.reduceat((lt[order, 0] >> 16).astype(np.uint64), start) & 0xffff
+    out = np.empty((len(start), 4), np.uint32)
+    first = order[start]
+    out[:, 0] = (hc.astype(np.uint32) << 16) | (lt[first, 0] & 0xffff)
+    out[:, 1] = np.minimum.reduceat(t[order], start).view(np.uint32)
+    out[:, 2] = lt[first, 2]
+    out[:, 3] = np.bitwise_or.reduceat(lt[order, 3], start)
+    # the photon record kept: the earliest in input order among the run's smallest times
+    run = np.repeat(np.arange(len(start)), np.diff(np.r_[start, len(ks)]))
+    pos = np.flatnonzero(t[order] == out[run, 1].view(np.float32))
+    keep = np.full(len(start), -1)
+    keep[run[pos][::-1]] = order[pos][::-1]
+    return out, keep
+
+
+# selected counts on both sides of the tiles of 2,048 (selection and sort) and 1,024 (runs), past the
+# 256 sort tiles of one step of a digit's sums, and past the 8,192 selection tiles of one step of theirs
+@pytest.mark.parametrize("n, lite_only", [(1023, False), (1024, False), (1025, False), (2047, False), (2048, False),
+                                          (2049, False), (600_001, False), (16_900_123, True)])
+def test_merge_of_all_records(sim_and_photons, n, lite_only):
+    sim, _ = sim_and_photons
+    rng = np.random.default_rng(n)
+    lt = np.empty((n, 4), np.uint32)
+    lt[:, 0] = (rng.integers(1, 5, n) << 16) | rng.integers(1, 3000, n)
+    lt[:, 1] = (rng.integers(0, 4000, n) * np.float32(0.125)).astype(np.float32).view(np.uint32)
+    lt[:, 2] = np.arange(n)
+    lt[:, 3] = 1 << rng.integers(0, 16, n)
+    want, keep = merged_lites(lt, 4.0)
+    if n < 3000:
+        assert np.array_equal(want, spm.merge_lites(lt, L.MI_MERGE_ALREADY_SELECTED, 4.0))
+    got = sim.merge_hits_device(torch.from_numpy(lt.view(np.int32)).to(DEV), L.MI_MERGE_ALREADY_SELECTED, 4.0)
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), want)
+    if lite_only:
+        return
+    P = np.zeros((n, 4, 4), np.uint32)
+    P[:, 0, 0], P[:, 0, 3], P[:, 3, 1], P[:, 3, 3] = lt[:, 2], lt[:, 1], lt[:, 0] & 0xffff, lt[:, 3]
+    P[:, 1, 3] = lt[:, 0] & 0xffff0000
+    ref = P[keep].copy()
+    ref[:, 1, 3], ref[:, 3, 3] = want[:, 0] & 0xffff0000, want[:, 3]
+    got = sim.merge_hits_device(torch.from_numpy(P.view(np.float32)).to(DEV), L.MI_MERGE_ALREADY_SELECTED, 4.0)
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), ref)
