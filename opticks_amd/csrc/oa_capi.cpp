@@ -331,7 +331,7 @@ struct mi_sim {
     DBuf<unsigned long long> next;       /* photon counter of the adjoint replay */
     PinnedBuf result;                    /* LaunchResult: the last launch's counts and clock */
     double clock_ms = 1e-5;              /* device wall clock tick */
-    int shape_key[5] = { -1, -1, -1, -1, -1 }, resident_blocks = 0;   /* wave_shape's last answer */
+    struct Resident { int block = -1, rng = -1, depth = -1, blocks = 0; } resident[4];   /* wave_shape's last answers */
     /* outputs of the host-array entry point */
     DBuf<float4> photon, hit;
     DBuf<uint64_t> seq;
@@ -988,14 +988,13 @@ struct WaveShape { int block, grid; int64_t waves; };
 static WaveShape wave_shape(mi_sim* sim, bool lite, bool tape)
 {
     const int block = sim_block(sim), waves_per_block = block / 64;
-    const int key[5] = { block, sim->cfg.rng_kind, sim->stack_depth, lite, tape };
-    if (std::memcmp(key, sim->shape_key, sizeof(key)) != 0) {
+    mi_sim::Resident& r = sim->resident[(lite ? 1 : 0) | (tape ? 2 : 0)];
+    if (r.block != block || r.rng != sim->cfg.rng_kind || r.depth != sim->stack_depth) {
         int nb = oa_launch::wave_blocks_per_cu(block, sim->cfg.rng_kind, sim->stack_depth, lite, sim->ext_leaves, tape);
         if (nb <= 0) nb = std::max(1, 8 / waves_per_block);
-        sim->resident_blocks = std::max(1, sim->n_cu * nb);
-        std::memcpy(sim->shape_key, key, sizeof(key));
+        r = { block, sim->cfg.rng_kind, sim->stack_depth, std::max(1, sim->n_cu * nb) };
     }
-    int grid = sim->resident_blocks;
+    int grid = r.blocks;
     if (sim->cfg.waves_per_cu > 0)
         grid = (int)std::max<int64_t>(1, std::min<int64_t>(grid, (int64_t)sim->n_cu * sim->cfg.waves_per_cu / waves_per_block));
     return { block, grid, (int64_t)grid * waves_per_block };

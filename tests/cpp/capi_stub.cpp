@@ -22,7 +22,7 @@ std::mutex g_m;
 std::map<const char*, size_t> g_alloc;         /* live allocations */
 size_t g_limit = (size_t)1 << 40, g_largest = 0;
 std::atomic<int> g_bad{0}, g_inside{0}, g_overlap{0};
-int g_adjoint_tape = 0, g_fail_trace = 0, g_resident = 4, g_waves_dealt = 0, g_grid = 0;
+int g_queries = 0, g_adjoint_tape = 0, g_fail_trace = 0, g_resident = 4, g_waves_dealt = 0, g_grid = 0;
 int64_t g_n = 0, g_stride = 0;
 
 hipError_t alloc(void** p, size_t n)
@@ -85,6 +85,7 @@ int stub_adjoint_tape() { return g_adjoint_tape; }
 int stub_tape_stride() { return (int)g_stride; }
 int stub_waves_dealt() { return g_waves_dealt; }
 int stub_grid() { return g_grid; }
+int stub_queries() { return g_queries; }
 int stub_resident() { return g_resident; }
 int stub_resident_lite() { return g_resident - 1; }
 
@@ -188,7 +189,11 @@ hipError_t compact_hits(unsigned long long* words, int64_t cap, const int64_t* n
     if (out) out->n_hit = m;
     return hipSuccess;
 }
-int wave_blocks_per_cu(int, int, int, bool lite, bool, bool) { return g_resident - (lite ? 1 : 0); }
+int wave_blocks_per_cu(int, int, int, bool lite, bool, bool)
+{
+    g_queries++;
+    return g_resident - (lite ? 1 : 0);
+}
 unsigned sim_lds(int, int, int) { return 1024; }
 hipError_t prefix_check(const int64_t*, const int64_t*, int64_t, unsigned long long*, hipStream_t) { return hipSuccess; }
 hipError_t zero_u64(unsigned long long*, int64_t, hipStream_t) { return hipSuccess; }

@@ -155,6 +155,12 @@ def test_first_photons_are_dealt_to_resident_waves(stub, waves_per_cu):
         else:
             assert run_device(stub, sim, gs) == (0, 500)
         assert stub.stub_grid() == stub.stub_waves_dealt() == 2 * min(waves_per_cu or fit, fit)
+    queries = stub.stub_queries()
+    for _ in range(3):                                         # asked once for each kernel
+        assert run_device(stub, sim, gs) == (0, 500)
+        assert stub.mi_sim_simulate_lite_device(sim.handle, 0, gs.ctypes.data, 1, -1, 0, lite.ctypes.data, None, None, None, 0,
+                                                L.C.byref(m), None) == 0
+    assert stub.stub_queries() == queries
     sim.close()
 
 
