@@ -1445,7 +1445,7 @@ static bool is_pinned(const void* p)
     return known;
 }
 
-static int fetch(mi_sim* sim, std::initializer_list<Staged::Array> arrays, hipStream_t s)
+static int fetch(mi_sim* sim, std::initializer_list<Staged::Array> arrays, hipStream_t s) try
 {
     std::vector<Staged::Array> ordinary;
     bool direct = false;
@@ -1462,6 +1462,9 @@ static int fetch(mi_sim* sim, std::initializer_list<Staged::Array> arrays, hipSt
     HIPCHECK(st.run(ordinary, sim->ring, s));
     if (direct) HIPCHECK(hipStreamSynchronize(s));
     return MI_OK;
+} catch (const std::bad_alloc&) {
+    (void)hipStreamSynchronize(s);                  /* a direct copy may be under way */
+    return fail(MI_ERR_HIP, "out of host memory");
 }
 
 int mi_sim_fetch(mi_sim* sim, float* photon, uint64_t* seq, float* hit)
