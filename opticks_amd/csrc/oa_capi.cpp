@@ -1533,19 +1533,19 @@ int mi_sim_simtrace_device(mi_sim* sim, const void* d_gensteps, int64_t n_gs, in
     hipStream_t s = stream ? (hipStream_t)stream : sim->stream;
     HIPCHECK(sim->prefix.reserve((size_t)oa_launch::gs_prefix_words(n_gs)));
     HIPCHECK(oa_launch::gs_prefix((const float*)d_gensteps, n_gs, sim->prefix.p, s));
-    int64_t total = 0;
-    HIPCHECK(hipMemcpyAsync(&total, sim->prefix.p + n_gs, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    HIPCHECK(hipStreamSynchronize(s));
-    if (n_photon >= 0 && n_photon != total) return fail(MI_ERR_ARG, "n_photon does not match the gensteps");
-    if (total == 0) return fail(MI_NOTHING_TO_DO, "gensteps carry no photons");
     SimParams P = base_params(sim);
     P.gensteps = (const float*)d_gensteps;
     P.gs_prefix = sim->prefix.p;
     P.n_gs = n_gs;
+    HIPCHECK(oa_launch::ray_sample(P, (LaunchResult*)sim->result.p, s));
+    HIPCHECK(hipStreamSynchronize(s));
+    const int64_t total = ((volatile LaunchResult*)sim->result.p)->total;
+    if (n_photon >= 0 && n_photon != total) return fail(MI_ERR_ARG, "n_photon does not match the gensteps");
+    if (total == 0) return fail(MI_NOTHING_TO_DO, "gensteps carry no photons");
     P.n_photon = total;
     HIPCHECK(sim->ray_next.reserve(1));
     P.next = sim->ray_next.p;
-    HIPCHECK(oa_launch::simtrace(P, (float4*)d_simtrace, s));
+    HIPCHECK(oa_launch::simtrace(P, (float4*)d_simtrace, (const LaunchResult*)sim->result.p, s));
     HIPCHECK(hipStreamSynchronize(s));
     return MI_OK;
 }

@@ -51,7 +51,10 @@ hipError_t compact_hits(unsigned long long* d_words, int64_t n_photon, const int
 hipError_t event_hit_offsets(const unsigned long long* d_bitmask, const int32_t* d_word_prefix,
                              const int64_t* d_block_total, const int64_t* d_ev_ph_begin, int32_t n_event,
                              int64_t n_words, int64_t* d_hit_offsets, hipStream_t s);
-hipError_t simtrace(const SimParams& P, float4* out, hipStream_t s);
+/* before a simtrace: the gensteps' rays, and a sample of where they end, into out */
+hipError_t ray_sample(const SimParams& P, LaunchResult* out, hipStream_t s);
+/* sample: ray_sample's, complete */
+hipError_t simtrace(const SimParams& P, float4* out, const LaunchResult* sample, hipStream_t s);
 hipError_t trace(const SimParams& P, const float4* rays, int64_t n, float4* out, hipStream_t s);
 hipError_t refit(BvhNode* d_tlas, int64_t n_tlas, uint32_t max_depth, const uint32_t* d_tlas_items,
                  const float* d_inst_box, hipStream_t s);

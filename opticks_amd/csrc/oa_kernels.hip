@@ -256,6 +256,33 @@ __global__ void __launch_bounds__(64) OA_OCC k_simtrace_few(SimParams P, float4*
     simtrace_record(P, out + 4 * i, o, d, prd);
 }
 
+/*
+ * What the host has to know before a simtrace: the number of rays, and from `least` rays on, of
+ * OA_RAY_SAMPLES of them, evenly spread, how many leave the free ball and go on to the instance walk
+ * (a count a block, at result_ends of out; none where there is no such ball). It takes the place of a
+ * copy of the number, and a few microseconds where it samples.
+ */
+#define OA_RAY_SAMPLES 4096
+__global__ void __launch_bounds__(64) k_ray_sample(SimParams P, LaunchResult* out, int64_t least)
+{
+    const int64_t n = P.gs_prefix[P.n_gs];
+    if (blockIdx.x == 0 && threadIdx.x == 0) out->total = n;
+    unsigned long long walkers = 0ull;
+    if (n >= least && P.front_plain && !P.tlas_empty) {
+        const int64_t k = (int64_t)blockIdx.x * 64 + threadIdx.x, i = n / OA_RAY_SAMPLES * k + n % OA_RAY_SAMPLES * k / OA_RAY_SAMPLES;
+        const int64_t gsi = upper_index(P.gs_prefix, 0, P.n_gs, i);
+        v3 o, d;
+        simtrace_ray(P, reinterpret_cast<const float4*>(P.gensteps + 24 * gsi), i, o, d);
+        Nearest best;
+        nearest_none(best, P.tmax);
+        trace_front(P, o, d, P.tmin, best);
+        float tlo = P.tmin;
+        const float4 fb = const_load(const_ptr(P.free_ball));
+        walkers = __ballot(fb.w > 0.f && beyond_free_ball(fb, o, d, P.tmin, best.t, tlo));
+    }
+    if (threadIdx.x == 0) result_ends(out)[blockIdx.x] = (uint64_t)__popcll(walkers);
+}
+
 /* words of a ray in a wave's queue */
 #define OA_RAY_WORDS 16
 
@@ -778,17 +805,33 @@ hipError_t zero_u64(unsigned long long* p, int64_t n, hipStream_t s)
 }
 
 /*
- * Persistent waves pay where they hold many rays each and the rays walk: every claim of rays is
- * an atomic on one word, and the last rays of a wave run alone. A ray to a lane / persistent /
- * a ray to a lane with sixteen-step genstep lookups, as it was, in us, 2,000 detectors: 0.4M rays
- * 162 / 269 / 186, 1M 273 / 398 / 394, 2M 420 / 591 / 556, 4M 731 / 721 / 901, 10M
- * 1,653 / 1,442 / 1,944. Without a TLAS (a water sphere) every ray is settled by the front
- * instances: 10M 392 / 612 / 690.
+ * Persistent waves pay where many rays walk: every claim of rays is an atomic on one word, about 14 ns
+ * apiece, which rays that the front instances settle do not repay, and the last rays of a wave run
+ * alone. A ray to a lane / persistent, in us, on grids of a 2,000-detector shell by the share of
+ * walkers: 4M rays, 0.16 459 / 615, 0.30 696 / 750, 0.36 780 / 792, 0.47 951 / 832; 10M, 0: 427 / 614,
+ * 0.16 1,043 / 1,081, 0.22 1,287 / 1,227, 0.42 1,968 / 1,568; 24M, 0.13 2,108 / 2,073, 0.19 2,638 / 2,407.
+ * With 20,000 and 60,000 detectors the persistent waves are ahead a little sooner (4M rays, 0.28;
+ * 10M, 0.15), on a line of gensteps later. So the line is a number of walkers, 1.6M, and a share of one in eight for
+ * the claims of the others; fewer than 4M rays (2M, all walking: 420 / 591) are not sampled. Without a
+ * free ball all rays walk, most of them a step or two and in step with their neighbours: a ray to a
+ * lane there (6M rays among clusters of prims 552 / 748, among Boolean solids 675 / 1,006 from one point
+ * and 1,298 / 985 from a hundred, among the extended leaves 1,040 / 1,170 and 1,127 / 1,011).
  */
 #define OA_RAY_MANY 4000000
-hipError_t simtrace(const SimParams& P, float4* out, hipStream_t s)
+#define OA_RAY_WALKERS 1600000
+hipError_t ray_sample(const SimParams& P, LaunchResult* out, hipStream_t s)
 {
-    if (P.n_photon < OA_RAY_MANY || P.tlas_empty) {
+    hipLaunchKernelGGL(k_ray_sample, dim3(OA_RAY_SAMPLES / 64), dim3(64), 0, s, P, out, (int64_t)OA_RAY_MANY);
+    return hipGetLastError();
+}
+
+hipError_t simtrace(const SimParams& P, float4* out, const LaunchResult* sample, hipStream_t s)
+{
+    int64_t of = 0;
+    if (P.n_photon >= OA_RAY_MANY)
+        for (int k = 0; k < OA_RAY_SAMPLES / 64; ++k) of += (int64_t)result_ends(sample)[k];
+    const int64_t walkers = P.n_photon / OA_RAY_SAMPLES * of;
+    if (walkers < OA_RAY_WALKERS || 8 * of < OA_RAY_SAMPLES) {
         const dim3 grid((unsigned)((P.n_photon + 63) / 64));
         const unsigned stacks = 64u * (unsigned)P.stack_depth * 4u;
         if (P.ext_leaves) hipLaunchKernelGGL(k_simtrace_few<true>, grid, dim3(64), stacks, s, P, out);

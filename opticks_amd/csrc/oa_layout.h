@@ -103,6 +103,7 @@ struct LaunchResult {
 __host__ __device__
 #endif
 inline uint64_t* result_ends(LaunchResult* r) { return reinterpret_cast<uint64_t*>(r + 1); }
+inline const uint64_t* result_ends(const LaunchResult* r) { return reinterpret_cast<const uint64_t*>(r + 1); }
 
 /*
  * Photons dealt to each of the n_wave waves of the propagation grid at its start: 64, or an

@@ -207,7 +207,12 @@ hipError_t clear_launch(unsigned long long*, int64_t, int64_t n_wave, hipStream_
     return hipSuccess;
 }
 hipError_t event_hit_offsets(const unsigned long long*, const int32_t*, const int64_t*, const int64_t*, int32_t, int64_t, int64_t*, hipStream_t) { return hipSuccess; }
-hipError_t simtrace(const SimParams& P, float4* out, hipStream_t)
+hipError_t ray_sample(const SimParams& P, LaunchResult* out, hipStream_t)
+{
+    out->total = P.gs_prefix[P.n_gs];
+    return hipSuccess;
+}
+hipError_t simtrace(const SimParams& P, float4* out, const LaunchResult*, hipStream_t)
 {
     if (g_fail_trace) return hipErrorLaunchFailure;
     if (holds(out, 64 * (size_t)P.n_photon)) std::memset((void*)out, 0xff, 64 * (size_t)P.n_photon);

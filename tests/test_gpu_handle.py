@@ -250,3 +250,60 @@ def test_hit_counts_of_busy_detectors(n):
             assert got.shape == (n_det,) and torch.equal(got, want[1:n_det + 1].to(torch.float32)), (name, n_det)
         times[name] = best_time(lambda: (hits_per_detector(hit, n, 2000), torch.cuda.synchronize()), 10)
     assert times["one"] < 2.0 * times["even"] + 100e-6, times
+
+
+@pytest.mark.parametrize("half, walk", [(2000.0, False), (9000.0, True)])
+def test_simtrace_around_the_persistent_kernel(half, walk):
+    """Grids of 4M rays that the front instances settle, and that walk: the checker's records, and
+    no step in the time where the choice of a kernel begins (the settled: 1.6 times where it went
+    by the number alone)."""
+    w = configs.config1(num_gs=1, per_gs=10)
+    sim = QSim(w.geometry, w.physics, SEventConfig(seed=9))
+    gs = configs.frame_gensteps((0, 0, 0, half), (-50, 49, 0, 0, -20, 19, 1000, 1), gridscale=0.02)
+    times = []
+    for last in (999, 1000, 1037):                             # 3,999,999, 4,000,000 and 4,000,037 rays
+        gs.view(np.uint32)[-1, 0, 3] = last
+        gs_t = torch.from_numpy(gs).to(DEV)
+        n = 3_999_000 + last
+        out_t = torch.empty((n, 4, 4), dtype=torch.float32, device=DEV)
+        times.append(best_time(lambda: sim.simtrace_device(gs_t, out_t, n_photon=n), 10))
+    ref = po.World(w.geometry, w.physics).simtrace(gs, seed=9)
+    out = out_t.cpu().numpy().view(np.uint32)
+    assert np.array_equal(out, ref.view(np.uint32))
+    instances = out[:, 3, 3] >> 16
+    assert (np.count_nonzero(instances[instances != 0xffff]) > 100_000) == walk
+    assert max(times[1:]) < 1.3 * times[0] + 30e-6, times
+    sim.close()
+
+
+def test_persistent_simtrace_of_extended_leaves():
+    """Rays that walk among hyperboloids and cones around a free ball, enough of them for the
+    persistent kernel's instantiation with those leaves."""
+    from opticks_amd.foundry import Foundry, Node
+    from opticks_amd.physics import BoundaryLib, Material, Surface, gaussian_icdf
+    lib = BoundaryLib()
+    lib.add_material(Material("Water", 1.33, 20000.0, 30000.0))
+    lib.add_material(Material("Acrylic", 1.5, 1e6, 1e6))
+    lib.add_surface(Surface("wallSurf", detect=0.5, absorb=0.5))
+    b_world = lib.boundary("Water/wallSurf/wallSurf/Water")
+    b_obj = lib.boundary("Water///Acrylic")
+    fd = Foundry()
+    s0 = fd.addSolid("world", [fd.addPrim(Node.box3(13000.0, 13000.0, 13000.0), b_world), fd.addPrim(Node.sphere(5000.0), b_obj)])
+    kinds = [fd.addSolid("hyperboloid", [fd.addPrim(Node.hyperboloid(120.0, 160.0, -200.0, 240.0), b_obj)]),
+             fd.addSolid("cone", [fd.addPrim(Node.cone(200.0, -100.0, 60.0, 160.0), b_obj)])]
+    fd.addInstance(np.eye(4), s0)
+    for i, d in enumerate(configs.fibonacci_sphere(400)):
+        t = configs.rotation_z_to(-d)
+        t[3, :3] = 5500.0 * d
+        fd.addInstance(t, kinds[i % 2])
+    phys = lib.arrays()
+    phys["icdf"], phys["icdf_hd_factor"] = gaussian_icdf()
+    gs = configs.frame_gensteps((0, 0, 0, 6000.0), (-50, 49, 0, 0, -20, 20, 1000, 1), gridscale=0.02)
+    gs[:, 5, 1] = 3000.0                                       # off the middle: more of them leave the ball
+    sim = QSim(fd.arrays(), phys, SEventConfig(seed=3))
+    out = sim.simtrace_device(torch.from_numpy(gs).to(DEV)).cpu().numpy().view(np.uint32)
+    ref = po.World(fd.arrays(), phys).simtrace(gs, seed=3).view(np.uint32)
+    assert np.array_equal(out, ref)
+    instances = out[:, 3, 3] >> 16
+    assert np.count_nonzero((instances > 0) & (instances != 0xffff)) > 50_000
+    sim.close()
