@@ -147,6 +147,81 @@ __global__ void __launch_bounds__(256) k_radix_scatter(const Key* __restrict__ k
     }
 }
 
+/*
+ * All passes over at most TILE pairs in one block's LDS, with k_radix_scatter's ranks: from (keys,
+ * vals) to (keys_out, vals_out), which may be the same. Bound by its latency (3.8 us for 200 pairs of
+ * 11-bit keys, 9.3 where one wave ranks all of them), which the launches of three kernels a pass exceed:
+ * with them the taped adjoint of 200 hits took 134 us, so 115; the merge of 1,000 hits in windows of
+ * 0.01 ns 107 and 65, of 2,000 128 and 79. One tile is the most that fits the kernel's LDS (52 KB).
+ */
+template <class Key>
+__global__ void __launch_bounds__(256) k_radix_small(const Key* keys, const uint32_t* vals, int32_t n, int np, int d,
+                                                     Key* keys_out, uint32_t* vals_out)
+{
+    __shared__ Key s_key[2][TILE];
+    __shared__ uint32_t s_val[2][TILE];
+    __shared__ uint32_t s_count[4][1 << MOST_BITS];
+    __shared__ uint32_t s_sum[4];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int rounds = (n + 255) / 256, first = wave * rounds * 64 + lane;     /* a quarter to each wave */
+    for (int i = t; i < n; i += 256) { s_key[0][i] = keys[i]; s_val[0][i] = vals[i]; }
+    for (int p = 0; p < np; ++p) {
+        const Key* ks = s_key[p & 1];
+        const uint32_t* vs = s_val[p & 1];
+        for (int b = t; b < 4 << MOST_BITS; b += 256) (&s_count[0][0])[b] = 0u;
+        __syncthreads();
+        volatile uint32_t* mine = s_count[wave];
+        const int shift = p * d;
+        uint32_t rank[ROUNDS];
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) {
+            if (r >= rounds) break;
+            const int i = first + r * 64;
+            const bool valid = i < n;
+            const uint32_t g = valid ? digit_of(ks[i], shift, d) : 0u;
+            unsigned long long same = __ballot(valid);
+            for (int b = 0; b < d; ++b) {
+                const bool bit = (g >> b & 1u) != 0u;
+                const unsigned long long m = __ballot(bit);
+                same &= bit ? m : ~m;
+            }
+            const uint32_t below = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+            const uint32_t so_far = mine[g];
+            __builtin_amdgcn_wave_barrier();
+            if (valid && below == 0u) mine[g] = so_far + (uint32_t)__popcll(same);
+            __builtin_amdgcn_wave_barrier();
+            rank[r] = so_far + below;
+        }
+        __syncthreads();
+        /* where each digit of each wave starts, a digit to a thread */
+        uint32_t c[4], all = 0u;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) { c[w] = s_count[w][t]; all += c[w]; }
+        uint32_t incl = all;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t x = (uint32_t)__shfl_up((int)incl, o);
+            if (lane >= o) incl += x;
+        }
+        if (lane == 63) s_sum[wave] = incl;
+        __syncthreads();
+        uint32_t at = incl - all;
+        for (int w = 0; w < wave; ++w) at += s_sum[w];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) { s_count[w][t] = at; at += c[w]; }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) {
+            const int i = first + r * 64;
+            if (r >= rounds || i >= n) break;
+            const uint32_t q = mine[digit_of(ks[i], shift, d)] + rank[r];
+            s_key[~p & 1][q] = ks[i];
+            s_val[~p & 1][q] = vs[i];
+        }
+        __syncthreads();
+    }
+    for (int i = t; i < n; i += 256) { keys_out[i] = s_key[np & 1][i]; vals_out[i] = s_val[np & 1][i]; }
+}
+
 /* Sorts by the low `bits` bits of the keys, back and forth between (k0, v0) and (k1, v1): it
    starts in (k0, v0) and ends in (k1, v1) after an odd number of passes, in (k0, v0) after an
    even one. n <= 2^31 - 1, tmp: words(n, bits). */
@@ -154,6 +229,11 @@ template <class Key>
 hipError_t sort(Key* k0, Key* k1, uint32_t* v0, uint32_t* v1, int64_t n, int bits, uint32_t* tmp, hipStream_t s)
 {
     const int np = passes(bits), d = digit_bits(bits);
+    if (n <= TILE) {
+        hipLaunchKernelGGL(k_radix_small<Key>, dim3(1), dim3(256), 0, s, k0, v0, (int32_t)n, np, d, np % 2 ? k1 : k0,
+                           np % 2 ? v1 : v0);
+        return hipGetLastError();
+    }
     const uint32_t nt = (uint32_t)tiles(n), bins = 1u << d;
     uint32_t* total = tmp + ((size_t)nt << d);
     for (int p = 0; p < np; ++p) {

@@ -277,3 +277,20 @@ def test_merge_of_all_records(sim_and_photons, n, lite_only):
     ref[:, 1, 3], ref[:, 3, 3] = want[:, 0] & 0xffff0000, want[:, 3]
     got = sim.merge_hits_device(torch.from_numpy(P.view(np.float32)).to(DEV), L.MI_MERGE_ALREADY_SELECTED, 4.0)
     assert np.array_equal(got.cpu().numpy().view(np.uint32), ref)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 511, 513, 1793, 2047, 2048, 2049])
+def test_merge_of_few_records_keeps_their_order(sim_and_photons, n):
+    """Numbers of pairs around a wave, a round of four waves and a tile of the sort; keys of one to
+    six bytes. The index of a run's first record and its flags show the order of equal keys."""
+    sim, _ = sim_and_photons
+    rng = np.random.default_rng(n)
+    for n_id, n_bucket in ((1, 1), (3, 2), (300, 1), (3000, 40), (3, 3_000_000), (65535, 60_000_000)):
+        lt = np.empty((n, 4), np.uint32)
+        lt[:, 0] = (rng.integers(1, 5, n) << 16) | rng.integers(max(1, n_id - 7), n_id + 1, n)
+        lt[:, 1] = (rng.integers(max(0, n_bucket - 5), n_bucket, n) * np.float32(1.0)).astype(np.float32).view(np.uint32)
+        lt[:, 2] = np.arange(n)
+        lt[:, 3] = 1 << rng.integers(0, 16, n)
+        ref = spm.merge_lites(lt, L.MI_MERGE_ALREADY_SELECTED, 1.0)
+        out = sim.merge_hits_device(torch.from_numpy(lt.view(np.int32)).to(DEV), L.MI_MERGE_ALREADY_SELECTED, 1.0)
+        assert np.array_equal(out.cpu().numpy().view(np.uint32), ref), (n_id, n_bucket)
