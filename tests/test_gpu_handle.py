@@ -81,7 +81,7 @@ def best_time(f, n=40):
 
 
 def test_small_events_after_a_large_one():
-    """After an event of 400M photons, events of a few photons have the checker's results, and do
+    """After an event of 400M photons, events of a few photons have the oracle's results, and do
     not pay for what that one needed."""
     w = configs.config0(num_photon=1000)
     ref = {}
@@ -128,7 +128,7 @@ def test_grids_beyond_residency_keep_results(n, waves_per_cu):
 @pytest.mark.parametrize("num_det, n", [(2000, 30_000), (20_000, 30_000), (20_000, 900_000)])
 def test_lite_output_of_deep_detectors(num_det, n):
     """Lite records of detectors whose traversal stack leaves a CU fewer blocks with lite output
-    than without: time and flags of the photon records, the checker's among them."""
+    than without: time and flags of the photon records, the oracle's among them."""
     w = configs.detector_shell(num_det=num_det, num_gs=6, per_gs=n // 6)
     ev = Device(w.gensteps)
     sim = QSim(w.geometry, w.physics, SEventConfig(seed=w.seed))
@@ -254,7 +254,7 @@ def test_hit_counts_of_busy_detectors(n):
 
 @pytest.mark.parametrize("half, walk", [(2000.0, False), (9000.0, True)])
 def test_simtrace_around_the_persistent_kernel(half, walk):
-    """Grids of 4M rays that the front instances settle, and that walk: the checker's records, and
+    """Grids of 4M rays that the front instances settle, and that walk: the oracle's records, and
     no step in the time where the choice of a kernel begins (the settled: 1.6 times where it went
     by the number alone)."""
     w = configs.config1(num_gs=1, per_gs=10)
